@@ -16,57 +16,76 @@
 
 namespace k2t {
 
+// One wave's chunk c of a row: sign flip with the chunk's mask, butterflies and int8.
+__device__ __forceinline__ void quant_chunk(float v, int c, size_t gc, uint32_t lane, const uint64_t *signs,
+                                            int8_t *q, float *scales, int32_t *sums) {
+    // (the context's table holds the masks of the first kSignBlocks chunks)
+    const uint32_t neg = c < kSignBlocks ? (uint32_t)(signs[c] >> lane) & 1u : hadamard_sign_bit((uint64_t)c, lane);
+    v = wave_butterflies64(flip_sign(v, neg) * 0.125f, lane);
+    quant_chunk_store(v, lane, q + gc * 64, scales + gc, sums + gc);
+}
+
 __global__ __launch_bounds__(256) void act_quant_kernel(const float *__restrict__ x,
                                                         const float *__restrict__ w,
                                                         const float *__restrict__ inv_rms, int K,
-                                                        int total_chunks, int8_t *__restrict__ q,
-                                                        float *__restrict__ scales,
+                                                        int total_chunks, const uint64_t *__restrict__ signs,
+                                                        int8_t *__restrict__ q, float *__restrict__ scales,
                                                         int32_t *__restrict__ sums) {
     const uint32_t lane = threadIdx.x & 63;
-    const int gc = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+    const int gc = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     if (gc >= total_chunks) return;
     const int nc = K / 64;
     const int tok = gc / nc, c = gc - tok * nc;
     float v = x[(size_t)gc * 64 + lane];
     if (w) v = (v * inv_rms[tok]) * w[(size_t)c * 64 + lane];
-    v = flip_sign(v, hadamard_sign_bit((uint64_t)c, lane)) * 0.125f;
-    v = wave_butterflies64(v, lane);
-    const float mx = wave_max_f(fabsf(v));
-    if (mx <= FLT_EPSILON) {
-        q[(size_t)gc * 64 + lane] = 0;
-        if (lane == 0) {
-            scales[gc] = 0.0f;
-            sums[gc] = 0;
-        }
-        return;
-    }
-    const float inv = 127.0f / mx;
-    const int qi = (int)rintf(v * inv);
-    const int s = wave_sum_i(qi);
-    q[(size_t)gc * 64 + lane] = (int8_t)qi;
-    if (lane == 0) {
-        scales[gc] = mx / 127.0f;
-        sums[gc] = s;
-    }
+    quant_chunk(v, c, (size_t)gc, lane, signs, q, scales, sums);
 }
 
-// inv_rms[t] = 1 / sqrt(sum(x^2)/K + eps) per token (real_llm.rs:6929), one block per token.
-__global__ __launch_bounds__(256) void inv_rms_kernel(const float *__restrict__ x, float eps, int K,
-                                                      float *__restrict__ out) {
+// RMSNorm + FWHT + int8 in one launch: inv_rms = 1 / sqrt(sum(x^2)/K + eps) (real_llm.rs:6929)
+// is computed by every workgroup of a row (thread t adds elements t, t + 256, ... in that
+// order, eight loads in flight, then the four waves' sums pairwise), then its waves take
+// the workgroup's share of the row's chunks.  The row is a few KB and stays in L2, so
+// reading it once per workgroup costs less than a second launch does: one token x 4096,
+// 4.1 + 2.9 us as two kernels; with the 14336 x 4096 NF4 GEMV behind it a pass went from 14.0 to 11.5 us.
+// The host picks the workgroups per row (launch_rmsnorm_quant).
+__global__ __launch_bounds__(256) void rmsnorm_quant_kernel(const float *__restrict__ x, const float *__restrict__ w,
+                                                            float eps, int K, const uint64_t *__restrict__ signs,
+                                                            int8_t *__restrict__ q, float *__restrict__ scales,
+                                                            int32_t *__restrict__ sums) {
     __shared__ float part[4];
-    const float *xt = x + (size_t)blockIdx.x * K;
+    const uint32_t lane = threadIdx.x & 63u;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nc = K / 64, tok = (int)blockIdx.y, step = 4 * (int)gridDim.x;
+    const float *xt = x + (size_t)tok * K;
+    // the first chunk's operands go out with the row's loads
+    const int c0 = (int)blockIdx.x * 4 + wave, cl = min(c0, nc - 1);
+    const float x0 = xt[cl * 64 + lane], w0 = w[cl * 64 + lane];
     float s = 0.0f;
-    for (int i = threadIdx.x; i < K; i += 256) {
-        const float v = xt[i];
-        s = fmaf(v, v, s);
+    int i = (int)threadIdx.x;
+    for (; i + 7 * 256 < K; i += 8 * 256) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = xt[i + u * 256];
+#pragma unroll
+        for (int u = 0; u < 8; u++) s = fmaf(v[u], v[u], s);
+    }
+    {
+        float v[7];  // the rest: clamped loads, masked below (all in flight together)
+#pragma unroll
+        for (int u = 0; u < 7; u++) v[u] = xt[min(i + u * 256, K - 1)];
+#pragma unroll
+        for (int u = 0; u < 7; u++) s = i + u * 256 < K ? fmaf(v[u], v[u], s) : s;
     }
     s = wave_sum_f(s);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+    if (lane == 0) part[wave] = s;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const float tot = (part[0] + part[1]) + (part[2] + part[3]);
-        out[blockIdx.x] = 1.0f / sqrtf(tot / (float)K + eps);
-    }
+    const float tot = (part[0] + part[1]) + (part[2] + part[3]);
+    const float inv_rms = 1.0f / sqrtf(tot / (float)K + eps);
+    if (c0 >= nc) return;
+    quant_chunk((x0 * inv_rms) * w0, c0, (size_t)tok * nc + c0, lane, signs, q, scales, sums);
+    for (int c = c0 + step; c < nc; c += step)
+        quant_chunk((xt[c * 64 + lane] * inv_rms) * w[c * 64 + lane], c, (size_t)tok * nc + c, lane, signs, q, scales,
+                    sums);
 }
 
 // inv_rms[t] = 1 / sqrt(sum(x^2)/K + eps) with the sum of squares in the reference's x86
@@ -126,14 +145,24 @@ void launch_act_quant(k2t_ctx *ctx, const float *x, const float *w, const float 
     const int total = (K / 64) * ntok;
     if (total <= 0) return;
     hipLaunchKernelGGL(act_quant_kernel, dim3((total + 3) / 4), dim3(256), 0, ctx->stream, x, w,
-                       inv_rms, K, total, q, scales, sums);
+                       inv_rms, K, total, ctx->signs, q, scales, sums);
     hip_check(hipGetLastError(), "act_quant launch");
 }
 
-void launch_inv_rms(k2t_ctx *ctx, const float *x, float eps, int K, int ntok, float *inv_rms) {
+void launch_rmsnorm_quant(k2t_ctx *ctx, const float *x, const float *w, float eps, int K, int ntok, int8_t *q,
+                          float *scales, int32_t *sums) {
     if (ntok <= 0) return;
-    hipLaunchKernelGGL(inv_rms_kernel, dim3(ntok), dim3(256), 0, ctx->stream, x, eps, K, inv_rms);
-    hip_check(hipGetLastError(), "inv_rms launch");
+    // Workgroups per row: four chunks each while the launch is small (latency), fewer where
+    // the tokens alone fill the chip, since every workgroup reads its whole row.
+    const int per_row = (K / 64 + 3) / 4, want = std::max(1, 4 * ctx->num_cus / ntok);
+    const int gx = std::min(per_row, want);
+    for (int t0 = 0; t0 < ntok; t0 += 65535) {  // (the grid's y extent)
+        const int n = std::min(65535, ntok - t0);
+        const size_t row = (size_t)t0 * K, ch = (size_t)t0 * (K / 64);
+        hipLaunchKernelGGL(rmsnorm_quant_kernel, dim3(gx, n), dim3(256), 0, ctx->stream, x + row, w, eps, K, ctx->signs,
+                           q + row, scales + ch, sums + ch);
+    }
+    hip_check(hipGetLastError(), "rmsnorm_quant launch");
 }
 
 // Streaming read of `bytes` (measurement of the single-launch HBM read ceiling that the

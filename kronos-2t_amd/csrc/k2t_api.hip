@@ -254,7 +254,6 @@ void k2t_ctx_destroy(k2t_ctx *ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->scratch) (void)hipFree(ctx->scratch);
-    if (ctx->rms_scratch) (void)hipFree(ctx->rms_scratch);
     if (ctx->gqa_words) (void)hipFree(ctx->gqa_words);
     if (ctx->signs) (void)hipFree(ctx->signs);
     delete ctx;
@@ -420,16 +419,7 @@ int32_t k2t_act_quant_rmsnorm(k2t_ctx *ctx, const float *d_x, const float *d_nor
         arg_check(ntok == 0 || (d_x && d_norm_w && d_q && d_scales && d_sums), "NULL buffer");
         if (ntok == 0) return;
         hip_check(hipSetDevice(ctx->device), "hipSetDevice");
-        if ((size_t)ntok > ctx->rms_cap) {
-            hip_check(hipStreamSynchronize(ctx->stream), "scratch sync");
-            if (ctx->rms_scratch) hip_check(hipFree(ctx->rms_scratch), "hipFree");
-            ctx->rms_scratch = nullptr;
-            size_t cap = std::max((size_t)ntok, (size_t)1024);
-            device_alloc((void **)&ctx->rms_scratch, cap * sizeof(float));
-            ctx->rms_cap = cap;
-        }
-        launch_inv_rms(ctx, d_x, eps, K, ntok, ctx->rms_scratch);
-        launch_act_quant(ctx, d_x, d_norm_w, ctx->rms_scratch, K, ntok, d_q, d_scales, d_sums);
+        launch_rmsnorm_quant(ctx, d_x, d_norm_w, eps, K, ntok, d_q, d_scales, d_sums);
     });
 }
 

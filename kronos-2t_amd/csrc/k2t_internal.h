@@ -19,8 +19,6 @@ struct k2t_ctx {
     // small device scratch (debug entry points): grown on demand
     float *scratch = nullptr;
     size_t scratch_cap = 0;  // floats
-    float *rms_scratch = nullptr;
-    size_t rms_cap = 0;
     // grouped-query attention span words of k2t_attn_decode ({payload, epoch}, zeroed when
     // allocated), then its counters {epoch, merges done} and timeout word
     unsigned long long *gqa_words = nullptr;
@@ -203,7 +201,9 @@ void model_adopt(k2t_model *m, k2t_mat *mat);
 
 void launch_act_quant(k2t_ctx *ctx, const float *x, const float *w, const float *inv_rms, int K,
                       int ntok, int8_t *q, float *scales, int32_t *sums);
-void launch_inv_rms(k2t_ctx *ctx, const float *x, float eps, int K, int ntok, float *inv_rms);
+// RMSNorm (inv_rms computed in the launch) + FWHT + int8.
+void launch_rmsnorm_quant(k2t_ctx *ctx, const float *x, const float *w, float eps, int K, int ntok, int8_t *q,
+                          float *scales, int32_t *sums);
 void launch_expf_map(hipStream_t st, const float *x, float *y, size_t n);
 // inv_rms per token with the x86 reference's sum-of-squares order (exact-order mode).
 void launch_inv_rms_x86(hipStream_t st, const float *x, float eps, int K, int ntok, float *inv_rms);
