@@ -80,7 +80,7 @@ int32_t k2t_ctx_set_splitk(k2t_ctx *ctx, int32_t max_segments);
  * within a few ulp of the reference, and faster for long K.  Integer per-(row, chunk)
  * dots are exact in both modes. */
 int32_t k2t_ctx_set_exact(k2t_ctx *ctx, int32_t exact);
-/* Batched NF4 and bit-plane (b4 / b5 / b6) GEMVs (16 or more tokens of a ready activation
+/* Batched NF4, NF3 and bit-plane (b4 / b5 / b6) GEMVs (16 or more tokens of a ready activation
  * over the whole matrix, k2t_gemv and the model's prefill): enable = 1 (default) runs
  * them on the int8 matrix cores, one weight pass per 64 tokens, with outputs equal to the
  * exact-order epilogue's in either mode; 0 runs the 4-token weight passes of the
@@ -165,7 +165,8 @@ int32_t k2t_act_quant_rmsnorm(k2t_ctx *ctx, const float *d_x, const float *d_nor
  * Weights are read once per 4 tokens.  d_xsum is required for bit-plane
  * matrices and ignored for NF ones.  Per-(row, chunk) integer dots are exact;
  * with split-K disabled the fp32 result is bit-identical to the reference's
- * in-order fmaf epilogue.  16 or more tokens over the whole matrix (NF4 or bit
+ * in-order fmaf epilogue.  16 or more tokens over the whole matrix (NF with scale
+ * groups of a power of two, or bit
  * planes, k2t_ctx_set_mfma): one weight pass per 64 tokens on the matrix
  * cores, outputs bit-identical to that epilogue in either mode; such a call
  * copies the activation into the context's scratch, which it grows first if it

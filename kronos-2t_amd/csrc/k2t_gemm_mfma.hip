@@ -1,7 +1,7 @@
 // Batched quantized GEMV (prefill) on the int8 matrix cores of gfx950: out[t][r] =
 // sum_c fmaf(float(dot_{r,c,t}) * sx[t][c], ws[r][c], ...) for up to 64 tokens per weight
-// pass, the chunk dots from v_mfma_i32_16x16x64_i8.  NF4 (NfSdotMatrix) and the bit-plane
-// formats b4 / b5 / b6 (Nibble4SdotMatrix) share the kernel.
+// pass, the chunk dots from v_mfma_i32_16x16x64_i8.  NF4 and NF3 (NfSdotMatrix) and the bit-plane
+// formats b4 / b5 / b6 (Nibble4SdotMatrix) share the kernel (FMT 1, 2, 0).
 //
 // The reference runs prefill through the same kernels as decode, four tokens per weight
 // pass (nf_sdot_decode_neon's 4-token tile, simd_lut.rs:6074-6364, and the Nibble4 tile
@@ -11,6 +11,9 @@
 // is read once per 64 tokens instead of once per 4.
 //  - NF4: the codebook value of each code (the codebook as two v_perm XOR tables,
 //    nf4_xlut); the MFMA gives the chunk dot.
+//  - NF3: the same through one v_perm per four codes, from the row's triplet of dwords, in
+//    the device's lane order or the reference's.  200 tokens x 5000 x 2112: 137.8 us as 4-token
+//    passes, 20 us here.
 //  - bit planes: the unsigned code u (4 + hp bits: the nibble and the hi-plane bits); the
 //    MFMA gives sum(u * x), and the chunk dot of the odd weights 2u - (2^(4+hp) - 1) is
 //    2 * sum(u * x) - (2^(4+hp) - 1) * sum(x), as the reference computes it (simd_lut.rs:
@@ -72,7 +75,8 @@ struct MfArgs {
     const uint8_t *pair, *tail;
     size_t ptot;  // bytes per pair stream
     int rows, nc, np, stripes, sgc_log2;  // NF scale group = 1 << sgc_log2 chunks
-    uint32_t t0, t1, u0, u1;  // NF4 codebook XOR tables (nf4_xor_tables)
+    uint32_t t0, t1, u0, u1;  // NF4 codebook XOR tables (nf4_xor_tables); NF3: t0, t1 the codebook
+    int lane;                 // NF3: stripe-chunks in lane order
     const int8_t *xt;  // activations tile-major: [16-token block][chunk][64 lanes][16 bytes]
     const float *st;   // their scales: [16-token block][chunk][16 tokens]
     const int32_t *ut;  // their code sums (bit planes): [16-token block][chunk][16 tokens]
@@ -95,7 +99,7 @@ struct MfArgs {
 template <int FMT, int NB, bool SH>
 struct MfChunk {
     uint32_t d0, d1;
-    uint32_t hv;  // bit planes with hi planes: this lane's hi-plane dword
+    uint32_t hv;  // bit planes with hi planes: this lane's hi-plane dword; NF3: its third dword
     uint2 sw;
     int4 x[SH ? (NB + 3) / 4 : NB];  // with sharing: blocks wave, wave + 4
     float sx[NB];
@@ -113,8 +117,8 @@ struct MfSrc {
 
 // Per-lane offsets of a stripe-chunk record, fixed for the wave's life.
 struct MfLane {
-    uint32_t a_off;  // the lane's first nibble dword (the second is 16 bytes further)
-    uint32_t h_off;  // its hi-plane dword (bit planes)
+    uint32_t a_off, b_off;  // the lane's first and second code dword
+    uint32_t h_off;  // its hi-plane dword (bit planes), its third code dword (NF3)
     uint32_t s_off;  // its rows' BF16 scale pair
     uint32_t x_off, sx_off;
 };
@@ -135,13 +139,14 @@ __device__ __forceinline__ void mf_fetch(const MfArgs &A, const MfSrc &R, const 
         sgb = rec;
     } else {
         const uint32_t sg = (uint32_t)c >> A.sgc_log2, sb = (uint32_t)c - (sg << A.sgc_log2);
-        const uint32_t cs = is_tail ? 512u : 1024u, gsz = is_tail ? 32u : 64u;
+        constexpr uint32_t CB = FMT == 2 ? 384u : 512u;  // bytes per stripe-chunk
+        const uint32_t cs = is_tail ? CB : 2u * CB, gsz = is_tail ? 32u : 64u;
         sgb = sg * gsz + (sg << A.sgc_log2) * cs;  // scale-group base
         rec = sgb + gsz + sb * cs;
     }
     f.d0 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(R.w, L.a_off, rec, 0);
-    f.d1 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(R.w, L.a_off + 16u, rec, 0);
-    if constexpr (FMT == 0 && HP > 0) f.hv = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(R.w, L.h_off, rec, 0);
+    f.d1 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(R.w, L.b_off, rec, 0);
+    if constexpr ((FMT == 0 && HP > 0) || FMT == 2) f.hv = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(R.w, L.h_off, rec, 0);
     const v2u sw = __builtin_amdgcn_raw_buffer_load_b64(R.w, L.s_off, sgb, 0);
     f.sw = make_uint2(sw[0], sw[1]);
     if constexpr (SH) {
@@ -210,6 +215,21 @@ __device__ __forceinline__ void mf_step(const MfArgs &A, const MfChunk<FMT, NB, 
         a[1] = (int)hi0;
         a[2] = (int)lo1;
         a[3] = (int)hi1;
+    } else if constexpr (FMT == 2) {
+        // NF3 triplet (v0, v1, v2) of this row and 32-column half: codes 0-3 (even lane
+        // group) or 4-7 (odd) are this lane's four column quads; code 2 / 5 has its third
+        // bit in v2.  v0 = i0 | i1 << 3 | i2 << 6, v1 = i3 | i4 << 3 | i5 << 6, v2 = i6 | i7 << 3
+        // | third bits of i2, i5.  One v_perm looks four codes up in the 8-entry codebook.
+        const bool odd = (lane & 16u) != 0u;
+        const uint32_t p = odd ? f.d1 : f.d0, r = odd ? f.hv : f.d1;
+        const uint32_t e = (odd ? f.hv >> 3 : f.d0) & 0x07070707u;              // i0 / i7
+        const uint32_t n = (p >> 3) & 0x07070707u;                              // i1 / i4
+        const uint32_t m = ((p >> 6) & 0x03030303u) | ((f.hv >> (odd ? 5 : 4)) & 0x04040404u);  // i2 / i5
+        const uint32_t l = r & 0x07070707u;                                     // i3 / i6
+        a[0] = (int)__builtin_amdgcn_perm(A.t1, A.t0, odd ? n : e);
+        a[1] = (int)__builtin_amdgcn_perm(A.t1, A.t0, odd ? m : n);
+        a[2] = (int)__builtin_amdgcn_perm(A.t1, A.t0, odd ? l : m);
+        a[3] = (int)__builtin_amdgcn_perm(A.t1, A.t0, odd ? e : l);
     } else {
         a[0] = (int)nf4_xlut(f.d0 & 0x0F0F0F0Fu, A.t0, A.t1, A.u0, A.u1);
         a[1] = (int)nf4_xlut((f.d0 >> 4) & 0x0F0F0F0Fu, A.t0, A.t1, A.u0, A.u1);
@@ -278,12 +298,23 @@ __global__ __launch_bounds__(SW ? 512 : 256) void gemm_mfma_kernel(MfArgs A) {
     const uint8_t *mbase = is_tail ? A.tail : A.pair + (size_t)(stripe >> 1) * A.ptot;
     const uint32_t li = lane & 15u, lg = lane >> 4;
     MfLane L;
-    L.a_off = (is_tail ? 0u : side * 512u) + lg * 128u + (li >> 2) * 32u + 4u * (li & 3u);
+    if constexpr (FMT == 2) {
+        // block (g, half): 16-byte pieces 128 bytes apart in lane order, 16 in the reference's
+        const uint32_t g = li >> 2, half = lg >> 1, ps = A.lane ? 128u : 16u;
+        L.a_off = (is_tail ? 0u : side * 384u) + (A.lane ? (2u * g + half) * 16u : half * 192u + g * 48u) +
+                  4u * (li & 3u);
+        L.b_off = L.a_off + ps;
+        L.h_off = L.a_off + 2u * ps;
+        L.s_off = (is_tail ? 0u : side * 32u) + 8u * lg;
+    } else {
+        L.a_off = (is_tail ? 0u : side * 512u) + lg * 128u + (li >> 2) * 32u + 4u * (li & 3u);
+        L.b_off = L.a_off + 16u;
+    }
     if constexpr (FMT == 0) {
         const uint32_t hib = is_tail ? 512u : 1024u + side * 128u * HP;  // the stripe's hi bytes
         L.h_off = hib + (HP == 2 ? lg : lg >> 1) * 64u + (li >> 2) * 16u + 4u * (li & 3u);
         L.s_off = (is_tail ? 512u + 128u * HP : 1024u + 256u * HP + side * 32u) + 8u * lg;  // rows 4lg .. 4lg+3
-    } else {
+    } else if constexpr (FMT == 1) {
         L.h_off = 0;
         L.s_off = (is_tail ? 0u : side * 32u) + 8u * lg;
     }
@@ -434,7 +465,7 @@ __global__ __launch_bounds__(256) void mf_tile_kernel(const int8_t *xq, const fl
 
 bool gemm_mfma_supported(const k2t_mat *m, int ntok) {
     if (ntok < kMfmaMinTokens || m->cols % 64 != 0) return false;
-    if (m->fmt == K2T_FMT_NF) return m->bits == 4 && (m->sgc & (m->sgc - 1)) == 0;
+    if (m->fmt == K2T_FMT_NF) return (m->bits == 3 || m->bits == 4) && (m->sgc & (m->sgc - 1)) == 0;
     return m->fmt == K2T_FMT_NIBBLE4 && m->hp >= 0 && m->hp <= 2;
 }
 
@@ -467,7 +498,11 @@ static int mfma_args(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const flo
     A.np = m->pairs;
     A.stripes = m->stripes;
     A.sgc_log2 = planes ? 0 : __builtin_ctz((unsigned)m->sgc);
-    if (!planes) nf4_xor_tables(m->cb[0], m->cb[1], m->cb[2], m->cb[3], A.t0, A.t1, A.u0, A.u1);
+    A.lane = m->nf3_lane;
+    if (!planes && m->bits == 3) {
+        A.t0 = m->cb[0];
+        A.t1 = m->cb[1];
+    } else if (!planes) nf4_xor_tables(m->cb[0], m->cb[1], m->cb[2], m->cb[3], A.t0, A.t1, A.u0, A.u1);
     const int blocks = (ntok + 15) / 16;
     int8_t *xt = tiles.xt;
     float *stile = tiles.st;
@@ -505,7 +540,8 @@ void launch_gemm_mfma(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const fl
     A.accum = accum ? 1 : 0;
     const dim3 grid((m->stripes + 3) / 4, (ntok + 16 * nb - 1) / (16 * nb));
     hipStream_t st = ctx->stream;
-    if (m->fmt == K2T_FMT_NF) launch_gemm_mfma_fmt<1, 0>(st, nb, grid, A);
+    if (m->fmt == K2T_FMT_NF && m->bits == 3) launch_gemm_mfma_fmt<2, 0>(st, nb, grid, A);
+    else if (m->fmt == K2T_FMT_NF) launch_gemm_mfma_fmt<1, 0>(st, nb, grid, A);
     else if (m->hp == 0) launch_gemm_mfma_fmt<0, 0>(st, nb, grid, A);
     else if (m->hp == 1) launch_gemm_mfma_fmt<0, 1>(st, nb, grid, A);
     else launch_gemm_mfma_fmt<0, 2>(st, nb, grid, A);
@@ -534,7 +570,8 @@ bool launch_gemm_mfma_qkv(k2t_ctx *ctx, const k2t_mat *qkv, ActTiles tiles, int 
     A.qp = qp;
     const dim3 grid(qkv->rows / 64, (ntok + 16 * nb - 1) / (16 * nb));
     hipStream_t st = ctx->stream;
-    if (qkv->fmt == K2T_FMT_NF) launch_qkv_fmt<1, 0>(st, nb, grid, A);
+    if (qkv->fmt == K2T_FMT_NF && qkv->bits == 3) launch_qkv_fmt<2, 0>(st, nb, grid, A);
+    else if (qkv->fmt == K2T_FMT_NF) launch_qkv_fmt<1, 0>(st, nb, grid, A);
     else if (qkv->hp == 0) launch_qkv_fmt<0, 0>(st, nb, grid, A);
     else if (qkv->hp == 1) launch_qkv_fmt<0, 1>(st, nb, grid, A);
     else launch_qkv_fmt<0, 2>(st, nb, grid, A);
@@ -563,7 +600,8 @@ bool launch_gemm_mfma_swiglu(k2t_ctx *ctx, const k2t_mat *gu, ActTiles tiles, in
     A.nci = gu->rows / 128;
     const dim3 grid(gu->rows / 128, (ntok + 63) / 64);
     hipStream_t st = ctx->stream;
-    if (gu->fmt == K2T_FMT_NF) launch_swiglu_fmt<1, 0>(st, grid, A);
+    if (gu->fmt == K2T_FMT_NF && gu->bits == 3) launch_swiglu_fmt<2, 0>(st, grid, A);
+    else if (gu->fmt == K2T_FMT_NF) launch_swiglu_fmt<1, 0>(st, grid, A);
     else if (gu->hp == 0) launch_swiglu_fmt<0, 0>(st, grid, A);
     else if (gu->hp == 1) launch_swiglu_fmt<0, 1>(st, grid, A);
     else launch_swiglu_fmt<0, 2>(st, grid, A);

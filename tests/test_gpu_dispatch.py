@@ -58,3 +58,46 @@ def test_rmsnorm_quant_equals_split_form(gpu_ctx, K, ntok):
         assert np.array_equal(a.cpu().numpy(), b.cpu().numpy())
     if ntok > 1:
         assert not got[0][1].any() and not got[1][1].any()
+
+
+def _gemv(ctx, m, xq, xs, xsum, rows, exact=False):
+    import torch
+    ntok = xq.shape[0]
+    out = torch.full((ntok, rows), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.set_exact(exact)
+    try:
+        ctx.gemv(m, _t(xq), _t(xs), _t(xsum), out, ntok=ntok, out_stride=rows)
+        ctx.sync()
+    finally:
+        ctx.set_exact(False)
+    return out.cpu().numpy()
+
+
+# one and several 16-token blocks per wave, partial blocks, a tail stripe, rows past the end of
+# the last stripe, scale groups of one, two and four chunks with a ragged last group
+@pytest.mark.parametrize("rows,cols,sgc,ntok", [(16, 64, 1, 16), (48, 320, 2, 17), (1030, 2048, 2, 64),
+                                                (2048, 576, 4, 200), (5000, 192, 2, 130)])
+@pytest.mark.parametrize("lane", [True, False])
+def test_mfma_nf3_equals_reference_chain(gpu_ctx, rows, cols, sgc, ntok, lane):
+    """NF3 batches of 16 or more tokens, stripe-chunks in lane order and in the reference's:
+    every output bit-identical to the oracle's per-token chain in chunk order, both modes."""
+    import oracle as O
+    from helpers import acts, random_nf_streams
+    rng = np.random.default_rng(rows + cols + ntok)
+    idx, sc, pair, tail = random_nf_streams(rng, rows, cols, sgc, bits=3)
+    cb = np.array([-127, -79, -45, -14, 14, 45, 79, 127] + 8 * [0], np.int8)
+    dp, dt = _t(pair if pair.size else np.zeros(16, np.uint8)), _t(tail if tail.size else np.zeros(16, np.uint8))
+    m = gpu_ctx.wrap_nf(rows, cols, 3, sgc, cb, dp, pair.size, dt if tail.size else None, tail.size)
+    if lane:
+        m.nf3_lane_order()
+    base = [acts(rng, cols, 20, outlier_frac=0.001, outlier_scale=30.0)]
+    xq, xs, xsum = (np.concatenate([a] * -(-ntok // 20))[:ntok] for a in base[0])
+    xs[3, 0] = 0.0
+    xq[3, :64] = 0
+    ref = np.stack([O.nf_gemv(pair, tail, rows, cols, 3, sgc, cb, xq[t], xs[t]) for t in range(min(ntok, 24))])
+    for exact in (False, True):
+        out = _gemv(gpu_ctx, m, xq, xs, xsum, rows, exact)
+        assert np.array_equal(out[:ref.shape[0]].view(np.uint32), ref.view(np.uint32))
+        assert np.array_equal(out[24:].view(np.uint32), out[4:][np.arange(ntok - 24) % 20].view(np.uint32)) \
+            if ntok > 24 else True
+    m.close()
