@@ -123,6 +123,86 @@ struct MfLane {
     uint32_t x_off, sx_off;
 };
 
+// A lane's 16 bytes of the A operand: the int8 values (NF: codebook entries; bit planes: the
+// unsigned codes) of its row's columns 16 (lane / 16) .. + 15, from its code dwords.
+template <int FMT, int HP>
+__device__ __forceinline__ v4i mf_decode(uint32_t d0, uint32_t d1, uint32_t hv, uint32_t t0, uint32_t t1, uint32_t u0,
+                                         uint32_t u1, uint32_t lane) {
+    v4i a;
+    if constexpr (FMT == 0) {
+        // the unsigned codes: nibble, then the hi-plane bits (as chunk_dots places them for
+        // kk = lane group, half 0 for the first dword and half 1 for the second)
+        uint32_t lo0 = d0 & 0x0F0F0F0Fu, hi0 = (d0 >> 4) & 0x0F0F0F0Fu;
+        uint32_t lo1 = d1 & 0x0F0F0F0Fu, hi1 = (d1 >> 4) & 0x0F0F0F0Fu;
+        if constexpr (HP == 2) {
+            lo0 |= hv & 0x30303030u;
+            hi0 |= __builtin_rotateright32(hv, 2u) & 0x30303030u;
+            lo1 |= __builtin_rotateright32(hv, 30u) & 0x30303030u;
+            hi1 |= __builtin_rotateright32(hv, 28u) & 0x30303030u;
+        } else if constexpr (HP == 1) {
+            // odd lane groups: the piece's upper bits
+            const uint32_t h = __builtin_rotateright32(hv, (lane & 16u) ? 28u : 0u);
+            lo0 |= h & 0x10101010u;
+            hi0 |= __builtin_rotateright32(h, 1u) & 0x10101010u;
+            lo1 |= __builtin_rotateright32(h, 2u) & 0x10101010u;
+            hi1 |= __builtin_rotateright32(h, 3u) & 0x10101010u;
+        }
+        a[0] = (int)lo0;
+        a[1] = (int)hi0;
+        a[2] = (int)lo1;
+        a[3] = (int)hi1;
+    } else if constexpr (FMT == 2) {
+        // NF3 triplet (v0, v1, v2) of this row and 32-column half: codes 0-3 (even lane
+        // group) or 4-7 (odd) are this lane's four column quads; code 2 / 5 has its third
+        // bit in v2.  v0 = i0 | i1 << 3 | i2 << 6, v1 = i3 | i4 << 3 | i5 << 6, v2 = i6 | i7 << 3
+        // | third bits of i2, i5.  One v_perm looks four codes up in the 8-entry codebook.
+        const bool odd = (lane & 16u) != 0u;
+        const uint32_t p = odd ? d1 : d0, r = odd ? hv : d1;
+        const uint32_t e = (odd ? hv >> 3 : d0) & 0x07070707u;              // i0 / i7
+        const uint32_t n = (p >> 3) & 0x07070707u;                              // i1 / i4
+        const uint32_t m = ((p >> 6) & 0x03030303u) | ((hv >> (odd ? 5 : 4)) & 0x04040404u);  // i2 / i5
+        const uint32_t l = r & 0x07070707u;                                     // i3 / i6
+        a[0] = (int)__builtin_amdgcn_perm(t1, t0, odd ? n : e);
+        a[1] = (int)__builtin_amdgcn_perm(t1, t0, odd ? m : n);
+        a[2] = (int)__builtin_amdgcn_perm(t1, t0, odd ? l : m);
+        a[3] = (int)__builtin_amdgcn_perm(t1, t0, odd ? e : l);
+    } else {
+        a[0] = (int)nf4_xlut(d0 & 0x0F0F0F0Fu, t0, t1, u0, u1);
+        a[1] = (int)nf4_xlut((d0 >> 4) & 0x0F0F0F0Fu, t0, t1, u0, u1);
+        a[2] = (int)nf4_xlut(d1 & 0x0F0F0F0Fu, t0, t1, u0, u1);
+        a[3] = (int)nf4_xlut((d1 >> 4) & 0x0F0F0F0Fu, t0, t1, u0, u1);
+    }
+    return a;
+}
+
+// Per-lane offsets inside the records of a stripe (side 0 / 1 of its pair, or the tail).
+template <int FMT, int HP>
+__device__ __forceinline__ MfLane mf_lane(uint32_t lane, bool is_tail, uint32_t side, int lane_order) {
+    MfLane L;
+    const uint32_t li = lane & 15u, lg = lane >> 4;
+    if constexpr (FMT == 2) {
+        // block (g, half): 16-byte pieces 128 bytes apart in lane order, 16 in the reference's
+        const uint32_t g = li >> 2, half = lg >> 1, ps = lane_order ? 128u : 16u;
+        L.a_off = (is_tail ? 0u : side * 384u) + (lane_order ? (2u * g + half) * 16u : half * 192u + g * 48u) +
+                  4u * (li & 3u);
+        L.b_off = L.a_off + ps;
+        L.h_off = L.a_off + 2u * ps;
+        L.s_off = (is_tail ? 0u : side * 32u) + 8u * lg;
+    } else {
+        L.a_off = (is_tail ? 0u : side * 512u) + lg * 128u + (li >> 2) * 32u + 4u * (li & 3u);
+        L.b_off = L.a_off + 16u;
+    }
+    if constexpr (FMT == 0) {
+        const uint32_t hib = is_tail ? 512u : 1024u + side * 128u * HP;  // the stripe's hi bytes
+        L.h_off = hib + (HP == 2 ? lg : lg >> 1) * 64u + (li >> 2) * 16u + 4u * (li & 3u);
+        L.s_off = (is_tail ? 512u + 128u * HP : 1024u + 256u * HP + side * 32u) + 8u * lg;  // rows 4lg .. 4lg+3
+    } else if constexpr (FMT == 1) {
+        L.h_off = 0;
+        L.s_off = (is_tail ? 0u : side * 32u) + 8u * lg;
+    }
+    return L;
+}
+
 // Every load is a buffer load: the wave-uniform part of its offset in an SGPR, the
 // per-lane part (fixed for the wave's life) in one VGPR, so no 64-bit address adds.
 //  - NF: group sg = c / sgc starts at sg * gsz + sg * sgc * cs (gsz = 64 bytes of scales,
@@ -130,20 +210,25 @@ struct MfLane {
 //    codes at that + gsz + (c - sg * sgc) * cs.
 //  - bit planes: chunk c's record at c * REC (REC = 1024 + 256 hp + 64, the tail's
 //    512 + 128 hp + 32): codes, hi bytes, scales; the lane offsets point inside it.
-template <int FMT, int HP, int NB, bool SH>
-__device__ __forceinline__ void mf_fetch(const MfArgs &A, const MfSrc &R, const MfLane &L, bool is_tail, int tb0,
-                                         uint32_t wave, int c, MfChunk<FMT, NB, SH> &f) {
-    uint32_t rec, sgb;
+template <int FMT, int HP>
+__device__ __forceinline__ void mf_record(int sgc_log2, bool is_tail, int c, uint32_t &rec, uint32_t &sgb) {
     if constexpr (FMT == 0) {
         rec = (uint32_t)c * (is_tail ? 512u + 128u * HP + 32u : 1024u + 256u * HP + 64u);
         sgb = rec;
     } else {
-        const uint32_t sg = (uint32_t)c >> A.sgc_log2, sb = (uint32_t)c - (sg << A.sgc_log2);
+        const uint32_t sg = (uint32_t)c >> sgc_log2, sb = (uint32_t)c - (sg << sgc_log2);
         constexpr uint32_t CB = FMT == 2 ? 384u : 512u;  // bytes per stripe-chunk
         const uint32_t cs = is_tail ? CB : 2u * CB, gsz = is_tail ? 32u : 64u;
-        sgb = sg * gsz + (sg << A.sgc_log2) * cs;  // scale-group base
+        sgb = sg * gsz + (sg << sgc_log2) * cs;  // scale-group base
         rec = sgb + gsz + sb * cs;
     }
+}
+
+template <int FMT, int HP, int NB, bool SH>
+__device__ __forceinline__ void mf_fetch(const MfArgs &A, const MfSrc &R, const MfLane &L, bool is_tail, int tb0,
+                                         uint32_t wave, int c, MfChunk<FMT, NB, SH> &f) {
+    uint32_t rec, sgb;
+    mf_record<FMT, HP>(A.sgc_log2, is_tail, c, rec, sgb);
     f.d0 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(R.w, L.a_off, rec, 0);
     f.d1 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(R.w, L.b_off, rec, 0);
     if constexpr ((FMT == 0 && HP > 0) || FMT == 2) f.hv = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(R.w, L.h_off, rec, 0);
@@ -193,49 +278,7 @@ __device__ __forceinline__ void mf_step(const MfArgs &A, const MfChunk<FMT, NB, 
             if ((int)wave + 4 * k < NB) bsh[(wave + 4 * k) * 64 + lane] = f.x[k];
         __syncthreads();
     }
-    v4i a;
-    if constexpr (FMT == 0) {
-        // the unsigned codes: nibble, then the hi-plane bits (as chunk_dots places them for
-        // kk = lane group, half 0 for the first dword and half 1 for the second)
-        uint32_t lo0 = f.d0 & 0x0F0F0F0Fu, hi0 = (f.d0 >> 4) & 0x0F0F0F0Fu;
-        uint32_t lo1 = f.d1 & 0x0F0F0F0Fu, hi1 = (f.d1 >> 4) & 0x0F0F0F0Fu;
-        if constexpr (HP == 2) {
-            lo0 |= f.hv & 0x30303030u;
-            hi0 |= __builtin_rotateright32(f.hv, 2u) & 0x30303030u;
-            lo1 |= __builtin_rotateright32(f.hv, 30u) & 0x30303030u;
-            hi1 |= __builtin_rotateright32(f.hv, 28u) & 0x30303030u;
-        } else if constexpr (HP == 1) {
-            const uint32_t e = (lane & 16u) ? 28u : 0u;  // odd lane group: the piece's upper bits
-            lo0 |= __builtin_rotateright32(f.hv, e) & 0x10101010u;
-            hi0 |= __builtin_rotateright32(f.hv, e + 1u) & 0x10101010u;
-            lo1 |= __builtin_rotateright32(f.hv, e + 2u) & 0x10101010u;
-            hi1 |= __builtin_rotateright32(f.hv, e + 3u) & 0x10101010u;
-        }
-        a[0] = (int)lo0;
-        a[1] = (int)hi0;
-        a[2] = (int)lo1;
-        a[3] = (int)hi1;
-    } else if constexpr (FMT == 2) {
-        // NF3 triplet (v0, v1, v2) of this row and 32-column half: codes 0-3 (even lane
-        // group) or 4-7 (odd) are this lane's four column quads; code 2 / 5 has its third
-        // bit in v2.  v0 = i0 | i1 << 3 | i2 << 6, v1 = i3 | i4 << 3 | i5 << 6, v2 = i6 | i7 << 3
-        // | third bits of i2, i5.  One v_perm looks four codes up in the 8-entry codebook.
-        const bool odd = (lane & 16u) != 0u;
-        const uint32_t p = odd ? f.d1 : f.d0, r = odd ? f.hv : f.d1;
-        const uint32_t e = (odd ? f.hv >> 3 : f.d0) & 0x07070707u;              // i0 / i7
-        const uint32_t n = (p >> 3) & 0x07070707u;                              // i1 / i4
-        const uint32_t m = ((p >> 6) & 0x03030303u) | ((f.hv >> (odd ? 5 : 4)) & 0x04040404u);  // i2 / i5
-        const uint32_t l = r & 0x07070707u;                                     // i3 / i6
-        a[0] = (int)__builtin_amdgcn_perm(A.t1, A.t0, odd ? n : e);
-        a[1] = (int)__builtin_amdgcn_perm(A.t1, A.t0, odd ? m : n);
-        a[2] = (int)__builtin_amdgcn_perm(A.t1, A.t0, odd ? l : m);
-        a[3] = (int)__builtin_amdgcn_perm(A.t1, A.t0, odd ? e : l);
-    } else {
-        a[0] = (int)nf4_xlut(f.d0 & 0x0F0F0F0Fu, A.t0, A.t1, A.u0, A.u1);
-        a[1] = (int)nf4_xlut((f.d0 >> 4) & 0x0F0F0F0Fu, A.t0, A.t1, A.u0, A.u1);
-        a[2] = (int)nf4_xlut(f.d1 & 0x0F0F0F0Fu, A.t0, A.t1, A.u0, A.u1);
-        a[3] = (int)nf4_xlut((f.d1 >> 4) & 0x0F0F0F0Fu, A.t0, A.t1, A.u0, A.u1);
-    }
+    const v4i a = mf_decode<FMT, HP>(f.d0, f.d1, f.hv, A.t0, A.t1, A.u0, A.u1, lane);
     const float ws[4] = {bf16_lo(f.sw.x), bf16_hi(f.sw.x), bf16_lo(f.sw.y), bf16_hi(f.sw.y)};
 #pragma unroll
     for (int b = 0; b < NB; b++) {
@@ -297,27 +340,7 @@ __global__ __launch_bounds__(SW ? 512 : 256) void gemm_mfma_kernel(MfArgs A) {
     const uint32_t side = is_tail ? 0u : (uint32_t)(stripe & 1);
     const uint8_t *mbase = is_tail ? A.tail : A.pair + (size_t)(stripe >> 1) * A.ptot;
     const uint32_t li = lane & 15u, lg = lane >> 4;
-    MfLane L;
-    if constexpr (FMT == 2) {
-        // block (g, half): 16-byte pieces 128 bytes apart in lane order, 16 in the reference's
-        const uint32_t g = li >> 2, half = lg >> 1, ps = A.lane ? 128u : 16u;
-        L.a_off = (is_tail ? 0u : side * 384u) + (A.lane ? (2u * g + half) * 16u : half * 192u + g * 48u) +
-                  4u * (li & 3u);
-        L.b_off = L.a_off + ps;
-        L.h_off = L.a_off + 2u * ps;
-        L.s_off = (is_tail ? 0u : side * 32u) + 8u * lg;
-    } else {
-        L.a_off = (is_tail ? 0u : side * 512u) + lg * 128u + (li >> 2) * 32u + 4u * (li & 3u);
-        L.b_off = L.a_off + 16u;
-    }
-    if constexpr (FMT == 0) {
-        const uint32_t hib = is_tail ? 512u : 1024u + side * 128u * HP;  // the stripe's hi bytes
-        L.h_off = hib + (HP == 2 ? lg : lg >> 1) * 64u + (li >> 2) * 16u + 4u * (li & 3u);
-        L.s_off = (is_tail ? 512u + 128u * HP : 1024u + 256u * HP + side * 32u) + 8u * lg;  // rows 4lg .. 4lg+3
-    } else if constexpr (FMT == 1) {
-        L.h_off = 0;
-        L.s_off = (is_tail ? 0u : side * 32u) + 8u * lg;
-    }
+    MfLane L = mf_lane<FMT, HP>(lane, is_tail, side, A.lane);
     L.x_off = lane * 16u;
     L.sx_off = li * 4u;
     const MfSrc R{mf_rsrc(mbase), mf_rsrc(A.xt), mf_rsrc(A.st), mf_rsrc(FMT == 0 ? (const void *)A.ut : A.st)};
@@ -461,12 +484,222 @@ __global__ __launch_bounds__(256) void mf_tile_kernel(const int8_t *xq, const fl
     if (lg == 1 && ut) ut[tile * 16 + li] = xsum[(size_t)tok * nc + c];
 }
 
+// ---------------------------------------------------------------- 2 .. 15 tokens, fast epilogue
+// The GEMV's own work split (plan_gemv: a workgroup per stripe pair, or per stripe where
+// pairs are fewer than CUs; its waves are K segments) with the chunk dots of up to 16 tokens
+// from one MFMA per stripe-chunk.  The 4-token passes it replaces decode every weight once
+// per 4 tokens and spend two v_dot4 per four codes and token; here the decode and the MFMA
+// cost the same for 2 tokens as for 16, so what bounds it is the weight stream and, past
+// about 8 tokens, the gather of the activation rows (16 lines per load).  NF4 14336 x 4096,
+// 4 / 8 / 15 tokens: 12.6 / 21.1 / 40.3 us as 4-token passes, 9.6 / 10.7 / 12.7 us here (one
+// token 8.7); b6 4096 x 14336: 15.3 / 27.7 / 54.8 us, 14.0 / 18.0 / 23.4 us here.
+// Sums: the order of gemv_kernel's fast epilogue, so a batch gives each token the bits of
+// the one-token GEMV.  A wave's chunks are dealt round-robin to G accumulators (the GEMV's
+// lane groups: 4 in pair mode, 8 in stripe mode), which are added pairwise as the lane
+// butterfly does, then the waves' sums in wave order.  (A chunk with scale 0 adds +-0.)
+struct GvArgs {
+    const uint8_t *pair, *tail;
+    size_t ptot;
+    int rows, K, nc, np, sgc_log2, s0, s1, rb_lo, nseg, cps, ntok, accum;
+    int tg;  // tokens per workgroup (blockIdx.y counts token groups)
+    uint32_t t0, t1, u0, u1;
+    int lane;
+    const int8_t *xq;
+    const float *xs;
+    const int32_t *xsum;
+    float *out;
+    size_t out_stride;
+};
+
+template <int FMT, int RS>
+struct GvFrag {
+    uint32_t d0[RS], d1[RS], hv[RS];
+    uint2 sw[RS];
+    v4i x;
+    float sx;
+    int32_t su;
+};
+
+template <int FMT, int HP, bool SM>
+__global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
+    constexpr int RS = SM ? 1 : 2, G = SM ? 8 : 4, RB = 16 * RS;
+    constexpr int P = SM && FMT == 0 && HP > 0 ? 4 : G;  // chunks in flight (128 VGPRs at 16 waves)
+    extern __shared__ float part[];  // [nseg][16 tokens][RB rows + 1]
+    const uint32_t lane = threadIdx.x & 63u, li = lane & 15u, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    int rbi = (int)blockIdx.x;
+    if (SM && (gridDim.x & 15u) == 0) {  // both stripes of a pair on one XCD, as in gemv_kernel
+        const int a = rbi >> 4, s8 = (rbi >> 3) & 1, j = rbi & 7;
+        rbi = 2 * (8 * a + j) + s8;
+    }
+    const int rb = A.rb_lo + rbi;  // pair index, or stripe index in stripe mode
+    const bool is_tail = SM ? rb >= 2 * A.np : rb >= A.np;
+    const int pidx = SM ? rb >> 1 : rb;
+    const uint8_t *mbase = is_tail ? A.tail : A.pair + (size_t)pidx * A.ptot;
+    MfLane L[RS];
+#pragma unroll
+    for (int s = 0; s < RS; s++)  // (pair mode on the tail stripe: side 1 repeats it, not stored)
+        L[s] = mf_lane<FMT, HP>(lane, is_tail, is_tail ? 0u : SM ? (uint32_t)(rb & 1) : (uint32_t)s, A.lane);
+    const int tok0 = (int)blockIdx.y * A.tg, nt = min(A.tg, A.ntok - tok0);
+    const uint32_t tok = (uint32_t)tok0 + min(li, (uint32_t)nt - 1u);  // columns past nt repeat the last token, not stored
+    const uint32_t x_off = tok * (uint32_t)A.K + lg * 16u, sx_off = tok * (uint32_t)A.nc * 4u;
+    const __amdgpu_buffer_rsrc_t rw = mf_rsrc(mbase), rx = mf_rsrc(A.xq), rs = mf_rsrc(A.xs),
+                                 ru = mf_rsrc(FMT == 0 ? (const void *)A.xsum : A.xs);
+    const int cw0 = wave * A.cps, cw1 = min(A.nc, cw0 + A.cps), n = cw1 - cw0;
+    auto fetch = [&](GvFrag<FMT, RS> &f, int c) {
+        uint32_t rec, sgb;
+        mf_record<FMT, HP>(A.sgc_log2, is_tail, c, rec, sgb);
+#pragma unroll
+        for (int s = 0; s < RS; s++) {
+            f.d0[s] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw, L[s].a_off, rec, 0);
+            f.d1[s] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw, L[s].b_off, rec, 0);
+            if constexpr ((FMT == 0 && HP > 0) || FMT == 2)
+                f.hv[s] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw, L[s].h_off, rec, 0);
+            const v2u sw = __builtin_amdgcn_raw_buffer_load_b64(rw, L[s].s_off, sgb, 0);
+            f.sw[s] = make_uint2(sw[0], sw[1]);
+        }
+        const v4u x = __builtin_amdgcn_raw_buffer_load_b128(rx, x_off, (uint32_t)c * 64u, 0);
+        f.x = v4i{(int)x[0], (int)x[1], (int)x[2], (int)x[3]};
+        f.sx = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, sx_off, (uint32_t)c * 4u, 0));
+        if constexpr (FMT == 0) f.su = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(ru, sx_off, (uint32_t)c * 4u, 0);
+    };
+    float acc[G][RS][4];
+#pragma unroll
+    for (int g = 0; g < G; g++)
+#pragma unroll
+        for (int s = 0; s < RS; s++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[g][s][r] = 0.0f;
+    auto compute = [&](const GvFrag<FMT, RS> &f, float (&o)[RS][4]) {
+#pragma unroll
+        for (int s = 0; s < RS; s++) {
+            const v4i a = mf_decode<FMT, HP>(f.d0[s], f.d1[s], f.hv[s], A.t0, A.t1, A.u0, A.u1, lane);
+            const v4i zero = {0, 0, 0, 0};
+            const v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, f.x, zero, 0, 0, 0);
+            const float ws[4] = {bf16_lo(f.sw[s].x), bf16_hi(f.sw[s].x), bf16_lo(f.sw[s].y), bf16_hi(f.sw[s].y)};
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                int dot = d[r];
+                if constexpr (FMT == 0) dot = 2 * dot - ((1 << (4 + HP)) - 1) * f.su;
+                o[s][r] = fmaf((float)dot * f.sx, ws[r], o[s][r]);
+            }
+        }
+    };
+    // One round = the G accumulators' next chunks; a chunk's registers take the load P chunks
+    // on as soon as it is computed.  The last round issues only what it will use itself.
+    GvFrag<FMT, RS> ring[P];
+#pragma unroll
+    for (int u = 0; u < P; u++) fetch(ring[u], min(cw0 + u, cw1 - 1));
+    int i0 = 0;
+    for (; i0 + G < n; i0 += G) {
+#pragma unroll
+        for (int u = 0; u < G; u++) {
+            compute(ring[u % P], acc[u]);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(ring[u % P], min(cw0 + i0 + P + u, cw1 - 1));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+        if (i0 + u < n) compute(ring[u % P], acc[u]);
+        if (u + P < G) fetch(ring[u % P], min(cw0 + i0 + P + u, cw1 - 1));
+    }
+    // the accumulators pairwise (neighbours, then pairs, ...), then into LDS
+    constexpr int RP = RB + 1;
+#pragma unroll
+    for (int s = 0; s < RS; s++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            float v[G];
+#pragma unroll
+            for (int g = 0; g < G; g++) v[g] = acc[g][s][r];
+#pragma unroll
+            for (int w = G; w > 1; w >>= 1)
+#pragma unroll
+                for (int g = 0; g < w / 2; g++) v[g] = v[2 * g] + v[2 * g + 1];
+            part[((size_t)wave * 16 + li) * RP + 16 * s + 4 * lg + r] = v[0];
+        }
+    __syncthreads();
+    const int first = SM ? rb : is_tail ? 2 * A.np : 2 * rb;
+    const int live = (!SM && is_tail) ? 16 : RB;
+    for (int idx = (int)threadIdx.x; idx < nt * RB; idx += (int)blockDim.x) {
+        const int t = idx / RB, rl = idx % RB, st = first + rl / 16, row = st * 16 + rl % 16;
+        if (rl >= live || row >= A.rows || st < A.s0 || st >= A.s1) continue;
+        float v = part[(size_t)t * RP + rl];
+        for (int w = 1; w < A.nseg; w++) v += part[((size_t)w * 16 + t) * RP + rl];
+        float *o = A.out + (size_t)(tok0 + t) * A.out_stride + row;
+        *o = A.accum ? *o + v : v;
+    }
+}
+
 }  // namespace
 
 bool gemm_mfma_supported(const k2t_mat *m, int ntok) {
     if (ntok < kMfmaMinTokens || m->cols % 64 != 0) return false;
     if (m->fmt == K2T_FMT_NF) return (m->bits == 3 || m->bits == 4) && (m->sgc & (m->sgc - 1)) == 0;
     return m->fmt == K2T_FMT_NIBBLE4 && m->hp >= 0 && m->hp <= 2;
+}
+
+bool gemv_mfma_supported(const k2t_mat *m, int ntok) {
+    if (ntok < 2 || ntok >= kMfmaMinTokens || !gemm_mfma_supported(m, kMfmaMinTokens)) return false;
+    // NF3 up to 4 tokens: the 4-token pass (its 16-byte loads stream the 384-byte chunks
+    // better than this kernel's dwords: 4096 x 14336, 2 / 3 / 4 tokens 8.8 / 9.9 / 10.9 us
+    // there, 10.5 / 11.3 / 11.9 here; 8 tokens 19.3 there, 14.3 here)
+    return m->fmt != K2T_FMT_NF || m->bits != 3 || ntok > 4;
+}
+
+template <int FMT, int HP>
+static void launch_gemv_mfma_fmt(hipStream_t st, const GemvPlan &plan, dim3 grid, size_t lds, const GvArgs &A) {
+    const dim3 block(64 * plan.nseg);
+    if (plan.stripe_mode) hipLaunchKernelGGL((gemv_mfma_kernel<FMT, HP, true>), grid, block, lds, st, A);
+    else hipLaunchKernelGGL((gemv_mfma_kernel<FMT, HP, false>), grid, block, lds, st, A);
+}
+
+void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, const int8_t *xq, const float *xs,
+                      const int32_t *xsum, int ntok, int s0, int s1, float *out, size_t out_stride, bool accum) {
+    const bool planes = m->fmt == K2T_FMT_NIBBLE4;
+    GvArgs A{};
+    A.pair = m->pair;
+    A.tail = m->tail;
+    A.ptot = m->pairs ? m->pair_len / m->pairs : 0;
+    A.rows = m->rows;
+    A.K = m->cols;
+    A.nc = m->nc;
+    A.np = m->pairs;
+    A.sgc_log2 = planes ? 0 : __builtin_ctz((unsigned)m->sgc);
+    A.s0 = s0;
+    A.s1 = s1;
+    A.rb_lo = plan.rb_lo;
+    A.nseg = plan.nseg;
+    A.cps = plan.cps;
+    A.ntok = ntok;
+    A.accum = accum ? 1 : 0;
+    A.lane = m->nf3_lane;
+    if (!planes && m->bits == 3) {
+        A.t0 = m->cb[0];
+        A.t1 = m->cb[1];
+    } else if (!planes) nf4_xor_tables(m->cb[0], m->cb[1], m->cb[2], m->cb[3], A.t0, A.t1, A.u0, A.u1);
+    A.xq = xq;
+    A.xs = xs;
+    A.xsum = xsum;
+    A.out = out;
+    A.out_stride = out_stride;
+    // A matrix with few row blocks leaves CUs idle: the tokens are then dealt to several
+    // workgroups (four or more tokens each), which shortens each one's activation gather.
+    // NF4 2048 x 8192, 8 / 15 tokens: 8.8 / 11.0 us in one group, 7.6 / 9.0 us.
+    const int wgs = plan.rb_hi - plan.rb_lo;
+    const int groups = std::max(1, std::min(ctx->num_cus / wgs, (ntok + 3) / 4));
+    A.tg = (ntok + groups - 1) / groups;
+    const dim3 grid(wgs, (ntok + A.tg - 1) / A.tg);
+    const size_t lds = (size_t)plan.nseg * 16 * ((plan.stripe_mode ? 16 : 32) + 1) * sizeof(float);
+    hipStream_t st = ctx->stream;
+    if (m->fmt == K2T_FMT_NF && m->bits == 3) launch_gemv_mfma_fmt<2, 0>(st, plan, grid, lds, A);
+    else if (m->fmt == K2T_FMT_NF) launch_gemv_mfma_fmt<1, 0>(st, plan, grid, lds, A);
+    else if (m->hp == 0) launch_gemv_mfma_fmt<0, 0>(st, plan, grid, lds, A);
+    else if (m->hp == 1) launch_gemv_mfma_fmt<0, 1>(st, plan, grid, lds, A);
+    else launch_gemv_mfma_fmt<0, 2>(st, plan, grid, lds, A);
+    hip_check(hipGetLastError(), "mfma gemv launch");
 }
 
 template <int FMT, int HP>

@@ -971,6 +971,12 @@ static void launch_gemv_impl(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, c
     }
     ctx->max_segments = saved;
     if (plan.rb_hi <= plan.rb_lo || ntok <= 0) return;
+    // 2 .. 15 tokens with the fast epilogue: one weight pass on the matrix cores, the same
+    // plan and sum order (each token's bits are the one-token GEMV's)
+    if (!dots && !grp && xsm == 0 && gu_split == 0 && !ctx->exact && ctx->mfma && gemv_mfma_supported(m, ntok)) {
+        launch_gemv_mfma(ctx, m, plan, xq, xs, xsum, ntok, s0, s1, out, out_stride, accum);
+        return;
+    }
     GemvParams P{};
     P.pair = m->pair;
     P.tail = m->tail;

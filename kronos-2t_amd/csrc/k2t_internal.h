@@ -138,6 +138,11 @@ constexpr int kMfmaMinTokens = 16;
 bool gemm_mfma_supported(const k2t_mat *m, int ntok);
 void launch_gemm_mfma(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const float *xs, const int32_t *xsum,
                       int ntok, float *out, size_t out_stride, bool accum, ActTiles tiles = ActTiles{});
+// 2 .. 15 tokens with the fast epilogue on the matrix cores: plan_gemv's split, the sums in
+// gemv_kernel's order.
+bool gemv_mfma_supported(const k2t_mat *m, int ntok);
+void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, const int8_t *xq, const float *xs,
+                      const int32_t *xsum, int ntok, int s0, int s1, float *out, size_t out_stride, bool accum);
 // gate_up (interleaved [gate64, up64] blocks) from producer tiles with the SwiGLU + FWHT +
 // int8 of the down input (q / s / sums [token][rows / 128], its tiles into out_tiles,
 // which must not be `tiles`) as the epilogue; false (nothing launched) when the plain

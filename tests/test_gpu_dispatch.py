@@ -101,3 +101,52 @@ def test_mfma_nf3_equals_reference_chain(gpu_ctx, rows, cols, sgc, ntok, lane):
         assert np.array_equal(out[24:].view(np.uint32), out[4:][np.arange(ntok - 24) % 20].view(np.uint32)) \
             if ntok > 24 else True
     m.close()
+
+
+def _matrix(ctx, rng, fmt, rows, cols, sgc=2):
+    """A matrix of random codes in any format (bit planes b4 .. b6, NF4, NF3)."""
+    from helpers import random_nf_streams, random_nibble4_streams
+    if fmt[0] == "b":
+        pair, tail = random_nibble4_streams(rng, rows, cols, int(fmt[1]) - 4)
+        return ctx.upload_nibble4(rows, cols, int(fmt[1]) - 4, pair, tail)
+    bits = int(fmt[2])
+    _, _, pair, tail = random_nf_streams(rng, rows, cols, sgc, bits=bits)
+    cb = np.sort(rng.choice(np.arange(-127, 128), 16, replace=False)).astype(np.int8)
+    return ctx.upload_nf(rows, cols, bits, sgc, cb, pair, tail)
+
+
+# stripe mode and pair mode (512 or more stripes), one and several rounds of a wave's chunks,
+# ragged last rounds, a tail stripe, rows past the last stripe's end, 2 and 15 tokens
+@pytest.mark.parametrize("fmt", ["nf4", "nf3", "b4", "b5", "b6"])
+@pytest.mark.parametrize("rows,cols,ntok", [(16, 64, 2), (40, 576, 15), (1030, 4160, 5), (8208, 192, 3),
+                                            (8300, 2112, 11), (9000, 8256, 4)])
+def test_small_batch_gemv_equals_one_token(gpu_ctx, fmt, rows, cols, ntok):
+    """2 .. 15 tokens: each token's outputs are the one-token GEMV's bit for bit (the same
+    exact chunk dots, summed in the same order), also for a stripe range and with the number
+    of K segments capped; outputs outside the range stay untouched."""
+    import torch
+    from helpers import acts
+    rng = np.random.default_rng(rows + cols + ntok)
+    m = _matrix(gpu_ctx, rng, fmt, rows, cols)
+    xq, xs, xsum = acts(rng, cols, ntok, outlier_frac=0.001, outlier_scale=30.0)
+    xs[ntok - 1, 0] = 0.0
+    xq[ntok - 1, :64] = 0
+    xsum[ntok - 1, 0] = 0
+    out = _gemv(gpu_ctx, m, xq, xs, xsum, rows)
+    one = np.concatenate([_gemv(gpu_ctx, m, xq[t:t + 1], xs[t:t + 1], xsum[t:t + 1], rows) for t in range(ntok)])
+    assert np.array_equal(out.view(np.uint32), one.view(np.uint32))
+    s0, s1 = m.info()[2] // 3, -(-2 * m.info()[2] // 3)
+    part = [torch.full((ntok, rows + 3), 7.0, device="cuda") for _ in range(2)]
+    args = _t(xq), _t(xs), _t(xsum)
+    gpu_ctx.set_splitk(3)
+    try:
+        gpu_ctx.gemv(m, *args, part[0], ntok=ntok, s0=s0, s1=s1, out_stride=rows + 3)
+        for t in range(ntok):
+            gpu_ctx.gemv(m, args[0][t], args[1][t], args[2][t], part[1][t], s0=s0, s1=s1)
+        gpu_ctx.sync()
+    finally:
+        gpu_ctx.set_splitk(0)
+    a, b = (p.cpu().numpy() for p in part)
+    assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    assert np.all(a[:, s1 * 16:] == 7.0) and np.all(a[:, :s0 * 16] == 7.0)
+    m.close()
