@@ -19,8 +19,6 @@
 #include "k2t_moe.h"
 
 namespace k2t {
-void launch_rmsnorm_act(hipStream_t st, const uint64_t *signs, const float *x, const float *w, float eps, int K,
-                        int ntok, int8_t *q, float *s, int32_t *sums, ActTiles tiles = ActTiles{});
 void launch_qkv_post(hipStream_t st, float *qkv, const float *bias, const float *qn, const float *kn, float eps,
                      const float *rope, const int *pos_dev, int nq,
                      int nkv, int hd, int ntok, int layer, KvRing kr, int8_t *kq, int8_t *vq, float *ks, float *vs,
@@ -216,6 +214,8 @@ struct k2t_model {
     KvRing ring{};                       // KV slots: cap = max_seq, or a sliding-window ring
     float *moe_ws = nullptr;             // MoE workspace (largest layer's need)
     size_t moe_ws_floats = 0;
+    uint8_t *moe_batch = nullptr;        // batch workspace (the largest layer's need; max_batch > 1)
+    size_t moe_batch_bytes = 0;
     float *rope = nullptr;  // [max_seq][hd] = cos | sin halves
     int8_t *kq = nullptr, *vq = nullptr;
     float *ks = nullptr, *vs = nullptr;
@@ -268,6 +268,16 @@ void *dalloc(k2t_model *m, size_t bytes) {
     }
     m->allocs.push_back(p);
     return p;
+}
+
+// Grows the model's MoE batch workspace to layer L's need.
+void ensure_moe_batch(k2t_model *m, const MoeLayer &L) {
+    if (m->max_batch < 2) return;
+    const int inter = L.sh_gu ? L.sh_gu->rows / 2 : 0;
+    const size_t need = moe_batch_bytes(L.bank, L.top_k, inter, moe_batch_tokens(L.bank, L.top_k, inter, m->max_batch));
+    if (need <= m->moe_batch_bytes) return;
+    m->moe_batch = (uint8_t *)dalloc(m, need);
+    m->moe_batch_bytes = need;
 }
 
 void arg(bool ok, const char *msg) {
@@ -422,7 +432,17 @@ void forward(k2t_model *m, int ntok, bool with_logits, int ctx_bound = 0) {
                          GqaWork{m->attn_words, m->attn_cnt, m->err_dev}, ctx_bound, to, ctx->mfma != 0);
         launch_gemv_ex(ctx, L.o, m->xq, m->xs, m->xsum, ntok, m->hidden, d, true, 0, to);
         if (L.has_moe) {
-            // one token at a time: each token has its own routes (forward_layer_single)
+            // each token has its own routes (forward_layer_single); a batch groups its tokens
+            // by expert
+            if (ntok > 1 && m->moe_batch && moe_batch_supported(ctx, L.moe)) {
+                const int inter = L.moe.sh_gu ? L.moe.sh_gu->rows / 2 : 0;
+                const int group = moe_batch_tokens(L.moe.bank, L.moe.top_k, inter, m->max_batch);
+                const MoeBatchWork bw = moe_batch_carve(m->moe_batch, L.moe.bank, L.moe.top_k, inter, group);
+                for (int t = 0; t < ntok; t += group)
+                    launch_moe_ffn_batch(ctx, L.moe, m->hidden + (size_t)t * d, std::min(group, ntok - t), L.post_norm,
+                                         c.rms_eps, bw, m->err_dev);
+                continue;
+            }
             MoeWork ws = moe_work_carve(m->moe_ws, L.moe.bank, L.moe.top_k);
             ws.err = m->err_dev;  // timeouts surface through the model's error word
             for (int t = 0; t < ntok; t++) launch_moe_ffn(ctx, L.moe, m->hidden + (size_t)t * d, L.post_norm, c.rms_eps, ws);
@@ -915,6 +935,7 @@ int32_t k2t_model_set_moe(k2t_model *m, int32_t layer, const k2t_experts *bank, 
         }
         L.moe = MoeLayer{bank, shard_layer, rw, rb, top_k, norm_topk_prob ? 1 : 0, scoring};
         L.has_moe = true;
+        ensure_moe_batch(m, L.moe);
         drop_graph(m);
     });
 }
@@ -951,6 +972,7 @@ int32_t k2t_model_set_moe_shared(k2t_model *m, int32_t layer, const k2t_mat *gat
         L.moe.sh_gu = gate_up;
         L.moe.sh_dn = down;
         L.moe.sh_gate = g;
+        ensure_moe_batch(m, L.moe);
     });
 }
 

@@ -509,6 +509,11 @@ struct GvArgs {
     const int32_t *xsum;
     float *out;
     size_t out_stride;
+    // Grouped form (sparse-MoE experts): blockIdx.y counts work items, each up to 16 (token,
+    // slot) pairs of one expert; the matrix and its codebook are at the expert's record, pair
+    // p reads activation row p / row_div and writes out + p * out_stride (gu_split: a [gate;
+    // up] matrix's rows in [gate64, up64] blocks).
+    GvGroup grp;
 };
 
 template <int FMT, int RS>
@@ -520,7 +525,7 @@ struct GvFrag {
     int32_t su;
 };
 
-template <int FMT, int HP, bool SM>
+template <int FMT, int HP, bool SM, bool GRP = false>
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
     constexpr int RS = SM ? 1 : 2, G = SM ? 8 : 4, RB = 16 * RS;
     constexpr int P = SM && FMT == 0 && HP > 0 ? 4 : G;  // chunks in flight (128 VGPRs at 16 waves)
@@ -536,12 +541,23 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
     const bool is_tail = SM ? rb >= 2 * A.np : rb >= A.np;
     const int pidx = SM ? rb >> 1 : rb;
     const uint8_t *mbase = is_tail ? A.tail : A.pair + (size_t)pidx * A.ptot;
+    int4 item = make_int4(0, 0, 0, 0);  // expert, first entry of the pair list, pairs
+    if constexpr (GRP) {
+        if ((int)blockIdx.y >= A.grp.n_items[0]) return;  // uniform: the grid covers the most items possible
+        item = A.grp.items[blockIdx.y];
+        const uint8_t *rec = A.grp.bank + (size_t)item.x * A.grp.bank_stride;
+        mbase = rec + A.grp.mat_off + (size_t)pidx * A.ptot;
+        const uint4 cb = *reinterpret_cast<const uint4 *>(rec + A.grp.cb_off);
+        if constexpr (FMT == 1) nf4_xor_tables(cb.x, cb.y, cb.z, cb.w, A.t0, A.t1, A.u0, A.u1);
+        else A.t0 = cb.x, A.t1 = cb.y;
+    }
     MfLane L[RS];
 #pragma unroll
     for (int s = 0; s < RS; s++)  // (pair mode on the tail stripe: side 1 repeats it, not stored)
         L[s] = mf_lane<FMT, HP>(lane, is_tail, is_tail ? 0u : SM ? (uint32_t)(rb & 1) : (uint32_t)s, A.lane);
-    const int tok0 = (int)blockIdx.y * A.tg, nt = min(A.tg, A.ntok - tok0);
-    const uint32_t tok = (uint32_t)tok0 + min(li, (uint32_t)nt - 1u);  // columns past nt repeat the last token, not stored
+    const int tok0 = GRP ? 0 : (int)blockIdx.y * A.tg, nt = GRP ? item.z : min(A.tg, A.ntok - tok0);
+    uint32_t tok = (uint32_t)tok0 + min(li, (uint32_t)nt - 1u);  // columns past nt repeat the last token, not stored
+    if constexpr (GRP) tok = (uint32_t)A.grp.list[item.y + (int)tok] / (uint32_t)A.grp.row_div;
     const uint32_t x_off = tok * (uint32_t)A.K + lg * 16u, sx_off = tok * (uint32_t)A.nc * 4u;
     const __amdgpu_buffer_rsrc_t rw = mf_rsrc(mbase), rx = mf_rsrc(A.xq), rs = mf_rsrc(A.xs),
                                  ru = mf_rsrc(FMT == 0 ? (const void *)A.xsum : A.xs);
@@ -628,6 +644,15 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
         if (rl >= live || row >= A.rows || st < A.s0 || st >= A.s1) continue;
         float v = part[(size_t)t * RP + rl];
         for (int w = 1; w < A.nseg; w++) v += part[((size_t)w * 16 + t) * RP + rl];
+        if constexpr (GRP) {
+            int r = row;  // gate / up rows in blocks of 64
+            if (A.grp.gu_split) {
+                const int inter = A.rows >> 1, up = row >= inter ? 1 : 0, rr = row - up * inter;
+                r = (rr >> 6) * 128 + up * 64 + (rr & 63);
+            }
+            A.out[(size_t)A.grp.list[item.y + t] * A.out_stride + r] = v;
+            continue;
+        }
         float *o = A.out + (size_t)(tok0 + t) * A.out_stride + row;
         *o = A.accum ? *o + v : v;
     }
@@ -656,8 +681,9 @@ static void launch_gemv_mfma_fmt(hipStream_t st, const GemvPlan &plan, dim3 grid
     else hipLaunchKernelGGL((gemv_mfma_kernel<FMT, HP, false>), grid, block, lds, st, A);
 }
 
-void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, const int8_t *xq, const float *xs,
-                      const int32_t *xsum, int ntok, int s0, int s1, float *out, size_t out_stride, bool accum) {
+// The arguments every launch over matrix m with this plan shares.
+static GvArgs gemv_mfma_args(const k2t_mat *m, const GemvPlan &plan, const int8_t *xq, const float *xs,
+                             const int32_t *xsum, float *out, size_t out_stride) {
     const bool planes = m->fmt == K2T_FMT_NIBBLE4;
     GvArgs A{};
     A.pair = m->pair;
@@ -668,13 +694,10 @@ void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, cons
     A.nc = m->nc;
     A.np = m->pairs;
     A.sgc_log2 = planes ? 0 : __builtin_ctz((unsigned)m->sgc);
-    A.s0 = s0;
-    A.s1 = s1;
+    A.s1 = m->stripes;
     A.rb_lo = plan.rb_lo;
     A.nseg = plan.nseg;
     A.cps = plan.cps;
-    A.ntok = ntok;
-    A.accum = accum ? 1 : 0;
     A.lane = m->nf3_lane;
     if (!planes && m->bits == 3) {
         A.t0 = m->cb[0];
@@ -685,6 +708,41 @@ void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, cons
     A.xsum = xsum;
     A.out = out;
     A.out_stride = out_stride;
+    return A;
+}
+
+static size_t gemv_mfma_lds(const GemvPlan &plan) {
+    return (size_t)plan.nseg * 16 * ((plan.stripe_mode ? 16 : 32) + 1) * sizeof(float);
+}
+
+bool gemv_mfma_grouped_supported(const k2t_mat *geom) {
+    return geom->fmt == K2T_FMT_NF && !geom->has_tail && gemm_mfma_supported(geom, kMfmaMinTokens);
+}
+
+void launch_gemv_mfma_grouped(k2t_ctx *ctx, const k2t_mat *geom, const GvGroup &g, int max_items, const int8_t *xq,
+                              const float *xs, float *out, size_t out_stride) {
+    if (!gemv_mfma_grouped_supported(geom) || max_items < 1 || max_items > 65535)
+        throw Error(K2T_E_INTERNAL, "grouped mfma gemv: shape");
+    const GemvPlan plan = plan_gemv(ctx, geom, 0, geom->stripes);
+    GvArgs A = gemv_mfma_args(geom, plan, xq, xs, nullptr, out, out_stride);
+    A.grp = g;
+    const dim3 grid(plan.rb_hi - plan.rb_lo, max_items), block(64 * plan.nseg);
+    const size_t lds = gemv_mfma_lds(plan);
+    hipStream_t st = ctx->stream;
+    if (geom->bits == 3 && plan.stripe_mode) hipLaunchKernelGGL((gemv_mfma_kernel<2, 0, true, true>), grid, block, lds, st, A);
+    else if (geom->bits == 3) hipLaunchKernelGGL((gemv_mfma_kernel<2, 0, false, true>), grid, block, lds, st, A);
+    else if (plan.stripe_mode) hipLaunchKernelGGL((gemv_mfma_kernel<1, 0, true, true>), grid, block, lds, st, A);
+    else hipLaunchKernelGGL((gemv_mfma_kernel<1, 0, false, true>), grid, block, lds, st, A);
+    hip_check(hipGetLastError(), "grouped mfma gemv launch");
+}
+
+void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, const int8_t *xq, const float *xs,
+                      const int32_t *xsum, int ntok, int s0, int s1, float *out, size_t out_stride, bool accum) {
+    GvArgs A = gemv_mfma_args(m, plan, xq, xs, xsum, out, out_stride);
+    A.s0 = s0;
+    A.s1 = s1;
+    A.ntok = ntok;
+    A.accum = accum ? 1 : 0;
     // A matrix with few row blocks leaves CUs idle: the tokens are then dealt to several
     // workgroups (four or more tokens each), which shortens each one's activation gather.
     // NF4 2048 x 8192, 8 / 15 tokens: 8.8 / 11.0 us in one group, 7.6 / 9.0 us.
@@ -692,7 +750,7 @@ void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, cons
     const int groups = std::max(1, std::min(ctx->num_cus / wgs, (ntok + 3) / 4));
     A.tg = (ntok + groups - 1) / groups;
     const dim3 grid(wgs, (ntok + A.tg - 1) / A.tg);
-    const size_t lds = (size_t)plan.nseg * 16 * ((plan.stripe_mode ? 16 : 32) + 1) * sizeof(float);
+    const size_t lds = gemv_mfma_lds(plan);
     hipStream_t st = ctx->stream;
     if (m->fmt == K2T_FMT_NF && m->bits == 3) launch_gemv_mfma_fmt<2, 0>(st, plan, grid, lds, A);
     else if (m->fmt == K2T_FMT_NF) launch_gemv_mfma_fmt<1, 0>(st, plan, grid, lds, A);

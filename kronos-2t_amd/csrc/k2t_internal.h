@@ -130,6 +130,8 @@ struct ActTiles {
 };
 void launch_gemv_ex(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const float *xs, const int32_t *xsum, int ntok,
                     float *out, size_t out_stride, bool accumulate, int gu_split = 0, ActTiles tiles = ActTiles{});
+void launch_rmsnorm_act(hipStream_t st, const uint64_t *signs, const float *x, const float *w, float eps, int K,
+                        int ntok, int8_t *q, float *s, int32_t *sums, ActTiles tiles = ActTiles{});
 void launch_swiglu_act(hipStream_t st, const uint64_t *signs, const float *gu, int inter, int ntok, int8_t *q,
                        float *s, int32_t *sums, bool exact, ActTiles tiles = ActTiles{});
 // Batched NF4 / bit-plane GEMV on the matrix cores (k2t_gemm_mfma.hip): kMfmaMinTokens or
@@ -143,6 +145,22 @@ void launch_gemm_mfma(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const fl
 bool gemv_mfma_supported(const k2t_mat *m, int ntok);
 void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, const int8_t *xq, const float *xs,
                       const int32_t *xsum, int ntok, int s0, int s1, float *out, size_t out_stride, bool accum);
+// The same over sparse-MoE experts: work items {expert, first entry of `list`, pairs (1 .. 16)}
+// of (token, slot) pairs, built on the device; n_items[0] of them are valid.
+struct GvGroup {
+    const int4 *items = nullptr;
+    const int *n_items = nullptr;
+    const int *list = nullptr;
+    int row_div = 1;  // pair p reads activation row p / row_div
+    const uint8_t *bank = nullptr;
+    size_t bank_stride = 0;
+    uint32_t mat_off = 0, cb_off = 0;
+    int gu_split = 0;
+};
+constexpr int kGvItemPairs = 16;
+bool gemv_mfma_grouped_supported(const k2t_mat *geom);
+void launch_gemv_mfma_grouped(k2t_ctx *ctx, const k2t_mat *geom, const GvGroup &g, int max_items, const int8_t *xq,
+                              const float *xs, float *out, size_t out_stride);
 // gate_up (interleaved [gate64, up64] blocks) from producer tiles with the SwiGLU + FWHT +
 // int8 of the down input (q / s / sums [token][rows / 128], its tiles into out_tiles,
 // which must not be `tiles`) as the epilogue; false (nothing launched) when the plain

@@ -70,4 +70,32 @@ void check_moe_args(const k2t_experts *bank, int shard_layer, int top_k, int sco
 void launch_moe_ffn(k2t_ctx *ctx, const MoeLayer &L, float *hidden, const float *post_norm, float eps,
                     const MoeWork &ws);
 
+// The same for a batch of tokens (a prompt's), up to moe_batch_tokens of them per call: each
+// expert's tokens share its weight passes.  Every token's result is launch_moe_ffn's, but
+// for a shared expert's down projection of 16 or more tokens (the matrix-core GEMV's order).
+struct MoeBatchWork {
+    float *gu, *eo;             // [tokens * top_k][2 * d_ff], [tokens * top_k][d_model]
+    unsigned long long *words;  // [tokens][2E + 2] router logits or partial dots and sums
+    float *wts;                 // [tokens * top_k]
+    int *ids, *list;            // [tokens * top_k]: routes; pairs sorted by expert
+    int4 *items;                // work items of the grouped GEMVs
+    int *n_items;
+    int8_t *aq, *mq;            // [tokens][d], [tokens * top_k][d_ff]
+    float *as, *ms;
+    int32_t *asum, *msum;
+    float *sh_gu, *sh_out, *sh_scale;  // shared expert: [tokens][2 * inter], [tokens][d], [tokens]
+    int8_t *sh_q;
+    float *sh_s;
+    int32_t *sh_sum;
+};
+// Tokens per call for prompts of up to max_batch: at most 512 (each expert's weights are then
+// read for 32 of them at top 8 of 128), and a workspace of at most 256 MiB.
+int moe_batch_tokens(const k2t_experts *b, int top_k, int shared_inter, int max_batch);
+bool moe_batch_supported(const k2t_ctx *ctx, const MoeLayer &L);
+// Bytes for `tokens` tokens, and the regions inside a buffer of that size.
+size_t moe_batch_bytes(const k2t_experts *b, int top_k, int shared_inter, int tokens);
+MoeBatchWork moe_batch_carve(uint8_t *base, const k2t_experts *b, int top_k, int shared_inter, int tokens);
+void launch_moe_ffn_batch(k2t_ctx *ctx, const MoeLayer &L, float *hidden, int ntok, const float *post_norm, float eps,
+                          const MoeBatchWork &ws, int *err);
+
 }  // namespace k2t

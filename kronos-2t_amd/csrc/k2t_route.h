@@ -265,6 +265,60 @@ __device__ __forceinline__ void route_logit_half(const float *__restrict__ x, co
     }
 }
 
+// route_logit_half for `n` tokens (rows of x, d apart; parts pstride words apart): the unit's
+// row half and norm weights are read once, the next token's values while one is summed; the
+// same sums in the same order.
+__device__ __forceinline__ void route_logit_half_batch(const float *__restrict__ x, int n, const float *__restrict__ nw,
+                                                       int d, const float *__restrict__ W, int u, uint32_t lane,
+                                                       int E, unsigned long long *__restrict__ parts, size_t pstride) {
+    constexpr int NJ = 4;
+    const int e = u >> 1, h = u & 1;
+    const int nh = d / 8;  // float4 per half
+    const float4 *w4 = reinterpret_cast<const float4 *>(nw) + h * nh;
+    const float4 *r4 = reinterpret_cast<const float4 *>(W + (size_t)e * d) + h * nh;
+    const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 wv[NJ], rv[NJ], nx[NJ];
+    auto load = [&](int t) {
+        const float4 *x4 = reinterpret_cast<const float4 *>(x + (size_t)t * d) + h * nh;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) nx[j] = x4[min((int)lane + 64 * j, nh - 1)];
+    };
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const int i = min((int)lane + 64 * j, nh - 1);
+        wv[j] = w4[i];
+        rv[j] = r4[i];
+    }
+    load(0);
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+        if ((int)lane + 64 * j >= nh) wv[j] = rv[j] = zero4;
+    for (int t = 0; t < n; t++) {
+        float4 xv[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; j++) xv[j] = (int)lane + 64 * j < nh ? nx[j] : zero4;
+        load(min(t + 1, n - 1));
+        float ss = 0.0f, acc = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            ss = fmaf(xv[j].x, xv[j].x, ss);
+            ss = fmaf(xv[j].y, xv[j].y, ss);
+            ss = fmaf(xv[j].z, xv[j].z, ss);
+            ss = fmaf(xv[j].w, xv[j].w, ss);
+            acc = fmaf(xv[j].x * wv[j].x, rv[j].x, acc);
+            acc = fmaf(xv[j].y * wv[j].y, rv[j].y, acc);
+            acc = fmaf(xv[j].z * wv[j].z, rv[j].z, acc);
+            acc = fmaf(xv[j].w * wv[j].w, rv[j].w, acc);
+        }
+        acc = wave_sum_f(acc);
+        if (e == 0) ss = wave_sum_f(ss);
+        if (lane == 0) {
+            word_store(parts + t * pstride + u, __float_as_uint(acc), 1u);
+            if (e == 0) word_store(parts + t * pstride + 2 * E + h, __float_as_uint(ss), 1u);
+        }
+    }
+}
+
 // Bounded wait for a word of this epoch (on timeout raises *err and returns 0).
 __device__ __forceinline__ float await_word(const unsigned long long *__restrict__ p, unsigned long long w,
                                             uint32_t epoch, uint32_t spin_limit, int *__restrict__ err, bool &ok) {

@@ -150,3 +150,49 @@ def test_small_batch_gemv_equals_one_token(gpu_ctx, fmt, rows, cols, ntok):
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
     assert np.all(a[:, s1 * 16:] == 7.0) and np.all(a[:, :s0 * 16] == 7.0)
     m.close()
+
+
+# all experts used by every token (items of 16 and a remainder), and few tokens over many
+# experts; the wide router (d > 2048); a shared expert; more tokens than one MoE call takes
+@pytest.mark.parametrize("bits,E,k,d,ntok,max_batch,shared", [(3, 4, 4, 256, 40, 64, False), (4, 16, 3, 256, 2, 8, False),
+                                                              (3, 32, 6, 256, 15, 15, True), (4, 8, 2, 2112, 9, 16, False),
+                                                              (3, 4, 2, 256, 37, 8, True)])
+def test_moe_prompt_equals_token_by_token(gpu_ctx, bits, E, k, d, ntok, max_batch, shared):
+    """A prompt through sparse-MoE layers (tokens grouped by expert) gives the logits of
+    decoding its tokens one by one, bit for bit.  (Three-chunk scale groups and the NF4 KV
+    cache keep the attention half on kernels with that property at any batch size; a shared
+    expert's matrices likewise.)"""
+    from k2tb_writer import random_moe_layer, write_k2tm
+    from model_oracle import quantize_matrix
+    cfg = dict(n_layers=2, hidden=d, n_heads=4, n_kv_heads=2, head_dim=64, intermediate=64, vocab=300, max_seq=64,
+               rms_eps=1e-6, rope_theta=10000.0)
+    rng = np.random.default_rng(E * 100 + ntok)
+    dff, hd = 192, 64
+    w = lambda r, c: (rng.standard_normal((r, c)) * 0.02).astype(np.float32)  # noqa: E731
+    moe = [random_moe_layer(rng, d, dff, E, bits=bits) for _ in range(2)]
+    bank = k2t.ExpertBank.upload(gpu_ctx, write_k2tm([m[0] for m in moe], d, dff, bits, 2))
+    m = k2t.Model(gpu_ctx, cfg, max_batch=max_batch)
+    mats = []
+
+    def up(rows, cols):
+        q = quantize_matrix(w(rows, cols), "nf4", sgc=3)
+        mats.append(gpu_ctx.upload_nf(rows, cols, 4, 3, q.cb, q.pair, q.tail))
+        return mats[-1]
+
+    for i in range(2):
+        m.set_layer(i, up((4 + 4) * hd, d), up(d, 4 * hd), None, None, 1 + w(1, d)[0], 1 + w(1, d)[0])
+        m.set_moe(i, bank, i, moe[i][1], k, True, i, router_bias=w(1, E)[0] if i else None)
+        if shared:
+            m.set_moe_shared(i, up(2 * 128, d), up(d, 128), w(1, d)[0] if i else None)
+    m.set_head(up(300, d), np.ones(d, np.float32))
+    m.set_kv_bits(4)
+    toks = rng.integers(0, 300, ntok).astype(np.int32)
+    a = m.prefill(toks)
+    m.reset()
+    for t in toks:
+        b = m.decode(int(t))
+    assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    m.close()
+    for x in mats:
+        x.close()
+    bank.close()
