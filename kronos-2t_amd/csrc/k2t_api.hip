@@ -254,7 +254,7 @@ void k2t_ctx_destroy(k2t_ctx *ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->scratch) (void)hipFree(ctx->scratch);
-    if (ctx->gqa_words) (void)hipFree(ctx->gqa_words);
+    if (ctx->span_words) (void)hipFree(ctx->span_words);
     if (ctx->signs) (void)hipFree(ctx->signs);
     delete ctx;
 }
@@ -271,7 +271,7 @@ int32_t k2t_ctx_sync(k2t_ctx *ctx) {
         arg_check(ctx != nullptr, "ctx is NULL");
         hip_check(hipSetDevice(ctx->device), "hipSetDevice");
         hip_check(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-        check_gqa_timeout(ctx);
+        check_span_timeout(ctx);
     });
 }
 

@@ -29,10 +29,9 @@ void launch_attention_exact(hipStream_t st, const float *q, int q_stride, const 
 void launch_attention(hipStream_t st, const float *q, int q_stride, int8_t *kq, int8_t *vq, float *ks, float *vs,
                       const AttnPost &post, const int *pos_dev, int layer, int nq, int nkv, int hd, KvRing kr,
                       float attn_scale, int nsplit, int ntok, float *part, float *out_f, int8_t *aq, float *as,
-                      int32_t *asum, const GqaWork &gqa, int ctx_bound = 0, ActTiles tiles = ActTiles{},
+                      int32_t *asum, const SpanWork &span, int ctx_bound = 0, ActTiles tiles = ActTiles{},
                       bool mfma = false);
 int attn_max_splits(int max_seq);
-int gqa_spans(int cap);
 void launch_embed(hipStream_t st, const k2t_mat *m, const int *tokens, int ntok, float *out);
 void launch_kv_synthetic(hipStream_t st, int8_t *kq, int8_t *vq, float *ks, float *vs, int layers_kv, int cap,
                          int n_pos, int hd, int bits, uint64_t seed);
@@ -103,15 +102,15 @@ void launch_argmax(hipStream_t st, const float *x, int n, int *out_idx) {
 
 // Device scratch of k2t_attn_decode_noalloc: the span partials (n_heads * splits *
 // (head_dim + 2) floats) and the position word in the first kNoAllocScratchFloats floats;
-// then the grouped-query kernel's span words (kNoAllocGqaWords 64-bit {payload, epoch}
+// then the span attention kernel's words (kNoAllocSpanWords 64-bit {payload, epoch}
 // words), its counters {epoch, merges done} and its timeout word.  Device memory starts
 // zeroed, and the words' epochs only grow, so nothing here is ever cleared (but after a
 // timeout).  One copy per GPU, held until the process ends.  Host code never passes this
 // name to a kernel or a copy: it is a host-side stand-in there; noalloc_scratch() looks up
 // each device's own address.
 constexpr size_t kNoAllocScratchFloats = (size_t)1 << 20;  // 4 MiB
-constexpr size_t kNoAllocGqaWords = (size_t)1 << 19;       // 4 MiB
-constexpr size_t kNoAllocTotalFloats = kNoAllocScratchFloats + 2 * (kNoAllocGqaWords + 2);
+constexpr size_t kNoAllocSpanWords = (size_t)1 << 19;       // 4 MiB
+constexpr size_t kNoAllocTotalFloats = kNoAllocScratchFloats + 2 * (kNoAllocSpanWords + 2);
 static __device__ __align__(256) float scratch[kNoAllocTotalFloats];
 
 namespace k2t {
@@ -139,56 +138,56 @@ float *noalloc_scratch(int device) {
     }
     return g_noalloc_ptr[device];
 }
-// The grouped-query words, counters and timeout word of one scratch region.
-GqaWork gqa_work_at(unsigned long long *words, size_t cap) {
-    return GqaWork{words, reinterpret_cast<unsigned int *>(words + cap), reinterpret_cast<int *>(words + cap + 1)};
+// The span words, counters and timeout word of one scratch region.
+SpanWork span_work_at(unsigned long long *words, size_t cap) {
+    return SpanWork{words, reinterpret_cast<unsigned int *>(words + cap), reinterpret_cast<int *>(words + cap + 1)};
 }
 
-GqaWork noalloc_gqa(int device) {
+SpanWork noalloc_span(int device) {
     float *base = noalloc_scratch(device);
-    return gqa_work_at(reinterpret_cast<unsigned long long *>(base + kNoAllocScratchFloats), kNoAllocGqaWords);
+    return span_work_at(reinterpret_cast<unsigned long long *>(base + kNoAllocScratchFloats), kNoAllocSpanWords);
 }
 
-// k2t_attn_decode's grouped-query workspace on the context (zeroed whenever it grows).
-GqaWork ctx_gqa(k2t_ctx *ctx, size_t words) {
-    if (words > ctx->gqa_cap) {
-        hip_check(hipStreamSynchronize(ctx->stream), "gqa workspace sync");
-        if (ctx->gqa_words) hip_check(hipFree(ctx->gqa_words), "hipFree");
-        ctx->gqa_words = nullptr;
-        ctx->gqa_cap = 0;
+// k2t_attn_decode's span workspace on the context (zeroed whenever it grows).
+SpanWork ctx_span(k2t_ctx *ctx, size_t words) {
+    if (words > ctx->span_cap) {
+        hip_check(hipStreamSynchronize(ctx->stream), "span workspace sync");
+        if (ctx->span_words) hip_check(hipFree(ctx->span_words), "hipFree");
+        ctx->span_words = nullptr;
+        ctx->span_cap = 0;
         const size_t bytes = (words + 2) * sizeof(unsigned long long);
-        hipError_t e = hipMalloc((void **)&ctx->gqa_words, bytes);
+        hipError_t e = hipMalloc((void **)&ctx->span_words, bytes);
         if (e != hipSuccess) {
             (void)hipGetLastError();
             throw Error(K2T_E_NOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));
         }
-        hip_check(hipMemset(ctx->gqa_words, 0, bytes), "gqa workspace clear");
-        ctx->gqa_cap = words;
+        hip_check(hipMemset(ctx->span_words, 0, bytes), "span workspace clear");
+        ctx->span_cap = words;
     }
-    return gqa_work_at(ctx->gqa_words, ctx->gqa_cap);
+    return span_work_at(ctx->span_words, ctx->span_cap);
 }
 
 // Reads a region's timeout word after a sync; on a timeout clears the region (its epochs
 // start over) and raises.
-void raise_gqa_timeout(const GqaWork &g, size_t cap) {
+void raise_span_timeout(const SpanWork &g, size_t cap) {
     int e = 0;
-    hip_check(hipMemcpy(&e, g.err, sizeof(int), hipMemcpyDeviceToHost), "gqa timeout word");
+    hip_check(hipMemcpy(&e, g.err, sizeof(int), hipMemcpyDeviceToHost), "span timeout word");
     if (!e) return;
-    hip_check(hipMemset(g.words, 0, (cap + 2) * sizeof(unsigned long long)), "gqa workspace clear");
-    throw Error(K2T_E_HIP, "grouped-query attention: span wait timed out");
+    hip_check(hipMemset(g.words, 0, (cap + 2) * sizeof(unsigned long long)), "span workspace clear");
+    throw Error(K2T_E_HIP, "span attention: span wait timed out");
 }
 
 }  // namespace
 
 namespace k2t {
-void check_gqa_timeout(k2t_ctx *ctx) {
-    if (ctx->gqa_words) raise_gqa_timeout(gqa_work_at(ctx->gqa_words, ctx->gqa_cap), ctx->gqa_cap);
+void check_span_timeout(k2t_ctx *ctx) {
+    if (ctx->span_words) raise_span_timeout(span_work_at(ctx->span_words, ctx->span_cap), ctx->span_cap);
     bool seen = false;
     {
         std::lock_guard<std::mutex> lock(g_noalloc_mu);
         seen = ctx->device >= 0 && ctx->device < kMaxNoAllocDevices && g_noalloc_ptr[ctx->device] != nullptr;
     }
-    if (seen) raise_gqa_timeout(noalloc_gqa(ctx->device), kNoAllocGqaWords);
+    if (seen) raise_span_timeout(noalloc_span(ctx->device), kNoAllocSpanWords);
 }
 }  // namespace k2t
 
@@ -223,7 +222,7 @@ struct k2t_model {
     int *tokens = nullptr;
     int max_batch = 0;
     float *hidden = nullptr, *qkv = nullptr, *gu = nullptr, *logits = nullptr, *attn_part = nullptr;
-    unsigned long long *attn_words = nullptr;  // grouped-query attention span words
+    unsigned long long *attn_words = nullptr;  // span attention words
     unsigned int *attn_cnt = nullptr;          // {its epoch, merge workgroups done}
     int8_t *xq = nullptr;
     float *xs = nullptr;
@@ -429,7 +428,7 @@ void forward(k2t_model *m, int ntok, bool with_logits, int ctx_bound = 0) {
         const ActTiles to = act_tiles_for(m, L.o, ntok);  // (none for one token: the grouped kernel writes none)
         launch_attention(st, m->qkv, (nq + 2 * nkv) * hd, m->kq, m->vq, m->ks, m->vs, post, m->pos_dev, l, nq, nkv,
                          hd, m->ring, attn_scale, nsplit, ntok, m->attn_part, nullptr, m->xq, m->xs, m->xsum,
-                         GqaWork{m->attn_words, m->attn_cnt, m->err_dev}, ctx_bound, to, ctx->mfma != 0);
+                         SpanWork{m->attn_words, m->attn_cnt, m->err_dev}, ctx_bound, to, ctx->mfma != 0);
         launch_gemv_ex(ctx, L.o, m->xq, m->xs, m->xsum, ntok, m->hidden, d, true, 0, to);
         if (L.has_moe) {
             // each token has its own routes (forward_layer_single); a batch groups its tokens
@@ -671,14 +670,13 @@ void check_mk_error(k2t_model *m) {
     hip_check(hipMemcpy(&e, m->err_dev, sizeof(int), hipMemcpyDeviceToHost), "error flag");
     if (e) {
         (void)hipMemset(m->err_dev, 0, sizeof(int));
-        // a timed-out wait leaves the grouped-query attention's counters and words
+        // a timed-out wait leaves the span attention's counters and words
         // inconsistent: start its epochs over
         (void)hipMemset(m->attn_cnt, 0, 2 * sizeof(unsigned int));
         (void)hipMemset(m->attn_words, 0,
-                        (size_t)gqa_spans(m->cfg.max_seq) * m->cfg.n_heads * (2 + m->cfg.head_dim) *
-                            sizeof(unsigned long long));
+                        attn_span_words(m->cfg.max_seq, m->cfg.n_heads, m->cfg.head_dim) * sizeof(unsigned long long));
         throw Error(K2T_E_INTERNAL, e == 2   ? "MoE route selection: router wait timed out"
-                                    : e == 3 ? "grouped-query attention: span wait timed out"
+                                    : e == 3 ? "span attention: span wait timed out"
                                              : "persistent decode kernel: dependency wait timed out");
     }
 }
@@ -768,9 +766,9 @@ int32_t k2t_model_create(k2t_ctx *ctx, const k2t_model_config *cfg, int32_t max_
             m->logits = (float *)dalloc(m, (size_t)c.vocab * sizeof(float));
             m->attn_part = (float *)dalloc(
                 m, (size_t)max_batch * c.n_heads * attn_max_splits(c.max_seq) * (2 + c.head_dim) * sizeof(float));
-            // grouped-query attention: span words (one token) and the epoch / done counters,
+            // span attention: its words (one token) and the epoch / done counters,
             // zeroed once (epochs only grow, so no launch clears them)
-            const size_t gw = (size_t)gqa_spans(c.max_seq) * c.n_heads * (2 + c.head_dim);
+            const size_t gw = attn_span_words(c.max_seq, c.n_heads, c.head_dim);
             m->attn_words = (unsigned long long *)dalloc(m, gw * sizeof(unsigned long long));
             hip_check(hipMemset(m->attn_words, 0, gw * sizeof(unsigned long long)), "span words clear");
             m->attn_cnt = (unsigned int *)dalloc(m, 2 * sizeof(unsigned int));
@@ -1279,29 +1277,35 @@ void attn_decode_impl(k2t_ctx *ctx, int32_t bits, const float *d_q, int32_t n_he
     const int act = window > 0 ? std::min(seq, window) : seq;
     const int nsplit = attn_max_splits(act);
     hip_check(hipSetDevice(ctx->device), "hipSetDevice");
-    // grouped queries at long context: the model's grouped-query kernel (each K / V tile
-    // read once for the G q heads of its KV head), with span words that persist across
-    // calls (context workspace, or the fixed no-alloc region)
-    GqaWork gq{};
-    if (gqa_eligible(nsplit, 1, n_heads, n_kv_heads, head_dim, kr)) {
-        const size_t words = gqa_words(cap, n_heads, head_dim, 1);
-        if (noalloc) {
-            if (words > kNoAllocGqaWords)
-                throw Error(K2T_E_ARG, "k2t_attn_decode_noalloc: ceil(cap / 128) * n_heads * (head_dim + 2) = " +
-                                           std::to_string(words) + " span words exceeds its fixed scratch region of " +
-                                           std::to_string(kNoAllocGqaWords));
-            gq = noalloc_gqa(ctx->device);
-        } else {
-            gq = ctx_gqa(ctx, words);
-        }
-    }
     const size_t part = (size_t)n_heads * nsplit * (2 + head_dim);
+    if (noalloc && part + 64 > kNoAllocScratchFloats)
+        throw Error(K2T_E_ARG, "k2t_attn_decode_noalloc: n_heads * ceil(positions / 256) * (head_dim + 2) = " +
+                                   std::to_string(part) + " floats exceeds its fixed scratch of " +
+                                   std::to_string(kNoAllocScratchFloats - 64) + " floats");
+    // Grouped queries over a long int8 cache: the no-alloc region is sized for the whole cache.
+    const int group = n_heads / n_kv_heads;
+    if (noalloc && nsplit > 1 && group >= 2 && group <= 8 && bits == 8 && window <= 0) {
+        const size_t words = attn_span_words(cap, n_heads, head_dim);
+        if (words > kNoAllocSpanWords)
+            throw Error(K2T_E_ARG, "k2t_attn_decode_noalloc: ceil(cap / 128) * n_heads * (head_dim + 2) = " +
+                                       std::to_string(words) + " span words exceeds its fixed scratch region of " +
+                                       std::to_string(kNoAllocSpanWords));
+    }
+    // One launch over spans of the cache, whose words persist across calls (context
+    // workspace, or the fixed no-alloc region); the position goes with the launch.
+    const size_t words = attn_span_words(act, n_heads, head_dim);
+    if (attn_span_supported(n_heads, n_kv_heads, head_dim, kr) && (!noalloc || words <= kNoAllocSpanWords)) {
+        const SpanWork sw = noalloc ? noalloc_span(ctx->device) : ctx_span(ctx, words);
+        launch_attn_span(ctx->stream, d_q, (int8_t *)d_kq, (int8_t *)d_vq, (float *)d_ks, (float *)d_vs, AttnPost{}, nullptr,
+                         seq - 1, 0, n_heads, n_kv_heads, head_dim, kr, attn_scale, act, d_out, nullptr, nullptr, nullptr,
+                         sw);
+        if (!noalloc) hip_check(hipStreamSynchronize(ctx->stream), "sync");
+        return;
+    }
+    // More than 8 q heads per KV head, or more spans than the no-alloc region holds: split
+    // partials and a merge.
     float *pp;
     if (noalloc) {
-        if (part + 64 > kNoAllocScratchFloats)
-            throw Error(K2T_E_ARG, "k2t_attn_decode_noalloc: n_heads * ceil(positions / 256) * (head_dim + 2) = " +
-                                       std::to_string(part) + " floats exceeds its fixed scratch of " +
-                                       std::to_string(kNoAllocScratchFloats - 64) + " floats");
         pp = noalloc_scratch(ctx->device);
     } else {
         ensure_scratch(ctx, part + 64);
@@ -1318,7 +1322,7 @@ void attn_decode_impl(k2t_ctx *ctx, int32_t bits, const float *d_q, int32_t n_he
     // read-only on the cache (no post stage: the caller's queries are final)
     launch_attention(ctx->stream, d_q, n_heads * head_dim, (int8_t *)d_kq, (int8_t *)d_vq, (float *)d_ks,
                      (float *)d_vs, AttnPost{}, pos, 0, n_heads, n_kv_heads, head_dim, kr, attn_scale, nsplit, 1, pp,
-                     d_out, nullptr, nullptr, nullptr, gq);
+                     d_out, nullptr, nullptr, nullptr, SpanWork{});
     // the copied position lives on this function's stack; the no-alloc variant stores it
     // with a kernel and stays asynchronous
     if (!noalloc) hip_check(hipStreamSynchronize(ctx->stream), "sync");

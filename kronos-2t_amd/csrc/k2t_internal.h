@@ -19,10 +19,10 @@ struct k2t_ctx {
     // small device scratch (debug entry points): grown on demand
     float *scratch = nullptr;
     size_t scratch_cap = 0;  // floats
-    // grouped-query attention span words of k2t_attn_decode ({payload, epoch}, zeroed when
+    // span attention words of k2t_attn_decode ({payload, epoch}, zeroed when
     // allocated), then its counters {epoch, merges done} and timeout word
-    unsigned long long *gqa_words = nullptr;
-    size_t gqa_cap = 0;  // words
+    unsigned long long *span_words = nullptr;
+    size_t span_cap = 0;  // words
     // Hadamard sign masks of 64-blocks 0..kSignBlocks-1 (bit i = sign of element i),
     // uploaded at creation for the GEMV's fused activation builder.
     uint64_t *signs = nullptr;
@@ -196,13 +196,13 @@ struct QkvPostDev {
 bool launch_gemm_mfma_qkv(k2t_ctx *ctx, const k2t_mat *qkv, ActTiles tiles, int ntok, float *out, size_t out_stride,
                           const QkvPostDev &qp);
 
-// Workspace of the grouped-query decode attention kernel: the span words
+// Workspace of the span attention kernel (k2t_attn_span.hip): the span words
 // ([q head][span][2 + hd] {payload, epoch}, zeroed once) and two counters {epoch of the
 // last launch, merge workgroups done} (zeroed once); err receives 3 on a wait timeout.
-struct GqaWork {
-    unsigned long long *words;
-    unsigned int *cnt;
-    int *err;
+struct SpanWork {
+    unsigned long long *words = nullptr;
+    unsigned int *cnt = nullptr;
+    int *err = nullptr;
 };
 
 // One-token decode attention that also does qkv_post's work (bias, QK-norm, RoPE, K/V
@@ -213,11 +213,17 @@ struct AttnPost {
     float eps;
 };
 
-bool gqa_eligible(int nsplit, int ntok, int nq, int nkv, int hd, const KvRing &kr);
-size_t gqa_words(int cap, int nq, int hd, int ntok);
-// Raises (and clears) a grouped-query attention wait timeout that a k2t_attn_decode call
+// Decode attention of one token in one launch over spans of the cache: up to 8 q heads per
+// KV head, head size 64 or 128.  The position is *pos_dev, or pos where pos_dev is NULL; no
+// more than max_positions are attended.  attn_span_words: the span words it needs.
+bool attn_span_supported(int nq, int nkv, int hd, const KvRing &kr);
+size_t attn_span_words(int positions, int nq, int hd);
+void launch_attn_span(hipStream_t st, const float *q, int8_t *kq, int8_t *vq, float *ks, float *vs, const AttnPost &post,
+                      const int *pos_dev, int pos, int layer, int nq, int nkv, int hd, KvRing kr, float attn_scale,
+                      int max_positions, float *out_f, int8_t *aq, float *as, int32_t *asum, const SpanWork &w);
+// Raises (and clears) a span attention wait timeout that a k2t_attn_decode call
 // on this context left in its span-word workspace; called after a stream sync.
-void check_gqa_timeout(k2t_ctx *ctx);
+void check_span_timeout(k2t_ctx *ctx);
 
 // The model takes ownership of `mat` (destroyed with the model).
 void model_adopt(k2t_model *m, k2t_mat *mat);

@@ -769,582 +769,10 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(const float *__restrict_
                               out_f, aq, as, asum, tiles);
 }
 
-// Long-context decode attention for grouped queries (int8 KV, no window), one launch.
-// Span workgroups, one per (KV head, span of kGqaSpan positions, token), score all
-// G = nq / nkv q heads of the group, so each K / V tile is read from memory once instead
-// of once per q head.  The tile is copied into LDS by direct-to-LDS loads issued first;
-// meanwhile each wave applies bias / QK-norm / RoPE and the Hadamard int8 quantization to
-// one q head (and, in the span holding the current position, waves 0 and 1 build that
-// position's K / V and store them in the cache).  Per head: s_t = float(q8 . k8_t) * ks_t *
-// (qs * scale) as causal_gqa_group_q8 (real_llm.rs:8471-8594), the span's maximum m and
-// sum of exp(s_t - m), and o = sum_t (exp(s_t - m) * vs_t) * v8_t, each V element
-// converted once for all G heads.  A span workgroup publishes its partials as
-// {payload, epoch} words (one agent-scope atomic store each).  Merge workgroups, one per
-// (KV head, q head, token), come first in dispatch order and poll (bounded) the words of
-// their head's spans until every one carries this launch's epoch, then combine the spans
-// (global maximum, exp-weighted sums in span order), apply ifwht64 (real_llm.rs:8588-8592),
-// and write the o_proj activation (populate_chunk_fwht_raw(None), real_llm.rs:7060-7084).
-// The epoch is one more than the last launch's; the last merge workgroup to finish
-// advances it, so the words never need clearing.
-#ifndef K2T_GQA_SPAN
-#define K2T_GQA_SPAN 128
-#endif
-constexpr int kGqaSpan = K2T_GQA_SPAN;  // 64 or 128
-constexpr int kGqaThreads = 512;
-constexpr int kGqaMaxGroup = 8;
-// q heads per span workgroup (8, or 4 in a measurement build): a group of more q heads
-// than this is split over ceil(G / heads) span workgroups of each span, which read the
-// same K / V tile.  Splitting config 5's 8 heads over two workgroups of 4 measured slower
-// (417.5 -> 391.7 tok/s: twice the span workgroups and tile reads for half the work each).
-#ifndef K2T_GQA_HEADS
-#define K2T_GQA_HEADS 8
-#endif
-constexpr int kGqaHeads = K2T_GQA_HEADS;
-// Scores and o sums on the matrix cores (needs one 16-position tile per wave: 128-position
-// spans, 8 waves); 0 in a measurement build keeps the dot-product form.
-#ifndef K2T_GQA_MFMA
-#define K2T_GQA_MFMA 1
-#endif
-constexpr bool kGqaMfma = K2T_GQA_MFMA != 0 && kGqaSpan == 16 * (kGqaThreads / 64);
-
-#ifdef K2T_GQA_TRACE
-// Measurement builds only: wall-clock stamps of layer 0's workgroups, 8 per (KV head, row).
-__device__ unsigned long long g_gqa_trace[8 * 128 * 8];
-#define GQA_TR(k)                                                                                  \
-    do {                                                                                           \
-        if (layer == 0 && threadIdx.x == 0 && blockIdx.y < 128 && blockIdx.x < 8)                 \
-            g_gqa_trace[((size_t)blockIdx.x * 128 + blockIdx.y) * 8 + (k)] = wall_clock64();       \
-    } while (0)
-#else
-#define GQA_TR(k) \
-    do {          \
-    } while (0)
-#endif
-
-struct GqaArgs {
-    const float *q;
-    int q_stride;
-    int8_t *kq, *vq;
-    float *ks, *vs;
-    const int *pos_dev;
-    int layer, nq, nkv;
-    KvRing kr;
-    float attn_scale;
-    int nspan;
-    int hsplit;  // span workgroups per span (each scores SH of the group's q heads)
-    AttnPost post;
-    unsigned long long *words;  // [token][q head][nspan][2 + hd] {payload, epoch} span words
-    unsigned int *cnt;          // {epoch of the last launch, merge workgroups done}
-    int *err;
-    unsigned int spin_limit;
-    float *out_f;
-    int8_t *aq;
-    float *as;
-    int32_t *asum;
-};
-
-// SH: q heads per span workgroup (the group's G heads are split over ceil(G / SH) span
-// workgroups of each span, which read the same K / V tile).
-// MF: steps 3-5 on the matrix cores (see below).
-template <int HD, int SH, bool MF>
-__global__ __launch_bounds__(kGqaThreads) void attn_gqa_kernel(GqaArgs A) {
-    constexpr int P = kGqaSpan, NTH = kGqaThreads, GM = SH;
-    constexpr int PW = P / 64, HW = NTH / 64 / PW;  // waves per 64 positions, heads per pass
-    static_assert(P % 64 == 0 && GM % HW == 0 && GM <= kGqaMaxGroup, "span shape");
-    // K and V tiles [position][hd] (the first half); after the o sums the whole array holds
-    // the position subsets' partial sums
-    constexpr int kTiles = 2 * P * 128 > NTH * 4 * GM * 4 ? 2 * P * 128 : NTH * 4 * GM * 4;
-    __shared__ __align__(16) int8_t tiles[kTiles];
-    __shared__ float kst[P], vst[P];
-    __shared__ __align__(16) int8_t qi[GM * 128];
-    __shared__ float qas[GM];
-    __shared__ __align__(16) float sc[P * GM];  // exp(s_t - m) * vs_t per (position, head)
-    __shared__ float red_m[GM][MF ? NTH / 64 : PW], red_l[GM][MF ? NTH / 64 : PW];
-    __shared__ __align__(16) int8_t kcur[128], vcur[128];
-    __shared__ float cur_s[2];
-    const int layer = A.layer, nq = A.nq, nkv = A.nkv;
-    constexpr int hd = HD;
-    const int G = nq / nkv;
-    constexpr int nb = HD / 64;
-    const int kvh = blockIdx.x, tok = blockIdx.z;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6;
-    GQA_TR(0);
-    const int seq = A.pos_dev[0] + tok + 1;
-    const int nact = (seq + P - 1) / P;
-    // this launch's epoch: one more than the last launch's (advanced by its last merge
-    // workgroup, after every span workgroup of that launch had read it)
-    const uint32_t ep = __hip_atomic_load(A.cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-    const size_t pstride = (size_t)A.nspan * (2 + hd);
-    if ((int)blockIdx.y < G) {
-        // ------------------------------------------------------------ merge workgroup
-        // thread (span subset sub, 4-column group cg): spans sub, sub + nsub, ... ascending;
-        // per span it polls the words {m, L, o[4 columns]} until they carry this epoch
-        const int head = kvh * G + (int)blockIdx.y;
-        const unsigned long long *pp = A.words + (size_t)(tok * nq + head) * pstride;
-        constexpr int ncg = HD / 4, nsub = NTH / ncg;
-        const int cg = (int)tid % ncg, sub = (int)tid / ncg;
-        constexpr int kPre = 4;  // spans per thread polled together
-        bool ok = true;
-        auto poll = [&](int s, unsigned long long (&w)[6]) {
-            // (the caller keeps s < nact)
-            const unsigned long long *ps = pp + (size_t)s * (2 + hd);
-            w[0] = ll_word_load(ps);
-            w[1] = ll_word_load(ps + 1);
-#pragma unroll
-            for (int k = 0; k < 4; k++) w[2 + k] = ll_word_load(ps + 2 + cg * 4 + k);
-        };
-        // Every slot's words are requested before any is examined (a slot past nact reads
-        // span nact - 1's and is then replaced by the empty span {-inf, 0, 0}): under a
-        // per-slot branch the compiler waited for each slot's loads before issuing the
-        // next slot's.
-        unsigned long long wv6[kPre][6];
-#pragma unroll
-        for (int j = 0; j < kPre; j++) poll(min(sub + j * nsub, nact - 1), wv6[j]);
-        uint32_t pending = 0;
-#pragma unroll
-        for (int j = 0; j < kPre; j++) {
-            const bool live = sub + j * nsub < nact;
-#pragma unroll
-            for (int k = 0; k < 6; k++) {
-                if (live && (uint32_t)(wv6[j][k] >> 32) != ep) pending |= 1u << (6 * j + k);
-                if (!live) wv6[j][k] = k == 0 ? (unsigned long long)__float_as_uint(-INFINITY) : 0ull;
-            }
-        }
-        for (uint32_t spins = 0; pending != 0 && ok; spins++) {
-            if ((spins & 31u) == 31u) {
-                if (spins > A.spin_limit) {
-                    __hip_atomic_store(A.err, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    ok = false;
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-            }
-#pragma unroll
-            for (int j = 0; j < kPre; j++) {
-                const unsigned long long *ps = pp + (size_t)(sub + j * nsub) * (2 + hd);
-#pragma unroll
-                for (int k = 0; k < 6; k++)
-                    if (pending & (1u << (6 * j + k)))
-                        wv6[j][k] = ll_word_load(ps + (k < 2 ? k : 2 + cg * 4 + (k - 2)));
-            }
-#pragma unroll
-            for (int j = 0; j < kPre; j++)
-#pragma unroll
-                for (int k = 0; k < 6; k++)
-                    if ((pending & (1u << (6 * j + k))) && (uint32_t)(wv6[j][k] >> 32) == ep)
-                        pending &= ~(1u << (6 * j + k));
-        }
-        GQA_TR(1);
-        // spans past kPre per thread (contexts above nsub * kPre * P positions): one by one
-        auto wait6 = [&](int s, unsigned long long (&w)[6]) {
-            poll(s, w);
-            for (uint32_t spins = 0; ok; spins++) {
-                bool cur = true;
-#pragma unroll
-                for (int k = 0; k < 6; k++) cur = cur && (uint32_t)(w[k] >> 32) == ep;
-                if (cur) break;
-                if (spins > A.spin_limit) {
-                    __hip_atomic_store(A.err, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    ok = false;
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-                poll(s, w);
-            }
-        };
-        auto wf = [](unsigned long long w) { return __uint_as_float((uint32_t)w); };
-        float *mred = reinterpret_cast<float *>(tiles);  // [NTH / 64] wave maxima
-        // global maximum of the span maxima
-        float M = -INFINITY;
-#pragma unroll
-        for (int j = 0; j < kPre; j++) M = fmaxf(M, wf(wv6[j][0]));
-        for (int s = sub + kPre * nsub; s < nact; s += nsub) {
-            unsigned long long w[6];
-            wait6(s, w);
-            M = fmaxf(M, wf(w[0]));
-        }
-        M = wave_max_f(M);
-        if (lane == 0) mred[wv] = M;
-        __syncthreads();
-        M = mred[0];
-        for (int w = 1; w < NTH / 64; w++) M = fmaxf(M, mred[w]);
-        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        float L = 0.0f;
-        auto add_span = [&](const unsigned long long (&w)[6]) {
-            const float e = expf(wf(w[0]) - M);
-            L = fmaf(wf(w[1]), e, L);
-            acc.x = fmaf(wf(w[2]), e, acc.x);
-            acc.y = fmaf(wf(w[3]), e, acc.y);
-            acc.z = fmaf(wf(w[4]), e, acc.z);
-            acc.w = fmaf(wf(w[5]), e, acc.w);
-        };
-#pragma unroll
-        for (int j = 0; j < kPre; j++)
-            if (sub + j * nsub < nact) add_span(wv6[j]);
-        for (int s = sub + kPre * nsub; s < nact; s += nsub) {
-            unsigned long long w[6];
-            wait6(s, w);
-            add_span(w);
-        }
-        // subsets added in order
-        float *osub = reinterpret_cast<float *>(tiles) + 64;  // [nsub][hd]
-        float *lsub = osub + nsub * hd;                      // [nsub]
-        *reinterpret_cast<float4 *>(osub + sub * hd + cg * 4) = acc;
-        if (cg == 0) lsub[sub] = L;
-        __syncthreads();
-        float *ofin = lsub + nsub;  // [hd]
-        if ((int)tid < hd) {
-            float Lt = lsub[0], o = osub[tid];
-            for (int u = 1; u < nsub; u++) {
-                Lt += lsub[u];
-                o += osub[u * hd + tid];
-            }
-            ofin[tid] = o * (1.0f / Lt);
-        }
-        __syncthreads();
-        if ((int)wv < nb) {
-            const int b = (int)wv;
-            const float o = ifwht_lane(ofin[b * 64 + lane], (uint64_t)b, lane);
-            const size_t hbase = (size_t)tok * nq * hd + (size_t)head * hd;
-            if (A.out_f) A.out_f[hbase + b * 64 + lane] = o;
-            if (A.aq) {
-                const size_t c = (size_t)head * nb + b, g = (size_t)tok * nq * nb + c;
-                quant_chunk_store(fwht_lane(o, c, lane), lane, A.aq + g * 64, A.as + g, A.asum + g);
-            }
-        }
-        // the last merge workgroup of the launch advances the epoch (every span workgroup
-        // of this launch has published, so all have read the epoch already)
-        if (tid == 0) {
-            const unsigned int total = gridDim.x * (unsigned int)G * gridDim.z;
-            if (__hip_atomic_fetch_add(A.cnt + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1u) {
-                __hip_atomic_store(A.cnt + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(A.cnt, ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-        GQA_TR(7);
-        return;
-    }
-    // ---------------------------------------------------------------- span workgroup
-    // (span, head part hs): q heads h0 .. h0 + GL - 1 of the group
-    const int span = ((int)blockIdx.y - G) / A.hsplit, hs = ((int)blockIdx.y - G) % A.hsplit;
-    const int h0 = hs * GM, GL = min(GM, G - h0);
-    const int t0 = span * P, t1 = min(seq, t0 + P), n = t1 - t0;
-    if (n <= 0 || GL <= 0) return;  // spans past the context take no part
-    const KvRing kr = A.kr;
-    const size_t base = ((size_t)layer * nkv + kvh) * kr.cap;
-    int8_t *kt = tiles, *vt = tiles + P * 128;
-    // 1. K / V rows t0 .. t0+P-1 (rows past t1 re-read row t1-1), 16 bytes per lane; the
-    //    scales by waves 0-3 (K rows 0-63, 64-127, then V)
-    {
-        constexpr int pieces = P * HD / 16, per_row = HD / 16;
-        const uint32_t mk = lds_offset(kt), mvv = lds_offset(vt);
-        for (int j = 0; j * NTH < pieces; j++) {
-            const int i = j * NTH + (int)tid;
-            const int r = min(i / per_row, n - 1), c = i % per_row;
-            const size_t off = (base + (size_t)(t0 + r)) * hd + (size_t)c * 16;
-            const uint32_t m0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(j * NTH + wv * 64) * 16);
-            lds_dma16(A.kq + off, mk + m0);
-            lds_dma16(A.vq + off, mvv + m0);
-        }
-        if ((int)wv < 2 * PW) {
-            const int row = (int)(wv % PW) * 64 + (int)lane;
-            const size_t sl = base + (size_t)(t0 + min(row, n - 1));
-            const uint32_t m0 = (uint32_t)__builtin_amdgcn_readfirstlane(
-                (int)(lds_offset((int)wv < PW ? kst : vst) + (wv % PW) * 256));
-            lds_dma4(((int)wv < PW ? A.ks : A.vs) + sl, m0);
-        }
-    }
-    // 2. q head wv (and the current position's K / V where this span holds it)
-    const AttnPost &post = A.post;
-    const int cur = seq - 1;
-    const bool covers = post.on && t0 <= cur && cur < t1;
-    if ((int)wv < GL) {
-        const int h = (int)wv, head = kvh * G + h0 + h;
-        const float *qh = A.q + (size_t)tok * A.q_stride + (size_t)head * hd;
-        float qv0, qv1;
-        if (post.on) {
-            head_post(qh, head, nq, nkv, hd, post.bias, post.qn, post.kn, post.eps, post.rope, cur, lane, qv0, qv1);
-        } else {
-            qv0 = qh[lane];
-            qv1 = nb > 1 ? qh[64 + lane] : 0.0f;
-        }
-        const float r0 = fwht_lane(qv0, 0, lane);
-        const float r1 = nb > 1 ? fwht_lane(qv1, 1, lane) : 0.0f;
-        const float mx = wave_max_f(fmaxf(fabsf(r0), fabsf(r1)));
-        int8_t *qd = qi + h * 128;
-        if (mx <= FLT_EPSILON) {
-            qd[lane] = 0;
-            if (nb > 1) qd[64 + lane] = 0;
-            if (lane == 0) qas[h] = 0.0f;
-        } else {
-            const float inv = 127.0f / mx;
-            qd[lane] = (int8_t)(int)rintf(r0 * inv);
-            if (nb > 1) qd[64 + lane] = (int8_t)(int)rintf(r1 * inv);
-            if (lane == 0) qas[h] = (mx / 127.0f) * A.attn_scale;
-        }
-    }
-    if (covers && wv < 2) {
-        const int hh = wv == 0 ? nq + kvh : nq + nkv + kvh;
-        float a0, a1;
-        head_post(A.q + (size_t)tok * A.q_stride + (size_t)hh * hd, hh, nq, nkv, hd, post.bias, post.qn, post.kn,
-                  post.eps, post.rope, cur, lane, a0, a1);
-        const float r0 = fwht_lane(a0, 0, lane);
-        const float r1 = nb > 1 ? fwht_lane(a1, 1, lane) : 0.0f;
-        kv_store_head(r0, r1, nb, lane, 8, hd, 0, wv == 0 ? kcur : vcur, cur_s + wv);
-        // (every head part builds the row for its own tile; the first stores it in the cache)
-        if (hs == 0)
-            kv_store_head(r0, r1, nb, lane, 8, hd, base + (size_t)cur, wv == 0 ? A.kq : A.vq,
-                          wv == 0 ? A.ks : A.vs);
-    }
-    GQA_TR(2);
-    wait_vmcnt<0>();  // this wave's tile copies have landed
-    __syncthreads();
-    if (covers) {  // the current position's row (its tile copy read the slot before it was written)
-        const int r = cur - t0;
-        if ((int)tid < hd) {
-            kt[r * hd + tid] = kcur[tid];
-            vt[r * hd + tid] = vcur[tid];
-        }
-        if (tid == 0) {
-            kst[r] = cur_s[0];
-            vst[r] = cur_s[1];
-        }
-        __syncthreads();
-    }
-    GQA_TR(3);
-    if constexpr (MF) {
-        // 3-5 on the matrix cores (the layout of attn_prefill_mfma_kernel with the group's q
-        // heads in place of its tokens).  Wave w takes positions 16w .. 16w + 15 of the span:
-        //  - scores: v_mfma_i32_16x16x64_i8 with A = K (lane l: position 16w + l%16) and
-        //    B = the int8 q heads (lane l: head l%16; heads past the part are zero): exact
-        //    integer dots, lane l holding positions 16w + 4(l/16) + r of head l%16;
-        //    s = (float(dot) * ks) * qas as before;
-        //  - the span's maximum and sum per head: each wave's over its positions, then the
-        //    waves' in wave order;
-        //  - o^T += V^T (p vs)^T: four v_mfma_f32_16x16x4f32 per 16 dims, the r-th over the
-        //    wave's positions 4g + r (g = 0..3), whose weights are the score tile's own
-        //    registers; the waves' partial o are added in wave order.
-        static_assert(P == 16 * (NTH / 64), "one 16-position tile per wave");
-        constexpr int NW = NTH / 64, DB = HD / 16;
-        const uint32_t li = lane & 15u, lg = lane >> 4;
-        const int pw0 = 16 * (int)wv;
-        const bool hl = (int)li < GL;
-        v4i_t acc = {0, 0, 0, 0};
-#pragma unroll
-        for (int k = 0; k < nb; k++) {
-            const int4 kv = *reinterpret_cast<const int4 *>(kt + (pw0 + (int)li) * HD + 64 * k + 16 * (int)lg);
-            const int4 qv = hl ? *reinterpret_cast<const int4 *>(qi + li * 128 + 64 * k + 16 * lg) : make_int4(0, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(v4i_t{kv.x, kv.y, kv.z, kv.w}, v4i_t{qv.x, qv.y, qv.z, qv.w}, acc,
-                                                         0, 0, 0);
-        }
-        const float qs = hl ? qas[li] : 0.0f;
-        const int pr = pw0 + 4 * (int)lg;  // this lane's first position
-        float sc4[4];
-        float tmax = -INFINITY;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            sc4[r] = hl && pr + r < n ? ((float)acc[r] * kst[pr + r]) * qs : -INFINITY;
-            tmax = fmaxf(tmax, sc4[r]);
-        }
-        tmax = fmaxf(tmax, xor_lane(tmax, 16));
-        tmax = fmaxf(tmax, xor_lane(tmax, 32));
-        if (lg == 0 && hl) red_m[li][wv] = tmax;
-        __syncthreads();
-        float m = -INFINITY;
-        if (hl) {
-            m = red_m[li][0];
-#pragma unroll
-            for (int u = 1; u < NW; u++) m = fmaxf(m, red_m[li][u]);
-        }
-        float psum = 0.0f, w[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const float pe = sc4[r] == -INFINITY ? 0.0f : expf(sc4[r] - m);
-            psum += pe;
-            w[r] = pe * vst[pr + r];
-        }
-        psum += xor_lane(psum, 16);
-        psum += xor_lane(psum, 32);
-        if (lg == 0 && hl) red_l[li][wv] = psum;
-        v4f o[DB];
-#pragma unroll
-        for (int b = 0; b < DB; b++) {
-            o[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const float a = (float)vt[(pr + r) * HD + 16 * b + (int)li];
-                o[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, w[r], o[b], 0, 0, 0);
-            }
-        }
-        // the waves' partial o [wave][head][dim] after the K / V tiles (still being read)
-        float *opw = reinterpret_cast<float *>(tiles + 2 * P * 128);
-        if (hl) {
-#pragma unroll
-            for (int b = 0; b < DB; b++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) opw[((int)wv * GM + (int)li) * HD + 16 * b + 4 * (int)lg + r] = o[b][r];
-        }
-        __syncthreads();
-        unsigned long long *pbase =
-            A.words + (size_t)(tok * nq + kvh * G + h0) * pstride + (size_t)span * (2 + hd);
-        for (int i = (int)tid; i < GL * hd; i += NTH) {
-            const int h = i / hd, c = i % hd;
-            float ov = opw[h * HD + c];
-            for (int u = 1; u < NW; u++) ov += opw[(u * GM + h) * HD + c];
-            unsigned long long *pp = pbase + (size_t)h * pstride;
-            ll_word_store(pp + 2 + c, __float_as_uint(ov), ep);
-            if (c == 0) {
-                float mm = red_m[h][0], l = red_l[h][0];
-                for (int u = 1; u < NW; u++) {
-                    mm = fmaxf(mm, red_m[h][u]);
-                    l += red_l[h][u];
-                }
-                ll_word_store(pp, __float_as_uint(mm), ep);
-                ll_word_store(pp + 1, __float_as_uint(l), ep);
-            }
-        }
-    } else {
-    // 3. scores: wave w takes position (w & 1) * 64 + lane for heads w / 2 and w / 2 + 4;
-    //    lane p reads its K row's 16-byte pieces starting at piece p (no bank conflicts)
-    const int p = (int)(wv % PW) * 64 + (int)lane;
-    const bool valid = p < n;
-    constexpr int KH = GM / HW;  // heads per wave
-    float s2[KH];
-    {
-        constexpr int npc = HD / 16;
-        uint4 kr4[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-            if (i < npc) kr4[i] = reinterpret_cast<const uint4 *>(kt + p * hd)[(i + p) & (npc - 1)];
-#pragma unroll
-        for (int k = 0; k < KH; k++) {
-            const int h = (int)(wv / PW) + HW * k;
-            s2[k] = -INFINITY;
-            if (h < GL) {
-                const uint4 *qr = reinterpret_cast<const uint4 *>(qi + h * 128);
-                int dot = 0;
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    if (i < npc) {
-                        const uint4 a = kr4[i], b = qr[(i + p) & (npc - 1)];
-                        dot = __builtin_amdgcn_sdot4((int)a.x, (int)b.x, dot, false);
-                        dot = __builtin_amdgcn_sdot4((int)a.y, (int)b.y, dot, false);
-                        dot = __builtin_amdgcn_sdot4((int)a.z, (int)b.z, dot, false);
-                        dot = __builtin_amdgcn_sdot4((int)a.w, (int)b.w, dot, false);
-                    }
-                }
-                s2[k] = valid ? ((float)dot * kst[p]) * qas[h] : -INFINITY;
-                const float m = wave_max_f(s2[k]);
-                if (lane == 0) red_m[h][wv % PW] = m;
-            }
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < KH; k++) {
-        const int h = (int)(wv / PW) + HW * k;
-        if (h < GL) {
-            float m = red_m[h][0];
-            for (int u = 1; u < PW; u++) m = fmaxf(m, red_m[h][u]);
-            const float e = valid ? expf(s2[k] - m) : 0.0f;
-            const float l = wave_sum_f(e);
-            sc[p * GM + h] = e * vst[p];
-            if (lane == 0) red_l[h][wv % PW] = l;
-        }
-    }
-    for (int i = (int)tid; i < P * GM; i += NTH)
-        if ((i & (GM - 1)) >= GL) sc[i] = 0.0f;  // heads past this part
-    __syncthreads();
-    GQA_TR(4);
-    // 4. o partials: thread (position subset sub, 4-column group cg) converts each V
-    //    element once and adds it into all heads; the subsets are added in order
-    constexpr int ncg = HD / 4, nsub = NTH / ncg, plen = P / nsub;
-    const int cg = (int)tid % ncg, sub = (int)tid / ncg;
-    float acc[GM][4];
-#pragma unroll
-    for (int h = 0; h < GM; h++) acc[h][0] = acc[h][1] = acc[h][2] = acc[h][3] = 0.0f;
-    {
-        const int ta = sub * plen, tb = min(n, ta + plen);
-        for (int t = ta; t < tb; t++) {
-            const int v = *reinterpret_cast<const int *>(vt + t * hd + cg * 4);
-            float w[GM];
-            const float4 w0 = *reinterpret_cast<const float4 *>(sc + t * GM);
-            w[0] = w0.x;
-            w[1] = w0.y;
-            w[2] = w0.z;
-            w[3] = w0.w;
-            if constexpr (GM > 4) {
-                const float4 w1 = *reinterpret_cast<const float4 *>(sc + t * GM + 4);
-                w[4] = w1.x;
-                w[5] = w1.y;
-                w[6] = w1.z;
-                w[7] = w1.w;
-            }
-            const float x0 = (float)(int8_t)(v & 0xFF), x1 = (float)(int8_t)((v >> 8) & 0xFF);
-            const float x2 = (float)(int8_t)((v >> 16) & 0xFF), x3 = (float)(int8_t)((v >> 24) & 0xFF);
-#pragma unroll
-            for (int h = 0; h < GM; h++) {
-                acc[h][0] = fmaf(w[h], x0, acc[h][0]);
-                acc[h][1] = fmaf(w[h], x1, acc[h][1]);
-                acc[h][2] = fmaf(w[h], x2, acc[h][2]);
-                acc[h][3] = fmaf(w[h], x3, acc[h][3]);
-            }
-        }
-    }
-    __syncthreads();  // the tiles are free: they take the subsets' sums [sub][head][hd]
-    float *opart = reinterpret_cast<float *>(tiles);
-#pragma unroll
-    for (int h = 0; h < GM; h++)
-        if (h < GL)
-            *reinterpret_cast<float4 *>(opart + ((size_t)sub * GL + h) * hd + cg * 4) =
-                make_float4(acc[h][0], acc[h][1], acc[h][2], acc[h][3]);
-    __syncthreads();
-    // 5. publish {m, L, o[hd]} per head as {payload, epoch} words (one agent-scope store
-    //    each: the value and its ready mark arrive together, no fence or counter)
-    unsigned long long *pbase =
-        A.words + (size_t)(tok * nq + kvh * G + h0) * pstride + (size_t)span * (2 + hd);
-    for (int i = (int)tid; i < GL * hd; i += NTH) {
-        const int h = i / hd, c = i % hd;
-        float o = opart[h * hd + c];
-        for (int u = 1; u < nsub; u++) o += opart[((size_t)u * GL + h) * hd + c];
-        unsigned long long *pp = pbase + (size_t)h * pstride;
-        ll_word_store(pp + 2 + c, __float_as_uint(o), ep);
-        if (c == 0) {
-            float m = red_m[h][0], l = red_l[h][0];
-            for (int u = 1; u < PW; u++) {
-                m = fmaxf(m, red_m[h][u]);
-                l += red_l[h][u];
-            }
-            ll_word_store(pp, __float_as_uint(m), ep);
-            ll_word_store(pp + 1, __float_as_uint(l), ep);
-        }
-    }
-    }
-    GQA_TR(5);
-}
-
-#ifdef K2T_GQA_TRACE
-extern "C" int k2t_gqa_trace_read(unsigned long long *dst) {
-    return hipMemcpyFromSymbol(dst, HIP_SYMBOL(g_gqa_trace), sizeof(g_gqa_trace)) == hipSuccess ? 0 : -1;
-}
-#endif
-
 // One split (the whole-context kernel) up to kAttnWhole positions, else 256-position spans.
 int attn_max_splits(int max_seq) {
     return max_seq <= kAttnWhole ? 1 : (max_seq + kAttnSplitLen - 1) / kAttnSplitLen;
 }
-
-// Spans of the grouped-query kernel over a cache of `cap` slots.
-int gqa_spans(int cap) { return (cap + kGqaSpan - 1) / kGqaSpan; }
-
-// Whether launch_attention runs the grouped-query kernel (given span words), and the
-// words it then needs: [token][q head][span][2 + hd].
-bool gqa_eligible(int nsplit, int ntok, int nq, int nkv, int hd, const KvRing &kr) {
-    const int group = nq / nkv;
-    return nsplit > 1 && ntok == 1 && group >= 2 && group <= kGqaMaxGroup && kr.bits == 8 && kr.window == 0 &&
-           (hd == 64 || hd == 128);
-}
-size_t gqa_words(int cap, int nq, int hd, int ntok) { return (size_t)gqa_spans(cap) * nq * (2 + hd) * ntok; }
 
 // attn_partial_kernel with or without the sliding-window ring arithmetic.
 template <int NTH, bool FINAL, int VORD, typename... Args>
@@ -1359,7 +787,7 @@ void launch_attention(hipStream_t st, const float *q, int q_stride, int8_t *kq, 
                       const AttnPost &post, const int *pos_dev, int layer, int nq, int nkv, int hd, KvRing kr,
                       float attn_scale,
                       int nsplit, int ntok, float *part, float *out_f, int8_t *aq, float *as, int32_t *asum,
-                      const GqaWork &gqa, int ctx_bound, ActTiles tiles, bool mfma) {
+                      const SpanWork &span, int ctx_bound, ActTiles tiles, bool mfma) {
     if (mfma && ntok >= 16 && !post.on && kr.bits == 8 && kr.window == 0 && kr.ring == 0 && (hd == 64 || hd == 128)) {
         const dim3 grid(nq, (ntok + 15) / 16);
         if (hd == 128)
@@ -1387,20 +815,10 @@ void launch_attention(hipStream_t st, const float *q, int q_stride, int8_t *kq, 
         hip_check(hipGetLastError(), "attention launch");
         return;
     }
-    const int group = nq / nkv;
-    if (gqa.words && ntok == 1 && group >= 2 && group <= kGqaMaxGroup && kr.bits == 8 && kr.window == 0 &&
-        (hd == 64 || hd == 128)) {
-        if (tiles.xt) throw Error(K2T_E_INTERNAL, "grouped-query attention writes no activation tiles");
-        const int hsplit = (group + kGqaHeads - 1) / kGqaHeads;
-        GqaArgs A{q,          q_stride,          kq,   vq,         ks,       vs,       pos_dev, layer,
-                  nq,         nkv,               kr,   attn_scale, gqa_spans(kr.cap), hsplit, post, gqa.words,
-                  gqa.cnt,    gqa.err,           1u << 20, out_f, aq, as, asum};
-        const dim3 grid(nkv, group + A.nspan * hsplit, ntok);
-        if (hd == 128)
-            hipLaunchKernelGGL((attn_gqa_kernel<128, kGqaHeads, kGqaMfma>), grid, dim3(kGqaThreads), 0, st, A);
-        else
-            hipLaunchKernelGGL((attn_gqa_kernel<64, kGqaHeads, kGqaMfma>), grid, dim3(kGqaThreads), 0, st, A);
-        hip_check(hipGetLastError(), "attn_gqa launch");
+    if (span.words && ntok == 1 && !tiles.xt && attn_span_supported(nq, nkv, hd, kr)) {
+        const int most = std::min(nsplit * kAttnSplitLen, kr.window > 0 ? kr.window : kr.cap);
+        launch_attn_span(st, q, kq, vq, ks, vs, post, pos_dev, 0, layer, nq, nkv, hd, kr, attn_scale, most, out_f, aq, as,
+                         asum, span);
         return;
     }
     launch_attn_partial<kAttnSplitLen, false, kAttnSplitLen>(

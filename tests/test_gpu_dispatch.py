@@ -196,3 +196,91 @@ def test_moe_prompt_equals_token_by_token(gpu_ctx, bits, E, k, d, ntok, max_batc
     for x in mats:
         x.close()
     bank.close()
+
+
+# one span (128- and 256-position form) and its edges, several spans, more spans than a merge
+# thread polls at once; 1 .. 8 q heads per KV head; windows not yet full, full and wrapped
+@pytest.mark.parametrize("nq,nkv,hd", [(3, 3, 64), (6, 2, 128), (8, 2, 64), (10, 2, 128), (8, 1, 64)])
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("seq,window,sinks", [(1, 0, 0), (127, 0, 0), (128, 0, 0), (129, 0, 0), (257, 0, 0), (1100, 0, 0),
+                                              (9000, 0, 0), (90, 100, 4), (1300, 300, 4), (2777, 1001, 0)])
+def test_span_attention_matches_reference(gpu_ctx, nq, nkv, hd, bits, seq, window, sinks):
+    """Decode attention against float64 softmax attention over the cache as stored (codes times
+    scales): 2e-5 of the largest output, about 40 ulp of fp32 for sums of up to 9000 terms."""
+    import torch
+    import oracle as O
+    rng = np.random.default_rng(nq * 1000 + seq + bits)
+    cap = window + 512 if window else seq + 3
+    heads = rng.standard_normal((2, nkv * cap, hd)).astype(np.float32)
+    q = (2 * rng.standard_normal((nq, hd))).astype(np.float32)
+    codes = [torch.empty((nkv * cap, hd if bits == 8 else hd // 2), dtype=torch.int8, device="cuda") for _ in range(2)]
+    scales = [torch.empty((nkv * cap, 1 if bits == 8 else hd // 64), device="cuda",
+                          dtype=torch.float32 if bits == 8 else torch.bfloat16) for _ in range(2)]
+    for i in range(2):
+        gpu_ctx.kv_store(bits, _t(heads[i]), nkv * cap, hd, codes[i], scales[i])
+    out = [torch.full((nq, hd), float("nan"), device="cuda") for _ in range(2)]
+    args = (bits, _t(q), nq, nkv, hd, codes[0], scales[0], codes[1], scales[1], cap, seq, hd ** -0.5)
+    gpu_ctx.attn_decode(*args, out[0], window, sinks)
+    gpu_ctx.attn_decode_noalloc(*args, out[1], window, sinks)
+    gpu_ctx.sync()
+    # the stored values
+    dense = []
+    for i in range(2):
+        c, s = codes[i].cpu().numpy(), scales[i].float().cpu().numpy().astype(np.float64)
+        if bits == 8:
+            v = c.astype(np.float64) * s
+        else:
+            cb = np.array([-127, -96, -75, -58, -44, -31, -18, -6, 6, 18, 31, 44, 58, 75, 96, 127], np.float64)
+            b = c.view(np.uint8).reshape(-1, hd // 64, 2, 1, 16)  # [block][half][nibble][16]
+            v = cb[np.concatenate([b & 15, b >> 4], axis=3)].reshape(-1, hd // 64, 64) * s[:, :, None]
+        dense.append(v.reshape(nkv, cap, hd))
+    pos = np.arange(seq)
+    if window and seq > window:
+        pos = np.concatenate([np.arange(sinks), np.arange(seq - (window - sinks), seq)])
+    if window:
+        pos = np.where(pos < sinks, pos, sinks + (pos - sinks) % (cap - sinks))
+    ref = np.zeros((nq, hd))
+    for h in range(nq):
+        qi, qs = O.kv_quant_head(q[h])
+        k, v = (d[h // (nq // nkv)][pos] for d in dense)
+        s = k @ (qi.astype(np.float64) * float(qs)) * hd ** -0.5
+        p = np.exp(s - s.max())
+        ref[h] = O.ifwht64(((p / p.sum()) @ v).astype(np.float32))
+    for o in out:
+        assert np.abs(o.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("nq,nkv,hd", [(4, 4, 64), (8, 2, 128), (8, 1, 64)])
+@pytest.mark.parametrize("bits,window", [(8, 0), (4, 0), (8, 1100), (4, 1100)])
+def test_span_attention_in_decode_steps(gpu_ctx, nq, nkv, hd, bits, window):
+    """Decode steps of a model whose cache is sized for the span kernel (more than 1024
+    positions) against the same model with a short cache (one workgroup per head): the
+    current position's K / V built and stored in the launch, one span and several."""
+    from model_oracle import random_model
+    cfg = dict(n_layers=2, hidden=256, n_heads=nq, n_kv_heads=nkv, head_dim=hd, intermediate=256, vocab=200,
+               rms_eps=1e-5, rope_theta=10000.0)
+    layers, head, fn = random_model(cfg, seed=nq + hd, fmt="nf4")
+    up = lambda m: gpu_ctx.upload_nf(m.rows, m.cols, 4, m.sgc, m.cb, m.pair, m.tail)  # noqa: E731
+    mats = [[up(L[k]) for k in ("qkv", "o", "gu", "down")] for L in layers]
+    hm = up(head)
+    logits = []
+    for max_seq, win in ((2048, window), (1000, 0)):
+        m = k2t.Model(gpu_ctx, dict(cfg, max_seq=max_seq), max_batch=300)
+        for i, L in enumerate(layers):
+            m.set_layer(i, *mats[i], L["in_norm"], L["post_norm"])
+        m.set_head(hm, fn)
+        m.set_persistent(False)
+        m.set_kv_bits(bits)
+        if win:
+            m.set_kv_window(win, 4)
+        toks = np.random.default_rng(1).integers(0, 200, 300)
+        got = [m.decode(int(t)) for t in toks[:3]]
+        m.prefill(toks[3:254].astype(np.int32), want_logits=False)
+        got += [m.decode(int(t)) for t in toks[254:260]]
+        logits.append(np.stack(got))
+        m.close()
+    a, b = logits
+    cos = (a * b).sum(1) / (np.linalg.norm(a, axis=1) * np.linalg.norm(b, axis=1))
+    assert cos.min() > 0.9998 and np.isfinite(a).all()
+    for x in [hm] + [x for r in mats for x in r]:
+        x.close()
