@@ -55,6 +55,8 @@ struct MkParams {
     const float *rope;
     int *pos_dev;      // advanced by the kernel's last step (with step_dev)
     int *tokens;       // input token; the kernel's last step writes the greedy next token
+    int token;         // >= 0: the input token itself (tokens is then only written)
+    int *next;         // where the greedy next token is written as well, or NULL
     uint32_t *step_dev;
     int8_t *kq, *vq;
     float *ks, *vs;

@@ -1052,7 +1052,7 @@ __global__ __launch_bounds__(NTH) void decode_mk_kernel(MkParams P) {
 
     // phase 0: embedding -> HA (one wave per 64-element chunk)
     {
-        const int token = P.tokens[0];
+        const int token = P.token >= 0 ? P.token : P.tokens[0];
         for (int c = (int)blockIdx.x * kWaves + wave; c < d / 64; c += (int)gridDim.x * kWaves)
         {
             float v;
@@ -1336,7 +1336,9 @@ __global__ __launch_bounds__(NTH) void decode_mk_kernel(MkParams P) {
                     bi = oi;
                 }
             }
-            P.tokens[0] = bi == 0x7fffffff ? 0 : bi;
+            const int pick = bi == 0x7fffffff ? 0 : bi;
+            P.tokens[0] = pick;
+            if (P.next) *P.next = pick;
             P.pos_dev[0] = pos + 1;
             P.step_dev[0] = step + 1u;
         }

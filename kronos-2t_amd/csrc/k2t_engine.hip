@@ -117,6 +117,12 @@ namespace k2t {
 __global__ void store_int_kernel(int *dst, int v) {
     if (threadIdx.x == 0) dst[0] = v;
 }
+
+// A host value into device memory as a launch argument (no staging buffer, graph-safe).
+static void launch_store_int(hipStream_t st, int *dst, int v) {
+    hipLaunchKernelGGL(store_int_kernel, dim3(1), dim3(64), 0, st, dst, v);
+    hip_check(hipGetLastError(), "store launch");
+}
 }  // namespace k2t
 
 using namespace k2t;
@@ -240,7 +246,10 @@ struct k2t_model {
     float *rms_x86 = nullptr;  // [max_batch] inv_rms of the exact-order steps
     float *attn_f = nullptr;   // [max_batch][n_heads * head_dim] exact-order attention output
     hipGraphExec_t graph = nullptr;
-    bool graph_pk = false;  // the captured step is the persistent kernel
+    // persistent kernel: whether it applies (-1: not yet looked at since the last change) and
+    // whether its layer table is on the device
+    mutable int mk_use = -1;
+    bool mk_table = false;
     std::vector<void *> allocs;
     // persistent single-launch decode step (fast epilogue, NF4 or 4-plane weights)
     int persistent = 1;  // 0 off, 1 single-format models, 2 also mixed 4/5-plane models
@@ -507,17 +516,23 @@ bool mk_format(const k2t_model *m, int &fmt, int &hp) {
 }
 
 bool use_persistent(const k2t_model *m) {
+    if (m->mk_use >= 0) return m->mk_use != 0;
     int fmt, hp;
     // the sliding-window ring and the NF4 KV cache run on the per-operation path
-    if (m->ring.window > 0 || m->ring.bits != 8) return false;
+    bool use = m->ring.window <= 0 && m->ring.bits == 8;
     for (const auto &L : m->layers)
-        if (L.has_moe || L.q_norm || L.k_norm) return false;  // these run on the per-operation path
-    return m->persistent && m->mk_ok && mk_format(m, fmt, hp);
+        if (L.has_moe || L.q_norm || L.k_norm) use = false;  // these run on the per-operation path
+    use = use && m->persistent && m->mk_ok && mk_format(m, fmt, hp);
+    m->mk_use = use ? 1 : 0;
+    return use;
 }
 
 // Destroys the captured decode graph after the stream has drained: a replay enqueued
 // earlier may still be reading the executable graph's kernel arguments.
+// (Called at every change of the model: the persistent kernel's state is looked at again too.)
 void drop_graph(k2t_model *m) {
+    m->mk_use = -1;
+    m->mk_table = false;
     if (!m->graph) return;
     hip_check(hipSetDevice(m->ctx->device), "hipSetDevice");
     hip_check(hipStreamSynchronize(m->stream), "sync before graph destroy");
@@ -579,8 +594,9 @@ void upload_mk_layers(k2t_model *m) {
     hip_check(hipMemcpy(m->mk_layers, h.data(), h.size() * sizeof(MkLayer), hipMemcpyHostToDevice), "layer table");
 }
 
-// One decode step as a single persistent kernel, then the position / step advance.
-void forward_mk(k2t_model *m) {
+// One decode step as a single persistent kernel, which advances the position and the step.
+// token >= 0: the input token (else the device's); next: where the greedy choice also goes.
+void forward_mk(k2t_model *m, int token, int *next) {
     const k2t_model_config &c = m->cfg;
     MkParams P{};
     P.layers = m->mk_layers;
@@ -610,6 +626,8 @@ void forward_mk(k2t_model *m) {
     P.rope = m->rope;
     P.pos_dev = m->pos_dev;
     P.tokens = m->tokens;
+    P.token = token;
+    P.next = next;
     P.step_dev = m->step_dev;
     P.kq = m->kq;
     P.vq = m->vq;
@@ -681,28 +699,35 @@ void check_mk_error(k2t_model *m) {
     }
 }
 
-// One decode step at host position m->pos (pk = persistent_at(m, m->pos)).
-void decode_step(k2t_model *m, bool pk) {
+// One decode step at host position m->pos (pk = persistent_at(m, m->pos)).  token >= 0 is
+// the input token; otherwise it is on the device already.  next (persistent kernel only)
+// also receives the greedy choice.
+// The persistent kernel is launched as it is, with the token and `next` as arguments: a
+// graph of one node saves nothing, and could not carry them (the copies they replace cost
+// a launch each: two layers of the 1.7B shape 84 -> MEASURED us a step).  The per-operation
+// step is captured once and replayed.
+void decode_step(k2t_model *m, bool pk, int token, int *next) {
     StreamSwap sw(m);
-    // the context crossed kMkMaxContext: capture the other path (an earlier step of a
-    // generate() loop may still be replaying the old graph; drop_graph waits for it)
-    if (m->graph && m->graph_pk != pk) drop_graph(m);
-    if (!m->use_graph) {
-        if (pk) {
+    if (pk) {
+        if (!m->mk_table) {
+            // an earlier step may still be reading the table
+            hip_check(hipStreamSynchronize(m->stream), "sync before the layer table changes");
             upload_mk_layers(m);
-            forward_mk(m);
-        } else {
-            forward(m, 1, true);
+            m->mk_table = true;
         }
+        forward_mk(m, token, next);
+        return;
+    }
+    if (token >= 0) launch_store_int(m->stream, m->tokens, token);
+    if (!m->use_graph) {
+        forward(m, 1, true);
         return;
     }
     if (!m->graph) {
-        if (pk) upload_mk_layers(m);
         hipGraph_t g = nullptr;
         hip_check(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal), "begin capture");
         try {
-            if (pk) forward_mk(m);
-            else forward(m, 1, true);
+            forward(m, 1, true);
         } catch (...) {
             (void)hipStreamEndCapture(m->stream, &g);
             if (g) (void)hipGraphDestroy(g);
@@ -712,7 +737,6 @@ void decode_step(k2t_model *m, bool pk) {
         hipError_t e = hipGraphInstantiate(&m->graph, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         hip_check(e, "graph instantiate");
-        m->graph_pk = pk;
     }
     hip_check(hipGraphLaunch(m->graph, m->stream), "graph launch");
 }
@@ -1126,8 +1150,7 @@ int32_t k2t_model_decode(k2t_model *m, int32_t token, float *logits_host) {
         arg(token >= 0 && token < m->cfg.vocab, "token out of range");
         arg(m->pos < m->cfg.max_seq, "context full (max_seq reached)");
         hip_check(hipSetDevice(m->ctx->device), "hipSetDevice");
-        hip_check(hipMemcpyAsync(m->tokens, &token, sizeof(int), hipMemcpyHostToDevice, m->stream), "token upload");
-        decode_step(m, persistent_at(m, m->pos));
+        decode_step(m, persistent_at(m, m->pos), token, nullptr);
         m->pos += 1;
         if (logits_host) {
             hip_check(hipMemcpyAsync(logits_host, m->logits, (size_t)m->cfg.vocab * sizeof(float),
@@ -1178,18 +1201,15 @@ int32_t k2t_model_generate(k2t_model *m, int32_t first_token, int32_t n_steps, i
         arg(first_token >= 0 && first_token < m->cfg.vocab, "token out of range");
         arg(m->pos + n_steps <= m->cfg.max_seq, "generation exceeds max_seq");
         hip_check(hipSetDevice(m->ctx->device), "hipSetDevice");
-        hip_check(hipMemcpyAsync(m->tokens, &first_token, sizeof(int), hipMemcpyHostToDevice, m->stream),
-                  "token upload");
-        std::vector<int> host;
         int *dev_out = nullptr;
         if (tokens_out && n_steps > 0) dev_out = (int *)dalloc(m, (size_t)n_steps * sizeof(int));
         for (int i = 0; i < n_steps; i++) {
             const bool pk = persistent_at(m, m->pos + i);
-            decode_step(m, pk);
             // greedy: the next input token is argmax of these logits, written on the device
             // (by the persistent kernel itself, or by argmax_kernel after the per-op step)
+            decode_step(m, pk, i == 0 ? first_token : -1, dev_out ? dev_out + i : nullptr);
             if (!pk) launch_argmax(m->stream, m->logits, m->cfg.vocab, m->tokens);
-            if (dev_out)
+            if (dev_out && !pk)
                 hip_check(hipMemcpyAsync(dev_out + i, m->tokens, sizeof(int), hipMemcpyDeviceToDevice, m->stream),
                           "token copy");
         }
@@ -1314,8 +1334,7 @@ void attn_decode_impl(k2t_ctx *ctx, int32_t bits, const float *d_q, int32_t n_he
     int *pos = reinterpret_cast<int *>(pp + part);
     const int p0 = seq - 1;
     if (noalloc) {
-        hipLaunchKernelGGL(store_int_kernel, dim3(1), dim3(64), 0, ctx->stream, pos, p0);
-        hip_check(hipGetLastError(), "position store launch");
+        launch_store_int(ctx->stream, pos, p0);
     } else {
         hip_check(hipMemcpyAsync(pos, &p0, sizeof(int), hipMemcpyHostToDevice, ctx->stream), "pos upload");
     }
