@@ -82,8 +82,8 @@ int32_t k2t_ctx_set_splitk(k2t_ctx *ctx, int32_t max_segments);
 int32_t k2t_ctx_set_exact(k2t_ctx *ctx, int32_t exact);
 /* Batched NF4, NF3 and bit-plane (b4 / b5 / b6) GEMVs (16 or more tokens of a ready activation
  * over the whole matrix, k2t_gemv and the model's prefill): enable = 1 (default) runs
- * them on the int8 matrix cores, one weight pass per 64 tokens, with outputs equal to the
- * exact-order epilogue's in either mode, and with the fast epilogue 2 .. 15 tokens in one
+ * them on the int8 matrix cores, one weight pass per 16 to 128 tokens, with outputs equal to the
+ * exact-order epilogue's in either mode (small NF3 products keep the 4-token passes), and with the fast epilogue 2 .. 15 tokens in one
  * weight pass with each token's one-token outputs; 0 runs the 4-token weight passes of the
  * reference's tiles (nf_sdot_decode_neon, simd_lut.rs:6074-6364;
  * nibble4_sdot_batch_stripe_range, 4101-4320).  2: matrix cores, but a model's prefill does not have the
@@ -169,11 +169,12 @@ int32_t k2t_act_quant_rmsnorm(k2t_ctx *ctx, const float *d_x, const float *d_nor
  * with split-K disabled the fp32 result is bit-identical to the reference's
  * in-order fmaf epilogue.  16 or more tokens over the whole matrix (NF with scale
  * groups of a power of two, or bit
- * planes, k2t_ctx_set_mfma): one weight pass per 64 tokens on the matrix
+ * planes, k2t_ctx_set_mfma): one weight pass per 16 to 128 tokens on the matrix
  * cores, outputs bit-identical to that epilogue in either mode; such a call
- * copies the activation into the context's scratch, which it grows first if it
- * is too small (a synchronous allocation, so the first such call of a size
- * must not be inside a stream capture). */
+ * copies the activation into the context's scratch (small ones read it as it is), which
+ * it grows first if it is too small (a synchronous allocation, so the first such call of a
+ * size must not be inside a stream capture; NF3, and small NF3 products always, then take the
+ * 4-token passes, which need none). */
 int32_t k2t_gemv(k2t_ctx *ctx, const k2t_mat *m, const int8_t *d_xq, const float *d_xs,
                  const int32_t *d_xsum, int32_t ntok, int32_t s0, int32_t s1, float *d_out,
                  size_t out_stride);

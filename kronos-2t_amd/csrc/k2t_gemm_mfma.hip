@@ -1,14 +1,13 @@
 // Batched quantized GEMV (prefill) on the int8 matrix cores of gfx950: out[t][r] =
-// sum_c fmaf(float(dot_{r,c,t}) * sx[t][c], ws[r][c], ...) for up to 64 tokens per weight
-// pass, the chunk dots from v_mfma_i32_16x16x64_i8.  NF4 and NF3 (NfSdotMatrix) and the bit-plane
+// sum_c fmaf(float(dot_{r,c,t}) * sx[t][c], ws[r][c], ...), the chunk dots from v_mfma_i32_16x16x64_i8.  NF4 and NF3 (NfSdotMatrix) and the bit-plane
 // formats b4 / b5 / b6 (Nibble4SdotMatrix) share the kernel (FMT 1, 2, 0).
 //
 // The reference runs prefill through the same kernels as decode, four tokens per weight
 // pass (nf_sdot_decode_neon's 4-token tile, simd_lut.rs:6074-6364, and the Nibble4 tile
-// nibble4_sdot_batch_stripe_range, 4101-4320).  Here one wave owns one 16-row stripe and 16 to 64 tokens: per 64-column
-// chunk it decodes the stripe-chunk's codes to int8 once, then runs one MFMA per 16-token
-// block (A: 16 rows x 64 codes, B: 64 activation bytes x 16 tokens), so each weight byte
-// is read once per 64 tokens instead of once per 4.
+// nibble4_sdot_batch_stripe_range, 4101-4320).  Here a 16-row stripe's codes of a 64-column
+// chunk are decoded to int8 once per up to 128 tokens, with one MFMA per 16-token block
+// (A: 16 rows x 64 codes, B: 64 activation bytes x 16 tokens).  Three kernels share that step and
+// differ in how stripes, tokens and chunks are dealt to waves (launch_plain_fmt's rule).
 //  - NF4: the codebook value of each code (the codebook as two v_perm XOR tables,
 //    nf4_xlut); the MFMA gives the chunk dot.
 //  - NF3: the same through one v_perm per four codes, from the row's triplet of dwords, in
@@ -39,6 +38,8 @@
 // group g (g*16 + 4j) holds the bits of row 4g + j for columns kk*16 .. kk*16+15, kk = 2p
 // and 2p + 1 (one hi plane) or kk = p (two), in the bit positions the decode kernels'
 // rotations select (chunk_dots in k2t_gemv_core.h).
+#include <type_traits>
+
 #include "../../include/k2t_hip.h"
 #include "k2t_device.h"
 #include "k2t_internal.h"
@@ -48,24 +49,7 @@ namespace k2t {
 
 namespace {
 
-#ifndef K2T_MFMA_DEPTH
-#define K2T_MFMA_DEPTH 4
-#endif
-#ifndef K2T_MFMA_MIN_WAVES
-#define K2T_MFMA_MIN_WAVES 2048
-#endif
-constexpr int kMfmaDepth = K2T_MFMA_DEPTH;         // chunks in flight per wave (unshared kernels)
-#ifndef K2T_MFMA_SH_DEPTH
-#define K2T_MFMA_SH_DEPTH 2
-#endif
-constexpr int kMfmaShDepth = K2T_MFMA_SH_DEPTH;    // the same, kernels sharing activation blocks
-constexpr long kMfmaMinWaves = K2T_MFMA_MIN_WAVES;  // 8 waves per CU
-#ifndef K2T_MFMA_MAX_BLOCKS
-#define K2T_MFMA_MAX_BLOCKS 4
-#endif
-// 16-token blocks per wave: 4, or 8 in a measurement build (16384 x 2048 at 256 tokens:
-// 40.0 -> 41.0 us at 188 VGPRs; 1.7B prefill unchanged)
-constexpr int kMfmaMaxBlocks = K2T_MFMA_MAX_BLOCKS;
+constexpr int kMfmaDepth = 4;  // chunks in flight per wave (gemm_mfma_kernel)
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
@@ -80,7 +64,8 @@ struct MfArgs {
     const int8_t *xt;  // activations tile-major: [16-token block][chunk][64 lanes][16 bytes]
     const float *st;   // their scales: [16-token block][chunk][16 tokens]
     const int32_t *ut;  // their code sums (bit planes): [16-token block][chunk][16 tokens]
-    int K, ntok, nblk;  // nblk: 16-token blocks in the tiles
+    int K, ntok, nblk;  // nblk: 16-token blocks
+    int tiled;          // gemm_ks_kernel: 0 = xt / st / ut are the [token] rows themselves
     float *out;
     size_t out_stride;
     int accum;
@@ -95,13 +80,13 @@ struct MfArgs {
 };
 
 // Everything one chunk needs (one ring stage): the stripe-chunk's codes and scales, the
-// activation blocks this wave loads (all NB, or with sharing its own one), their scales.
-template <int FMT, int NB, bool SH>
+// activation blocks and their scales.
+template <int FMT, int NB>
 struct MfChunk {
     uint32_t d0, d1;
     uint32_t hv;  // bit planes with hi planes: this lane's hi-plane dword; NF3: its third dword
     uint2 sw;
-    int4 x[SH ? (NB + 3) / 4 : NB];  // with sharing: blocks wave, wave + 4
+    int4 x[NB];
     float sx[NB];
     int32_t su[FMT == 0 ? NB : 1];  // bit planes: the tokens' code sums
 };
@@ -224,9 +209,9 @@ __device__ __forceinline__ void mf_record(int sgc_log2, bool is_tail, int c, uin
     }
 }
 
-template <int FMT, int HP, int NB, bool SH>
+template <int FMT, int HP, int NB>
 __device__ __forceinline__ void mf_fetch(const MfArgs &A, const MfSrc &R, const MfLane &L, bool is_tail, int tb0,
-                                         uint32_t wave, int c, MfChunk<FMT, NB, SH> &f) {
+                                         int c, MfChunk<FMT, NB> &f) {
     uint32_t rec, sgb;
     mf_record<FMT, HP>(A.sgc_log2, is_tail, c, rec, sgb);
     f.d0 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(R.w, L.a_off, rec, 0);
@@ -234,28 +219,12 @@ __device__ __forceinline__ void mf_fetch(const MfArgs &A, const MfSrc &R, const 
     if constexpr ((FMT == 0 && HP > 0) || FMT == 2) f.hv = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(R.w, L.h_off, rec, 0);
     const v2u sw = __builtin_amdgcn_raw_buffer_load_b64(R.w, L.s_off, sgb, 0);
     f.sw = make_uint2(sw[0], sw[1]);
-    if constexpr (SH) {
-        // With sharing, wave w loads blocks w, w + 4, ...  The load is unconditional (a
-        // wave past the blocks re-reads the last one and stores nothing), so the ring
-        // stage's registers hold only the new value: a conditional load kept the old one
-        // alive, which cost copies, and a wait for nearly every load, at the loop's back
-        // edge.
-#pragma unroll
-        for (int k = 0; k < (NB + 3) / 4; k++) {
-            const int b = min((int)wave + 4 * k, NB - 1);
-            const uint32_t tile = (uint32_t)min(tb0 + b, A.nblk - 1) * (uint32_t)A.nc + (uint32_t)c;
-            const v4u x = __builtin_amdgcn_raw_buffer_load_b128(R.x, L.x_off, tile * 1024u, 0);
-            f.x[k] = make_int4((int)x[0], (int)x[1], (int)x[2], (int)x[3]);
-        }
-    }
 #pragma unroll
     for (int b = 0; b < NB; b++) {
         // blocks past the last repeat it; their outputs are never stored
         const uint32_t tile = (uint32_t)min(tb0 + b, A.nblk - 1) * (uint32_t)A.nc + (uint32_t)c;
-        if constexpr (!SH) {
-            const v4u x = __builtin_amdgcn_raw_buffer_load_b128(R.x, L.x_off, tile * 1024u, 0);
-            f.x[b] = make_int4((int)x[0], (int)x[1], (int)x[2], (int)x[3]);
-        }
+        const v4u x = __builtin_amdgcn_raw_buffer_load_b128(R.x, L.x_off, tile * 1024u, 0);
+        f.x[b] = make_int4((int)x[0], (int)x[1], (int)x[2], (int)x[3]);
         f.sx[b] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(R.s, L.sx_off, tile * 64u, 0));
         if constexpr (FMT == 0) f.su[b] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(R.u, L.sx_off, tile * 64u, 0);
     }
@@ -265,25 +234,13 @@ __device__ __forceinline__ void mf_fetch(const MfArgs &A, const MfSrc &R, const 
 // needs no select: its term float(d) * 0 * ws is +-0, and adding +-0 leaves every
 // accumulator unchanged (each starts at +0 and a round-to-nearest sum is -0 only when
 // both addends are -0, so no accumulator is ever -0).
-// With sharing, `bsh` is this chunk's LDS slot ([NB][64 lanes] of 16 bytes): the waves
-// that loaded a block store it, one barrier, then every wave reads every block.  Two
-// slots alternate: a wave stores into a slot only after the barrier that all waves
-// passed once done reading it.
-template <int FMT, int HP, int NB, bool SH>
-__device__ __forceinline__ void mf_step(const MfArgs &A, const MfChunk<FMT, NB, SH> &f, float (&acc)[NB][4],
-                                        int4 *bsh, uint32_t wave, uint32_t lane) {
-    if (SH) {
-#pragma unroll
-        for (int k = 0; k < (NB + 3) / 4; k++)
-            if ((int)wave + 4 * k < NB) bsh[(wave + 4 * k) * 64 + lane] = f.x[k];
-        __syncthreads();
-    }
+template <int FMT, int HP, int NB>
+__device__ __forceinline__ void mf_step(const MfArgs &A, const MfChunk<FMT, NB> &f, float (&acc)[NB][4], uint32_t lane) {
     const v4i a = mf_decode<FMT, HP>(f.d0, f.d1, f.hv, A.t0, A.t1, A.u0, A.u1, lane);
     const float ws[4] = {bf16_lo(f.sw.x), bf16_hi(f.sw.x), bf16_lo(f.sw.y), bf16_hi(f.sw.y)};
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-        const int4 xb = SH ? bsh[b * 64 + lane] : f.x[b];
-        const v4i bv = {xb.x, xb.y, xb.z, xb.w};
+        const v4i bv = {f.x[b].x, f.x[b].y, f.x[b].z, f.x[b].w};
         const v4i zero = {0, 0, 0, 0};
         const v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bv, zero, 0, 0, 0);
 #pragma unroll
@@ -295,47 +252,105 @@ __device__ __forceinline__ void mf_step(const MfArgs &A, const MfChunk<FMT, NB, 
     }
 }
 
+// qkv (head size 64): qkv_post_kernel's work on a head's 64 rows of up to 64 tokens in LDS
+// (ep[token][row], RP floats a token): bias, q / k RMSNorm and RoPE, then q into the qkv
+// rows, k and v rotated and stored in the cache slot of their position.  The same arithmetic
+// on the same values, so the cache and q equal the separate kernel's.
+template <int RP, int W, int TOK>
+__device__ __forceinline__ void mf_qkv_epilogue(const MfArgs &A, const float *ep, int tokb, int wave, uint32_t lane) {
+    const QkvPostDev &Q = A.qp;
+    const int head = (int)blockIdx.x, pos0 = Q.pos_dev[0];
+    const uint32_t lg = lane >> 4;
+    if (Q.kr.bits == 8) {
+        // Four tokens per wave pass: lanes 16k .. 16k + 15 hold token 4 (pass * W + w) + k,
+        // four consecutive elements each (head_post4; the K / V rotation and int8 by
+        // rotate_quant4 with block 0's signs: fwht_lane + kv_store_head's int8 branch).
+        const uint32_t sl = lane & 15u;
+        const uint64_t m0 = __ballot(hadamard_sign_bit(0, lane) != 0u);
+        for (int tl0 = 4 * wave; tl0 < TOK; tl0 += 4 * W) {
+            if (tokb + tl0 >= A.ntok) break;  // wave-uniform
+            const int t = tokb + tl0 + (int)lg;
+            const bool live = t < A.ntok;
+            const float4 e4 = *reinterpret_cast<const float4 *>(ep + (tl0 + (int)lg) * RP + 4 * sl);
+            float v[4] = {e4.x, e4.y, e4.z, e4.w};
+            head_post4(head, Q.nq, Q.nkv, Q.bias, Q.qn, Q.kn, Q.eps, Q.rope, pos0 + min(t, A.ntok - 1), sl, v);
+            if (head < Q.nq) {
+                if (live)
+                    *reinterpret_cast<float4 *>(A.out + (size_t)t * A.out_stride + (size_t)head * 64 + 4 * sl) =
+                        make_float4(v[0], v[1], v[2], v[3]);
+                continue;
+            }
+            const Chunk4 r = rotate_quant4(v, m0, sl);
+            if (live) {
+                const bool is_k = head < Q.nq + Q.nkv;
+                const int kvh = is_k ? head - Q.nq : head - Q.nq - Q.nkv;
+                const size_t slot = ((size_t)Q.layer * Q.nkv + kvh) * Q.kr.cap + ring_slot(Q.kr, pos0 + t);
+                *reinterpret_cast<uint32_t *>((is_k ? Q.kq : Q.vq) + slot * 64 + 4 * sl) = r.w;
+                if (sl == 0) (is_k ? Q.ks : Q.vs)[slot] = r.scale;
+            }
+        }
+        return;
+    }
+    for (int tl = wave; tl < TOK; tl += W) {
+        const int t = tokb + tl;
+        if (t >= A.ntok) break;  // wave-uniform
+        float v0 = ep[tl * RP + (int)lane], v1 = 0.0f;
+        head_post_vals(head, Q.nq, Q.nkv, 64, Q.bias, Q.qn, Q.kn, Q.eps, Q.rope, pos0 + t, lane, v0, v1);
+        if (head < Q.nq) {
+            A.out[(size_t)t * A.out_stride + (size_t)head * 64 + lane] = v0;
+            continue;
+        }
+        const bool is_k = head < Q.nq + Q.nkv;
+        const int kvh = is_k ? head - Q.nq : head - Q.nq - Q.nkv;
+        const size_t slot = ((size_t)Q.layer * Q.nkv + kvh) * Q.kr.cap + ring_slot(Q.kr, pos0 + t);
+        kv_store_head(fwht_lane(v0, 0, lane), 0.0f, 1, lane, Q.kr.bits, 64, slot, is_k ? Q.kq : Q.vq,
+                      is_k ? Q.ks : Q.vs);
+    }
+}
+
+// gate_up: swiglu_act_kernel's work on an interleaved block of 128 rows ([gate64(ic), up64(ic)],
+// simd_lut.rs:3310-3325) of up to 64 tokens in LDS: per token v = (g / (1 + exp(-g))) * u
+// (swiglu_activate_scalar, real_llm.rs:9801-9805), the FWHT of chunk ic and the int8
+// quantization (populate_chunk_fwht_raw) of the down input, with its tile-major copy.  The
+// same arithmetic in the same order as that kernel, so the outputs are the same.
+template <int RP, int W, int TOK>
+__device__ __forceinline__ void mf_swiglu_epilogue(const MfArgs &A, const float *ep, int tokb, int wave, uint32_t lane) {
+    const int ic = (int)blockIdx.x;
+    // Four tokens per wave at a time: lanes 16k .. 16k + 15 hold token tl0 + k, four
+    // consecutive elements each (rotate_quant4: the arithmetic of fwht_lane +
+    // quant_chunk_store in that layout, so the codes, scales and sums are the same).
+    const uint64_t smask = __ballot(hadamard_sign_bit((uint64_t)ic, lane) != 0u);
+    const uint32_t sl = lane & 15u;
+    for (int tl0 = 4 * wave; tl0 < TOK; tl0 += 4 * W) {
+        if (tokb + tl0 >= A.ntok) break;  // wave-uniform
+        const int tl = tl0 + (int)(lane >> 4), t = tokb + tl;
+        const float4 g4 = *reinterpret_cast<const float4 *>(ep + tl * RP + 4 * sl);
+        const float4 u4 = *reinterpret_cast<const float4 *>(ep + tl * RP + 64 + 4 * sl);
+        const float gs[4] = {g4.x, g4.y, g4.z, g4.w}, us[4] = {u4.x, u4.y, u4.z, u4.w};
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = (gs[j] / (1.0f + expf(-gs[j]))) * us[j];
+        const Chunk4 r = rotate_quant4(v, smask, sl);
+        if (t < A.ntok)
+            chunk4_store(r, sl, t, ic, A.nci, A.sq, A.ss, A.ssum, A.stiles.xt, A.stiles.st, A.stiles.ut);
+    }
+}
+
+// Many stripes, up to 32 tokens: a wave per stripe and NB 16-token blocks, which walks the
+// stripe's K; bound by the weight stream and the latency of each wave's chain.
 // P chunks in flight per wave: a register ring of P stages, unrolled so that each stage
 // is a fixed set of registers (no copies, so the compiler's load waits count only the
 // stages issued after the one consumed).  Stage i holds chunks i, i + P, i + 2P, ...;
 // fetches past the last chunk re-read the last chunk and are never consumed.  Scheduling
 // barriers keep each refill right after the step that frees its stage: left to itself,
 // the compiler sank every load of a round below the round's last MFMA and a wait for all
-// loads, so no load was in flight during compute (256-token 1.7B prefill: o / down 24.8
-// -> 22.9 us, gate_up 40.7 -> 39.6 us).  A software-pipelined form (chunk c's MFMAs
-// issued before chunk c - 1's epilogue) measured slower (25.3 / 41.5 us): the register
-// allocator then copied ring registers at the loop head, which drained the ring.
-//
-// SH: the waves of a workgroup share their tokens' activation blocks through LDS (wave
-// w < NB loads block w; one barrier per chunk) instead of each loading all NB.  Measured
-// (256 tokens): 16384 x 2048 at NB 4, 45.7 -> 40.4 us with P 2; 2048 x 8192 at NB 1,
-// 36.9 -> 44-49 us (one loader and a barrier per chunk for 128 chunks): on for NB 4 only.
-//
-// SW (gate_up only): 8 waves per workgroup, so a workgroup holds one interleaved block ic
-// of 128 rows ([gate64(ic), up64(ic)], simd_lut.rs:3310-3325) for its 64 tokens, and its
-// epilogue is swiglu_act_kernel's instead of a store: per token, v = (g / (1 + exp(-g)))
-// * u (swiglu_activate_scalar, real_llm.rs:9801-9805), the FWHT of chunk ic and the int8
-// quantization (populate_chunk_fwht_raw) of the down input, with its tile-major copy.
-// The same arithmetic in the same order as that kernel, so the outputs are the same.
-//
-// QP (qkv, head size 64): a workgroup's 4 stripes are one head's 64 rows, and its epilogue
-// is qkv_post_kernel's for each of its tokens: bias, q / k RMSNorm and RoPE
-// (head_post_vals), then q back into the qkv rows, k and v rotated and stored in the
-// cache slot of their position.  The same arithmetic on the same values, so the cache
-// and q equal the separate kernel's.
-template <int FMT, int HP, int NB, int P, bool SH, bool SW = false, bool QP = false>
-__global__ __launch_bounds__(SW ? 512 : 256) void gemm_mfma_kernel(MfArgs A) {
-    constexpr int W = SW ? 8 : 4;  // waves (stripes) per workgroup
-    static_assert(!SW || (SH && NB == 4), "the SwiGLU epilogue runs on 64-token workgroups");
+// loads, so no load was in flight during compute.
+template <int FMT, int HP, int NB, int P, bool QP = false>
+__global__ __launch_bounds__(256) void gemm_mfma_kernel(MfArgs A) {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: stripe math on SGPRs
-    const int stripe_id = (int)blockIdx.x * W + (int)wave;
-    // With sharing every wave takes part in every barrier: a wave past the last stripe
-    // runs the last stripe's chunks and stores nothing.
-    if (!SH && stripe_id >= A.stripes) return;
-    const int stripe = min(stripe_id, A.stripes - 1);
-    __shared__ int4 bsh[2][SH ? NB * 64 : 1];
-    const int tokb = (int)blockIdx.y * 16 * NB;
+    const int stripe = (int)blockIdx.x * 4 + (int)wave;
+    if (stripe >= A.stripes) return;
     const bool is_tail = stripe >= 2 * A.np;
     const uint32_t side = is_tail ? 0u : (uint32_t)(stripe & 1);
     const uint8_t *mbase = is_tail ? A.tail : A.pair + (size_t)(stripe >> 1) * A.ptot;
@@ -351,110 +366,35 @@ __global__ __launch_bounds__(SW ? 512 : 256) void gemm_mfma_kernel(MfArgs A) {
 #pragma unroll
         for (int r = 0; r < 4; r++) acc[b][r] = 0.0f;
     const int nc = A.nc, last = nc - 1;
-    MfChunk<FMT, NB, SH> ring[P];
+    MfChunk<FMT, NB> ring[P];
 #pragma unroll
-    for (int i = 0; i < P; i++) mf_fetch<FMT, HP, NB, SH>(A, R, L, is_tail, tb0, wave, min(i, last), ring[i]);
+    for (int i = 0; i < P; i++) mf_fetch<FMT, HP, NB>(A, R, L, is_tail, tb0, min(i, last), ring[i]);
     int c0 = 0;
     for (; c0 + P <= nc; c0 += P) {
 #pragma unroll
         for (int i = 0; i < P; i++) {
-            mf_step<FMT, HP, NB, SH>(A, ring[i], acc, bsh[(c0 + i) & 1], wave, lane);
+            mf_step<FMT, HP, NB>(A, ring[i], acc, lane);
             __builtin_amdgcn_sched_barrier(0);
-            mf_fetch<FMT, HP, NB, SH>(A, R, L, is_tail, tb0, wave, min(c0 + P + i, last), ring[i]);
+            mf_fetch<FMT, HP, NB>(A, R, L, is_tail, tb0, min(c0 + P + i, last), ring[i]);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
 #pragma unroll
     for (int i = 0; i < P - 1; i++)
-        if (c0 + i < nc) mf_step<FMT, HP, NB, SH>(A, ring[i], acc, bsh[(c0 + i) & 1], wave, lane);
+        if (c0 + i < nc) mf_step<FMT, HP, NB>(A, ring[i], acc, lane);
     if constexpr (QP) {
-        __shared__ __align__(16) float eq[16 * NB][68];  // [token][row of the head] (padded rows)
+        __shared__ __align__(16) float ep[16 * NB * 68];
 #pragma unroll
         for (int b = 0; b < NB; b++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) eq[16 * b + li][wave * 16 + 4 * lg + r] = acc[b][r];
+            *reinterpret_cast<float4 *>(ep + (16 * b + (int)li) * 68 + 16 * (int)wave + 4 * (int)lg) =
+                make_float4(acc[b][0], acc[b][1], acc[b][2], acc[b][3]);
         __syncthreads();
-        const QkvPostDev &Q = A.qp;
-        const int head = (int)blockIdx.x, pos0 = Q.pos_dev[0];
-        if (Q.kr.bits == 8) {
-            // Four tokens per wave pass: lanes 16k .. 16k + 15 hold token 4 (pass * W + w) + k,
-            // four consecutive elements each (head_post4; the K / V rotation and int8 by
-            // rotate_quant4 with block 0's signs: fwht_lane + kv_store_head's int8 branch).
-            const uint32_t sl = lane & 15u;
-            const uint64_t m0 = __ballot(hadamard_sign_bit(0, lane) != 0u);
-            for (int tl0 = 4 * (int)wave; tl0 < 16 * NB; tl0 += 4 * W) {
-                if (tokb + tl0 >= A.ntok) break;  // wave-uniform
-                const int t = tokb + tl0 + (int)lg;
-                const bool live = t < A.ntok;
-                const float4 e4 = *reinterpret_cast<const float4 *>(&eq[tl0 + (int)lg][4 * sl]);
-                float v[4] = {e4.x, e4.y, e4.z, e4.w};
-                head_post4(head, Q.nq, Q.nkv, Q.bias, Q.qn, Q.kn, Q.eps, Q.rope, pos0 + min(t, A.ntok - 1), sl, v);
-                if (head < Q.nq) {
-                    if (live)
-                        *reinterpret_cast<float4 *>(A.out + (size_t)t * A.out_stride + (size_t)head * 64 + 4 * sl) =
-                            make_float4(v[0], v[1], v[2], v[3]);
-                    continue;
-                }
-                const Chunk4 r = rotate_quant4(v, m0, sl);
-                if (live) {
-                    const bool is_k = head < Q.nq + Q.nkv;
-                    const int kvh = is_k ? head - Q.nq : head - Q.nq - Q.nkv;
-                    const size_t slot = ((size_t)Q.layer * Q.nkv + kvh) * Q.kr.cap + ring_slot(Q.kr, pos0 + t);
-                    *reinterpret_cast<uint32_t *>((is_k ? Q.kq : Q.vq) + slot * 64 + 4 * sl) = r.w;
-                    if (sl == 0) (is_k ? Q.ks : Q.vs)[slot] = r.scale;
-                }
-            }
-            return;
-        }
-        for (int tl = (int)wave; tl < 16 * NB; tl += W) {
-            const int t = tokb + tl;
-            if (t >= A.ntok) break;  // wave-uniform
-            float v0 = eq[tl][lane], v1 = 0.0f;
-            head_post_vals(head, Q.nq, Q.nkv, 64, Q.bias, Q.qn, Q.kn, Q.eps, Q.rope, pos0 + t, lane, v0, v1);
-            if (head < Q.nq) {
-                A.out[(size_t)t * A.out_stride + (size_t)head * 64 + lane] = v0;
-                continue;
-            }
-            const bool is_k = head < Q.nq + Q.nkv;
-            const int kvh = is_k ? head - Q.nq : head - Q.nq - Q.nkv;
-            const size_t slot = ((size_t)Q.layer * Q.nkv + kvh) * Q.kr.cap + ring_slot(Q.kr, pos0 + t);
-            kv_store_head(fwht_lane(v0, 0, lane), 0.0f, 1, lane, Q.kr.bits, 64, slot, is_k ? Q.kq : Q.vq,
-                          is_k ? Q.ks : Q.vs);
-        }
+        mf_qkv_epilogue<68, 4, 16 * NB>(A, ep, tb0 * 16, (int)wave, lane);
         return;
     }
-    if constexpr (SW) {
-        __shared__ float4 ep4[64][33];  // [token][row of the block / 4] (+1 float4 of padding)
-        float *ep = reinterpret_cast<float *>(ep4);
-#pragma unroll
-        for (int b = 0; b < NB; b++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) ep[(16 * b + li) * 132 + wave * 16 + 4 * lg + r] = acc[b][r];
-        __syncthreads();
-        const int ic = (int)blockIdx.x;
-        // Four tokens per wave at a time: lanes 16k .. 16k + 15 hold token tl0 + k, four
-        // consecutive elements each (rotate_quant4: the arithmetic of fwht_lane +
-        // quant_chunk_store in that layout, so the codes, scales and sums are the same).
-        const uint64_t smask = __ballot(hadamard_sign_bit((uint64_t)ic, lane) != 0u);
-        const uint32_t sl = lane & 15u;
-        for (int tl0 = 4 * (int)wave; tl0 < 16 * NB; tl0 += 4 * W) {
-            if (tokb + tl0 >= A.ntok) break;  // wave-uniform
-            const int tl = tl0 + (int)(lane >> 4), t = tokb + tl;
-            const float4 g4 = ep4[tl][sl], u4 = ep4[tl][16 + sl];
-            const float gs[4] = {g4.x, g4.y, g4.z, g4.w}, us[4] = {u4.x, u4.y, u4.z, u4.w};
-            float v[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = (gs[j] / (1.0f + expf(-gs[j]))) * us[j];
-            const Chunk4 r = rotate_quant4(v, smask, sl);
-            if (t < A.ntok)
-                chunk4_store(r, sl, t, ic, A.nci, A.sq, A.ss, A.ssum, A.stiles.xt, A.stiles.st, A.stiles.ut);
-        }
-        return;
-    }
-    if (stripe_id >= A.stripes) return;
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-        const int t = tokb + 16 * b + (int)li;
+        const int t = (tb0 + b) * 16 + (int)li;
         if (t >= A.ntok) continue;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
@@ -462,6 +402,371 @@ __global__ __launch_bounds__(SW ? 512 : 256) void gemm_mfma_kernel(MfArgs A) {
             if (row >= A.rows) continue;
             float *o = A.out + (size_t)t * A.out_stride + row;
             *o = A.accum ? *o + acc[b][r] : acc[b][r];
+        }
+    }
+}
+
+// ---------------------------------------------------------------- few waves: K dealt over a workgroup
+// One stripe and up to 64 tokens per workgroup of 8 waves.  gemm_mfma_kernel gives a wave its
+// stripe's whole K, so a matrix with few stripes leaves SIMDs idle while each wave walks its
+// chunks one after the other (NF4 4096 x 14336, 16 tokens: 40.5 us for 30 MB).  Here the waves
+// take the chunks of a round of 8 side by side: decode, MFMA and the terms float(dot) * sx go
+// to LDS, one barrier a round (two buffers), and the chain f = fmaf(term, scale, f) runs over
+// the round's terms in chunk order, each wave owning one (block, row mod 4) part of the
+// outputs.  The same operations in the same order, so the outputs equal gemm_mfma_kernel's;
+// 16.5 us for that shape.  Bound by the exchange (2 KB of LDS traffic per tile of 16 x 16
+// outputs and chunk) and the issue rate of the chain.
+constexpr int kKsWaves = 8;
+
+template <int FMT, int NB>
+struct KsFrag {
+    uint32_t d0, d1, hv;
+    uint2 sw;
+    v4i x[NB];
+    float sx[NB];
+    int32_t su[FMT == 0 ? NB : 1];
+};
+
+template <int FMT, int HP, int NB>
+__global__ __launch_bounds__(64 * kKsWaves, 4) void gemm_ks_kernel(MfArgs A) {
+    constexpr int W = kKsWaves, P = NB == 4 ? 2 : NB == 2 ? 3 : 4;  // rounds in flight
+    constexpr int OWN = NB == 4 ? 2 : 1;              // chains per wave
+    __shared__ float tt[2][W][NB][4][64];             // terms [chunk of the round][block][row mod 4][lane]
+    __shared__ __align__(16) float wss[2][W][16];     // the chunks' row scales
+    const uint32_t lane = threadIdx.x & 63u, li = lane & 15u, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    int stripe = (int)blockIdx.x;
+    if ((gridDim.x & 15u) == 0) {  // both stripes of a pair on one XCD, as in gemv_kernel
+        const int a = stripe >> 4, s8 = (stripe >> 3) & 1, j = stripe & 7;
+        stripe = 2 * (8 * a + j) + s8;
+    }
+    const bool is_tail = stripe >= 2 * A.np;
+    const MfLane L = mf_lane<FMT, HP>(lane, is_tail, is_tail ? 0u : (uint32_t)(stripe & 1), A.lane);
+    const __amdgpu_buffer_rsrc_t rw = mf_rsrc(is_tail ? A.tail : A.pair + (size_t)(stripe >> 1) * A.ptot),
+                                 rx = mf_rsrc(A.xt), rs = mf_rsrc(A.st), ru = mf_rsrc(FMT == 0 ? (const void *)A.ut : A.st);
+    const int tokb = (int)blockIdx.y * 16 * NB;
+    uint32_t xo[NB], so[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {  // (blocks and tokens past the end repeat the last one, not stored)
+        if (A.tiled) {
+            const uint32_t t = (uint32_t)min((int)blockIdx.y * NB + b, A.nblk - 1) * (uint32_t)A.nc;
+            xo[b] = t * 1024u + lane * 16u;
+            so[b] = t * 64u + li * 4u;
+        } else {
+            const uint32_t t = (uint32_t)min(tokb + 16 * b + (int)li, A.ntok - 1);
+            xo[b] = t * (uint32_t)A.K + lg * 16u;
+            so[b] = t * (uint32_t)A.nc * 4u;
+        }
+    }
+    const uint32_t xstep = A.tiled ? 1024u : 64u, sstep = A.tiled ? 64u : 4u;
+    auto fetch = [&](KsFrag<FMT, NB> &f, int c) {
+        uint32_t rec, sgb;
+        mf_record<FMT, HP>(A.sgc_log2, is_tail, c, rec, sgb);
+        f.d0 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw, L.a_off, rec, 0);
+        f.d1 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw, L.b_off, rec, 0);
+        if constexpr ((FMT == 0 && HP > 0) || FMT == 2)
+            f.hv = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw, L.h_off, rec, 0);
+        const v2u sw = __builtin_amdgcn_raw_buffer_load_b64(rw, L.s_off, sgb, 0);
+        f.sw = make_uint2(sw[0], sw[1]);
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const v4u x = __builtin_amdgcn_raw_buffer_load_b128(rx, xo[b], (uint32_t)c * xstep, 0);
+            f.x[b] = v4i{(int)x[0], (int)x[1], (int)x[2], (int)x[3]};
+            f.sx[b] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, so[b], (uint32_t)c * sstep, 0));
+            if constexpr (FMT == 0)
+                f.su[b] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(ru, so[b], (uint32_t)c * sstep, 0);
+        }
+    };
+    // this wave's chains: row 4 lg + r of token li, blocks ob, ob + 2
+    const int r_own = wave & 3, ob = wave >> 2;
+    float acc[OWN];
+#pragma unroll
+    for (int k = 0; k < OWN; k++) acc[k] = 0.0f;
+    const int nc = A.nc, last = nc - 1;
+    auto round = [&](const KsFrag<FMT, NB> &f, int i) {
+        const int buf = i & 1;
+        const v4i a = mf_decode<FMT, HP>(f.d0, f.d1, f.hv, A.t0, A.t1, A.u0, A.u1, lane);
+        if (li == 0)
+            *reinterpret_cast<float4 *>(&wss[buf][wave][4 * lg]) =
+                make_float4(bf16_lo(f.sw.x), bf16_hi(f.sw.x), bf16_lo(f.sw.y), bf16_hi(f.sw.y));
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const v4i zero = {0, 0, 0, 0};
+            const v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, f.x[b], zero, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                int dot = d[r];
+                if constexpr (FMT == 0) dot = 2 * dot - ((1 << (4 + HP)) - 1) * f.su[b];
+                tt[buf][wave][b][r][lane] = (float)dot * f.sx[b];
+            }
+        }
+        __syncthreads();
+        if (NB > 1 || ob == 0) {
+            const int n = min(W, nc - i * W);  // (a wave past the last chunk repeated it; not added)
+#pragma unroll
+            for (int h = 0; h < W; h += 4) {
+                float ws[4], t[OWN][4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    ws[k] = wss[buf][h + k][4 * lg + r_own];
+#pragma unroll
+                    for (int o = 0; o < OWN; o++) t[o][k] = tt[buf][h + k][NB == 1 ? 0 : ob + 2 * o][r_own][lane];
+                }
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (h + k < n)
+#pragma unroll
+                        for (int o = 0; o < OWN; o++) acc[o] = fmaf(t[o][k], ws[k], acc[o]);
+            }
+        }
+    };
+    KsFrag<FMT, NB> ring[P];
+#pragma unroll
+    for (int k = 0; k < P; k++) fetch(ring[k], min(W * k + wave, last));
+    const int rounds = (nc + W - 1) / W;
+    int i = 0;
+    for (; i + P <= rounds; i += P) {
+#pragma unroll
+        for (int k = 0; k < P; k++) {
+            round(ring[k], i + k);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(ring[k], min(W * (i + k + P) + wave, last));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < P - 1; k++)
+        if (i + k < rounds) round(ring[k], i + k);
+    // through LDS, so that a token's 16 rows are stored together
+    __syncthreads();
+    float *ot = &tt[0][0][0][0][0];  // [16 NB tokens][17]
+    if (NB > 1 || ob == 0)
+#pragma unroll
+        for (int o = 0; o < OWN; o++)
+            ot[(16 * (NB == 1 ? 0 : ob + 2 * o) + (int)li) * 17 + 4 * lg + r_own] = acc[o];
+    __syncthreads();
+    for (int k = (int)threadIdx.x; k < 16 * NB * 16; k += 64 * W) {
+        const int t = tokb + k / 16, row = stripe * 16 + k % 16;
+        if (t >= A.ntok || row >= A.rows) continue;
+        const float v = ot[(k / 16) * 17 + k % 16];
+        float *o = A.out + (size_t)t * A.out_stride + row;
+        *o = A.accum ? *o + v : v;
+    }
+}
+
+// ---------------------------------------------------------------- tile kernel
+// NP stripe pairs x 64 tokens per workgroup of 4 waves, 4 chunks per stage:
+//  - wave w loads and decodes chunk 4 i + w of the NP pairs into LDS (A operands and row
+//    scales as floats; two buffers, one barrier per stage), so a decode serves 4 token blocks
+//    whatever the number of waves the launch has;
+//  - wave w then runs the stage's 4 chunks over all 2 NP stripes for its own token block w
+//    (TB: its TB blocks) whose activation it loads straight in B order, while stage i + 1 is
+//    decoded into the other buffer.
+// Per output tile (16 x 16, one chunk) that is 12 instructions of epilogue (convert, multiply,
+// fma per output, the reference's chain) and 6 / TB of decode next to an MFMA of 16 cycles
+// that the other instructions do not overlap: the issue rate bounds the kernel (NF4 14336 x
+// 4096, 512 tokens: 81 us for 1.8 M tiles, 94 us when a wave decoded for its own blocks).
+// Weights and activations of the next D stages are in flight in registers.
+// MODE 0 stores the outputs; 1 (gate_up, NP 4: one interleaved block of 128 rows) has
+// swiglu_act_kernel's work as its epilogue; 2 (qkv at head size 64, NP 2: one head of 64 rows)
+// qkv_post_kernel's.
+template <int FMT, int HP, int NP, int TB, int D, int MODE>
+__global__ __launch_bounds__(256, NP* TB >= 4 ? 1 : 2) void gemm_tile_kernel(MfArgs A) {
+    constexpr int W = 4, NS = 2 * NP, TOK = 16 * W * TB;
+    constexpr uint32_t CB = FMT == 2 ? 384u : 512u;  // bytes per stripe-chunk
+    extern __shared__ __align__(16) unsigned char tile_lds[];
+    int4(*al)[W][NS][64] = reinterpret_cast<int4(*)[W][NS][64]>(tile_lds);                          // [2] decoded A
+    float(*wl)[W][NS][16] = reinterpret_cast<float(*)[W][NS][16]>(tile_lds + 2 * W * NS * 1024);  // [2] row scales
+    const uint32_t lane = threadIdx.x & 63u, li = lane & 15u, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int npt = (A.stripes + 1) >> 1, p0 = (int)blockIdx.x * NP;  // pairs, the odd last stripe among them
+    bool tail[NP];
+    __amdgpu_buffer_rsrc_t rw[NP];
+#pragma unroll
+    for (int k = 0; k < NP; k++) {  // (pairs past the last repeat it, not stored)
+        const int pk = min(p0 + k, npt - 1);
+        tail[k] = pk >= A.np;
+        rw[k] = mf_rsrc(tail[k] ? A.tail : A.pair + (size_t)pk * A.ptot);
+    }
+    const __amdgpu_buffer_rsrc_t rx = mf_rsrc(A.xt), rs = mf_rsrc(A.st), ru = mf_rsrc(FMT == 0 ? (const void *)A.ut : A.st);
+    const MfLane L = mf_lane<FMT, HP>(lane, true, 0u, A.lane);  // offsets from the stripe's codes, hi bytes, scales
+    const uint32_t ah = FMT == 0 ? L.h_off - 512u : L.h_off, as = 8u * lg;
+    struct Wt {
+        uint32_t d0[NS], d1[NS], hv[NS];
+        uint2 sw[NS];
+    };
+    struct Bt {
+        v4i x[TB];
+        float sx[TB];
+        int32_t su[TB];
+    };
+    const int nc = A.nc, last = nc - 1;
+    auto fetch_w = [&](Wt &f, int stage) {
+        const int c = min(W * stage + wave, last);
+#pragma unroll
+        for (int k = 0; k < NP; k++) {
+            uint32_t rec, sgb;
+            mf_record<FMT, HP>(A.sgc_log2, tail[k], c, rec, sgb);
+#pragma unroll
+            for (int s = 0; s < 2; s++) {  // (side 1 of the tail stripe repeats side 0, not stored)
+                const uint32_t sd = tail[k] ? 0u : (uint32_t)s;
+                const uint32_t code = rec + sd * CB;
+                uint32_t sc = sgb + sd * 32u;
+                if constexpr (FMT == 0) sc = rec + (tail[k] ? 512u + 128u * HP : 1024u + 256u * HP + sd * 32u);
+                f.d0[2 * k + s] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw[k], L.a_off, code, 0);
+                f.d1[2 * k + s] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw[k], L.b_off, code, 0);
+                if constexpr (FMT == 2)
+                    f.hv[2 * k + s] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw[k], ah, code, 0);
+                if constexpr (FMT == 0 && HP > 0)
+                    f.hv[2 * k + s] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(
+                        rw[k], ah, rec + (tail[k] ? 512u : 1024u + sd * 128u * HP), 0);
+                const v2u sw = __builtin_amdgcn_raw_buffer_load_b64(rw[k], as, sc, 0);
+                f.sw[2 * k + s] = make_uint2(sw[0], sw[1]);
+            }
+        }
+    };
+    const int tb = ((int)blockIdx.y * W + wave) * TB, tokb = (int)blockIdx.y * TOK;
+    uint32_t t0[TB];
+#pragma unroll
+    for (int b = 0; b < TB; b++) t0[b] = (uint32_t)min(tb + b, A.nblk - 1) * (uint32_t)nc;
+    auto fetch_b = [&](Bt &f, int c) {
+#pragma unroll
+        for (int b = 0; b < TB; b++) {
+            const uint32_t t = t0[b] + (uint32_t)min(c, last);
+            const v4u x = __builtin_amdgcn_raw_buffer_load_b128(rx, lane * 16u, t * 1024u, 0);
+            f.x[b] = v4i{(int)x[0], (int)x[1], (int)x[2], (int)x[3]};
+            f.sx[b] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, li * 4u, t * 64u, 0));
+            if constexpr (FMT == 0) f.su[b] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(ru, li * 4u, t * 64u, 0);
+        }
+    };
+    float acc[NS][TB][4];
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+#pragma unroll
+        for (int b = 0; b < TB; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[s][b][r] = 0.0f;
+    const int stages = (nc + W - 1) / W;
+    auto decode = [&](const Wt &f, int buf) {
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            const v4i a = mf_decode<FMT, HP>(f.d0[s], f.d1[s], f.hv[s], A.t0, A.t1, A.u0, A.u1, lane);
+            al[buf][wave][s][lane] = make_int4(a[0], a[1], a[2], a[3]);
+            // (every lane of a group of 16 writes the same 16 bytes)
+            *reinterpret_cast<float4 *>(&wl[buf][wave][s][4 * lg]) =
+                make_float4(bf16_lo(f.sw[s].x), bf16_hi(f.sw[s].x), bf16_lo(f.sw[s].y), bf16_hi(f.sw[s].y));
+        }
+    };
+    struct Ld {
+        int4 a[2];
+        float4 w[2];
+    };
+    auto read = [&](Ld &f, int buf, int g) {  // group g: chunk g / NP, pair g % NP
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            f.a[s] = al[buf][g / NP][2 * (g % NP) + s][lane];
+            f.w[s] = *reinterpret_cast<const float4 *>(&wl[buf][g / NP][2 * (g % NP) + s][4 * lg]);
+        }
+    };
+    auto mul = [&](const Ld &f, const Bt &x, int k) {
+        v4i d[2][TB];
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int b = 0; b < TB; b++) {
+                const v4i zero = {0, 0, 0, 0};
+                d[s][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v4i{f.a[s].x, f.a[s].y, f.a[s].z, f.a[s].w}, x.x[b], zero, 0, 0, 0);
+            }
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            const float wv[4] = {f.w[s].x, f.w[s].y, f.w[s].z, f.w[s].w};
+#pragma unroll
+            for (int b = 0; b < TB; b++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    int dot = d[s][b][r];
+                    if constexpr (FMT == 0) dot = 2 * dot - ((1 << (4 + HP)) - 1) * x.su[b];
+                    acc[2 * k + s][b][r] = fmaf((float)dot * x.sx[b], wv[r], acc[2 * k + s][b][r]);
+                }
+        }
+    };
+    auto run = [&](auto active) {  // active: this wave has a token block (the others only decode)
+        constexpr bool kActive = decltype(active)::value;
+        Wt wr[D];
+        Bt br[D][W];
+        // Stage i's products while the next stage is decoded into the other buffer.
+        auto step = [&](Wt &wf, Bt(&bf)[W], int i, int live) {
+            const int buf = i & 1;
+            Ld ld[2];
+            if constexpr (kActive) read(ld[0], buf, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            decode(wf, buf ^ 1);
+            fetch_w(wf, i + 1 + D);
+            if constexpr (kActive) {
+#pragma unroll
+                for (int g = 0; g < W * NP; g++) {
+                    const int q = g / NP;
+                    if (q >= live) break;
+                    if (g + 1 < W * NP) read(ld[(g + 1) & 1], buf, g + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    mul(ld[g & 1], bf[q], g % NP);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (g % NP == NP - 1) fetch_b(bf[q], W * (i + D) + q);
+                }
+            }
+            __syncthreads();
+        };
+        fetch_w(wr[0], 0);
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            if (d > 0) fetch_w(wr[d], d);
+            if constexpr (kActive)
+#pragma unroll
+                for (int q = 0; q < W; q++) fetch_b(br[d][q], W * d + q);
+        }
+        decode(wr[0], 0);
+        fetch_w(wr[0], D);
+        __syncthreads();
+        const int full = nc / W;
+        int i = 0;
+        for (; i + D <= full; i += D)
+#pragma unroll
+            for (int d = 0; d < D; d++) step(wr[(d + 1) % D], br[d], i + d, W);
+#pragma unroll
+        for (int d = 0; d < D; d++)
+            if (i + d < stages) step(wr[(d + 1) % D], br[d], i + d, nc - W * (i + d));
+    };
+    if (tb < A.nblk) run(std::true_type{});
+    else run(std::false_type{});
+    if constexpr (MODE != 0) {
+        // the epilogues work on [token][row] in LDS
+        constexpr int RP = 32 * NP + 4;
+        float *ep = reinterpret_cast<float *>(tile_lds);
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int b = 0; b < TB; b++)
+                *reinterpret_cast<float4 *>(ep + (16 * (TB * wave + b) + (int)li) * RP + 16 * s + 4 * (int)lg) =
+                    make_float4(acc[s][b][0], acc[s][b][1], acc[s][b][2], acc[s][b][3]);
+        __syncthreads();
+        if constexpr (MODE == 1) mf_swiglu_epilogue<RP, W, TOK>(A, ep, tokb, wave, lane);
+        else mf_qkv_epilogue<RP, W, TOK>(A, ep, tokb, wave, lane);
+        return;
+    }
+#pragma unroll
+    for (int b = 0; b < TB; b++) {
+        const int t = (tb + b) * 16 + (int)li;
+        if (t >= A.ntok) return;
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            const int stripe = 2 * p0 + s, row0 = 16 * stripe + 4 * (int)lg;
+            if (stripe >= A.stripes) break;
+            float *o = A.out + (size_t)t * A.out_stride + row0;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if (row0 + r >= A.rows) break;
+                o[r] = A.accum ? o[r] + acc[s][b][r] : acc[s][b][r];
+            }
         }
     }
 }
@@ -660,6 +965,17 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
 
 }  // namespace
 
+// Lookup words of an NF matrix: NF4's XOR tables, NF3's codebook (bit planes: none).
+static void mf_tables(const k2t_mat *m, uint32_t &t0, uint32_t &t1, uint32_t &u0, uint32_t &u1) {
+    if (m->fmt != K2T_FMT_NF) return;
+    if (m->bits == 3) {
+        t0 = m->cb[0];
+        t1 = m->cb[1];
+    } else {
+        nf4_xor_tables(m->cb[0], m->cb[1], m->cb[2], m->cb[3], t0, t1, u0, u1);
+    }
+}
+
 bool gemm_mfma_supported(const k2t_mat *m, int ntok) {
     if (ntok < kMfmaMinTokens || m->cols % 64 != 0) return false;
     if (m->fmt == K2T_FMT_NF) return (m->bits == 3 || m->bits == 4) && (m->sgc & (m->sgc - 1)) == 0;
@@ -699,10 +1015,7 @@ static GvArgs gemv_mfma_args(const k2t_mat *m, const GemvPlan &plan, const int8_
     A.nseg = plan.nseg;
     A.cps = plan.cps;
     A.lane = m->nf3_lane;
-    if (!planes && m->bits == 3) {
-        A.t0 = m->cb[0];
-        A.t1 = m->cb[1];
-    } else if (!planes) nf4_xor_tables(m->cb[0], m->cb[1], m->cb[2], m->cb[3], A.t0, A.t1, A.u0, A.u1);
+    mf_tables(m, A.t0, A.t1, A.u0, A.u1);
     A.xq = xq;
     A.xs = xs;
     A.xsum = xsum;
@@ -760,24 +1073,47 @@ void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, cons
     hip_check(hipGetLastError(), "mfma gemv launch");
 }
 
-template <int FMT, int HP>
-static void launch_gemm_mfma_fmt(hipStream_t st, int nb, dim3 grid, const MfArgs &A) {
-    switch (nb) {
-        case 1: hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 1, kMfmaDepth, false>), grid, dim3(256), 0, st, A); break;
-        case 2: hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 2, kMfmaDepth, false>), grid, dim3(256), 0, st, A); break;
-        case 3: hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 3, kMfmaDepth, false>), grid, dim3(256), 0, st, A); break;
-        case 4: hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 4, kMfmaShDepth, true>), grid, dim3(256), 0, st, A); break;
-        default:
-            if constexpr (kMfmaMaxBlocks >= 8)
-                hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 8, kMfmaShDepth, true>), grid, dim3(256), 0, st, A);
-            break;
+// Whether `blocks` 16-token blocks run on gemm_ks_kernel: few stripes, and no more (stripe,
+// block) pairs than keep its exchange through LDS cheaper than a long chain per wave.  NF4
+// 4096 x 14336 (256 stripes), 16 / 64 / 128 / 256 tokens: 16.5 / 28.9 / 41.5 / 76 us there,
+// 40.5 / 46 / 47 / 58 us on the others; 2048 x 2048, 128: 8.6 and 10.8.  The bit planes' chains
+// also subtract the code sums: b6 4096 x 14336, 64 / 128 tokens 33 / 63 us there, 40 / 49 us.
+static bool ks_split(const k2t_mat *m, int blocks) {
+    return m->stripes < 512 && (long)m->stripes * blocks <= (m->fmt == K2T_FMT_NIBBLE4 ? 1024 : 2048);
+}
+
+// Whether gemm_ks_kernel then reads a plain activation as its rows lie, rather than a tile-major
+// copy made first: worth the copy's launch (2.5 us) only for short rows and few stripes (each
+// gathers them again).  960 x 576, 16 tokens 7.3 -> 4.2 us, NF4 128 tokens 7.4 -> 6.6; NF4
+// 2048 x 2048, 16 tokens 7.1 -> 6.0; not taken: 32 tokens of it 7.2 -> 8.1, 6144 x 2048, 16 tokens
+// 7.6 -> 10.2, b6 960 x 576, 64 tokens 7.4 -> 8.0.
+static bool ks_rows(const k2t_mat *m, int blocks) {
+    return ks_split(m, blocks) && (long)m->stripes * m->nc * blocks <= 6000 &&
+           m->nc * (blocks < 4 ? blocks : 4) <= (m->fmt == K2T_FMT_NIBBLE4 ? 20 : 40);
+}
+
+// Scratch floats the tile-major copy of ntok tokens takes (0: no copy is made).
+static size_t tile_scratch(const k2t_mat *m, int ntok) {
+    const int blocks = (ntok + 15) / 16;
+    return ks_rows(m, blocks) ? 0 : (size_t)blocks * m->nc * (1024 + 64 + 64) / sizeof(float);
+}
+
+bool gemm_mfma_nf3_passes(k2t_ctx *ctx, const k2t_mat *m, int ntok) {
+    if (m->fmt != K2T_FMT_NF || m->bits != 3) return false;
+    if (ntok <= 128 && (long)m->stripes * m->nc * ((ntok + 3) / 4) <= 36000) return true;
+    if (tile_scratch(m, ntok) <= ctx->scratch_cap) return false;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
     }
+    return cap != hipStreamCaptureStatusNone;
 }
 
 // Arguments of one launch over all of m's stripes, and the tile-major activation (the
 // producer's, else copied here into the context's scratch: 1 KB + 64 B of scales + 64 B
-// of code sums per tile).  Returns the 16-token blocks per wave the launch will use.
-static int mfma_args(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const float *xs, const int32_t *xsum,
+// of code sums per tile).
+static void mfma_args(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const float *xs, const int32_t *xsum,
                      int ntok, ActTiles tiles, MfArgs &A) {
     const bool planes = m->fmt == K2T_FMT_NIBBLE4;
     A = MfArgs{};
@@ -790,17 +1126,20 @@ static int mfma_args(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const flo
     A.stripes = m->stripes;
     A.sgc_log2 = planes ? 0 : __builtin_ctz((unsigned)m->sgc);
     A.lane = m->nf3_lane;
-    if (!planes && m->bits == 3) {
-        A.t0 = m->cb[0];
-        A.t1 = m->cb[1];
-    } else if (!planes) nf4_xor_tables(m->cb[0], m->cb[1], m->cb[2], m->cb[3], A.t0, A.t1, A.u0, A.u1);
+    mf_tables(m, A.t0, A.t1, A.u0, A.u1);
     const int blocks = (ntok + 15) / 16;
     int8_t *xt = tiles.xt;
     float *stile = tiles.st;
     int32_t *utile = tiles.ut;
-    if (!xt || (planes && !utile)) {
+    A.tiled = 1;
+    if ((!xt || (planes && !utile)) && ks_rows(m, blocks)) {
+        xt = const_cast<int8_t *>(xq);
+        stile = const_cast<float *>(xs);
+        utile = const_cast<int32_t *>(xsum);
+        A.tiled = 0;
+    } else if (!xt || (planes && !utile)) {
         const size_t ntile = (size_t)blocks * m->nc;
-        ensure_scratch(ctx, ntile * (1024 + 64 + 64) / sizeof(float));
+        ensure_scratch(ctx, tile_scratch(m, ntok));
         xt = reinterpret_cast<int8_t *>(ctx->scratch);
         stile = ctx->scratch + ntile * 256;
         utile = reinterpret_cast<int32_t *>(ctx->scratch + ntile * 272);
@@ -813,41 +1152,78 @@ static int mfma_args(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const flo
     A.ut = utile;
     A.K = m->cols;
     A.ntok = ntok;
-    // Tokens per wave: the most 16-token blocks (fewest weight passes) that still give
-    // the launch kMfmaMinWaves waves.
-    int nb = std::min(kMfmaMaxBlocks, blocks);
-    if (nb > 4 && nb < 8) nb = 4;
-    while (nb > 1 && (long)m->stripes * ((blocks + nb - 1) / nb) < kMfmaMinWaves) nb = nb > 4 ? 4 : nb > 2 ? 2 : 1;
-    return nb;
+}
+
+template <int FMT, int HP, int NP, int TB, int D, int MODE>
+static void launch_tile(hipStream_t st, const MfArgs &A) {
+    const dim3 grid(((A.stripes + 1) / 2 + NP - 1) / NP, (A.nblk + 4 * TB - 1) / (4 * TB));
+    const size_t lds = (size_t)2 * 4 * 2 * NP * (1024 + 64);
+    hipLaunchKernelGGL((gemm_tile_kernel<FMT, HP, NP, TB, D, MODE>), grid, dim3(256), lds, st, A);
+}
+
+// f<FMT, HP>(...) for matrix m's format.
+#define MF_FORMATS(m, f, ...)                                                 \
+    do {                                                                      \
+        if ((m)->fmt == K2T_FMT_NF && (m)->bits == 3) f<2, 0>(__VA_ARGS__);   \
+        else if ((m)->fmt == K2T_FMT_NF) f<1, 0>(__VA_ARGS__);                \
+        else if ((m)->hp == 0) f<0, 0>(__VA_ARGS__);                          \
+        else if ((m)->hp == 1) f<0, 1>(__VA_ARGS__);                          \
+        else f<0, 2>(__VA_ARGS__);                                            \
+    } while (0)
+
+template <int FMT, int HP>
+static void launch_plain_fmt(hipStream_t st, bool ks, const MfArgs &A) {
+    const int S = A.stripes, B = A.nblk;
+    // Many stripes and up to 32 tokens: a wave per stripe (NF4 14336 x 4096, 16 tokens 16 us,
+    // 18.6 in 64-token tiles).  Above, tiles of 32 rows x 64 tokens, or x 128 once those give 448
+    // workgroups: NF4 14336 x 4096, 64 / 128 / 512 tokens 22 / 38 / 105 us in 64-token tiles,
+    // 25 / 30 / 81 in 128-token ones (a wave per stripe and block, or 16 rows x 64 tokens per
+    // wave: 31 / 41 / 94); 2048 x 8192, 512 tokens (256 workgroups of 128) 38 and 42.5.
+    if (ks) {
+        const dim3 blk(64 * kKsWaves);
+        const int nb = B <= 1 ? 1 : B == 2 ? 2 : 4;
+        const dim3 grid(S, (B + nb - 1) / nb);
+        if (nb == 1) hipLaunchKernelGGL((gemm_ks_kernel<FMT, HP, 1>), grid, blk, 0, st, A);
+        else if (nb == 2) hipLaunchKernelGGL((gemm_ks_kernel<FMT, HP, 2>), grid, blk, 0, st, A);
+        else hipLaunchKernelGGL((gemm_ks_kernel<FMT, HP, 4>), grid, blk, 0, st, A);
+    } else if (B <= 2) {
+        // two blocks per wave only where that leaves 8 waves per CU
+        const int nb = B == 2 && S >= 2048 ? 2 : 1;
+        const dim3 grid((S + 3) / 4, (B + nb - 1) / nb);
+        if (nb == 1) hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 1, kMfmaDepth>), grid, dim3(256), 0, st, A);
+        else hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 2, kMfmaDepth>), grid, dim3(256), 0, st, A);
+    } else if (B >= 8 && (long)((S + 1) / 2) * ((B + 7) / 8) >= 448) {
+        launch_tile<FMT, HP, 1, 2, 1, 0>(st, A);
+    } else {
+        launch_tile<FMT, HP, 1, 1, 3, 0>(st, A);
+    }
+}
+
+template <int FMT, int HP>
+static void launch_swiglu_fmt(hipStream_t st, const MfArgs &A) {
+    if ((long)A.nci * ((A.nblk + 7) / 8) >= 384) launch_tile<FMT, HP, 4, 2, 1, 1>(st, A);
+    else launch_tile<FMT, HP, 4, 1, 1, 1>(st, A);
+}
+
+template <int FMT, int HP>
+static void launch_qkv_fmt(hipStream_t st, const MfArgs &A) {
+    // A head and 16 tokens per workgroup while those are few: 48 heads, K 2048, 128 tokens (384
+    // workgroups) 3.5 us a layer less than 64-token tiles, 512 tokens 14 us more.
+    const dim3 grid(A.stripes / 4, A.nblk);
+    if (grid.x * grid.y <= 512) hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 1, kMfmaDepth, true>), grid, dim3(256), 0, st, A);
+    else launch_tile<FMT, HP, 2, 1, 2, 2>(st, A);
 }
 
 void launch_gemm_mfma(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const float *xs, const int32_t *xsum,
                       int ntok, float *out, size_t out_stride, bool accum, ActTiles tiles) {
     if (!gemm_mfma_supported(m, ntok)) throw Error(K2T_E_INTERNAL, "mfma gemm: unsupported matrix");
     MfArgs A;
-    const int nb = mfma_args(ctx, m, xq, xs, xsum, ntok, tiles, A);
+    mfma_args(ctx, m, xq, xs, xsum, ntok, tiles, A);
     A.out = out;
     A.out_stride = out_stride;
     A.accum = accum ? 1 : 0;
-    const dim3 grid((m->stripes + 3) / 4, (ntok + 16 * nb - 1) / (16 * nb));
-    hipStream_t st = ctx->stream;
-    if (m->fmt == K2T_FMT_NF && m->bits == 3) launch_gemm_mfma_fmt<2, 0>(st, nb, grid, A);
-    else if (m->fmt == K2T_FMT_NF) launch_gemm_mfma_fmt<1, 0>(st, nb, grid, A);
-    else if (m->hp == 0) launch_gemm_mfma_fmt<0, 0>(st, nb, grid, A);
-    else if (m->hp == 1) launch_gemm_mfma_fmt<0, 1>(st, nb, grid, A);
-    else launch_gemm_mfma_fmt<0, 2>(st, nb, grid, A);
+    MF_FORMATS(m, launch_plain_fmt, ctx->stream, ks_split(m, A.nblk), A);
     hip_check(hipGetLastError(), "mfma gemm launch");
-}
-
-template <int FMT, int HP>
-static void launch_qkv_fmt(hipStream_t st, int nb, dim3 grid, const MfArgs &A) {
-    const dim3 blk(256);
-    switch (nb) {
-        case 1: hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 1, kMfmaDepth, false, false, true>), grid, blk, 0, st, A); break;
-        case 2: hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 2, kMfmaDepth, false, false, true>), grid, blk, 0, st, A); break;
-        case 3: hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 3, kMfmaDepth, false, false, true>), grid, blk, 0, st, A); break;
-        default: hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 4, kMfmaShDepth, true, false, true>), grid, blk, 0, st, A);
-    }
 }
 
 bool launch_gemm_mfma_qkv(k2t_ctx *ctx, const k2t_mat *qkv, ActTiles tiles, int ntok, float *out, size_t out_stride,
@@ -855,47 +1231,31 @@ bool launch_gemm_mfma_qkv(k2t_ctx *ctx, const k2t_mat *qkv, ActTiles tiles, int 
     if (!gemm_mfma_supported(qkv, ntok) || !tiles.xt || qkv->rows % 64 != 0) return false;
     if (qkv->fmt == K2T_FMT_NIBBLE4 && !tiles.ut) return false;
     MfArgs A;
-    const int nb = std::min(4, mfma_args(ctx, qkv, nullptr, nullptr, nullptr, ntok, tiles, A));
+    mfma_args(ctx, qkv, nullptr, nullptr, nullptr, ntok, tiles, A);
     A.out = out;
     A.out_stride = out_stride;
     A.qp = qp;
-    const dim3 grid(qkv->rows / 64, (ntok + 16 * nb - 1) / (16 * nb));
-    hipStream_t st = ctx->stream;
-    if (qkv->fmt == K2T_FMT_NF && qkv->bits == 3) launch_qkv_fmt<2, 0>(st, nb, grid, A);
-    else if (qkv->fmt == K2T_FMT_NF) launch_qkv_fmt<1, 0>(st, nb, grid, A);
-    else if (qkv->hp == 0) launch_qkv_fmt<0, 0>(st, nb, grid, A);
-    else if (qkv->hp == 1) launch_qkv_fmt<0, 1>(st, nb, grid, A);
-    else launch_qkv_fmt<0, 2>(st, nb, grid, A);
+    MF_FORMATS(qkv, launch_qkv_fmt, ctx->stream, A);
     hip_check(hipGetLastError(), "mfma qkv launch");
     return true;
-}
-
-template <int FMT, int HP>
-static void launch_swiglu_fmt(hipStream_t st, dim3 grid, const MfArgs &A) {
-    hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 4, kMfmaShDepth, true, true>), grid, dim3(512), 0, st, A);
 }
 
 bool launch_gemm_mfma_swiglu(k2t_ctx *ctx, const k2t_mat *gu, ActTiles tiles, int ntok, int8_t *q, float *s,
                              int32_t *sums, ActTiles out_tiles) {
     if (!gemm_mfma_supported(gu, ntok) || !tiles.xt || !out_tiles.xt || gu->rows % 128 != 0) return false;
     if (gu->fmt == K2T_FMT_NIBBLE4 && !tiles.ut) return false;
-    // Only where the plain GEMV would take 64-token workgroups anyway: forcing them on a
-    // small gate_up (135M: 3072 rows, 768 waves at 256 tokens) cost more than the launch
-    // the fusion saves (135M prefill 130k -> 123k tok/s).
+    // 512 or more workgroups of 128 rows x 64 tokens; with fewer the plain launch and the
+    // activation's own spread better: 16384 x 2048 NF4, two layers, 512 / 256 tokens 403 / 282 us
+    // apart and 375 / 275 fused; 128 / 64 tokens (256 / 128 workgroups) 219 / 202 and 228 / 222.
+    if ((long)(gu->rows / 128) * ((ntok + 63) / 64) < 512) return false;
     MfArgs A;
-    if (mfma_args(ctx, gu, nullptr, nullptr, nullptr, ntok, tiles, A) != 4) return false;
+    mfma_args(ctx, gu, nullptr, nullptr, nullptr, ntok, tiles, A);
     A.sq = q;
     A.ss = s;
     A.ssum = sums;
     A.stiles = out_tiles;
     A.nci = gu->rows / 128;
-    const dim3 grid(gu->rows / 128, (ntok + 63) / 64);
-    hipStream_t st = ctx->stream;
-    if (gu->fmt == K2T_FMT_NF && gu->bits == 3) launch_swiglu_fmt<2, 0>(st, grid, A);
-    else if (gu->fmt == K2T_FMT_NF) launch_swiglu_fmt<1, 0>(st, grid, A);
-    else if (gu->hp == 0) launch_swiglu_fmt<0, 0>(st, grid, A);
-    else if (gu->hp == 1) launch_swiglu_fmt<0, 1>(st, grid, A);
-    else launch_swiglu_fmt<0, 2>(st, grid, A);
+    MF_FORMATS(gu, launch_swiglu_fmt, ctx->stream, A);
     hip_check(hipGetLastError(), "mfma gate_up + swiglu launch");
     return true;
 }

@@ -138,6 +138,11 @@ void launch_swiglu_act(hipStream_t st, const uint64_t *signs, const float *gu, i
 // more tokens of a ready int8 activation, outputs equal to the exact-order GEMV's.
 constexpr int kMfmaMinTokens = 16;
 bool gemm_mfma_supported(const k2t_mat *m, int ntok);
+// Whether an NF3 matrix takes the 4-token passes of gemv_kernel instead when no producer wrote
+// the tiles: small products, where the copy into tiles costs more than the passes (NF3 1000 x
+// 4096, 16 tokens 6.2 us and 8.6; 8192 x 512, 32 tokens 6.7 and 7.3; 64 tokens 11.3 and 7.6:
+// not taken), and captures whose context has no scratch for the copy yet.
+bool gemm_mfma_nf3_passes(k2t_ctx *ctx, const k2t_mat *m, int ntok);
 void launch_gemm_mfma(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const float *xs, const int32_t *xsum,
                       int ntok, float *out, size_t out_stride, bool accum, ActTiles tiles = ActTiles{});
 // 2 .. 15 tokens with the fast epilogue on the matrix cores: plan_gemv's split, the sums in
@@ -163,8 +168,8 @@ void launch_gemv_mfma_grouped(k2t_ctx *ctx, const k2t_mat *geom, const GvGroup &
                               const float *xs, float *out, size_t out_stride);
 // gate_up (interleaved [gate64, up64] blocks) from producer tiles with the SwiGLU + FWHT +
 // int8 of the down input (q / s / sums [token][rows / 128], its tiles into out_tiles,
-// which must not be `tiles`) as the epilogue; false (nothing launched) when the plain
-// launch would not take 64-token workgroups, or for other shapes.
+// which must not be `tiles`) as the epilogue; false (nothing launched) when too few
+// workgroups would run, or for other shapes.
 bool launch_gemm_mfma_swiglu(k2t_ctx *ctx, const k2t_mat *gu, ActTiles tiles, int ntok, int8_t *q, float *s,
                              int32_t *sums, ActTiles out_tiles);
 void launch_gemv_grouped(k2t_ctx *ctx, const k2t_mat *geom, const GemvGroup &g, int xs_mode, const float *src,
