@@ -963,6 +963,111 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
     }
 }
 
+// The grouped form where an expert's matrix is split by stripes and a wave's K segment is at most
+// 8 chunks (one per accumulator of the GEMV's order: most experts): a workgroup takes one item
+// and R stripes after each other, its activation in registers for all of them.  With a
+// workgroup per stripe the gather of the activation rows and scales (16 lines a load) kept
+// the address units busy 73% of the time; the weights alone are 3 or 2 loads per chunk.
+// (Two thirds of a wave's time is still waiting for them.)
+template <int FMT>
+__global__ __launch_bounds__(1024) void gemv_mfma_items_kernel(GvArgs A, int R) {
+    constexpr int G = 8;
+    constexpr uint32_t CB = FMT == 2 ? 384u : 512u;  // bytes per stripe-chunk
+    extern __shared__ float part[];                  // [2][nseg][16 tokens][17]
+    const uint32_t lane = threadIdx.x & 63u, li = lane & 15u, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if ((int)blockIdx.y >= A.grp.n_items[0]) return;  // uniform: the grid covers the most items possible
+    const int4 item = A.grp.items[blockIdx.y];        // expert, first entry of the pair list, pairs
+    const uint8_t *rec0 = A.grp.bank + (size_t)item.x * A.grp.bank_stride;
+    const MfLane L = mf_lane<FMT, 0>(lane, false, 0u, A.lane);
+    const __amdgpu_buffer_rsrc_t rw = mf_rsrc(rec0 + A.grp.mat_off), rx = mf_rsrc(A.xq), rs = mf_rsrc(A.xs);
+    const int cw0 = wave * A.cps, cw1 = min(A.nc, cw0 + A.cps), n = cw1 - cw0;
+    struct Wt {
+        uint32_t d0, d1, hv;
+        uint2 sw;
+    };
+    const int s_first = (int)blockIdx.x * R, s_last = min(s_first + R, 2 * A.np) - 1;
+    auto fetch = [&](Wt &f, int stripe, int u) {
+        const int c = min(cw0 + u, cw1 - 1);
+        uint32_t rec, sgb;
+        mf_record<FMT, 0>(A.sgc_log2, false, c, rec, sgb);
+        const uint32_t base = (uint32_t)(stripe >> 1) * (uint32_t)A.ptot, side = (uint32_t)(stripe & 1);
+        const uint32_t code = base + rec + side * CB;
+        f.d0 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw, L.a_off, code, 0);
+        f.d1 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw, L.b_off, code, 0);
+        if constexpr (FMT == 2) f.hv = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw, L.h_off, code, 0);
+        const v2u sw = __builtin_amdgcn_raw_buffer_load_b64(rw, L.s_off, base + sgb + side * 32u, 0);
+        f.sw = make_uint2(sw[0], sw[1]);
+    };
+    Wt wt[G];
+    v4i x[G];
+    float sx[G];
+#pragma unroll
+    for (int u = 0; u < G; u++)
+        if (u < n) fetch(wt[u], s_first, u);
+    __builtin_amdgcn_sched_barrier(0);
+    const int nt = item.z;
+    const uint32_t pr = (uint32_t)A.grp.list[item.y + (int)min(li, (uint32_t)nt - 1u)], tok = pr / (uint32_t)A.grp.row_div;
+    // (kept in LDS: a global load in the stripes' loop would wait for the weights in flight)
+    __shared__ uint32_t pairs[16];
+    if (threadIdx.x < 16) pairs[threadIdx.x] = pr;
+    const uint32_t x_off = tok * (uint32_t)A.K + lg * 16u, sx_off = tok * (uint32_t)A.nc * 4u;
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+        if (u >= n) break;  // (uniform)
+        const uint32_t c = (uint32_t)(cw0 + u);
+        const v4u xv = __builtin_amdgcn_raw_buffer_load_b128(rx, x_off, c * 64u, 0);
+        x[u] = v4i{(int)xv[0], (int)xv[1], (int)xv[2], (int)xv[3]};
+        sx[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, sx_off, c * 4u, 0));
+    }
+    const uint4 cb = *reinterpret_cast<const uint4 *>(rec0 + A.grp.cb_off);
+    if constexpr (FMT == 1) nf4_xor_tables(cb.x, cb.y, cb.z, cb.w, A.t0, A.t1, A.u0, A.u1);
+    else A.t0 = cb.x, A.t1 = cb.y;
+    for (int stripe = s_first; stripe <= s_last; stripe++) {
+        float acc[G][4];
+#pragma unroll
+        for (int u = 0; u < G; u++) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[u][r] = 0.0f;
+            if (u < n) {
+                const v4i a = mf_decode<FMT, 0>(wt[u].d0, wt[u].d1, wt[u].hv, A.t0, A.t1, A.u0, A.u1, lane);
+                const v4i zero = {0, 0, 0, 0};
+                const v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, x[u], zero, 0, 0, 0);
+                const float ws[4] = {bf16_lo(wt[u].sw.x), bf16_hi(wt[u].sw.x), bf16_lo(wt[u].sw.y), bf16_hi(wt[u].sw.y)};
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[u][r] = fmaf((float)d[r] * sx[u], ws[r], 0.0f);
+                __builtin_amdgcn_sched_barrier(0);
+                fetch(wt[u], min(stripe + 1, s_last), u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        float *pt = part + (size_t)(stripe & 1) * A.nseg * 16 * 17;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            float v[G];
+#pragma unroll
+            for (int g = 0; g < G; g++) v[g] = acc[g][r];
+#pragma unroll
+            for (int w = G; w > 1; w >>= 1)
+#pragma unroll
+                for (int g = 0; g < w / 2; g++) v[g] = v[2 * g] + v[2 * g + 1];
+            pt[((size_t)wave * 16 + li) * 17 + 4 * lg + r] = v[0];
+        }
+        __syncthreads();
+        for (int idx = (int)threadIdx.x; idx < nt * 16; idx += (int)blockDim.x) {
+            const int t = idx >> 4, row = stripe * 16 + (idx & 15);
+            float v = pt[(size_t)t * 17 + (idx & 15)];
+            for (int w = 1; w < A.nseg; w++) v += pt[((size_t)w * 16 + t) * 17 + (idx & 15)];
+            int r = row;  // gate / up rows in blocks of 64
+            if (A.grp.gu_split) {
+                const int inter = A.rows >> 1, up = row >= inter ? 1 : 0, rr = row - up * inter;
+                r = (rr >> 6) * 128 + up * 64 + (rr & 63);
+            }
+            A.out[(size_t)pairs[t] * A.out_stride + r] = v;
+        }
+    }
+}
+
 }  // namespace
 
 // Lookup words of an NF matrix: NF4's XOR tables, NF3's codebook (bit planes: none).
@@ -1039,9 +1144,23 @@ void launch_gemv_mfma_grouped(k2t_ctx *ctx, const k2t_mat *geom, const GvGroup &
     const GemvPlan plan = plan_gemv(ctx, geom, 0, geom->stripes);
     GvArgs A = gemv_mfma_args(geom, plan, xq, xs, nullptr, out, out_stride);
     A.grp = g;
-    const dim3 grid(plan.rb_hi - plan.rb_lo, max_items), block(64 * plan.nseg);
-    const size_t lds = gemv_mfma_lds(plan);
+    const dim3 block(64 * plan.nseg);
     hipStream_t st = ctx->stream;
+    // Items that are half full or more (the rows to gather are what the loop over stripes saves)
+    // and two waves per SIMD with that: per layer, 300 tokens with 8 of 128 experts 396 -> 347 us
+    // NF3; 96 tokens 212 -> 210 NF3, 208 -> 212 NF4; 32 tokens 147 -> 154.
+    constexpr int R = 4;  // 2 / 8 stripes: 367 / 359 us
+    const int groups = (geom->stripes + R - 1) / R;
+    if (plan.stripe_mode && plan.cps <= 8 && g.pairs >= 8 * g.experts && (long)groups * max_items * plan.nseg >= 2048) {
+        const dim3 grid(groups, max_items);
+        const size_t lds = (size_t)2 * plan.nseg * 16 * 17 * sizeof(float);
+        if (geom->bits == 3) hipLaunchKernelGGL((gemv_mfma_items_kernel<2>), grid, block, lds, st, A, R);
+        else hipLaunchKernelGGL((gemv_mfma_items_kernel<1>), grid, block, lds, st, A, R);
+        hip_check(hipGetLastError(), "grouped mfma gemv launch");
+        return;
+    }
+    const dim3 grid(plan.rb_hi - plan.rb_lo, max_items);
+    const size_t lds = gemv_mfma_lds(plan);
     if (geom->bits == 3 && plan.stripe_mode) hipLaunchKernelGGL((gemv_mfma_kernel<2, 0, true, true>), grid, block, lds, st, A);
     else if (geom->bits == 3) hipLaunchKernelGGL((gemv_mfma_kernel<2, 0, false, true>), grid, block, lds, st, A);
     else if (plan.stripe_mode) hipLaunchKernelGGL((gemv_mfma_kernel<1, 0, true, true>), grid, block, lds, st, A);

@@ -161,6 +161,7 @@ struct GvGroup {
     size_t bank_stride = 0;
     uint32_t mat_off = 0, cb_off = 0;
     int gu_split = 0;
+    int pairs = 0, experts = 0;  // of the whole launch
 };
 constexpr int kGvItemPairs = 16;
 bool gemv_mfma_grouped_supported(const k2t_mat *geom);

@@ -498,7 +498,9 @@ void launch_moe_ffn(k2t_ctx *ctx, const MoeLayer &L, float *hidden, const float 
 //   4. the combine, per token as before.
 // The arithmetic of each step is the one-token path's in its order (the GEMV's fast sums
 // included, gemv_mfma_kernel), so a prompt's tokens get the bits that decoding them gives.
-constexpr int kRouteTokens = 16;  // tokens per router wave
+// Tokens per router wave: 96 tokens over 128 experts, two layers with 16 / 8 / 4 / 2 tokens 424 / 404 /
+// 407 / 420 us (more waves hide the reductions, fewer read the router rows less often).
+constexpr int kRouteTokens = 8;
 
 __global__ __launch_bounds__(256) void moe_logits_batch_kernel(const float *__restrict__ x, int ntok,
                                                                const float *__restrict__ nw, int d,
@@ -688,6 +690,8 @@ void launch_moe_ffn_batch(k2t_ctx *ctx, const MoeLayer &L, float *hidden, int nt
     g.mat_off = (uint32_t)b->lay.gu_pair_off;
     g.cb_off = (uint32_t)b->lay.gu_cb_off;
     g.gu_split = 1;
+    g.pairs = P;
+    g.experts = E;
     const int max_items = std::min(P, E + P / kGvItemPairs);  // at most one partial item per expert
     launch_gemv_mfma_grouped(ctx, &b->gu, g, max_items, ws.aq, ws.as, ws.gu, (size_t)2 * dff);
     launch_swiglu_act(st, ctx->signs, ws.gu, dff, P, ws.mq, ws.ms, ws.msum, false);

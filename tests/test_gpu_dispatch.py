@@ -223,10 +223,12 @@ def test_prefill_epilogues_equal_separate_kernels(gpu_ctx, fmt, planes, kv_bits,
 
 
 # all experts used by every token (items of 16 and a remainder), and few tokens over many
-# experts; the wide router (d > 2048); a shared expert; more tokens than one MoE call takes
+# experts; the wide router (d > 2048); a shared expert; more tokens than one MoE call takes; enough
+# pairs per expert for a workgroup to take several stripes
 @pytest.mark.parametrize("bits,E,k,d,ntok,max_batch,shared", [(3, 4, 4, 256, 40, 64, False), (4, 16, 3, 256, 2, 8, False),
                                                               (3, 32, 6, 256, 15, 15, True), (4, 8, 2, 2112, 9, 16, False),
-                                                              (3, 4, 2, 256, 37, 8, True)])
+                                                              (3, 4, 2, 256, 37, 8, True), (3, 4, 4, 320, 500, 500, False),
+                                                              (4, 4, 4, 576, 500, 500, False)])
 def test_moe_prompt_equals_token_by_token(gpu_ctx, bits, E, k, d, ntok, max_batch, shared):
     """A prompt through sparse-MoE layers (tokens grouped by expert) gives the logits of
     decoding its tokens one by one, bit for bit.  (Three-chunk scale groups and the NF4 KV
@@ -234,10 +236,10 @@ def test_moe_prompt_equals_token_by_token(gpu_ctx, bits, E, k, d, ntok, max_batc
     expert's matrices likewise.)"""
     from k2tb_writer import random_moe_layer, write_k2tm
     from model_oracle import quantize_matrix
-    cfg = dict(n_layers=2, hidden=d, n_heads=4, n_kv_heads=2, head_dim=64, intermediate=64, vocab=300, max_seq=64,
+    cfg = dict(n_layers=2, hidden=d, n_heads=4, n_kv_heads=2, head_dim=64, intermediate=64, vocab=300, max_seq=512,
                rms_eps=1e-6, rope_theta=10000.0)
     rng = np.random.default_rng(E * 100 + ntok)
-    dff, hd = 192, 64
+    dff, hd = 192 if ntok < 500 else 1088, 64
     w = lambda r, c: (rng.standard_normal((r, c)) * 0.02).astype(np.float32)  # noqa: E731
     moe = [random_moe_layer(rng, d, dff, E, bits=bits) for _ in range(2)]
     bank = k2t.ExpertBank.upload(gpu_ctx, write_k2tm([m[0] for m in moe], d, dff, bits, 2))
