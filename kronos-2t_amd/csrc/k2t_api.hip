@@ -240,10 +240,15 @@ int32_t k2t_ctx_create(int32_t device, k2t_ctx **out) {
         for (int b = 0; b < kSignBlocks; b++) masks[b] = hadamard_sign_mask_host((uint64_t)b);
         hipError_t e = hipMalloc(&c->signs, sizeof(masks));
         if (e == hipSuccess) e = hipMemcpy(c->signs, masks, sizeof(masks), hipMemcpyHostToDevice);
+        const size_t moe_bytes = kMoeStateWords * sizeof(unsigned long long);
+        if (e == hipSuccess) e = hipMalloc(&c->moe_state, moe_bytes);
+        if (e == hipSuccess) e = hipMemset(c->moe_state, 0, moe_bytes);
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
         if (e != hipSuccess) {
             if (c->signs) (void)hipFree(c->signs);
+            if (c->moe_state) (void)hipFree(c->moe_state);
             delete c;
-            hip_check(e, "sign table");
+            hip_check(e, "context tables");
         }
         *out = c;
     });
@@ -256,6 +261,7 @@ void k2t_ctx_destroy(k2t_ctx *ctx) {
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     if (ctx->span_words) (void)hipFree(ctx->span_words);
     if (ctx->signs) (void)hipFree(ctx->signs);
+    if (ctx->moe_state) (void)hipFree(ctx->moe_state);
     delete ctx;
 }
 

@@ -23,11 +23,16 @@ struct k2t_ctx {
     // allocated), then its counters {epoch, merges done} and timeout word
     unsigned long long *span_words = nullptr;
     size_t span_cap = 0;  // words
+    // hand-off words of k2t_moe_ffn's routing (kMoeStateWords, zeroed at creation): {epoch, value}
+    // words that no later call's epoch matches, then the call counter and the timeout word
+    unsigned long long *moe_state = nullptr;
     // Hadamard sign masks of 64-blocks 0..kSignBlocks-1 (bit i = sign of element i),
     // uploaded at creation for the GEMV's fused activation builder.
     uint64_t *signs = nullptr;
 };
 constexpr int kSignBlocks = 512;  // K <= 32768
+// moe_state: 2 E + 2 words of up to 256 experts, the published route, counter and timeout word
+constexpr size_t kMoeStatePub = 2 * 256 + 2, kMoeStateWords = kMoeStatePub + K2T_MOE_MAX_TOPK + 1;
 
 enum k2t_fmt : int32_t { K2T_FMT_NIBBLE4 = 1, K2T_FMT_NF = 2 };
 

@@ -51,6 +51,9 @@ struct MoeWork {
     int *ids;                   // [top_k]
     uint32_t *ctr;              // route-call counter (epoch source)
     int *err;                   // raised when the route wait times out
+    int *out_ids = nullptr;     // where the combine copies the sorted route and its weights to, if
+    float *out_wts = nullptr;   // anywhere
+    bool clear_err = false;     // the combine resets err (a call of its own, not a model's layer)
     // exact-order mode (the context's exact flag): inv_rms, the int8 activation of x_norm
     // and the slots' down activations
     float *rms;
@@ -59,10 +62,9 @@ struct MoeWork {
     int32_t *asum, *msum;
 };
 
-// Workspace size; the words and the counter must start zeroed (model: at allocation;
-// the standalone entry point: launch_moe_clear before each call).
+// Workspace size; the words and the counter must start zeroed (model: at allocation; the
+// standalone entry point has its own in the context).
 size_t moe_work_floats(const k2t_experts *b, int top_k);
-void launch_moe_clear(hipStream_t st, const MoeWork &ws, int E);
 MoeWork moe_work_carve(float *base, const k2t_experts *b, int top_k);
 void check_moe_args(const k2t_experts *bank, int shard_layer, int top_k, int scoring);
 

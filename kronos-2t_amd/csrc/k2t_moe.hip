@@ -139,22 +139,6 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float *__restrict_
     if (lane == 0) *ctr = epoch;
 }
 
-// Clears the hand-off words and the call counter of a fresh workspace (a kernel, so that a
-// captured graph holds no memset node).
-__global__ void moe_clear_kernel(unsigned long long *words, int E, unsigned long long *pub, uint32_t *ctr, int *err) {
-    for (int i = (int)threadIdx.x; i < 2 * E + 2; i += (int)blockDim.x) words[i] = 0ull;
-    if (threadIdx.x < K2T_MOE_MAX_TOPK) pub[threadIdx.x] = 0ull;
-    if (threadIdx.x == 0) {
-        *ctr = 0u;
-        *err = 0;
-    }
-}
-
-void launch_moe_clear(hipStream_t st, const MoeWork &ws, int E) {
-    hipLaunchKernelGGL(moe_clear_kernel, dim3(1), dim3(256), 0, st, ws.words, E, ws.pub, ws.ctr, ws.err);
-    hip_check(hipGetLastError(), "moe clear launch");
-}
-
 // out.fill(0); out += w_z * expert_z in route order; hidden += out
 // (sparse_moe.rs:1001-1003, 1041-1043; real_llm.rs:6714).
 // Up to kCombineMax slots have all their loads in flight together (slot min(z, k - 1) is
@@ -163,15 +147,27 @@ void launch_moe_clear(hipStream_t st, const MoeWork &ws, int E) {
 constexpr int kCombineMax = 8;
 // With ctr set, thread 0 advances the route-call counter (routing ran inside the gate_up
 // launch, whose workgroups have all read it by now).
+// A one-token call's copies of the route (ids, weights) and the reset of its timeout word are
+// co's: as copies of their own, and with a clearing launch before the routing, they took 5.6
+// of the call's 26.9 us (d 2048, 8 of 128 NF3 experts).
 // With a shared expert (sh != NULL) the sum starts from its output, times the gate scale
 // when a gate is present and the scale differs from 1 by more than FLT_EPSILON
 // (forward_single then forward_layer_single, sparse_moe.rs:252-312, 989-1000).
+struct MoeCombineOut {
+    const int *route = nullptr;
+    int *ids = nullptr;
+    float *wts = nullptr;
+    int *err = nullptr;
+};
 __global__ __launch_bounds__(256) void moe_combine_kernel(float *__restrict__ hidden, const float *__restrict__ eo,
                                                           const float *__restrict__ wts, int k, int d,
                                                           uint32_t *__restrict__ ctr, const float *__restrict__ sh,
-                                                          const float *__restrict__ sh_scale) {
+                                                          const float *__restrict__ sh_scale, MoeCombineOut co) {
     const int r = (int)blockIdx.x * 256 + (int)threadIdx.x;
     if (ctr && r == 0) *ctr = *ctr + 1u;  // (one token)
+    if (r < k && co.ids) co.ids[r] = co.route[r];
+    if (r < k && co.wts) co.wts[r] = wts[r];
+    if (r == 0 && co.err) *co.err = 0;
     if (r >= d) return;
     const size_t t = blockIdx.y;  // token of the batch
     hidden += t * d;
@@ -200,6 +196,10 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(float *__restrict__ hi
     }
     for (int z = 0; z < k; z++) p = p + wts[z] * eo[(size_t)z * d + r];
     hidden[r] = hidden[r] + p;
+}
+
+static MoeCombineOut combine_out(const MoeWork &ws) {
+    return MoeCombineOut{ws.ids, ws.out_ids, ws.out_wts, ws.clear_err ? ws.err : nullptr};
 }
 
 // Exact-order routing (the x86 reference's order; one workgroup): x_norm[i] = (h[i] *
@@ -408,7 +408,7 @@ static void launch_moe_ffn_exact(k2t_ctx *ctx, const MoeLayer &L, float *hidden,
     g.slot_act = 1;
     launch_gemv_grouped(ctx, &b->dn, g, 0, nullptr, nullptr, 0.0f, ws.eo);
     hipLaunchKernelGGL(moe_combine_kernel, dim3((d + 255) / 256), dim3(256), 0, st, hidden, ws.eo, ws.wts, L.top_k,
-                       d, nullptr, sh_out, sh_scale);
+                       d, nullptr, sh_out, sh_scale, combine_out(ws));
     hip_check(hipGetLastError(), "moe combine launch");
 }
 
@@ -481,7 +481,7 @@ void launch_moe_ffn(k2t_ctx *ctx, const MoeLayer &L, float *hidden, const float 
     g.gu_split = 0;
     launch_gemv_grouped(ctx, &b->dn, g, K2T_XS_SWIGLU, ws.gu, nullptr, 0.0f, ws.eo);
     hipLaunchKernelGGL(moe_combine_kernel, dim3((d + 255) / 256), dim3(256), 0, st, hidden, ws.eo, ws.wts, L.top_k,
-                       d, fused ? ws.ctr : nullptr, sh_out, sh_scale);
+                       d, fused ? ws.ctr : nullptr, sh_out, sh_scale, combine_out(ws));
     hip_check(hipGetLastError(), "moe combine launch");
 }
 
@@ -701,7 +701,7 @@ void launch_moe_ffn_batch(k2t_ctx *ctx, const MoeLayer &L, float *hidden, int nt
     g.gu_split = 0;
     launch_gemv_mfma_grouped(ctx, &b->dn, g, max_items, ws.mq, ws.ms, ws.eo, (size_t)d);
     hipLaunchKernelGGL(moe_combine_kernel, dim3((d + 255) / 256, ntok), dim3(256), 0, st, hidden, ws.eo, ws.wts, k, d,
-                       nullptr, sh_out, sh_scale);
+                       nullptr, sh_out, sh_scale, MoeCombineOut{});
     hip_check(hipGetLastError(), "moe combine launch");
 }
 
@@ -927,17 +927,26 @@ int32_t k2t_moe_ffn(k2t_ctx *ctx, const k2t_experts *bank, int32_t shard_layer, 
         if (bank->ctx != ctx) throw Error(K2T_E_ARG, "expert bank of another context");
         MoeLayer L{bank, shard_layer, d_router_w, d_router_bias, top_k, norm_topk_prob ? 1 : 0, scoring};
         ensure_scratch(ctx, moe_work_floats(bank, top_k));
-        const MoeWork ws = moe_work_carve(ctx->scratch, bank, top_k);
-        launch_moe_clear(ctx->stream, ws, (int)bank->hdr.experts_per_layer);  // the scratch is shared
-        launch_moe_ffn(ctx, L, d_hidden, d_post_norm, eps, ws);
-        if (d_route_ids)
-            hip_check(hipMemcpyAsync(d_route_ids, ws.ids, (size_t)top_k * sizeof(int), hipMemcpyDeviceToDevice,
-                                     ctx->stream),
-                      "route copy");
-        if (d_route_weights)
-            hip_check(hipMemcpyAsync(d_route_weights, ws.wts, (size_t)top_k * sizeof(float), hipMemcpyDeviceToDevice,
-                                     ctx->stream),
-                      "route copy");
+        MoeWork ws = moe_work_carve(ctx->scratch, bank, top_k);
+        // the hand-off words are the context's own: the scratch is shared, so in it they would
+        // have to be cleared by a launch before every call
+        ws.words = ctx->moe_state;
+        ws.pub = ctx->moe_state + kMoeStatePub;
+        ws.ctr = reinterpret_cast<uint32_t *>(ctx->moe_state + kMoeStatePub + K2T_MOE_MAX_TOPK);
+        ws.err = reinterpret_cast<int *>(ws.ctr + 1);
+        ws.out_ids = d_route_ids;
+        ws.out_wts = d_route_weights;
+        ws.clear_err = true;
+        try {
+            launch_moe_ffn(ctx, L, d_hidden, d_post_norm, eps, ws);
+        } catch (...) {
+            // a part of the launches may have left words of an epoch that the counter has not passed
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
+                hipStreamSynchronize(ctx->stream) == hipSuccess)
+                (void)hipMemset(ctx->moe_state, 0, kMoeStateWords * sizeof(unsigned long long));
+            throw;
+        }
     });
 }
 

@@ -356,3 +356,45 @@ def test_span_attention_in_decode_steps(gpu_ctx, nq, nkv, hd, bits, window):
     assert cos.min() > 0.9998 and np.isfinite(a).all()
     for x in [hm] + [x for r in mats for x in r]:
         x.close()
+
+
+# banks of different expert counts on one context (its hand-off words are shared), calls with and
+# without the route's outputs, the wide router (d > 2048)
+def test_moe_ffn_calls_share_the_context_state(gpu_ctx):
+    """Each call's hidden state and route equal those of the same call on a fresh context."""
+    import torch
+    from k2tb_writer import random_moe_layer, write_k2tm
+    rng = np.random.default_rng(77)
+    shapes = [(256, 128, 128, 8), (2112, 64, 8, 2), (256, 64, 16, 3)]
+    banks, calls = [], []
+    for d, dff, E, k in shapes:
+        exp, router = random_moe_layer(rng, d, dff, E, bits=3)
+        banks.append((write_k2tm([exp], d, dff, 3, 2), _t(np.asarray(router, np.float32)), d, k))
+
+    def run(ctx, bank, i, x, outs):
+        _, router, d, k = banks[i]
+        h, ids, wts = x.clone(), torch.full((k,), -1, dtype=torch.int32, device="cuda"), torch.full((k,), -1.0, device="cuda")
+        kw = dict(route_ids=ids, route_weights=wts) if outs else {}
+        ctx.moe_ffn(bank, 0, router, h, torch.ones(d, device="cuda"), 1e-5, k, **kw)
+        ctx.sync()
+        return h, ids, wts
+
+    shared = [k2t.ExpertBank.upload(gpu_ctx, b[0]) for b in banks]
+    xs = [_t(rng.standard_normal(b[2]).astype(np.float32)) for b in banks]
+    for i, outs in ((0, True), (1, True), (2, False), (0, False), (2, True), (1, False), (0, True)):
+        calls.append((i, outs, run(gpu_ctx, shared[i], i, xs[i], outs)))
+    want = []
+    for i, b in enumerate(banks):
+        ctx = k2t.Ctx(0)
+        bank = k2t.ExpertBank.upload(ctx, b[0])
+        want.append(run(ctx, bank, i, xs[i], True))
+        bank.close()
+        ctx.close()
+    for i, outs, got in calls:
+        assert torch.isfinite(got[0]).all() and torch.equal(got[0], want[i][0])
+        if outs:
+            assert torch.equal(got[1], want[i][1]) and torch.equal(got[2], want[i][2])
+        else:
+            assert (got[1] == -1).all() and (got[2] == -1).all()
+    for bank in shared:
+        bank.close()
