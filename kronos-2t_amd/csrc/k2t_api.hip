@@ -236,20 +236,18 @@ int32_t k2t_ctx_create(int32_t device, k2t_ctx **out) {
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0)
             c->num_cus = cus;
-        uint64_t masks[kSignBlocks];
-        for (int b = 0; b < kSignBlocks; b++) masks[b] = hadamard_sign_mask_host((uint64_t)b);
-        hipError_t e = hipMalloc(&c->signs, sizeof(masks));
-        if (e == hipSuccess) e = hipMemcpy(c->signs, masks, sizeof(masks), hipMemcpyHostToDevice);
-        const size_t moe_bytes = kMoeStateWords * sizeof(unsigned long long);
-        if (e == hipSuccess) e = hipMalloc(&c->moe_state, moe_bytes);
-        if (e == hipSuccess) e = hipMemset(c->moe_state, 0, moe_bytes);
-        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+        // one allocation and upload: the sign masks, then k2t_moe_ffn's zeroed hand-off words
+        static_assert(sizeof(unsigned long long) == sizeof(uint64_t), "one element type");
+        uint64_t tables[kSignBlocks + kMoeStateWords] = {};
+        for (int b = 0; b < kSignBlocks; b++) tables[b] = hadamard_sign_mask_host((uint64_t)b);
+        hipError_t e = hipMalloc(&c->signs, sizeof(tables));
+        if (e == hipSuccess) e = hipMemcpy(c->signs, tables, sizeof(tables), hipMemcpyHostToDevice);
         if (e != hipSuccess) {
             if (c->signs) (void)hipFree(c->signs);
-            if (c->moe_state) (void)hipFree(c->moe_state);
             delete c;
             hip_check(e, "context tables");
         }
+        c->moe_state = reinterpret_cast<unsigned long long *>(c->signs + kSignBlocks);
         *out = c;
     });
 }
@@ -261,7 +259,6 @@ void k2t_ctx_destroy(k2t_ctx *ctx) {
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     if (ctx->span_words) (void)hipFree(ctx->span_words);
     if (ctx->signs) (void)hipFree(ctx->signs);
-    if (ctx->moe_state) (void)hipFree(ctx->moe_state);
     delete ctx;
 }
 

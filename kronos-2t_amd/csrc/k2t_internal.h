@@ -23,8 +23,9 @@ struct k2t_ctx {
     // allocated), then its counters {epoch, merges done} and timeout word
     unsigned long long *span_words = nullptr;
     size_t span_cap = 0;  // words
-    // hand-off words of k2t_moe_ffn's routing (kMoeStateWords, zeroed at creation): {epoch, value}
-    // words that no later call's epoch matches, then the call counter and the timeout word
+    // hand-off words of k2t_moe_ffn's routing (kMoeStateWords after the sign masks, zeroed at
+    // creation): {epoch, value} words that no later call's epoch matches, then the call counter and
+    // the timeout word
     unsigned long long *moe_state = nullptr;
     // Hadamard sign masks of 64-blocks 0..kSignBlocks-1 (bit i = sign of element i),
     // uploaded at creation for the GEMV's fused activation builder.
