@@ -119,8 +119,10 @@ __global__ __launch_bounds__(kSpanThreads, HD == 128 && G8 ? 4 : 6) void attn_sp
         const unsigned long long *pp = A.words + (size_t)head * pstride;
         constexpr int ncg = HD / 4, nsub = NTH / ncg;
         const int cg = (int)tid % ncg, sub = (int)tid / ncg;
-        // spans per thread polled together (4: 127 VGPRs, and 13.0 -> 13.4 us at 52 spans)
-        constexpr int kPre = 2;
+        // spans per thread polled together; the large kernel has the registers for 3 (30B-A3B
+        // decode at 6600 positions, 52 spans: 420.6 tok/s with 2, 422 with 3, 419 with 4 at 127
+        // VGPRs)
+        constexpr int kPre = HD == 128 && G8 ? 3 : 2;
         bool ok = true;
         auto poll = [&](int s, unsigned long long (&w)[6]) {
             // (the caller keeps s < nact)
