@@ -88,10 +88,13 @@ __device__ inline void select_routes(float sc[4], int lane, int E, int k, int no
             sc[j] = lane + 64 * j < E && sc[j] == sc[j] ? 1.0f / (1.0f + expf(-sc[j])) : -INFINITY;
     }
     // Selection round r leaves its (id, score) in lane r's registers; a picked key is
-    // replaced by 0, below every real key (-inf's included), for the later rounds.
+    // replaced by 0, below every real key, for the later rounds.  So are the lanes past E:
+    // a softmax over no finite logit (a hidden state with NaNs, every bias -inf) gives NaN
+    // scores, which as keys may lie below -inf's; the k picks have to be k experts even so,
+    // since they index the bank's records and sort the pairs of a batch.
     unsigned long long key[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) key[j] = score_key(sc[j], lane + 64 * j);
+    for (int j = 0; j < 4; j++) key[j] = lane + 64 * j < E ? score_key(sc[j], lane + 64 * j) : 0ull;
     int my_id = 0;
     float my_w = 0.0f;
     for (int r = 0; r < k; r++) {
@@ -101,7 +104,7 @@ __device__ inline void select_routes(float sc[4], int lane, int E, int k, int no
         b = wave_max_key(b);
         const int bi = key_index(b);
         if (lane == r) {
-            my_id = min(bi, E - 1);  // every id indexes a record of the bank, whatever the scores
+            my_id = bi;  // (below E: k <= E lanes hold keys above 0)
             my_w = key_score(b);
         }
 #pragma unroll

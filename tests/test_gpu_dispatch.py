@@ -398,3 +398,62 @@ def test_moe_ffn_calls_share_the_context_state(gpu_ctx):
             assert (got[1] == -1).all() and (got[2] == -1).all()
     for bank in shared:
         bank.close()
+
+
+# the router in the gate_up launch (d <= 2048) and in its own (above); one token and a batch
+@pytest.mark.parametrize("d,E,k,scoring", [(256, 8, 4, 0), (256, 128, 8, 0), (256, 16, 16, 1), (256, 16, 3, 2), (2112, 8, 4, 0)])
+@pytest.mark.parametrize("bad", ["bias", "hidden"])
+def test_moe_routes_without_a_finite_logit(gpu_ctx, d, E, k, scoring, bad):
+    """Logits that are all -inf (bias) or NaN (hidden state): softmax scores are NaN then.  The
+    route is still k different experts of the bank in ascending order, a prompt with such a
+    token ends, and the model's next prompts are those of a model that never saw one."""
+    import torch
+    from k2tb_writer import random_moe_layer, write_k2tm
+    from model_oracle import quantize_matrix
+    rng = np.random.default_rng(d + E + scoring)
+    dff = 64
+    exp, router = random_moe_layer(rng, d, dff, E, bits=3)
+    bank = k2t.ExpertBank.upload(gpu_ctx, write_k2tm([exp], d, dff, 3, 2))
+    bias = np.full(E, -np.inf if bad == "bias" else 0.0, np.float32)
+    h = _t(rng.standard_normal(d).astype(np.float32))
+    if bad == "hidden":
+        h[5] = float("nan")
+    ids = torch.full((k,), -1, dtype=torch.int32, device="cuda")
+    for exact in (False, True):
+        gpu_ctx.set_exact(exact)
+        try:
+            gpu_ctx.moe_ffn(bank, 0, _t(np.asarray(router, np.float32)), h, torch.ones(d, device="cuda"), 1e-5, k,
+                            scoring=scoring, router_bias=_t(bias), route_ids=ids)
+            gpu_ctx.sync()
+        finally:
+            gpu_ctx.set_exact(False)
+        got = ids.cpu().numpy()
+        assert (np.diff(got) > 0).all() and got[0] >= 0 and got[-1] < E
+    cfg = dict(n_layers=1, hidden=d, n_heads=2, n_kv_heads=1, head_dim=64, intermediate=64, vocab=64, max_seq=64,
+               rms_eps=1e-6, rope_theta=10000.0)
+    m = k2t.Model(gpu_ctx, cfg, max_batch=32)
+    w = lambda r, c: (rng.standard_normal((r, c)) * 0.02).astype(np.float32)  # noqa: E731
+    mats = []
+    for r, c in ((4 * 64, d), (d, 2 * 64), (64, d)):
+        q = quantize_matrix(w(r, c), "nf4")
+        mats.append(gpu_ctx.upload_nf(r, c, 4, q.sgc, q.cb, q.pair, q.tail))
+    m.set_layer(0, mats[0], mats[1], None, None, np.ones(d, np.float32), np.ones(d, np.float32))
+    m.set_moe(0, bank, 0, np.asarray(router, np.float32), k, True, scoring, router_bias=bias if bad == "bias" else None)
+    m.set_head(mats[2], np.ones(d, np.float32))
+    rows = rng.standard_normal((64, d)).astype(np.float32)
+    if bad == "hidden":
+        rows[63] = np.nan
+    m.set_embedding(k2t.EMBED_F32, rows)
+    toks = np.arange(20, dtype=np.int32)
+    first = m.prefill(toks)
+    m.reset()
+    m.prefill(np.append(toks, 63).astype(np.int32))
+    m.decode(63)
+    m.reset()
+    again = m.prefill(toks)
+    assert np.array_equal(first.view(np.uint32), again.view(np.uint32))
+    assert bad == "bias" or np.isfinite(first).all()
+    m.close()
+    for x in mats:
+        x.close()
+    bank.close()
