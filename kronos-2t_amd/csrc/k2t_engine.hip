@@ -278,14 +278,29 @@ void *dalloc(k2t_model *m, size_t bytes) {
     return p;
 }
 
-// Grows the model's MoE batch workspace to layer L's need.
+int moe_shared_inter(const MoeLayer &L) { return L.sh_gu ? L.sh_gu->rows / 2 : 0; }
+
+// Bytes of layer L's batch workspace; group receives the tokens it holds.
+size_t moe_batch_need(const k2t_model *m, const MoeLayer &L, int &group) {
+    const int inter = moe_shared_inter(L);
+    group = moe_batch_tokens(L.bank, L.top_k, inter, m->max_batch);
+    return moe_batch_bytes(L.bank, L.top_k, inter, group);
+}
+
+// Grows the model's MoE batch workspace to layer L's need.  The larger one is allocated first:
+// a failure leaves the model as it was.
 void ensure_moe_batch(k2t_model *m, const MoeLayer &L) {
     if (m->max_batch < 2) return;
-    const int inter = L.sh_gu ? L.sh_gu->rows / 2 : 0;
-    const size_t need = moe_batch_bytes(L.bank, L.top_k, inter, moe_batch_tokens(L.bank, L.top_k, inter, m->max_batch));
+    int group;
+    const size_t need = moe_batch_need(m, L, group);
     if (need <= m->moe_batch_bytes) return;
+    uint8_t *old = m->moe_batch;
     m->moe_batch = (uint8_t *)dalloc(m, need);
     m->moe_batch_bytes = need;
+    if (!old) return;
+    hip_check(hipStreamSynchronize(m->stream), "moe workspace sync");  // a prompt may still be using it
+    m->allocs.erase(std::find(m->allocs.begin(), m->allocs.end(), (void *)old));
+    hip_check(hipFree(old), "hipFree");
 }
 
 void arg(bool ok, const char *msg) {
@@ -442,10 +457,10 @@ void forward(k2t_model *m, int ntok, bool with_logits, int ctx_bound = 0) {
         if (L.has_moe) {
             // each token has its own routes (forward_layer_single); a batch groups its tokens
             // by expert
-            if (ntok > 1 && m->moe_batch && moe_batch_supported(ctx, L.moe)) {
-                const int inter = L.moe.sh_gu ? L.moe.sh_gu->rows / 2 : 0;
-                const int group = moe_batch_tokens(L.moe.bank, L.moe.top_k, inter, m->max_batch);
-                const MoeBatchWork bw = moe_batch_carve(m->moe_batch, L.moe.bank, L.moe.top_k, inter, group);
+            int group = 0;
+            if (ntok > 1 && moe_batch_supported(ctx, L.moe) && moe_batch_need(m, L.moe, group) <= m->moe_batch_bytes) {
+                const MoeBatchWork bw =
+                    moe_batch_carve(m->moe_batch, L.moe.bank, L.moe.top_k, moe_shared_inter(L.moe), group);
                 for (int t = 0; t < ntok; t += group)
                     launch_moe_ffn_batch(ctx, L.moe, m->hidden + (size_t)t * d, std::min(group, ntok - t), L.post_norm,
                                          c.rms_eps, bw, m->err_dev);
@@ -950,15 +965,18 @@ int32_t k2t_model_set_moe(k2t_model *m, int32_t layer, const k2t_experts *bank, 
         }
         const size_t need = moe_work_floats(bank, top_k);
         if (need > m->moe_ws_floats) {
-            m->moe_ws = (float *)dalloc(m, need * sizeof(float));
-            m->moe_ws_floats = need;
+            float *ws = (float *)dalloc(m, need * sizeof(float));
             // the route hand-off words and the call counter start at epoch 0
-            hip_check(hipMemset(m->moe_ws, 0, need * sizeof(float)), "moe workspace clear");
+            hip_check(hipMemset(ws, 0, need * sizeof(float)), "moe workspace clear");
+            m->moe_ws = ws;
+            m->moe_ws_floats = need;
         }
-        L.moe = MoeLayer{bank, shard_layer, rw, rb, top_k, norm_topk_prob ? 1 : 0, scoring};
-        L.has_moe = true;
-        ensure_moe_batch(m, L.moe);
+        // (the layer changes once nothing can fail any more)
+        const MoeLayer moe{bank, shard_layer, rw, rb, top_k, norm_topk_prob ? 1 : 0, scoring};
+        ensure_moe_batch(m, moe);
         drop_graph(m);
+        L.moe = moe;
+        L.has_moe = true;
     });
 }
 
@@ -985,16 +1003,18 @@ int32_t k2t_model_set_moe_shared(k2t_model *m, int32_t layer, const k2t_mat *gat
         hip_check(hipSetDevice(m->ctx->device), "hipSetDevice");
         // [2 * inter gate_up | d output | 64 (gate scale) | exact mode: inter int8 codes,
         //  inter / 64 scales and sums of the down activation]
-        L.moe.sh_buf = (float *)dalloc(m, ((size_t)2 * inter + d + 64 + inter / 4 + 2 * (inter / 64) + 64) * sizeof(float));
+        MoeLayer moe = L.moe;
+        moe.sh_buf = (float *)dalloc(m, ((size_t)2 * inter + d + 64 + inter / 4 + 2 * (inter / 64) + 64) * sizeof(float));
         float *g = nullptr;
         if (gate_weight) {
             g = (float *)dalloc(m, (size_t)d * sizeof(float));
             hip_check(hipMemcpy(g, gate_weight, (size_t)d * sizeof(float), hipMemcpyHostToDevice), "gate upload");
         }
-        L.moe.sh_gu = gate_up;
-        L.moe.sh_dn = down;
-        L.moe.sh_gate = g;
-        ensure_moe_batch(m, L.moe);
+        moe.sh_gu = gate_up;
+        moe.sh_dn = down;
+        moe.sh_gate = g;
+        ensure_moe_batch(m, moe);
+        L.moe = moe;
     });
 }
 

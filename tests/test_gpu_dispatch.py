@@ -457,3 +457,58 @@ def test_moe_routes_without_a_finite_logit(gpu_ctx, d, E, k, scoring, bad):
     for x in mats:
         x.close()
     bank.close()
+
+
+def test_moe_layer_unchanged_by_a_failed_allocation(gpu_ctx):
+    """k2t_model_set_moe / _shared whose batch workspace does not fit in the GPU's memory raise
+    and leave the layer as it was: its prompts give the same logits as before, and the same
+    calls succeed once there is memory."""
+    import torch
+    from k2tb_writer import random_moe_layer, write_k2tm
+    rng = np.random.default_rng(5)
+    d, dff, E, inter = 2048, 1024, 8, 8192
+    exp, router = random_moe_layer(rng, d, dff, 1, bits=3)
+    bank = k2t.ExpertBank.upload(gpu_ctx, write_k2tm([exp * E], d, dff, 3, 2))
+    router = (0.05 * rng.standard_normal((E, d))).astype(np.float32)
+    cfg = dict(n_layers=1, hidden=d, n_heads=2, n_kv_heads=1, head_dim=64, intermediate=64, vocab=64, max_seq=512,
+               rms_eps=1e-6, rope_theta=10000.0)
+    m = k2t.Model(gpu_ctx, cfg, max_batch=512)
+    mats = [_matrix(gpu_ctx, rng, "nf4", r, c) for r, c in ((4 * 64, d), (d, 2 * 64), (64, d), (2 * inter, d), (d, inter))]
+    m.set_layer(0, mats[0], mats[1], None, None, np.ones(d, np.float32), np.ones(d, np.float32))
+    m.set_head(mats[2], np.ones(d, np.float32))
+    m.set_moe(0, bank, 0, router, 2, False)
+    toks = rng.integers(0, 64, 300).astype(np.int32)
+
+    def logits():
+        m.reset()
+        return m.prefill(toks).view(np.uint32).copy()
+
+    before = logits()
+    room = torch.empty(1 << 25, dtype=torch.uint8, device="cuda")
+    hold, size = [], 1 << 36
+    while size >= 1 << 24:  # all but 32 .. 48 MiB; the workspaces need 59 (shared) and 73 MiB (top 8)
+        try:
+            hold.append(torch.empty(size, dtype=torch.uint8, device="cuda"))
+        except torch.OutOfMemoryError:
+            size //= 2
+    del room
+    torch.cuda.empty_cache()
+    try:
+        for call in (lambda: m.set_moe_shared(0, mats[3], mats[4]), lambda: m.set_moe(0, bank, 0, router, 8, False)):
+            with pytest.raises(k2t.K2TError, match="hipMalloc"):
+                call()
+            assert np.array_equal(logits(), before)
+    finally:
+        hold.clear()
+        torch.cuda.empty_cache()
+    m.set_moe(0, bank, 0, router, 8, False)
+    top8 = logits()
+    m.set_moe_shared(0, mats[3], mats[4])
+    shared = logits()
+    assert not np.array_equal(top8, before) and not np.array_equal(shared, top8)
+    m.set_moe(0, bank, 0, router, 2, False)
+    assert np.array_equal(logits(), before)
+    m.close()
+    for x in mats:
+        x.close()
+    bank.close()
