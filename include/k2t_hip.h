@@ -173,8 +173,9 @@ int32_t k2t_act_quant_rmsnorm(k2t_ctx *ctx, const float *d_x, const float *d_nor
  * cores, outputs bit-identical to that epilogue in either mode; such a call
  * copies the activation into the context's scratch (small ones read it as it is), which
  * it grows first if it is too small (a synchronous allocation, so the first such call of a
- * size must not be inside a stream capture; NF3, and small NF3 products always, then take the
- * 4-token passes, which need none). */
+ * size must not be inside a stream capture; a graph of such a call holds that scratch, so it
+ * is valid until a later call on the context grows it).  Small NF3 products, and under capture
+ * every NF3 product that would be copied, take the 4-token passes, which need no scratch. */
 int32_t k2t_gemv(k2t_ctx *ctx, const k2t_mat *m, const int8_t *d_xq, const float *d_xs,
                  const int32_t *d_xsum, int32_t ntok, int32_t s0, int32_t s1, float *d_out,
                  size_t out_stride);

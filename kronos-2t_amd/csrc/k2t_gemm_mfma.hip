@@ -1220,7 +1220,7 @@ static size_t tile_scratch(const k2t_mat *m, int ntok) {
 bool gemm_mfma_nf3_passes(k2t_ctx *ctx, const k2t_mat *m, int ntok) {
     if (m->fmt != K2T_FMT_NF || m->bits != 3) return false;
     if (ntok <= 128 && (long)m->stripes * m->nc * ((ntok + 3) / 4) <= 36000) return true;
-    if (tile_scratch(m, ntok) <= ctx->scratch_cap) return false;
+    if (tile_scratch(m, ntok) == 0) return false;  // no copy
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) {
         (void)hipGetLastError();

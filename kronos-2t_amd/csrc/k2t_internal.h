@@ -147,7 +147,9 @@ bool gemm_mfma_supported(const k2t_mat *m, int ntok);
 // Whether an NF3 matrix takes the 4-token passes of gemv_kernel instead when no producer wrote
 // the tiles: small products, where the copy into tiles costs more than the passes (NF3 1000 x
 // 4096, 16 tokens 6.2 us and 8.6; 8192 x 512, 32 tokens 6.7 and 7.3; 64 tokens 11.3 and 7.6:
-// not taken), and captures whose context has no scratch for the copy yet.
+// not taken), and under stream capture every product that would be copied: a graph that held
+// the context's scratch would outlive it (a later call may grow, so free, it), and whether the
+// scratch is large enough already depends on the calls before.
 bool gemm_mfma_nf3_passes(k2t_ctx *ctx, const k2t_mat *m, int ntok);
 void launch_gemm_mfma(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const float *xs, const int32_t *xsum,
                       int ntok, float *out, size_t out_stride, bool accum, ActTiles tiles = ActTiles{});

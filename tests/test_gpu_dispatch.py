@@ -512,3 +512,47 @@ def test_moe_layer_unchanged_by_a_failed_allocation(gpu_ctx):
     for x in mats:
         x.close()
     bank.close()
+
+
+# a product that the matrix cores take after a copy into tiles, and one that they take as its
+# rows lie (no copy)
+@pytest.mark.parametrize("rows,cols,ntok", [(1030, 4160, 64), (1040, 576, 80)])
+def test_captured_nf3_batch_needs_no_scratch(rows, cols, ntok):
+    """A captured NF3 batch keeps its outputs over replays while other calls use, and grow (so
+    free), the context's scratch: the graph holds none of it.  Its bits are those of the same
+    capture on a context that has not been used before."""
+    import torch
+    from helpers import acts
+    rng = np.random.default_rng(rows)
+    outs = []
+    for used in (False, True):
+        ctx, s = k2t.Ctx(0), torch.cuda.Stream()
+        ctx.set_stream(s.cuda_stream)
+        rng2 = np.random.default_rng(rows + 1)
+        m, big = _matrix(ctx, rng2, "nf3", rows, cols), _matrix(ctx, rng2, "nf4", 64, 4160)
+        a = [_t(x) for x in acts(rng2, cols, ntok)]
+        n = 16 * ntok
+        b = [_t(x) for x in acts(rng, 4160, 16)]
+        b = [x.repeat(n // 16, 1) for x in b]
+        out, bout = torch.zeros((ntok, rows), device="cuda"), torch.zeros((n, 64), device="cuda")
+        torch.cuda.synchronize()
+        if used:  # the scratch now holds the tiles of either product
+            ctx.gemv(m, *a, out, ntok=ntok, out_stride=rows)
+            ctx.gemv(big, *[x[:ntok] for x in b], bout, ntok=ntok, out_stride=64)
+        ctx.sync()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            ctx.gemv(m, *a, out, ntok=ntok, out_stride=rows)
+        for k in range(3):
+            ctx.gemv(big, *[x[:(4 + 6 * k) * ntok] for x in b], bout, ntok=(4 + 6 * k) * ntok, out_stride=64)
+            ctx.sync()
+            out.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(s):
+                g.replay()
+            torch.cuda.synchronize()
+            outs.append(out.cpu().numpy().view(np.uint32))
+        m.close()
+        big.close()
+        ctx.close()
+    assert outs[0].any() and all(np.array_equal(outs[0], o) for o in outs[1:])
