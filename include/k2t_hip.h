@@ -83,8 +83,9 @@ int32_t k2t_ctx_set_exact(k2t_ctx *ctx, int32_t exact);
 /* Batched NF4, NF3 and bit-plane (b4 / b5 / b6) GEMVs (16 or more tokens of a ready activation
  * over the whole matrix, k2t_gemv and the model's prefill): enable = 1 (default) runs
  * them on the int8 matrix cores, one weight pass per 16 to 128 tokens, with outputs equal to the
- * exact-order epilogue's in either mode (small NF3 products keep the 4-token passes), and with the fast epilogue 2 .. 15 tokens in one
- * weight pass with each token's one-token outputs; 0 runs the 4-token weight passes of the
+ * exact-order epilogue's in either mode (NF3: in exact mode; otherwise each token's one-token
+ * outputs), and with the fast epilogue 2 .. 15 tokens in one weight pass with each token's
+ * one-token outputs; 0 runs the 4-token weight passes of the
  * reference's tiles (nf_sdot_decode_neon, simd_lut.rs:6074-6364;
  * nibble4_sdot_batch_stripe_range, 4101-4320).  2: matrix cores, but a model's prefill does not have the
  * activation's producer write the tile-major copy the GEMV reads (the GEMV copies it
@@ -174,8 +175,8 @@ int32_t k2t_act_quant_rmsnorm(k2t_ctx *ctx, const float *d_x, const float *d_nor
  * copies the activation into the context's scratch (small ones read it as it is), which
  * it grows first if it is too small (a synchronous allocation, so the first such call of a
  * size must not be inside a stream capture; a graph of such a call holds that scratch, so it
- * is valid until a later call on the context grows it).  Small NF3 products, and under capture
- * every NF3 product that would be copied, take the 4-token passes, which need no scratch. */
+ * is valid until a later call on the context grows it).  NF3: outside exact mode each token's
+ * outputs are the one-token call's; small products, and under capture all, need no scratch. */
 int32_t k2t_gemv(k2t_ctx *ctx, const k2t_mat *m, const int8_t *d_xq, const float *d_xs,
                  const int32_t *d_xsum, int32_t ntok, int32_t s0, int32_t s1, float *d_out,
                  size_t out_stride);

@@ -11,15 +11,16 @@
 //  - NF4: the codebook value of each code (the codebook as two v_perm XOR tables,
 //    nf4_xlut); the MFMA gives the chunk dot.
 //  - NF3: the same through one v_perm per four codes, from the row's triplet of dwords, in
-//    the device's lane order or the reference's.  200 tokens x 5000 x 2112: 137.8 us as 4-token
-//    passes, 20 us here.
+//    the device's lane order or the reference's.  With the fast epilogue its sums keep the
+//    one-token GEMV's order (launch_gemm_ordered).
 //  - bit planes: the unsigned code u (4 + hp bits: the nibble and the hi-plane bits); the
 //    MFMA gives sum(u * x), and the chunk dot of the odd weights 2u - (2^(4+hp) - 1) is
 //    2 * sum(u * x) - (2^(4+hp) - 1) * sum(x), as the reference computes it (simd_lut.rs:
 //    4030-4045 and 4304-4309: the sdot of the codes acc, then 2 * acc - max_odd * xsum).
 // The epilogue is the reference's per-row chain in chunk order (simd_lut.rs:4030-4059,
 // 6334-6335: f = fmaf(float(dot) * sx, scale, f), chunks with sx == 0 skipped), so every
-// output equals the exact-order GEMV's (k2t_ctx_set_exact) bit for bit.
+// output (but NF3's with the fast epilogue) equals the exact-order GEMV's (k2t_ctx_set_exact) bit
+// for bit.
 //
 // Operand layouts of v_mfma_i32_16x16x64_i8 (checked on the GPU): lane l holds 16 bytes of
 // A row l % 16 and of B column l % 16; the products pair lane l's byte b of A with lane
@@ -66,6 +67,7 @@ struct MfArgs {
     const int32_t *ut;  // their code sums (bit planes): [16-token block][chunk][16 tokens]
     int K, ntok, nblk;  // nblk: 16-token blocks
     int tiled;          // gemm_ks_kernel: 0 = xt / st / ut are the [token] rows themselves
+    int nseg, cps, g_log2;  // gemm_ks_kernel, one-token order: plan_gemv's K segments and accumulators
     float *out;
     size_t out_stride;
     int accum;
@@ -416,6 +418,13 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(MfArgs A) {
 // outputs.  The same operations in the same order, so the outputs equal gemm_mfma_kernel's;
 // 16.5 us for that shape.  Bound by the exchange (2 KB of LDS traffic per tile of 16 x 16
 // outputs and chunk) and the issue rate of the chain.
+// ORD (NF3 with the fast epilogue): the sums in the order of gemv_kernel's fast epilogue, so a batch
+// gives each token the bits of the one-token GEMV, as its 4-token passes did, and their error (one
+// chain over K has up to three times it).  A wave holds one accumulator of a K segment in
+// registers; the exchange is one value per output, accumulator and segment, added pairwise and
+// then segment by segment by the outputs' owners.  NF3 5000 x 2112, 200 tokens 128.5 us as 4-token
+// passes, 23.1 here (one chain over K in tiles: 18.1); 14336 x 4096, 200 tokens 277 and 74 (46);
+// 4096 x 14336, 64 tokens 127 and 25 (30).
 constexpr int kKsWaves = 8;
 
 template <int FMT, int NB>
@@ -427,12 +436,12 @@ struct KsFrag {
     int32_t su[FMT == 0 ? NB : 1];
 };
 
-template <int FMT, int HP, int NB>
+template <int FMT, int HP, int NB, bool ORD = false>
 __global__ __launch_bounds__(64 * kKsWaves, 4) void gemm_ks_kernel(MfArgs A) {
     constexpr int W = kKsWaves, P = NB == 4 ? 2 : NB == 2 ? 3 : 4;  // rounds in flight
     constexpr int OWN = NB == 4 ? 2 : 1;              // chains per wave
     __shared__ float tt[2][W][NB][4][64];             // terms [chunk of the round][block][row mod 4][lane]
-    __shared__ __align__(16) float wss[2][W][16];     // the chunks' row scales
+    __shared__ __align__(16) float wss[2][W][16];     // the chunks' row scales (not ORD)
     const uint32_t lane = threadIdx.x & 63u, li = lane & 15u, lg = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     int stripe = (int)blockIdx.x;
@@ -481,7 +490,7 @@ __global__ __launch_bounds__(64 * kKsWaves, 4) void gemm_ks_kernel(MfArgs A) {
     const int r_own = wave & 3, ob = wave >> 2;
     float acc[OWN];
 #pragma unroll
-    for (int k = 0; k < OWN; k++) acc[k] = 0.0f;
+    for (int k = 0; k < OWN; k++) acc[k] = ORD ? -0.0f : 0.0f;  // (-0 + v is v)
     const int nc = A.nc, last = nc - 1;
     auto round = [&](const KsFrag<FMT, NB> &f, int i) {
         const int buf = i & 1;
@@ -520,23 +529,105 @@ __global__ __launch_bounds__(64 * kKsWaves, 4) void gemm_ks_kernel(MfArgs A) {
             }
         }
     };
-    KsFrag<FMT, NB> ring[P];
+    // ORD: this wave's accumulator u of segment h, h + 8 / G, ...; `len` visits per segment
+    const int G = ORD ? 1 << A.g_log2 : W, u = wave & (G - 1), h = ORD ? wave >> A.g_log2 : 0;
+    const int len = ORD ? (A.cps + G - 1) >> A.g_log2 : 1, seg_step = W / G;
+    const int rounds = ORD ? (A.nseg + seg_step - 1) / seg_step * len : (nc + W - 1) / W;
+    struct At {  // a round's place: first segment of the step, visit within it, parity of the step
+        int seg, v, buf;
+    };
+    auto next = [&](At &a) {
+        if (++a.v < len) return;
+        a.v = 0;
+        a.seg += seg_step;
+        a.buf ^= 1;
+    };
+    auto chunk_of = [&](const At &a, bool &live) {
+        const int off = u + a.v * G, c = (a.seg + h) * A.cps + off;
+        live = off < A.cps && c < nc;
+        return min(c, last);
+    };
+    float po[ORD ? NB : 1][4];
+    auto round_ord = [&](const KsFrag<FMT, NB> &f, const At &at) {
+        bool live;
+        (void)chunk_of(at, live);
+        if (at.v == 0)
 #pragma unroll
-    for (int k = 0; k < P; k++) fetch(ring[k], min(W * k + wave, last));
-    const int rounds = (nc + W - 1) / W;
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) po[ORD ? b : 0][r] = 0.0f;
+        if (live) {
+            const v4i a = mf_decode<FMT, HP>(f.d0, f.d1, f.hv, A.t0, A.t1, A.u0, A.u1, lane);
+            const float ws[4] = {bf16_lo(f.sw.x), bf16_hi(f.sw.x), bf16_lo(f.sw.y), bf16_hi(f.sw.y)};
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                const v4i zero = {0, 0, 0, 0};
+                const v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, f.x[b], zero, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    int dot = d[r];
+                    if constexpr (FMT == 0) dot = 2 * dot - ((1 << (4 + HP)) - 1) * f.su[b];
+                    float &o = po[ORD ? b : 0][r];
+                    o = fmaf((float)dot * f.sx[b], ws[r], o);
+                }
+            }
+        }
+        if (at.v != len - 1) return;
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) tt[at.buf][wave][b][r][lane] = po[ORD ? b : 0][r];
+        __syncthreads();
+        if (NB > 1 || ob == 0) {
+#pragma unroll
+            for (int o = 0; o < OWN; o++) {
+                float t[W];
+#pragma unroll
+                for (int k = 0; k < W; k++) t[k] = tt[at.buf][k][NB == 1 ? 0 : ob + 2 * o][r_own][lane];
+                const float lo = (t[0] + t[1]) + (t[2] + t[3]), hi = (t[4] + t[5]) + (t[6] + t[7]);
+                if (A.g_log2 == 3) {
+                    acc[o] += lo + hi;
+                } else {
+                    acc[o] += lo;
+                    if (at.seg + 1 < A.nseg) acc[o] += hi;
+                }
+            }
+        }
+    };
+    KsFrag<FMT, NB> ring[P];
+    At now{0, 0, 0}, ahead{0, 0, 0};
+    auto refill = [&](KsFrag<FMT, NB> &f, int i) {  // round i's chunk
+        if constexpr (ORD) {
+            bool live;
+            fetch(f, chunk_of(ahead, live));
+            next(ahead);
+        } else {
+            fetch(f, min(W * i + wave, last));
+        }
+    };
+    auto take = [&](const KsFrag<FMT, NB> &f, int i) {
+        if constexpr (ORD) {
+            round_ord(f, now);
+            next(now);
+        } else {
+            round(f, i);
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < P; k++) refill(ring[k], k);
     int i = 0;
     for (; i + P <= rounds; i += P) {
 #pragma unroll
         for (int k = 0; k < P; k++) {
-            round(ring[k], i + k);
+            take(ring[k], i + k);
             __builtin_amdgcn_sched_barrier(0);
-            fetch(ring[k], min(W * (i + k + P) + wave, last));
+            refill(ring[k], i + k + P);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
 #pragma unroll
     for (int k = 0; k < P - 1; k++)
-        if (i + k < rounds) round(ring[k], i + k);
+        if (i + k < rounds) take(ring[k], i + k);
     // through LDS, so that a token's 16 rows are stored together
     __syncthreads();
     float *ot = &tt[0][0][0][0][0];  // [16 NB tokens][17]
@@ -802,6 +893,7 @@ __global__ __launch_bounds__(256) void mf_tile_kernel(const int8_t *xq, const fl
 // the one-token GEMV.  A wave's chunks are dealt round-robin to G accumulators (the GEMV's
 // lane groups: 4 in pair mode, 8 in stripe mode), which are added pairwise as the lane
 // butterfly does, then the waves' sums in wave order.  (A chunk with scale 0 adds +-0.)
+// Any number of tokens in groups of up to 16, a weight pass each.
 struct GvArgs {
     const uint8_t *pair, *tail;
     size_t ptot;
@@ -861,11 +953,14 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
     for (int s = 0; s < RS; s++)  // (pair mode on the tail stripe: side 1 repeats it, not stored)
         L[s] = mf_lane<FMT, HP>(lane, is_tail, is_tail ? 0u : SM ? (uint32_t)(rb & 1) : (uint32_t)s, A.lane);
     const int tok0 = GRP ? 0 : (int)blockIdx.y * A.tg, nt = GRP ? item.z : min(A.tg, A.ntok - tok0);
-    uint32_t tok = (uint32_t)tok0 + min(li, (uint32_t)nt - 1u);  // columns past nt repeat the last token, not stored
+    uint32_t tok = min(li, (uint32_t)nt - 1u);  // columns past nt repeat the last token, not stored
     if constexpr (GRP) tok = (uint32_t)A.grp.list[item.y + (int)tok] / (uint32_t)A.grp.row_div;
+    // (offsets count from the workgroup's first token, so they stay small for any batch)
+    const size_t row0 = GRP ? 0 : (size_t)tok0;
     const uint32_t x_off = tok * (uint32_t)A.K + lg * 16u, sx_off = tok * (uint32_t)A.nc * 4u;
-    const __amdgpu_buffer_rsrc_t rw = mf_rsrc(mbase), rx = mf_rsrc(A.xq), rs = mf_rsrc(A.xs),
-                                 ru = mf_rsrc(FMT == 0 ? (const void *)A.xsum : A.xs);
+    const float *xs0 = A.xs + row0 * A.nc;
+    const __amdgpu_buffer_rsrc_t rw = mf_rsrc(mbase), rx = mf_rsrc(A.xq + row0 * A.K), rs = mf_rsrc(xs0),
+                                 ru = mf_rsrc(FMT == 0 ? (const void *)(A.xsum + row0 * A.nc) : xs0);
     const int cw0 = wave * A.cps, cw1 = min(A.nc, cw0 + A.cps), n = cw1 - cw0;
     auto fetch = [&](GvFrag<FMT, RS> &f, int c) {
         uint32_t rec, sgb;
@@ -1179,7 +1274,7 @@ void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, cons
     // workgroups (four or more tokens each), which shortens each one's activation gather.
     // NF4 2048 x 8192, 8 / 15 tokens: 8.8 / 11.0 us in one group, 7.6 / 9.0 us.
     const int wgs = plan.rb_hi - plan.rb_lo;
-    const int groups = std::max(1, std::min(ctx->num_cus / wgs, (ntok + 3) / 4));
+    const int groups = std::max((ntok + 15) / 16, std::min(ctx->num_cus / wgs, (ntok + 3) / 4));
     A.tg = (ntok + groups - 1) / groups;
     const dim3 grid(wgs, (ntok + A.tg - 1) / A.tg);
     const size_t lds = gemv_mfma_lds(plan);
@@ -1211,16 +1306,7 @@ static bool ks_rows(const k2t_mat *m, int blocks) {
            m->nc * (blocks < 4 ? blocks : 4) <= (m->fmt == K2T_FMT_NIBBLE4 ? 20 : 40);
 }
 
-// Scratch floats the tile-major copy of ntok tokens takes (0: no copy is made).
-static size_t tile_scratch(const k2t_mat *m, int ntok) {
-    const int blocks = (ntok + 15) / 16;
-    return ks_rows(m, blocks) ? 0 : (size_t)blocks * m->nc * (1024 + 64 + 64) / sizeof(float);
-}
-
-bool gemm_mfma_nf3_passes(k2t_ctx *ctx, const k2t_mat *m, int ntok) {
-    if (m->fmt != K2T_FMT_NF || m->bits != 3) return false;
-    if (ntok <= 128 && (long)m->stripes * m->nc * ((ntok + 3) / 4) <= 36000) return true;
-    if (tile_scratch(m, ntok) == 0) return false;  // no copy
+static bool stream_captured(k2t_ctx *ctx) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) {
         (void)hipGetLastError();
@@ -1229,11 +1315,16 @@ bool gemm_mfma_nf3_passes(k2t_ctx *ctx, const k2t_mat *m, int ntok) {
     return cap != hipStreamCaptureStatusNone;
 }
 
+bool gemm_mfma_nf3_passes(k2t_ctx *ctx, const k2t_mat *m, int ntok) {
+    if (ntok <= 128 && (long)m->stripes * m->nc * ((ntok + 3) / 4) <= 36000) return true;
+    return !ks_rows(m, (ntok + 15) / 16) && stream_captured(ctx);
+}
+
 // Arguments of one launch over all of m's stripes, and the tile-major activation (the
 // producer's, else copied here into the context's scratch: 1 KB + 64 B of scales + 64 B
 // of code sums per tile).
 static void mfma_args(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const float *xs, const int32_t *xsum,
-                     int ntok, ActTiles tiles, MfArgs &A) {
+                     int ntok, ActTiles tiles, bool rows, MfArgs &A) {
     const bool planes = m->fmt == K2T_FMT_NIBBLE4;
     A = MfArgs{};
     A.pair = m->pair;
@@ -1251,14 +1342,14 @@ static void mfma_args(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const fl
     float *stile = tiles.st;
     int32_t *utile = tiles.ut;
     A.tiled = 1;
-    if ((!xt || (planes && !utile)) && ks_rows(m, blocks)) {
+    if ((!xt || (planes && !utile)) && rows) {
         xt = const_cast<int8_t *>(xq);
         stile = const_cast<float *>(xs);
         utile = const_cast<int32_t *>(xsum);
         A.tiled = 0;
     } else if (!xt || (planes && !utile)) {
         const size_t ntile = (size_t)blocks * m->nc;
-        ensure_scratch(ctx, tile_scratch(m, ntok));
+        ensure_scratch(ctx, ntile * (1024 + 64 + 64) / sizeof(float));
         xt = reinterpret_cast<int8_t *>(ctx->scratch);
         stile = ctx->scratch + ntile * 256;
         utile = reinterpret_cast<int32_t *>(ctx->scratch + ntile * 272);
@@ -1280,15 +1371,26 @@ static void launch_tile(hipStream_t st, const MfArgs &A) {
     hipLaunchKernelGGL((gemm_tile_kernel<FMT, HP, NP, TB, D, MODE>), grid, dim3(256), lds, st, A);
 }
 
-// f<FMT, HP>(...) for matrix m's format.
-#define MF_FORMATS(m, f, ...)                                                 \
-    do {                                                                      \
-        if ((m)->fmt == K2T_FMT_NF && (m)->bits == 3) f<2, 0>(__VA_ARGS__);   \
-        else if ((m)->fmt == K2T_FMT_NF) f<1, 0>(__VA_ARGS__);                \
-        else if ((m)->hp == 0) f<0, 0>(__VA_ARGS__);                          \
-        else if ((m)->hp == 1) f<0, 1>(__VA_ARGS__);                          \
-        else f<0, 2>(__VA_ARGS__);                                            \
+// f<FMT, HP>(...) for matrix m's format (NF4 or bit planes).
+#define MF_FORMATS(m, f, ...)                             \
+    do {                                                  \
+        if ((m)->fmt == K2T_FMT_NF) f<1, 0>(__VA_ARGS__); \
+        else if ((m)->hp == 0) f<0, 0>(__VA_ARGS__);      \
+        else if ((m)->hp == 1) f<0, 1>(__VA_ARGS__);      \
+        else f<0, 2>(__VA_ARGS__);                        \
     } while (0)
+
+static bool is_nf3(const k2t_mat *m) { return m->fmt == K2T_FMT_NF && m->bits == 3; }
+
+template <int FMT, int HP, bool ORD = false>
+static void launch_ks(hipStream_t st, const MfArgs &A) {
+    const dim3 blk(64 * kKsWaves);
+    const int B = A.nblk, nb = B <= 1 ? 1 : B == 2 ? 2 : 4;
+    const dim3 grid(A.stripes, (B + nb - 1) / nb);
+    if (nb == 1) hipLaunchKernelGGL((gemm_ks_kernel<FMT, HP, 1, ORD>), grid, blk, 0, st, A);
+    else if (nb == 2) hipLaunchKernelGGL((gemm_ks_kernel<FMT, HP, 2, ORD>), grid, blk, 0, st, A);
+    else hipLaunchKernelGGL((gemm_ks_kernel<FMT, HP, 4, ORD>), grid, blk, 0, st, A);
+}
 
 template <int FMT, int HP>
 static void launch_plain_fmt(hipStream_t st, bool ks, const MfArgs &A) {
@@ -1299,12 +1401,7 @@ static void launch_plain_fmt(hipStream_t st, bool ks, const MfArgs &A) {
     // 25 / 30 / 81 in 128-token ones (a wave per stripe and block, or 16 rows x 64 tokens per
     // wave: 31 / 41 / 94); 2048 x 8192, 512 tokens (256 workgroups of 128) 38 and 42.5.
     if (ks) {
-        const dim3 blk(64 * kKsWaves);
-        const int nb = B <= 1 ? 1 : B == 2 ? 2 : 4;
-        const dim3 grid(S, (B + nb - 1) / nb);
-        if (nb == 1) hipLaunchKernelGGL((gemm_ks_kernel<FMT, HP, 1>), grid, blk, 0, st, A);
-        else if (nb == 2) hipLaunchKernelGGL((gemm_ks_kernel<FMT, HP, 2>), grid, blk, 0, st, A);
-        else hipLaunchKernelGGL((gemm_ks_kernel<FMT, HP, 4>), grid, blk, 0, st, A);
+        launch_ks<FMT, HP>(st, A);
     } else if (B <= 2) {
         // two blocks per wave only where that leaves 8 waves per CU
         const int nb = B == 2 && S >= 2048 ? 2 : 1;
@@ -1337,20 +1434,52 @@ void launch_gemm_mfma(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const fl
                       int ntok, float *out, size_t out_stride, bool accum, ActTiles tiles) {
     if (!gemm_mfma_supported(m, ntok)) throw Error(K2T_E_INTERNAL, "mfma gemm: unsupported matrix");
     MfArgs A;
-    mfma_args(ctx, m, xq, xs, xsum, ntok, tiles, A);
+    mfma_args(ctx, m, xq, xs, xsum, ntok, tiles, ks_rows(m, (ntok + 15) / 16), A);
     A.out = out;
     A.out_stride = out_stride;
     A.accum = accum ? 1 : 0;
-    MF_FORMATS(m, launch_plain_fmt, ctx->stream, ks_split(m, A.nblk), A);
+    const bool ks = ks_split(m, A.nblk);
+    if (is_nf3(m)) launch_plain_fmt<2, 0>(ctx->stream, ks, A);
+    else MF_FORMATS(m, launch_plain_fmt, ctx->stream, ks, A);
+    hip_check(hipGetLastError(), "mfma gemm launch");
+}
+
+// Whether `blocks` 16-token blocks of an ordered batch run on gemv_mfma_kernel, 16 tokens per weight
+// pass, instead of gemm_ks_kernel: small products, whose copy into tiles costs more than it saves
+// (NF3 5000 x 2112, 32 / 64 tokens 8.1 / 12.7 us there, 9.6 / 11.6 on gemm_ks_kernel; 2048 x 8192,
+// 32 / 64 tokens 11.6 / 22.0 and 15.0 / 20.3); one block over many stripes (14336 x 4096, 13.4 and
+// 16.3; 4096 x 14336, 18.2 and 16.1: not taken); rows of a round or two, which leave a K segment's
+// exchange nothing to pay for it (8200 x 576, 512 tokens 26 and 43).
+static bool ordered_gemv(const k2t_mat *m, int blocks) {
+    return (long)m->stripes * m->nc * blocks <= 36000 || (blocks == 1 && m->stripes >= 512) || m->nc <= 12;
+}
+
+void launch_gemm_ordered(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, const int8_t *xq, const float *xs,
+                         int ntok, float *out, size_t out_stride, bool accum, ActTiles tiles) {
+    if (!gemm_mfma_supported(m, ntok) || !is_nf3(m)) throw Error(K2T_E_INTERNAL, "ordered mfma gemm: unsupported matrix");
+    // (a captured graph holds no scratch: gemm_mfma_nf3_passes' note; the bits are the same)
+    if (ordered_gemv(m, (ntok + 15) / 16) || (!tiles.xt && stream_captured(ctx))) {
+        launch_gemv_mfma(ctx, m, plan, xq, xs, nullptr, ntok, 0, m->stripes, out, out_stride, accum);
+        return;
+    }
+    MfArgs A;
+    mfma_args(ctx, m, xq, xs, nullptr, ntok, tiles, false, A);
+    A.out = out;
+    A.out_stride = out_stride;
+    A.accum = accum ? 1 : 0;
+    A.nseg = plan.nseg;
+    A.cps = plan.cps;
+    A.g_log2 = plan.stripe_mode ? 3 : 2;
+    launch_ks<2, 0, true>(ctx->stream, A);
     hip_check(hipGetLastError(), "mfma gemm launch");
 }
 
 bool launch_gemm_mfma_qkv(k2t_ctx *ctx, const k2t_mat *qkv, ActTiles tiles, int ntok, float *out, size_t out_stride,
                           const QkvPostDev &qp) {
-    if (!gemm_mfma_supported(qkv, ntok) || !tiles.xt || qkv->rows % 64 != 0) return false;
+    if (!gemm_mfma_supported(qkv, ntok) || is_nf3(qkv) || !tiles.xt || qkv->rows % 64 != 0) return false;
     if (qkv->fmt == K2T_FMT_NIBBLE4 && !tiles.ut) return false;
     MfArgs A;
-    mfma_args(ctx, qkv, nullptr, nullptr, nullptr, ntok, tiles, A);
+    mfma_args(ctx, qkv, nullptr, nullptr, nullptr, ntok, tiles, false, A);
     A.out = out;
     A.out_stride = out_stride;
     A.qp = qp;
@@ -1361,14 +1490,14 @@ bool launch_gemm_mfma_qkv(k2t_ctx *ctx, const k2t_mat *qkv, ActTiles tiles, int 
 
 bool launch_gemm_mfma_swiglu(k2t_ctx *ctx, const k2t_mat *gu, ActTiles tiles, int ntok, int8_t *q, float *s,
                              int32_t *sums, ActTiles out_tiles) {
-    if (!gemm_mfma_supported(gu, ntok) || !tiles.xt || !out_tiles.xt || gu->rows % 128 != 0) return false;
+    if (!gemm_mfma_supported(gu, ntok) || is_nf3(gu) || !tiles.xt || !out_tiles.xt || gu->rows % 128 != 0) return false;
     if (gu->fmt == K2T_FMT_NIBBLE4 && !tiles.ut) return false;
     // 512 or more workgroups of 128 rows x 64 tokens; with fewer the plain launch and the
     // activation's own spread better: 16384 x 2048 NF4, two layers, 512 / 256 tokens 403 / 282 us
     // apart and 375 / 275 fused; 128 / 64 tokens (256 / 128 workgroups) 219 / 202 and 228 / 222.
     if ((long)(gu->rows / 128) * ((ntok + 63) / 64) < 512) return false;
     MfArgs A;
-    mfma_args(ctx, gu, nullptr, nullptr, nullptr, ntok, tiles, A);
+    mfma_args(ctx, gu, nullptr, nullptr, nullptr, ntok, tiles, false, A);
     A.sq = q;
     A.ss = s;
     A.ssum = sums;

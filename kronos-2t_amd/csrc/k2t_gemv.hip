@@ -954,10 +954,13 @@ static void launch_gemv_impl(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, c
                              const int32_t *xsum, int ntok, int s0, int s1, float *out, size_t out_stride,
                              int32_t *dots, bool accum, int xsm, const float *src, const float *w, float eps,
                              const GemvGroup *grp, int gu_split, ActTiles tiles) {
-    // 16 or more tokens of a ready activation through an NF4 matrix: the matrix-core
-    // kernel (one weight pass per 64 tokens; its outputs equal the exact-order GEMV's)
-    if (!dots && !grp && xsm == 0 && gu_split == 0 && s0 == 0 && s1 == m->stripes && ctx->mfma &&
-        gemm_mfma_supported(m, ntok) && (tiles.xt || !gemm_mfma_nf3_passes(ctx, m, ntok))) {
+    // 16 or more tokens of a ready activation: the matrix cores (one weight pass per 16 to 128
+    // tokens; outputs equal to the exact-order GEMV's, or NF3's with the fast epilogue to the
+    // one-token GEMV's)
+    const bool batch = !dots && !grp && xsm == 0 && gu_split == 0 && s0 == 0 && s1 == m->stripes && ctx->mfma &&
+                       gemm_mfma_supported(m, ntok);
+    const bool nf3 = m->fmt == K2T_FMT_NF && m->bits == 3;
+    if (batch && (!nf3 || (ctx->exact && !gemm_mfma_nf3_passes(ctx, m, ntok)))) {
         launch_gemm_mfma(ctx, m, xq, xs, xsum, ntok, out, out_stride, accum, tiles);
         return;
     }
@@ -971,6 +974,10 @@ static void launch_gemv_impl(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, c
     }
     ctx->max_segments = saved;
     if (plan.rb_hi <= plan.rb_lo || ntok <= 0) return;
+    if (batch && nf3 && !ctx->exact) {
+        launch_gemm_ordered(ctx, m, plan, xq, xs, ntok, out, out_stride, accum, tiles);
+        return;
+    }
     // 2 .. 15 tokens with the fast epilogue: one weight pass on the matrix cores, the same
     // plan and sum order (each token's bits are the one-token GEMV's)
     if (!dots && !grp && xsm == 0 && gu_split == 0 && !ctx->exact && ctx->mfma && gemv_mfma_supported(m, ntok)) {

@@ -140,21 +140,23 @@ void launch_rmsnorm_act(hipStream_t st, const uint64_t *signs, const float *x, c
                         int ntok, int8_t *q, float *s, int32_t *sums, ActTiles tiles = ActTiles{});
 void launch_swiglu_act(hipStream_t st, const uint64_t *signs, const float *gu, int inter, int ntok, int8_t *q,
                        float *s, int32_t *sums, bool exact, ActTiles tiles = ActTiles{});
-// Batched NF4 / bit-plane GEMV on the matrix cores (k2t_gemm_mfma.hip): kMfmaMinTokens or
-// more tokens of a ready int8 activation, outputs equal to the exact-order GEMV's.
+// Batched GEMV on the matrix cores (k2t_gemm_mfma.hip): kMfmaMinTokens or more tokens of a
+// ready int8 activation, outputs equal to the exact-order GEMV's (NF3: in exact mode).
 constexpr int kMfmaMinTokens = 16;
 bool gemm_mfma_supported(const k2t_mat *m, int ntok);
-// Whether an NF3 matrix takes the 4-token passes of gemv_kernel instead when no producer wrote
-// the tiles: small products, where the copy into tiles costs more than the passes (NF3 1000 x
-// 4096, 16 tokens 6.2 us and 8.6; 8192 x 512, 32 tokens 6.7 and 7.3; 64 tokens 11.3 and 7.6:
-// not taken), and under stream capture every product that would be copied: a graph that held
-// the context's scratch would outlive it (a later call may grow, so free, it), and whether the
-// scratch is large enough already depends on the calls before.
+// Whether an NF3 matrix takes the 4-token passes of gemv_kernel in exact mode: small products,
+// where the copy into tiles costs more than the passes (NF3 1000 x 4096, 16 tokens 6.2 us and 8.6;
+// 8192 x 512, 32 tokens 6.7 and 7.3; 64 tokens 11.3 and 7.6: not taken), and under stream capture
+// every product that would be copied: a graph that held the context's scratch would outlive it (a
+// later call may grow, so free, it).
 bool gemm_mfma_nf3_passes(k2t_ctx *ctx, const k2t_mat *m, int ntok);
 void launch_gemm_mfma(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const float *xs, const int32_t *xsum,
                       int ntok, float *out, size_t out_stride, bool accum, ActTiles tiles = ActTiles{});
-// 2 .. 15 tokens with the fast epilogue on the matrix cores: plan_gemv's split, the sums in
-// gemv_kernel's order.
+// NF3 batches with the fast epilogue: plan_gemv's split, the sums in gemv_kernel's order.
+void launch_gemm_ordered(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, const int8_t *xq, const float *xs,
+                         int ntok, float *out, size_t out_stride, bool accum, ActTiles tiles);
+// 2 .. 15 tokens with the fast epilogue on the matrix cores (any number of tokens where asked
+// for): the same split and order.
 bool gemv_mfma_supported(const k2t_mat *m, int ntok);
 void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, const int8_t *xq, const float *xs,
                       const int32_t *xsum, int ntok, int s0, int s1, float *out, size_t out_stride, bool accum);
