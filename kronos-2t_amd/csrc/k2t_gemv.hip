@@ -934,6 +934,14 @@ void launch_gemv_ex(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const floa
                      nullptr, 0.0f, nullptr, gu_split, tiles);
 }
 
+void launch_gemv_token_order(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const float *xs, const int32_t *xsum,
+                             int ntok, float *out, size_t out_stride) {
+    if (ntok >= kMfmaMinTokens && gemm_mfma_supported(m, ntok))
+        launch_gemv_mfma(ctx, m, plan_gemv(ctx, m, 0, m->stripes), xq, xs, xsum, ntok, 0, m->stripes, out, out_stride, false);
+    else
+        launch_gemv_ex(ctx, m, xq, xs, xsum, ntok, out, out_stride, false);
+}
+
 void launch_gemv_fused(k2t_ctx *ctx, const k2t_mat *m, int xs_mode, const float *src, const float *w, float eps,
                        float *out, bool accumulate, int gu_split) {
     launch_gemv_impl(ctx, m, nullptr, nullptr, nullptr, 1, 0, m->stripes, out, (size_t)m->rows, nullptr, accumulate,

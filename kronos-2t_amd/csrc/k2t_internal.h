@@ -136,6 +136,11 @@ struct ActTiles {
 };
 void launch_gemv_ex(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const float *xs, const int32_t *xsum, int ntok,
                     float *out, size_t out_stride, bool accumulate, int gu_split = 0, ActTiles tiles = ActTiles{});
+// A batch's outputs with each token's one-token bits at any size and without scratch (a model's
+// stream, where the context's scratch may be in use by a call on the context's): fast epilogue,
+// matrix cores on.
+void launch_gemv_token_order(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const float *xs, const int32_t *xsum,
+                             int ntok, float *out, size_t out_stride);
 void launch_rmsnorm_act(hipStream_t st, const uint64_t *signs, const float *x, const float *w, float eps, int K,
                         int ntok, int8_t *q, float *s, int32_t *sums, ActTiles tiles = ActTiles{});
 void launch_swiglu_act(hipStream_t st, const uint64_t *signs, const float *gu, int inter, int ntok, int8_t *q,

@@ -73,8 +73,7 @@ void launch_moe_ffn(k2t_ctx *ctx, const MoeLayer &L, float *hidden, const float 
                     const MoeWork &ws);
 
 // The same for a batch of tokens (a prompt's), up to moe_batch_tokens of them per call: each
-// expert's tokens share its weight passes.  Every token's result is launch_moe_ffn's, but
-// for a shared expert's down projection of 16 or more tokens (the matrix-core GEMV's order).
+// expert's tokens share its weight passes.  Every token's result is launch_moe_ffn's.
 struct MoeBatchWork {
     float *gu, *eo;             // [tokens * top_k][2 * d_ff], [tokens * top_k][d_model]
     unsigned long long *words;  // [tokens][2E + 2] router logits or partial dots and sums

@@ -665,7 +665,7 @@ void launch_moe_ffn_batch(k2t_ctx *ctx, const MoeLayer &L, float *hidden, int nt
         }
         launch_gemv_ex(ctx, L.sh_gu, ws.aq, ws.as, ws.asum, ntok, ws.sh_gu, (size_t)2 * inter, false, 1);
         launch_swiglu_act(st, ctx->signs, ws.sh_gu, inter, ntok, ws.sh_q, ws.sh_s, ws.sh_sum, false);
-        launch_gemv_ex(ctx, L.sh_dn, ws.sh_q, ws.sh_s, ws.sh_sum, ntok, sh_out, (size_t)d, false);
+        launch_gemv_token_order(ctx, L.sh_dn, ws.sh_q, ws.sh_s, ws.sh_sum, ntok, sh_out, (size_t)d);
     }
     const bool halves = d <= 2048;  // the one-token path's two forms of the router dot
     if (halves)

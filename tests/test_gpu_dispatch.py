@@ -255,19 +255,20 @@ def test_prefill_epilogues_equal_separate_kernels(gpu_ctx, fmt, planes, kv_bits,
 
 
 # all experts used by every token (items of 16 and a remainder), and few tokens over many
-# experts; the wide router (d > 2048); a shared expert; more tokens than one MoE call takes; enough
-# pairs per expert for a workgroup to take several stripes
-@pytest.mark.parametrize("bits,E,k,d,ntok,max_batch,shared", [(3, 4, 4, 256, 40, 64, False), (4, 16, 3, 256, 2, 8, False),
-                                                              (3, 32, 6, 256, 15, 15, True), (4, 8, 2, 2112, 9, 16, False),
-                                                              (3, 4, 2, 256, 37, 8, True), (3, 4, 4, 320, 500, 500, False),
-                                                              (4, 4, 4, 576, 500, 500, False)])
+# experts; the wide router (d > 2048); a shared expert (its width), on the 4-token passes (three-chunk
+# scale groups) and with 2-chunk ones on the matrix cores, at fewer and more than 16 tokens a call;
+# more tokens than one MoE call takes; enough pairs per expert for a workgroup to take several stripes
+@pytest.mark.parametrize("bits,E,k,d,ntok,max_batch,shared", [(3, 4, 4, 256, 40, 64, 0), (4, 16, 3, 256, 2, 8, 0),
+                                                              (3, 32, 6, 256, 15, 15, 128), (4, 8, 2, 2112, 9, 16, 0),
+                                                              (3, 4, 2, 256, 37, 8, 128), (3, 4, 4, 320, 500, 500, 0),
+                                                              (4, 4, 4, 576, 500, 500, 0), (3, 4, 2, 256, 40, 64, 1024),
+                                                              (4, 4, 2, 320, 150, 160, 1088), (3, 4, 2, 256, 20, 12, 1024)])
 def test_moe_prompt_equals_token_by_token(gpu_ctx, bits, E, k, d, ntok, max_batch, shared):
     """A prompt through sparse-MoE layers (tokens grouped by expert) gives the logits of
     decoding its tokens one by one, bit for bit.  (Three-chunk scale groups and the NF4 KV
-    cache keep the attention half on kernels with that property at any batch size; a shared
-    expert's matrices likewise.)"""
+    cache keep the attention half on kernels with that property at any batch size.)"""
+    import oracle as O
     from k2tb_writer import random_moe_layer, write_k2tm
-    from model_oracle import quantize_matrix
     cfg = dict(n_layers=2, hidden=d, n_heads=4, n_kv_heads=2, head_dim=64, intermediate=64, vocab=300, max_seq=512,
                rms_eps=1e-6, rope_theta=10000.0)
     rng = np.random.default_rng(E * 100 + ntok)
@@ -278,16 +279,19 @@ def test_moe_prompt_equals_token_by_token(gpu_ctx, bits, E, k, d, ntok, max_batc
     m = k2t.Model(gpu_ctx, cfg, max_batch=max_batch)
     mats = []
 
-    def up(rows, cols):
-        q = quantize_matrix(w(rows, cols), "nf4", sgc=3)
-        mats.append(gpu_ctx.upload_nf(rows, cols, 4, 3, q.cb, q.pair, q.tail))
+    def up(rows, cols, sgc=3, b=4):
+        W = w(rows, cols)
+        cb, mu = O.nf_fit_codebook(W, b, sgc)
+        idx, sc = O.nf_rtn(W, b, sgc, cb, mu)
+        mats.append(gpu_ctx.upload_nf(rows, cols, b, sgc, cb, *O.nf_from_indices(idx, sc, rows, cols, b, sgc)))
         return mats[-1]
 
     for i in range(2):
         m.set_layer(i, up((4 + 4) * hd, d), up(d, 4 * hd), None, None, 1 + w(1, d)[0], 1 + w(1, d)[0])
         m.set_moe(i, bank, i, moe[i][1], k, True, i, router_bias=w(1, E)[0] if i else None)
         if shared:
-            m.set_moe_shared(i, up(2 * 128, d), up(d, 128), w(1, d)[0] if i else None)
+            sgc = 3 if shared == 128 else 2
+            m.set_moe_shared(i, up(2 * shared, d, sgc), up(d, shared, sgc, 4 if i else bits), w(1, d)[0] if i else None)
     m.set_head(up(300, d), np.ones(d, np.float32))
     m.set_kv_bits(4)
     toks = rng.integers(0, 300, ntok).astype(np.int32)
