@@ -1178,6 +1178,8 @@ static void mf_tables(const k2t_mat *m, uint32_t &t0, uint32_t &t1, uint32_t &u0
 
 bool gemm_mfma_supported(const k2t_mat *m, int ntok) {
     if (ntok < kMfmaMinTokens || m->cols % 64 != 0) return false;
+    // (the tiles are read at 32-bit offsets inside 2 GiB)
+    if ((long)((ntok + 15) / 16) * m->nc * 1024 > 0x7FFFFFFFl) return false;
     if (m->fmt == K2T_FMT_NF) return (m->bits == 3 || m->bits == 4) && (m->sgc & (m->sgc - 1)) == 0;
     return m->fmt == K2T_FMT_NIBBLE4 && m->hp >= 0 && m->hp <= 2;
 }

@@ -592,3 +592,25 @@ def test_captured_nf3_batch_needs_no_scratch(rows, cols, ntok):
         big.close()
         ctx.close()
     assert outs[0].any() and all(np.array_equal(outs[0], o) for o in outs[1:])
+
+
+@pytest.mark.parametrize("fmt", ["nf3", "nf4", "b5"])
+def test_batch_past_two_gib_of_activations(gpu_ctx, fmt):
+    """Tokens past the first 2 GiB of int8 activations: their outputs are those of a call of their
+    own (1e-5 of the largest: another order of fp32 sums over 512 chunks)."""
+    import torch
+    rng = np.random.default_rng(3)
+    rows, cols, n, last = 16, 32768, 65536 + 20, 24
+    m = _matrix(gpu_ctx, rng, fmt, rows, cols)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    xq = torch.empty((n, cols), dtype=torch.int8, device="cuda").random_(-127, 128, generator=g)
+    xs = torch.rand((n, cols // 64), device="cuda", generator=g) * 0.01
+    xsum = torch.empty((n, cols // 64), dtype=torch.int32, device="cuda")
+    for i in range(0, n, 4096):
+        xsum[i:i + 4096] = xq[i:i + 4096].view(-1, cols // 64, 64).sum(2, dtype=torch.int32)
+    out, own = torch.zeros((n, rows), device="cuda"), torch.zeros((last, rows), device="cuda")
+    gpu_ctx.gemv(m, xq, xs, xsum, out, ntok=n, out_stride=rows)
+    gpu_ctx.gemv(m, xq[-last:], xs[-last:], xsum[-last:], own, ntok=last, out_stride=rows)
+    gpu_ctx.sync()
+    assert own.any() and (out[-last:] - own).abs().max() <= 1e-5 * own.abs().max()
+    m.close()
