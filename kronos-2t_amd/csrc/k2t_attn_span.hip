@@ -578,10 +578,9 @@ __global__ __launch_bounds__(kSpanThreads, HD == 128 && G8 ? 4 : 6) void attn_sp
 // spans until their workgroups are more than the CUs, then 256 (8 KV heads x 128, 4100 positions:
 // 264 workgroups 14.4 us, 136 of twice the length 11.1 us; 32 KV heads x 64, 1024 positions:
 // 256 workgroups 8.7 us, 128 8.3 us).
-constexpr int kSpanMaxWgs = 256;  // CUs
-int span_tiles(int nkv, int positions) {
+int span_tiles(int num_cus, int nkv, int positions) {
     if (positions <= 256) return positions <= 128 ? 1 : 2;
-    return (long)nkv * ((positions + 127) / 128) > kSpanMaxWgs ? 2 : 1;
+    return (long)nkv * ((positions + 127) / 128) > num_cus ? 2 : 1;
 }
 
 template <int HD, int BITS, bool RING>
@@ -595,9 +594,13 @@ void launch_span(hipStream_t st, int tpw, bool g8, dim3 grid, size_t lds, const 
 
 }  // namespace
 
-bool attn_span_supported(int nq, int nkv, int hd, const KvRing &kr) {
-    return nq / nkv <= kSpanMaxGroup && (hd == 64 || hd == 128) && (kr.bits == 8 || kr.bits == 4) &&
-           (kr.window == 0 || kr.ring >= kr.window - kr.sinks);
+// The nq merge workgroups come first in dispatch order and wait for the span workgroups', so
+// those must find room beside them.  At least two workgroups fit on a CU (at most 76 KB of LDS,
+// 8 waves of 128 VGPRs): with one merge workgroup per two CUs a launch uses at most a quarter of
+// the places for waiting, and up to three launches on streams of their own still end.
+bool attn_span_supported(int num_cus, int nq, int nkv, int hd, const KvRing &kr) {
+    return nq / nkv <= kSpanMaxGroup && nq <= num_cus / 2 && (hd == 64 || hd == 128) &&
+           (kr.bits == 8 || kr.bits == 4) && (kr.window == 0 || kr.ring >= kr.window - kr.sinks);
 }
 
 size_t attn_span_words(int positions, int nq, int hd) { return (size_t)((positions + 127) / 128) * nq * (2 + hd); }
@@ -605,7 +608,7 @@ size_t attn_span_words(int positions, int nq, int hd) { return (size_t)((positio
 void launch_attn_span(hipStream_t st, const float *q, int8_t *kq, int8_t *vq, float *ks, float *vs, const AttnPost &post,
                       const int *pos_dev, int pos, int layer, int nq, int nkv, int hd, KvRing kr, float attn_scale,
                       int max_positions, float *out_f, int8_t *aq, float *as, int32_t *asum, const SpanWork &w) {
-    const int tpw = span_tiles(nkv, max_positions), P = 128 * tpw, G = nq / nkv;
+    const int tpw = span_tiles(w.num_cus, nkv, max_positions), P = 128 * tpw, G = nq / nkv;
     const int nspan = (max_positions + P - 1) / P;
     SpanArgs A{q, kq, vq, ks, vs, pos_dev, pos, layer, nq, nkv, kr, attn_scale, nspan, post, w.words,
                w.cnt, w.err, 1u << 20, out_f, aq, as, asum};

@@ -145,13 +145,14 @@ float *noalloc_scratch(int device) {
     return g_noalloc_ptr[device];
 }
 // The span words, counters and timeout word of one scratch region.
-SpanWork span_work_at(unsigned long long *words, size_t cap) {
-    return SpanWork{words, reinterpret_cast<unsigned int *>(words + cap), reinterpret_cast<int *>(words + cap + 1)};
+SpanWork span_work_at(const k2t_ctx *ctx, unsigned long long *words, size_t cap) {
+    return SpanWork{words, reinterpret_cast<unsigned int *>(words + cap), reinterpret_cast<int *>(words + cap + 1),
+                    ctx->num_cus};
 }
 
-SpanWork noalloc_span(int device) {
-    float *base = noalloc_scratch(device);
-    return span_work_at(reinterpret_cast<unsigned long long *>(base + kNoAllocScratchFloats), kNoAllocSpanWords);
+SpanWork noalloc_span(const k2t_ctx *ctx) {
+    float *base = noalloc_scratch(ctx->device);
+    return span_work_at(ctx, reinterpret_cast<unsigned long long *>(base + kNoAllocScratchFloats), kNoAllocSpanWords);
 }
 
 // k2t_attn_decode's span workspace on the context (zeroed whenever it grows).
@@ -170,7 +171,7 @@ SpanWork ctx_span(k2t_ctx *ctx, size_t words) {
         hip_check(hipMemset(ctx->span_words, 0, bytes), "span workspace clear");
         ctx->span_cap = words;
     }
-    return span_work_at(ctx->span_words, ctx->span_cap);
+    return span_work_at(ctx, ctx->span_words, ctx->span_cap);
 }
 
 // Reads a region's timeout word after a sync; on a timeout clears the region (its epochs
@@ -187,13 +188,13 @@ void raise_span_timeout(const SpanWork &g, size_t cap) {
 
 namespace k2t {
 void check_span_timeout(k2t_ctx *ctx) {
-    if (ctx->span_words) raise_span_timeout(span_work_at(ctx->span_words, ctx->span_cap), ctx->span_cap);
+    if (ctx->span_words) raise_span_timeout(span_work_at(ctx, ctx->span_words, ctx->span_cap), ctx->span_cap);
     bool seen = false;
     {
         std::lock_guard<std::mutex> lock(g_noalloc_mu);
         seen = ctx->device >= 0 && ctx->device < kMaxNoAllocDevices && g_noalloc_ptr[ctx->device] != nullptr;
     }
-    if (seen) raise_span_timeout(noalloc_span(ctx->device), kNoAllocSpanWords);
+    if (seen) raise_span_timeout(noalloc_span(ctx), kNoAllocSpanWords);
 }
 }  // namespace k2t
 
@@ -452,7 +453,7 @@ void forward(k2t_model *m, int ntok, bool with_logits, int ctx_bound = 0) {
         const ActTiles to = act_tiles_for(m, L.o, ntok);  // (none for one token: the grouped kernel writes none)
         launch_attention(st, m->qkv, (nq + 2 * nkv) * hd, m->kq, m->vq, m->ks, m->vs, post, m->pos_dev, l, nq, nkv,
                          hd, m->ring, attn_scale, nsplit, ntok, m->attn_part, nullptr, m->xq, m->xs, m->xsum,
-                         SpanWork{m->attn_words, m->attn_cnt, m->err_dev}, ctx_bound, to, ctx->mfma != 0);
+                         SpanWork{m->attn_words, m->attn_cnt, m->err_dev, ctx->num_cus}, ctx_bound, to, ctx->mfma != 0);
         launch_gemv_ex(ctx, L.o, m->xq, m->xs, m->xsum, ntok, m->hidden, d, true, 0, to);
         if (L.has_moe) {
             // each token has its own routes (forward_layer_single); a batch groups its tokens
@@ -1334,16 +1335,16 @@ void attn_decode_impl(k2t_ctx *ctx, int32_t bits, const float *d_q, int32_t n_he
     // One launch over spans of the cache, whose words persist across calls (context
     // workspace, or the fixed no-alloc region); the position goes with the launch.
     const size_t words = attn_span_words(act, n_heads, head_dim);
-    if (attn_span_supported(n_heads, n_kv_heads, head_dim, kr) && (!noalloc || words <= kNoAllocSpanWords)) {
-        const SpanWork sw = noalloc ? noalloc_span(ctx->device) : ctx_span(ctx, words);
+    if (attn_span_supported(ctx->num_cus, n_heads, n_kv_heads, head_dim, kr) && (!noalloc || words <= kNoAllocSpanWords)) {
+        const SpanWork sw = noalloc ? noalloc_span(ctx) : ctx_span(ctx, words);
         launch_attn_span(ctx->stream, d_q, (int8_t *)d_kq, (int8_t *)d_vq, (float *)d_ks, (float *)d_vs, AttnPost{}, nullptr,
                          seq - 1, 0, n_heads, n_kv_heads, head_dim, kr, attn_scale, act, d_out, nullptr, nullptr, nullptr,
                          sw);
         if (!noalloc) hip_check(hipStreamSynchronize(ctx->stream), "sync");
         return;
     }
-    // More than 8 q heads per KV head, or more spans than the no-alloc region holds: split
-    // partials and a merge.
+    // More than 8 q heads per KV head, more heads than a launch can keep waiting, or more spans
+    // than the no-alloc region holds: split partials and a merge.
     float *pp;
     if (noalloc) {
         pp = noalloc_scratch(ctx->device);

@@ -224,6 +224,7 @@ struct SpanWork {
     unsigned long long *words = nullptr;
     unsigned int *cnt = nullptr;
     int *err = nullptr;
+    int num_cus = 0;
 };
 
 // One-token decode attention that also does qkv_post's work (bias, QK-norm, RoPE, K/V
@@ -235,9 +236,9 @@ struct AttnPost {
 };
 
 // Decode attention of one token in one launch over spans of the cache: up to 8 q heads per
-// KV head, head size 64 or 128.  The position is *pos_dev, or pos where pos_dev is NULL; no
+// KV head, a q head per two CUs, head size 64 or 128.  The position is *pos_dev, or pos where pos_dev is NULL; no
 // more than max_positions are attended.  attn_span_words: the span words it needs.
-bool attn_span_supported(int nq, int nkv, int hd, const KvRing &kr);
+bool attn_span_supported(int num_cus, int nq, int nkv, int hd, const KvRing &kr);
 size_t attn_span_words(int positions, int nq, int hd);
 void launch_attn_span(hipStream_t st, const float *q, int8_t *kq, int8_t *vq, float *ks, float *vs, const AttnPost &post,
                       const int *pos_dev, int pos, int layer, int nq, int nkv, int hd, KvRing kr, float attn_scale,

@@ -815,7 +815,7 @@ void launch_attention(hipStream_t st, const float *q, int q_stride, int8_t *kq, 
         hip_check(hipGetLastError(), "attention launch");
         return;
     }
-    if (span.words && ntok == 1 && !tiles.xt && attn_span_supported(nq, nkv, hd, kr)) {
+    if (span.words && ntok == 1 && !tiles.xt && attn_span_supported(span.num_cus, nq, nkv, hd, kr)) {
         const int most = std::min(nsplit * kAttnSplitLen, kr.window > 0 ? kr.window : kr.cap);
         launch_attn_span(st, q, kq, vq, ks, vs, post, pos_dev, 0, layer, nq, nkv, hd, kr, attn_scale, most, out_f, aq, as,
                          asum, span);

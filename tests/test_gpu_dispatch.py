@@ -306,6 +306,33 @@ def test_moe_prompt_equals_token_by_token(gpu_ctx, bits, E, k, d, ntok, max_batc
     bank.close()
 
 
+# more heads than may wait in one launch (half the CUs): split partials and a merge
+@pytest.mark.parametrize("nq,nkv,hd,seq,window", [(136, 136, 64, 1100, 0), (512, 64, 64, 300, 0), (600, 150, 128, 700, 300)])
+@pytest.mark.parametrize("bits", [8, 4])
+def test_attention_of_many_heads(gpu_ctx, nq, nkv, hd, bits, seq, window):
+    """A call of many heads gives each group of them what a call of its own gives (4e-5 of the
+    largest output: two fp32 orders), and never waits for workgroups that have no place to run."""
+    import torch
+    rng = np.random.default_rng(nq + seq)
+    cap, sinks = (window + 512, 4) if window else (seq, 0)
+    codes = [torch.empty((nkv, cap, hd if bits == 8 else hd // 2), dtype=torch.int8, device="cuda") for _ in range(2)]
+    scales = [torch.empty((nkv, cap, 1 if bits == 8 else hd // 64), device="cuda",
+                          dtype=torch.float32 if bits == 8 else torch.bfloat16) for _ in range(2)]
+    for c, s in zip(codes, scales):
+        gpu_ctx.kv_store(bits, _t(rng.standard_normal((nkv * cap, hd)).astype(np.float32)), nkv * cap, hd, c, s)
+    q = _t((2 * rng.standard_normal((nq, hd))).astype(np.float32))
+    out, own = torch.full((nq, hd), float("nan"), device="cuda"), torch.full((nq, hd), float("nan"), device="cuda")
+    for call in (gpu_ctx.attn_decode, gpu_ctx.attn_decode_noalloc):
+        call(bits, q, nq, nkv, hd, codes[0], scales[0], codes[1], scales[1], cap, seq, hd ** -0.5, out, window, sinks)
+        gpu_ctx.sync()
+        g = nq // nkv
+        for k in range(0, nkv, 10):
+            n = min(10, nkv - k)
+            gpu_ctx.attn_decode(bits, q[k * g:], n * g, n, hd, codes[0][k:], scales[0][k:], codes[1][k:], scales[1][k:], cap,
+                                seq, hd ** -0.5, own[k * g:], window, sinks)
+        assert (out - own).abs().max() <= 4e-5 * own.abs().max()
+
+
 # one span (128- and 256-position form) and its edges, several spans, more spans than a merge
 # thread polls at once; 1 .. 8 q heads per KV head; windows not yet full, full and wrapped
 @pytest.mark.parametrize("nq,nkv,hd", [(3, 3, 64), (6, 2, 128), (8, 2, 64), (10, 2, 128), (8, 1, 64)])
