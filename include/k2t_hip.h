@@ -74,6 +74,10 @@ int32_t k2t_ctx_set_stream(k2t_ctx *ctx, void *hip_stream);
 int32_t k2t_ctx_sync(k2t_ctx *ctx);
 /* Cap on the K segments (waves per workgroup) k2t_gemv may use: 0 = automatic. */
 int32_t k2t_ctx_set_splitk(k2t_ctx *ctx, int32_t max_segments);
+/* Polls (about 0.5 us each) after which a wait inside k2t_attn_decode / _noalloc gives up, for
+ * callers that want a shorter bound; 0 = the default (1 << 20).  Such a call's output is not
+ * valid: k2t_attn_decode, or the next k2t_ctx_sync after the no-alloc variant, returns K2T_E_HIP. */
+int32_t k2t_ctx_set_span_wait(k2t_ctx *ctx, int32_t polls);
 /* fp32 epilogue of k2t_gemv.  exact = 1 replays the reference's per-row fmaf chain
  * in chunk order (simd_lut.rs:4030-4059, 6334-6335) and is bit-identical to it;
  * exact = 0 (default) sums per-segment chains in a fixed order: deterministic and

@@ -258,6 +258,7 @@ void k2t_ctx_destroy(k2t_ctx *ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     if (ctx->span_words) (void)hipFree(ctx->span_words);
+    if (ctx->span_err) (void)hipHostFree(ctx->span_err);
     if (ctx->signs) (void)hipFree(ctx->signs);
     delete ctx;
 }
@@ -290,6 +291,14 @@ int32_t k2t_ctx_set_exact(k2t_ctx *ctx, int32_t exact) {
     return guarded([&] {
         arg_check(ctx != nullptr, "ctx is NULL");
         ctx->exact = exact ? 1 : 0;
+    });
+}
+
+int32_t k2t_ctx_set_span_wait(k2t_ctx *ctx, int32_t polls) {
+    return guarded([&] {
+        arg_check(ctx != nullptr, "ctx is NULL");
+        arg_check(polls >= 0, "polls must be >= 0");
+        ctx->span_wait = polls == 0 ? kSpanWait : (unsigned int)polls;
     });
 }
 

@@ -611,7 +611,7 @@ void launch_attn_span(hipStream_t st, const float *q, int8_t *kq, int8_t *vq, fl
     const int tpw = span_tiles(w.num_cus, nkv, max_positions), P = 128 * tpw, G = nq / nkv;
     const int nspan = (max_positions + P - 1) / P;
     SpanArgs A{q, kq, vq, ks, vs, pos_dev, pos, layer, nq, nkv, kr, attn_scale, nspan, post, w.words,
-               w.cnt, w.err, 1u << 20, out_f, aq, as, asum};
+               w.cnt, w.err, w.wait, out_f, aq, as, asum};
     const dim3 grid(nkv, G + nspan);
     const size_t lds = std::max(span_lds(hd, P, G), (size_t)(64 + 4 * kSpanThreads + 64) * sizeof(float));
     const bool ring = kr.window > 0;

@@ -144,15 +144,14 @@ float *noalloc_scratch(int device) {
     }
     return g_noalloc_ptr[device];
 }
-// The span words, counters and timeout word of one scratch region.
-SpanWork span_work_at(const k2t_ctx *ctx, unsigned long long *words, size_t cap) {
-    return SpanWork{words, reinterpret_cast<unsigned int *>(words + cap), reinterpret_cast<int *>(words + cap + 1),
-                    ctx->num_cus};
+// The span words and counters of one scratch region and its timeout word.
+SpanWork span_work_at(const k2t_ctx *ctx, unsigned long long *words, size_t cap, int *err) {
+    return SpanWork{words, reinterpret_cast<unsigned int *>(words + cap), err, ctx->num_cus, ctx->span_wait};
 }
 
 SpanWork noalloc_span(const k2t_ctx *ctx) {
-    float *base = noalloc_scratch(ctx->device);
-    return span_work_at(ctx, reinterpret_cast<unsigned long long *>(base + kNoAllocScratchFloats), kNoAllocSpanWords);
+    auto *words = reinterpret_cast<unsigned long long *>(noalloc_scratch(ctx->device) + kNoAllocScratchFloats);
+    return span_work_at(ctx, words, kNoAllocSpanWords, reinterpret_cast<int *>(words + kNoAllocSpanWords + 1));
 }
 
 // k2t_attn_decode's span workspace on the context (zeroed whenever it grows).
@@ -162,7 +161,13 @@ SpanWork ctx_span(k2t_ctx *ctx, size_t words) {
         if (ctx->span_words) hip_check(hipFree(ctx->span_words), "hipFree");
         ctx->span_words = nullptr;
         ctx->span_cap = 0;
-        const size_t bytes = (words + 2) * sizeof(unsigned long long);
+        if (!ctx->span_err) {
+            void *p = nullptr;
+            hip_check(hipHostMalloc(&p, sizeof(int), hipHostMallocMapped | hipHostMallocCoherent), "span timeout word");
+            ctx->span_err = static_cast<int *>(p);
+            *ctx->span_err = 0;
+        }
+        const size_t bytes = (words + 1) * sizeof(unsigned long long);
         hipError_t e = hipMalloc((void **)&ctx->span_words, bytes);
         if (e != hipSuccess) {
             (void)hipGetLastError();
@@ -171,30 +176,38 @@ SpanWork ctx_span(k2t_ctx *ctx, size_t words) {
         hip_check(hipMemset(ctx->span_words, 0, bytes), "span workspace clear");
         ctx->span_cap = words;
     }
-    return span_work_at(ctx, ctx->span_words, ctx->span_cap);
+    return span_work_at(ctx, ctx->span_words, ctx->span_cap, ctx->span_err);
 }
 
-// Reads a region's timeout word after a sync; on a timeout clears the region (its epochs
-// start over) and raises.
-void raise_span_timeout(const SpanWork &g, size_t cap) {
-    int e = 0;
-    hip_check(hipMemcpy(&e, g.err, sizeof(int), hipMemcpyDeviceToHost), "span timeout word");
-    if (!e) return;
-    hip_check(hipMemset(g.words, 0, (cap + 2) * sizeof(unsigned long long)), "span workspace clear");
+// After a wait that timed out: clears `words` (the region's epochs start over) and raises.
+void raise_span_timeout(k2t_ctx *ctx, unsigned long long *words, size_t n) {
+    hip_check(hipMemsetAsync(words, 0, n * sizeof(unsigned long long), ctx->stream), "span workspace clear");
+    hip_check(hipStreamSynchronize(ctx->stream), "span workspace clear");
     throw Error(K2T_E_HIP, "span attention: span wait timed out");
+}
+
+// The timeout word of k2t_attn_decode's workspace, after a sync.
+void check_ctx_span(k2t_ctx *ctx) {
+    if (!ctx->span_err || !__atomic_load_n(ctx->span_err, __ATOMIC_RELAXED)) return;
+    *ctx->span_err = 0;
+    if (ctx->span_words) raise_span_timeout(ctx, ctx->span_words, ctx->span_cap + 1);
 }
 
 }  // namespace
 
 namespace k2t {
 void check_span_timeout(k2t_ctx *ctx) {
-    if (ctx->span_words) raise_span_timeout(span_work_at(ctx, ctx->span_words, ctx->span_cap), ctx->span_cap);
+    check_ctx_span(ctx);
     bool seen = false;
     {
         std::lock_guard<std::mutex> lock(g_noalloc_mu);
         seen = ctx->device >= 0 && ctx->device < kMaxNoAllocDevices && g_noalloc_ptr[ctx->device] != nullptr;
     }
-    if (seen) raise_span_timeout(noalloc_span(ctx), kNoAllocSpanWords);
+    if (!seen) return;
+    const SpanWork g = noalloc_span(ctx);
+    int e = 0;
+    hip_check(hipMemcpy(&e, g.err, sizeof(int), hipMemcpyDeviceToHost), "span timeout word");
+    if (e) raise_span_timeout(ctx, g.words, kNoAllocSpanWords + 2);
 }
 }  // namespace k2t
 
@@ -1340,7 +1353,10 @@ void attn_decode_impl(k2t_ctx *ctx, int32_t bits, const float *d_q, int32_t n_he
         launch_attn_span(ctx->stream, d_q, (int8_t *)d_kq, (int8_t *)d_vq, (float *)d_ks, (float *)d_vs, AttnPost{}, nullptr,
                          seq - 1, 0, n_heads, n_kv_heads, head_dim, kr, attn_scale, act, d_out, nullptr, nullptr, nullptr,
                          sw);
-        if (!noalloc) hip_check(hipStreamSynchronize(ctx->stream), "sync");
+        if (!noalloc) {
+            hip_check(hipStreamSynchronize(ctx->stream), "sync");
+            check_ctx_span(ctx);
+        }
         return;
     }
     // More than 8 q heads per KV head, more heads than a launch can keep waiting, or more spans

@@ -8,6 +8,8 @@
 #include <stdexcept>
 #include <string>
 
+constexpr unsigned int kSpanWait = 1u << 20;
+
 struct k2t_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -20,9 +22,12 @@ struct k2t_ctx {
     float *scratch = nullptr;
     size_t scratch_cap = 0;  // floats
     // span attention words of k2t_attn_decode ({payload, epoch}, zeroed when
-    // allocated), then its counters {epoch, merges done} and timeout word
+    // allocated), then its counters {epoch, merges done}; its timeout word in pinned host
+    // memory (read after each call's sync without a copy)
     unsigned long long *span_words = nullptr;
     size_t span_cap = 0;  // words
+    int *span_err = nullptr;
+    unsigned int span_wait = kSpanWait;  // polls before a wait gives up
     // hand-off words of k2t_moe_ffn's routing (kMoeStateWords after the sign masks, zeroed at
     // creation): {epoch, value} words that no later call's epoch matches, then the call counter and
     // the timeout word
@@ -225,6 +230,7 @@ struct SpanWork {
     unsigned int *cnt = nullptr;
     int *err = nullptr;
     int num_cus = 0;
+    unsigned int wait = kSpanWait;
 };
 
 // One-token decode attention that also does qkv_post's work (bias, QK-norm, RoPE, K/V

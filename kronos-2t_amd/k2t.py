@@ -49,6 +49,7 @@ SIGNATURES = {
     "k2t_ctx_sync": (I32, [VP]),
     "k2t_ctx_set_splitk": (I32, [VP, I32]),
     "k2t_ctx_set_exact": (I32, [VP, I32]),
+    "k2t_ctx_set_span_wait": (I32, [VP, I32]),
     "k2t_ctx_set_mfma": (I32, [VP, I32]),
     "k2t_malloc": (I32, [VP, SZ, C.POINTER(VP)]),
     "k2t_free": (I32, [VP, VP]),
@@ -212,6 +213,10 @@ class Ctx:
 
     def set_splitk(self, n):
         check(lib().k2t_ctx_set_splitk(self.h, int(n)))
+
+    def set_span_wait(self, polls):
+        """k2t_ctx_set_span_wait: polls before attn_decode's wait gives up (0: the default)."""
+        check(lib().k2t_ctx_set_span_wait(self.h, int(polls)))
 
     def set_exact(self, on):
         check(lib().k2t_ctx_set_exact(self.h, int(bool(on))))

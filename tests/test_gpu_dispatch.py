@@ -641,3 +641,30 @@ def test_batch_past_two_gib_of_activations(gpu_ctx, fmt):
     gpu_ctx.sync()
     assert own.any() and (out[-last:] - own).abs().max() <= 1e-5 * own.abs().max()
     m.close()
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_attention_wait_that_gives_up_is_reported(gpu_ctx, noalloc):
+    """A merge that stops waiting before its spans are there (32 polls, a context whose spans take
+    ten times as long) makes k2t_attn_decode, or the sync after the no-alloc variant, raise; the
+    next call, with the usual bound, is right again."""
+    import torch
+    rng = np.random.default_rng(9)
+    nq, hd, seq = (128, 64, 40000) if not noalloc else (32, 64, 31000)
+    code = [torch.from_numpy(rng.integers(-100, 100, (nq, seq, hd), np.int8)).cuda() for _ in range(2)]
+    scale = [torch.full((nq, seq), 0.01, device="cuda") for _ in range(2)]
+    q, out = _t(rng.standard_normal((nq, hd)).astype(np.float32)), [torch.zeros((nq, hd), device="cuda") for _ in range(2)]
+    call = gpu_ctx.attn_decode_noalloc if noalloc else gpu_ctx.attn_decode
+    args = (8, q, nq, nq, hd, code[0], scale[0], code[1], scale[1], seq, seq, hd ** -0.5)
+    call(*args, out[0])
+    gpu_ctx.sync()
+    gpu_ctx.set_span_wait(1)
+    try:
+        with pytest.raises(k2t.K2TError, match="timed out"):
+            call(*args, out[1])
+            gpu_ctx.sync()
+    finally:
+        gpu_ctx.set_span_wait(0)
+    call(*args, out[1])
+    gpu_ctx.sync()
+    assert out[0].any() and torch.equal(out[0], out[1])
