@@ -383,11 +383,11 @@ int32_t k2t_attn_decode(k2t_ctx *ctx, int32_t bits, const float *d_q, int32_t n_
 /* k2t_attn_decode without any allocation.  No counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  Same arguments and results as k2t_attn_decode
- * (the same kernels), but the span partials and the position word live in a fixed 4 MiB
- * device array inside the library (one per GPU, kept until the process ends): calls with
- * n_heads * ceil(min(seq, window or seq) / 256) * (head_dim + 2) > 1048512 floats (for
- * contexts above 1024 positions; at most 1024 positions use a single span) return
- * K2T_E_ARG.  Asynchronous on the context's stream (the caller synchronizes).  Every call
+ * (the same kernels), but its workspaces live in a fixed 8 MiB device array inside the
+ * library (one per GPU, kept until the process ends).  With n = min(seq, window or seq):
+ * calls with n_heads * (n > 1024 ? ceil(n / 256) : 1) * (head_dim + 2) > 1048512, and above
+ * 1024 positions grouped queries (2 .. 8 q heads per KV head) over an int8 cache without a
+ * window with ceil(cap / 128) * n_heads * (head_dim + 2) > 524288, return K2T_E_ARG.  Asynchronous on the context's stream (the caller synchronizes).  Every call
  * on one GPU shares that array: calls that overlap on one GPU (other streams, other
  * contexts, other host threads) race. */
 int32_t k2t_attn_decode_noalloc(k2t_ctx *ctx, int32_t bits, const float *d_q, int32_t n_heads, int32_t n_kv_heads,

@@ -154,10 +154,28 @@ SpanWork noalloc_span(const k2t_ctx *ctx) {
     return span_work_at(ctx, words, kNoAllocSpanWords, reinterpret_cast<int *>(words + kNoAllocSpanWords + 1));
 }
 
-// k2t_attn_decode's span workspace on the context (zeroed whenever it grows).
-SpanWork ctx_span(k2t_ctx *ctx, size_t words) {
+// After a wait that timed out: clears `words` (the region's epochs start over) and raises.
+void raise_span_timeout(k2t_ctx *ctx, unsigned long long *words, size_t n) {
+    hip_check(hipMemsetAsync(words, 0, n * sizeof(unsigned long long), ctx->stream), "span workspace clear");
+    hip_check(hipStreamSynchronize(ctx->stream), "span workspace clear");
+    throw Error(K2T_E_HIP, "span attention: span wait timed out");
+}
+
+// The timeout word of k2t_attn_decode's workspace, after a sync.
+void check_ctx_span(k2t_ctx *ctx) {
+    if (!ctx->span_err || !__atomic_load_n(ctx->span_err, __ATOMIC_RELAXED)) return;
+    *ctx->span_err = 0;
+    if (ctx->span_words) raise_span_timeout(ctx, ctx->span_words, ctx->span_cap + 1);
+}
+
+// k2t_attn_decode's span workspace on the context (zeroed whenever it grows).  It grows to
+// twice what it was, up to `most` (the whole cache's words): a loop over a growing context
+// allocates a few times in all.
+SpanWork ctx_span(k2t_ctx *ctx, size_t words, size_t most) {
     if (words > ctx->span_cap) {
+        words = std::max(words, std::min(most, 2 * ctx->span_cap));
         hip_check(hipStreamSynchronize(ctx->stream), "span workspace sync");
+        check_ctx_span(ctx);  // (an earlier call's timeout, before its words go)
         if (ctx->span_words) hip_check(hipFree(ctx->span_words), "hipFree");
         ctx->span_words = nullptr;
         ctx->span_cap = 0;
@@ -173,24 +191,10 @@ SpanWork ctx_span(k2t_ctx *ctx, size_t words) {
             (void)hipGetLastError();
             throw Error(K2T_E_NOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));
         }
-        hip_check(hipMemset(ctx->span_words, 0, bytes), "span workspace clear");
+        hip_check(hipMemsetAsync(ctx->span_words, 0, bytes, ctx->stream), "span workspace clear");
         ctx->span_cap = words;
     }
     return span_work_at(ctx, ctx->span_words, ctx->span_cap, ctx->span_err);
-}
-
-// After a wait that timed out: clears `words` (the region's epochs start over) and raises.
-void raise_span_timeout(k2t_ctx *ctx, unsigned long long *words, size_t n) {
-    hip_check(hipMemsetAsync(words, 0, n * sizeof(unsigned long long), ctx->stream), "span workspace clear");
-    hip_check(hipStreamSynchronize(ctx->stream), "span workspace clear");
-    throw Error(K2T_E_HIP, "span attention: span wait timed out");
-}
-
-// The timeout word of k2t_attn_decode's workspace, after a sync.
-void check_ctx_span(k2t_ctx *ctx) {
-    if (!ctx->span_err || !__atomic_load_n(ctx->span_err, __ATOMIC_RELAXED)) return;
-    *ctx->span_err = 0;
-    if (ctx->span_words) raise_span_timeout(ctx, ctx->span_words, ctx->span_cap + 1);
 }
 
 }  // namespace
@@ -1336,7 +1340,8 @@ void attn_decode_impl(k2t_ctx *ctx, int32_t bits, const float *d_q, int32_t n_he
         throw Error(K2T_E_ARG, "k2t_attn_decode_noalloc: n_heads * ceil(positions / 256) * (head_dim + 2) = " +
                                    std::to_string(part) + " floats exceeds its fixed scratch of " +
                                    std::to_string(kNoAllocScratchFloats - 64) + " floats");
-    // Grouped queries over a long int8 cache: the no-alloc region is sized for the whole cache.
+    // Grouped queries over a long int8 cache: refused when the whole cache's words exceed the
+    // no-alloc region, so that a caller learns of it before its context has grown.
     const int group = n_heads / n_kv_heads;
     if (noalloc && nsplit > 1 && group >= 2 && group <= 8 && bits == 8 && window <= 0) {
         const size_t words = attn_span_words(cap, n_heads, head_dim);
@@ -1349,7 +1354,8 @@ void attn_decode_impl(k2t_ctx *ctx, int32_t bits, const float *d_q, int32_t n_he
     // workspace, or the fixed no-alloc region); the position goes with the launch.
     const size_t words = attn_span_words(act, n_heads, head_dim);
     if (attn_span_supported(ctx->num_cus, n_heads, n_kv_heads, head_dim, kr) && (!noalloc || words <= kNoAllocSpanWords)) {
-        const SpanWork sw = noalloc ? noalloc_span(ctx) : ctx_span(ctx, words);
+        const SpanWork sw = noalloc ? noalloc_span(ctx)
+                                    : ctx_span(ctx, words, attn_span_words(window > 0 ? window : cap, n_heads, head_dim));
         launch_attn_span(ctx->stream, d_q, (int8_t *)d_kq, (int8_t *)d_vq, (float *)d_ks, (float *)d_vs, AttnPost{}, nullptr,
                          seq - 1, 0, n_heads, n_kv_heads, head_dim, kr, attn_scale, act, d_out, nullptr, nullptr, nullptr,
                          sw);

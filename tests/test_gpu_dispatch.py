@@ -668,3 +668,31 @@ def test_attention_wait_that_gives_up_is_reported(gpu_ctx, noalloc):
     call(*args, out[1])
     gpu_ctx.sync()
     assert out[0].any() and torch.equal(out[0], out[1])
+
+
+def test_attention_of_a_growing_context_allocates_a_few_times():
+    """A decode loop over a growing cache: the context's span workspace (2 MB per 2048 positions of
+    these heads, which the free memory shows) doubles instead of growing with every call, and
+    every call equals the same call on a context whose workspace was large from the start."""
+    import torch
+    nq, hd, cap = 128, 128, 32768
+    g = torch.Generator(device="cuda").manual_seed(4)
+    code = [torch.empty((nq, cap, hd), dtype=torch.int8, device="cuda").random_(-100, 100, generator=g) for _ in range(2)]
+    scale = [torch.full((nq, cap), 0.01, device="cuda") for _ in range(2)]
+    q, out = torch.randn((nq, hd), device="cuda", generator=g), [torch.zeros((nq, hd), device="cuda") for _ in range(2)]
+    grown, large = k2t.Ctx(0), k2t.Ctx(0)
+    args = lambda n: (8, q, nq, nq, hd, code[0], scale[0], code[1], scale[1], cap, n, hd ** -0.5)  # noqa: E731
+    large.attn_decode(*args(cap), out[1])
+    grown.attn_decode(*args(1), out[0])
+    torch.cuda.synchronize()
+    free, steps = torch.cuda.mem_get_info()[0], 0
+    for n in range(300, cap, 2048):
+        grown.attn_decode(*args(n), out[0])
+        large.attn_decode(*args(n), out[1])
+        assert torch.equal(out[0], out[1])
+        now = torch.cuda.mem_get_info()[0]
+        steps += now != free
+        free = now
+    assert 2 <= steps <= 7  # 16 calls
+    grown.close()
+    large.close()
