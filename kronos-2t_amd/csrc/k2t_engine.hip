@@ -1353,7 +1353,12 @@ void attn_decode_impl(k2t_ctx *ctx, int32_t bits, const float *d_q, int32_t n_he
     // One launch over spans of the cache, whose words persist across calls (context
     // workspace, or the fixed no-alloc region); the position goes with the launch.
     const size_t words = attn_span_words(act, n_heads, head_dim);
-    if (attn_span_supported(ctx->num_cus, n_heads, n_kv_heads, head_dim, kr) && (!noalloc || words <= kNoAllocSpanWords)) {
+    // (16-byte V pieces and, at head size 128, both blocks' BF16 scales in one load: a cache at
+    // an odd address takes the kernels with the smaller loads)
+    const auto at = [](const void *p) { return reinterpret_cast<uintptr_t>(p); };
+    const bool aligned = (at(d_kq) | at(d_vq)) % 16 == 0 && (at(d_ks) | at(d_vs)) % (bits == 8 || head_dim == 128 ? 4 : 2) == 0;
+    if (aligned && attn_span_supported(ctx->num_cus, n_heads, n_kv_heads, head_dim, kr) &&
+        (!noalloc || words <= kNoAllocSpanWords)) {
         const SpanWork sw = noalloc ? noalloc_span(ctx)
                                     : ctx_span(ctx, words, attn_span_words(window > 0 ? window : cap, n_heads, head_dim));
         launch_attn_span(ctx->stream, d_q, (int8_t *)d_kq, (int8_t *)d_vq, (float *)d_ks, (float *)d_vs, AttnPost{}, nullptr,
@@ -1365,7 +1370,7 @@ void attn_decode_impl(k2t_ctx *ctx, int32_t bits, const float *d_q, int32_t n_he
         }
         return;
     }
-    // More than 8 q heads per KV head, more heads than a launch can keep waiting, or more spans
+    // An odd address, more than 8 q heads per KV head, more heads than a launch can keep waiting, or more spans
     // than the no-alloc region holds: split partials and a merge.
     float *pp;
     if (noalloc) {

@@ -696,3 +696,36 @@ def test_attention_of_a_growing_context_allocates_a_few_times():
     assert 2 <= steps <= 7  # 16 calls
     grown.close()
     large.close()
+
+
+@pytest.mark.parametrize("bits,hd,seq", [(8, 64, 1500), (8, 128, 300), (4, 64, 700), (4, 128, 1500)])
+def test_attention_of_a_cache_at_any_address(gpu_ctx, bits, hd, seq):
+    """V codes at a 4-byte address and, for the NF4 cache, scales at a 2-byte one: the output is
+    that of the aligned cache (4e-5 of the largest: two fp32 orders)."""
+    import torch
+    rng = np.random.default_rng(seq + bits)
+    nq, nkv = 8, 4
+    code, scale = [], []
+    for _ in range(2):
+        code.append(torch.empty((nkv, seq, hd if bits == 8 else hd // 2), dtype=torch.int8, device="cuda"))
+        scale.append(torch.empty((nkv, seq, 1 if bits == 8 else hd // 64), device="cuda",
+                                 dtype=torch.float32 if bits == 8 else torch.bfloat16))
+        gpu_ctx.kv_store(bits, _t(rng.standard_normal((nkv * seq, hd)).astype(np.float32)), nkv * seq, hd, code[-1], scale[-1])
+
+    def moved(t, n):
+        """A copy of t, n bytes past an aligned address."""
+        raw = t.reshape(-1).view(torch.uint8)
+        buf = torch.zeros(raw.numel() + n, dtype=torch.uint8, device="cuda")
+        buf[n:] = raw
+        return buf[n:]
+
+    q = _t(rng.standard_normal((nq, hd)).astype(np.float32))
+    out = torch.zeros((3, nq, hd), device="cuda")
+    v = moved(code[1], 4)
+    ks, vs = (moved(s, 2) if bits == 4 else s for s in scale)
+    gpu_ctx.attn_decode(bits, q, nq, nkv, hd, code[0], scale[0], code[1], scale[1], seq, seq, hd ** -0.5, out[0])
+    gpu_ctx.attn_decode(bits, q, nq, nkv, hd, code[0], ks, v, vs, seq, seq, hd ** -0.5, out[1])
+    gpu_ctx.attn_decode_noalloc(bits, q, nq, nkv, hd, code[0], ks, v, vs, seq, seq, hd ** -0.5, out[2])
+    gpu_ctx.sync()
+    assert out[0].any() and (out[1:] - out[0]).abs().max() <= 4e-5 * out[0].abs().max()
+    assert torch.equal(out[1], out[2])
