@@ -233,9 +233,10 @@ __device__ __forceinline__ void mf_fetch(const MfArgs &A, const MfSrc &R, const 
 }
 
 // One chunk's decode, MFMAs and epilogue steps.  A chunk whose activation scale is 0
-// needs no select: its term float(d) * 0 * ws is +-0, and adding +-0 leaves every
-// accumulator unchanged (each starts at +0 and a round-to-nearest sum is -0 only when
-// both addends are -0, so no accumulator is ever -0).
+// needs no select (NF4, bit planes) where ws is finite: its term float(d) * 0 * ws is +-0, and
+// adding +-0 leaves every accumulator unchanged (each starts at +0 and a round-to-nearest sum is
+// -0 only when both addends are -0, so no accumulator is ever -0).  Where the passes before these
+// kernels skipped such a chunk whatever ws (NF3, 2 .. 15 tokens, experts), its ws is taken as 0.
 template <int FMT, int HP, int NB>
 __device__ __forceinline__ void mf_step(const MfArgs &A, const MfChunk<FMT, NB> &f, float (&acc)[NB][4], uint32_t lane) {
     const v4i a = mf_decode<FMT, HP>(f.d0, f.d1, f.hv, A.t0, A.t1, A.u0, A.u1, lane);
@@ -249,7 +250,7 @@ __device__ __forceinline__ void mf_step(const MfArgs &A, const MfChunk<FMT, NB> 
         for (int r = 0; r < 4; r++) {
             int dot = d[r];
             if constexpr (FMT == 0) dot = 2 * dot - ((1 << (4 + HP)) - 1) * f.su[b];
-            acc[b][r] = fmaf((float)dot * f.sx[b], ws[r], acc[b][r]);
+            acc[b][r] = fmaf((float)dot * f.sx[b], FMT == 2 && f.sx[b] == 0.0f ? 0.0f : ws[r], acc[b][r]);
         }
     }
 }
@@ -506,7 +507,8 @@ __global__ __launch_bounds__(64 * kKsWaves, 4) void gemm_ks_kernel(MfArgs A) {
             for (int r = 0; r < 4; r++) {
                 int dot = d[r];
                 if constexpr (FMT == 0) dot = 2 * dot - ((1 << (4 + HP)) - 1) * f.su[b];
-                tt[buf][wave][b][r][lane] = (float)dot * f.sx[b];
+                // (NF3: -0 marks a chunk to skip, mf_step's note)
+                tt[buf][wave][b][r][lane] = FMT == 2 && f.sx[b] == 0.0f ? -0.0f : (float)dot * f.sx[b];
             }
         }
         __syncthreads();
@@ -525,7 +527,8 @@ __global__ __launch_bounds__(64 * kKsWaves, 4) void gemm_ks_kernel(MfArgs A) {
                 for (int k = 0; k < 4; k++)
                     if (h + k < n)
 #pragma unroll
-                        for (int o = 0; o < OWN; o++) acc[o] = fmaf(t[o][k], ws[k], acc[o]);
+                        for (int o = 0; o < OWN; o++)
+                            acc[o] = fmaf(t[o][k], FMT == 2 && __float_as_uint(t[o][k]) == 0x80000000u ? 0.0f : ws[k], acc[o]);
             }
         }
     };
@@ -558,9 +561,10 @@ __global__ __launch_bounds__(64 * kKsWaves, 4) void gemm_ks_kernel(MfArgs A) {
                 for (int r = 0; r < 4; r++) po[ORD ? b : 0][r] = 0.0f;
         if (live) {
             const v4i a = mf_decode<FMT, HP>(f.d0, f.d1, f.hv, A.t0, A.t1, A.u0, A.u1, lane);
-            const float ws[4] = {bf16_lo(f.sw.x), bf16_hi(f.sw.x), bf16_lo(f.sw.y), bf16_hi(f.sw.y)};
 #pragma unroll
             for (int b = 0; b < NB; b++) {
+                const uint2 sw = f.sx[b] == 0.0f ? make_uint2(0u, 0u) : f.sw;  // (mf_step's note)
+                const float ws[4] = {bf16_lo(sw.x), bf16_hi(sw.x), bf16_lo(sw.y), bf16_hi(sw.y)};
                 const v4i zero = {0, 0, 0, 0};
                 const v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, f.x[b], zero, 0, 0, 0);
 #pragma unroll
@@ -777,7 +781,8 @@ __global__ __launch_bounds__(256, NP* TB >= 4 ? 1 : 2) void gemm_tile_kernel(MfA
                 for (int r = 0; r < 4; r++) {
                     int dot = d[s][b][r];
                     if constexpr (FMT == 0) dot = 2 * dot - ((1 << (4 + HP)) - 1) * x.su[b];
-                    acc[2 * k + s][b][r] = fmaf((float)dot * x.sx[b], wv[r], acc[2 * k + s][b][r]);
+                    const float w = FMT == 2 && x.sx[b] == 0.0f ? 0.0f : wv[r];
+                    acc[2 * k + s][b][r] = fmaf((float)dot * x.sx[b], w, acc[2 * k + s][b][r]);
                 }
         }
     };
@@ -992,7 +997,8 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
             const v4i a = mf_decode<FMT, HP>(f.d0[s], f.d1[s], f.hv[s], A.t0, A.t1, A.u0, A.u1, lane);
             const v4i zero = {0, 0, 0, 0};
             const v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, f.x, zero, 0, 0, 0);
-            const float ws[4] = {bf16_lo(f.sw[s].x), bf16_hi(f.sw[s].x), bf16_lo(f.sw[s].y), bf16_hi(f.sw[s].y)};
+            const uint2 sw = f.sx == 0.0f ? make_uint2(0u, 0u) : f.sw[s];  // (mf_step's note)
+            const float ws[4] = {bf16_lo(sw.x), bf16_hi(sw.x), bf16_lo(sw.y), bf16_hi(sw.y)};
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 int dot = d[r];
@@ -1128,7 +1134,8 @@ __global__ __launch_bounds__(1024) void gemv_mfma_items_kernel(GvArgs A, int R) 
                 const v4i a = mf_decode<FMT, 0>(wt[u].d0, wt[u].d1, wt[u].hv, A.t0, A.t1, A.u0, A.u1, lane);
                 const v4i zero = {0, 0, 0, 0};
                 const v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, x[u], zero, 0, 0, 0);
-                const float ws[4] = {bf16_lo(wt[u].sw.x), bf16_hi(wt[u].sw.x), bf16_lo(wt[u].sw.y), bf16_hi(wt[u].sw.y)};
+                const uint2 sw = sx[u] == 0.0f ? make_uint2(0u, 0u) : wt[u].sw;  // (mf_step's note)
+                const float ws[4] = {bf16_lo(sw.x), bf16_hi(sw.x), bf16_lo(sw.y), bf16_hi(sw.y)};
 #pragma unroll
                 for (int r = 0; r < 4; r++) acc[u][r] = fmaf((float)d[r] * sx[u], ws[r], 0.0f);
                 __builtin_amdgcn_sched_barrier(0);

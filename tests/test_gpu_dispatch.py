@@ -729,3 +729,45 @@ def test_attention_of_a_cache_at_any_address(gpu_ctx, bits, hd, seq):
     gpu_ctx.sync()
     assert out[0].any() and (out[1:] - out[0]).abs().max() <= 4e-5 * out[0].abs().max()
     assert torch.equal(out[1], out[2])
+
+
+# every kernel of batches whose passes skip a chunk of zero activation: 2 .. 15 tokens, NF3 on the
+# small-batch kernel, the K-split one (ordered and chain) and the tiles; rows 0 and 33 have an
+# infinite and a NaN scale in the first chunk
+@pytest.mark.parametrize("fmt,ntok,rows,cols", [("nf4", 5, 64, 576), ("b4", 7, 64, 576), ("b6", 15, 64, 576), ("nf3", 5, 64, 576),
+                                                ("nf3", 20, 64, 576), ("nf3", 200, 1040, 4160), ("nf3", 40, 8200, 1088),
+                                                ("nf3", 16, 8200, 2112), ("nf3", 130, 8200, 576)])
+@pytest.mark.parametrize("exact", [False, True])
+def test_chunk_of_zero_activation_is_skipped(gpu_ctx, fmt, ntok, rows, cols, exact):
+    """A chunk whose activation scale is 0 takes no part whatever the row's scale, as in the
+    4-token passes, whose outputs every batch equals."""
+    import torch
+    from helpers import acts, random_nf_streams, random_nibble4_streams
+    rng = np.random.default_rng(rows + ntok)
+    if fmt[0] == "b":
+        hp = int(fmt[1]) - 4
+        pair, tail = random_nibble4_streams(rng, rows, cols, hp)
+        per, at = pair.size // (rows // 32), 1024 + 256 * hp
+    else:
+        _, _, pair, tail = random_nf_streams(rng, rows, cols, 2, bits=int(fmt[2]))
+        per, at = pair.size // (rows // 32), 0
+    pair[at:at + 2] = np.frombuffer(b"\x80\x7f", np.uint8)  # row 0: inf
+    pair[per + at + 2:per + at + 4] = np.frombuffer(b"\xc0\x7f", np.uint8)  # row 33: NaN
+    if fmt[0] == "b":
+        m = gpu_ctx.upload_nibble4(rows, cols, hp, pair, tail)
+    else:
+        cb = np.sort(rng.choice(np.arange(-127, 128), 16, replace=False)).astype(np.int8)
+        m = gpu_ctx.upload_nf(rows, cols, int(fmt[2]), 2, cb, pair, tail)
+    xq, xs, xsum = acts(rng, cols, ntok, outlier_frac=0.001, outlier_scale=30.0)
+    n = 2 if fmt[0] != "b" else 1  # the chunks of that scale
+    for t in (0, ntok - 1):
+        xq[t, :64 * n], xs[t, :n], xsum[t, :n] = 0, 0.0, 0
+    got = _gemv(gpu_ctx, m, xq, xs, xsum, rows, exact)
+    gpu_ctx.set_mfma(False)
+    try:
+        want = _gemv(gpu_ctx, m, xq, xs, xsum, rows, exact)
+    finally:
+        gpu_ctx.set_mfma(True)
+    assert np.array_equal(got, want, equal_nan=True)
+    assert np.isfinite(got[[0, ntok - 1]]).all() and not np.isfinite(got[1, [0, 33]]).any()
+    m.close()
