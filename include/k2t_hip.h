@@ -88,8 +88,8 @@ int32_t k2t_ctx_set_exact(k2t_ctx *ctx, int32_t exact);
  * over the whole matrix, k2t_gemv and the model's prefill): enable = 1 (default) runs
  * them on the int8 matrix cores, one weight pass per 16 to 128 tokens, with outputs equal to the
  * exact-order epilogue's in either mode (NF3: in exact mode; otherwise each token's one-token
- * outputs), and with the fast epilogue 2 .. 15 tokens in one weight pass with each token's
- * one-token outputs; 0 runs the 4-token weight passes of the
+ * outputs), and with the fast epilogue 2 .. 15 tokens, where that is faster, in one weight pass
+ * with each token's one-token outputs; 0 runs the 4-token weight passes of the
  * reference's tiles (nf_sdot_decode_neon, simd_lut.rs:6074-6364;
  * nibble4_sdot_batch_stripe_range, 4101-4320).  2: matrix cores, but a model's prefill does not have the
  * activation's producer write the tile-major copy the GEMV reads (the GEMV copies it
@@ -168,7 +168,7 @@ int32_t k2t_act_quant_rmsnorm(k2t_ctx *ctx, const float *d_x, const float *d_nor
  * and for ntok > 1 their batch variants nibble4_sdot_batch_stripe_range /
  * nf_sdot_batch_stripe_range (4101, 6689): token t reads d_xq + t*K,
  * d_xs + t*K/64, d_xsum + t*K/64 and writes d_out[t*out_stride + row].
- * Weights are read once per 4 tokens (once for 2 .. 15 tokens on the matrix cores, see
+ * Weights are read once per 4 tokens (or once for up to 15 tokens on the matrix cores, see
  * k2t_ctx_set_mfma).  d_xsum is required for bit-plane
  * matrices and ignored for NF ones.  Per-(row, chunk) integer dots are exact;
  * with split-K disabled the fp32 result is bit-identical to the reference's

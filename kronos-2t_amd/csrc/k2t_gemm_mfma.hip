@@ -891,9 +891,11 @@ __global__ __launch_bounds__(256) void mf_tile_kernel(const int8_t *xq, const fl
 // from one MFMA per stripe-chunk.  The 4-token passes it replaces decode every weight once
 // per 4 tokens and spend two v_dot4 per four codes and token; here the decode and the MFMA
 // cost the same for 2 tokens as for 16, so what bounds it is the weight stream and, past
-// about 8 tokens, the gather of the activation rows (16 lines per load).  NF4 14336 x 4096,
-// 4 / 8 / 15 tokens: 12.6 / 21.1 / 40.3 us as 4-token passes, 9.6 / 10.7 / 12.7 us here (one
-// token 8.7); b6 4096 x 14336: 15.3 / 27.7 / 54.8 us, 14.0 / 18.0 / 23.4 us here.
+// about 8 tokens, the gather of the activation rows (16 lines per load).  Weights from the
+// Infinity Cache, NF4 14336 x 4096, 4 / 8 / 15 tokens: 12.6 / 21.1 / 40.3 us as 4-token passes,
+// 9.2 / 10.6 / 12.7 us here (one token 8.7); b6 4096 x 14336, 8 / 15 tokens: 27.7 / 54.8 us, 18.2 /
+// 23.8 us here; from HBM, 4 / 8 tokens of the first 13.0 / 21.8 us and 11.8 / 12.3 us.
+// gemv_four_token_passes says where the passes stay.
 // Sums: the order of gemv_kernel's fast epilogue, so a batch gives each token the bits of
 // the one-token GEMV.  A wave's chunks are dealt round-robin to G accumulators (the GEMV's
 // lane groups: 4 in pair mode, 8 in stripe mode), which are added pairwise as the lane
@@ -1192,11 +1194,30 @@ bool gemm_mfma_supported(const k2t_mat *m, int ntok) {
 }
 
 bool gemv_mfma_supported(const k2t_mat *m, int ntok) {
-    if (ntok < 2 || ntok >= kMfmaMinTokens || !gemm_mfma_supported(m, kMfmaMinTokens)) return false;
-    // NF3 up to 4 tokens: the 4-token pass (its 16-byte loads stream the 384-byte chunks
-    // better than this kernel's dwords: 4096 x 14336, 2 / 3 / 4 tokens 8.8 / 9.9 / 10.9 us
-    // there, 10.5 / 11.3 / 11.9 here; 8 tokens 19.3 there, 14.3 here)
-    return m->fmt != K2T_FMT_NF || m->bits != 3 || ntok > 4;
+    return ntok >= 2 && ntok < kMfmaMinTokens && gemm_mfma_supported(m, kMfmaMinTokens);
+}
+
+// Where the 4-token passes stay the better form.  Their 16-byte loads stream weights better than
+// this kernel's dwords; what they pay is decode and dots per token.  So only calls that are one
+// launch of one round of workgroups count (up to 4 tokens, or whole groups of 4 side by side),
+// and of those (weights from HBM, us in passes and here):
+//  - 2 tokens: NF4 14336 x 4096 10.1 and 11.4, b4 4096 x 4096 5.4 and 6.9, b6 4096 x 14336 12.4 and
+//    15.8 (b5 2048 x 2048 6.7 and 5.6, the one kind of exception);
+//  - NF3 up to 4 tokens, or with long rows: 4096 x 14336, 4 tokens 11.0 and 11.3; 2048 x 8192, 8
+//    tokens 7.9 and 8.9; not taken: 2048 x 4096, 8 tokens 6.6 and 5.8;
+//  - pair mode, b4 with 3 tokens: 14336 x 4096 11.5 and 12.2 (4 tokens 12.8 and 12.5; b5 3 tokens
+//    14.2 and 13.8, NF4 12.1 and 11.4: not taken);
+//  - stripe mode, by the row length where they meet: b4 4096 x 4096, 4 tokens 6.8 and 7.4; b5 2048 x
+//    8192, 4 tokens 9.5 and 9.9 (2048 x 5632: 8.0 and 7.6); NF4, b6 4096 x 14336, 3 tokens 12.1 and
+//    12.9, 15.6 and 16.1, 2048 x 16384, 8 tokens 12.9 and 13.5, 15.5 and 16.9 (2048 x 8192: 8.7 and
+//    8.8, 10.1 and 10.0; NF4 with 3 tokens 8.0 and 8.5).
+bool gemv_four_token_passes(const k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, int ntok) {
+    if (ntok > 4 && (ntok % 4 != 0 || (plan.rb_hi - plan.rb_lo) * (ntok / 4) > ctx->num_cus)) return false;
+    if (m->fmt == K2T_FMT_NF && m->bits == 3) return ntok <= 4 || m->nc > 96;
+    if (ntok == 2) return true;
+    const bool b4 = m->fmt == K2T_FMT_NIBBLE4 && m->hp == 0, b5 = m->fmt == K2T_FMT_NIBBLE4 && m->hp == 1;
+    if (!plan.stripe_mode) return b4 && ntok == 3;
+    return b4 || m->nc > (b5 || (ntok == 3 && m->fmt == K2T_FMT_NF) ? 96 : 160);
 }
 
 template <int FMT, int HP>
