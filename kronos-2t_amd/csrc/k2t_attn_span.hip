@@ -68,10 +68,16 @@ struct SpanArgs {
     int32_t *asum;
 };
 
-// LDS of a workgroup: the int8 K and V tiles [position][HD], later (the tiles no longer
-// read) the waves' partial o [wave][head][HD].
+// LDS of a workgroup: the int8 K and V tiles [position][HD], and the waves' partial o
+// [wave][head][o_stride(HD)]: behind the tiles in the kernel of more than four heads over 128-position
+// spans, which saves it the barrier before their first store, else in the tiles' place once
+// those are read.  The stride: heads HD floats apart lie in the same banks, and the stores of
+// eight heads took 0.6 us longer.
+constexpr int o_stride(int hd) { return hd + 4; }
+constexpr bool o_behind(int tiles_per_wave, bool g8) { return g8 && tiles_per_wave == 1; }
 size_t span_lds(int hd, int positions, int group) {
-    return std::max((size_t)2 * positions * hd, (size_t)kSpanWaves * group * hd * sizeof(float));
+    const size_t t = (size_t)2 * positions * hd, o = (size_t)kSpanWaves * group * o_stride(hd) * sizeof(float);
+    return o_behind(positions / 128, group > 4) ? t + o : std::max(t, o);
 }
 
 // o (this wave's 64-block b of q head `head`, one element per lane, rotated domain) through
@@ -120,8 +126,7 @@ __global__ __launch_bounds__(kSpanThreads, HD == 128 && G8 ? 4 : 6) void attn_sp
         constexpr int ncg = HD / 4, nsub = NTH / ncg;
         const int cg = (int)tid % ncg, sub = (int)tid / ncg;
         // spans per thread polled together; the large kernel has the registers for 3 (30B-A3B
-        // decode at 6600 positions, 52 spans: 420.6 tok/s with 2, 422 with 3, 419 with 4 at 127
-        // VGPRs)
+        // decode at 6600 positions, 52 spans: 422 tok/s with 3, 420 with 4 at 127 VGPRs)
         constexpr int kPre = HD == 128 && G8 ? 3 : 2;
         bool ok = true;
         auto poll = [&](int s, unsigned long long (&w)[6]) {
@@ -173,7 +178,8 @@ __global__ __launch_bounds__(kSpanThreads, HD == 128 && G8 ? 4 : 6) void attn_sp
                     if ((pending & (1u << (6 * j + k))) && (uint32_t)(wv6[j][k] >> 32) == ep)
                         pending &= ~(1u << (6 * j + k));
         }
-        // spans past kPre per thread (contexts above nsub * kPre * P positions): one by one
+        // spans past kPre per thread (contexts above nsub * kPre * P positions): one by one, the
+        // first of them kept (read again after the maximum, it cost another 0.3 us)
         auto wait6 = [&](int s, unsigned long long (&w)[6]) {
             poll(s, w);
             for (uint32_t spins = 0; ok; spins++) {
@@ -190,13 +196,17 @@ __global__ __launch_bounds__(kSpanThreads, HD == 128 && G8 ? 4 : 6) void attn_sp
                 poll(s, w);
             }
         };
+        const int sx = sub + kPre * nsub;
+        unsigned long long wx[6] = {(unsigned long long)__float_as_uint(-INFINITY)};
+        if (sx < nact) wait6(sx, wx);
         auto wf = [](unsigned long long w) { return __uint_as_float((uint32_t)w); };
         float *mred = reinterpret_cast<float *>(tiles);  // [NW] wave maxima
         // global maximum of the span maxima
         float M = -INFINITY;
 #pragma unroll
         for (int j = 0; j < kPre; j++) M = fmaxf(M, wf(wv6[j][0]));
-        for (int s = sub + kPre * nsub; s < nact; s += nsub) {
+        M = fmaxf(M, wf(wx[0]));
+        for (int s = sx + nsub; s < nact; s += nsub) {
             unsigned long long w[6];
             wait6(s, w);
             M = fmaxf(M, wf(w[0]));
@@ -219,7 +229,8 @@ __global__ __launch_bounds__(kSpanThreads, HD == 128 && G8 ? 4 : 6) void attn_sp
 #pragma unroll
         for (int j = 0; j < kPre; j++)
             if (sub + j * nsub < nact) add_span(wv6[j]);
-        for (int s = sub + kPre * nsub; s < nact; s += nsub) {
+        if (sx < nact) add_span(wx);
+        for (int s = sx + nsub; s < nact; s += nsub) {
             unsigned long long w[6];
             wait6(s, w);
             add_span(w);
@@ -521,8 +532,10 @@ __global__ __launch_bounds__(kSpanThreads, HD == 128 && G8 ? 4 : 6) void attn_sp
     psum += xor_lane(psum, 16);
     psum += xor_lane(psum, 32);
     if (lane < (uint32_t)GC && hl) red_l[lane][wv] = psum;
-    __syncthreads();  // the tiles are read: their place takes the waves' partial o
-    float *opw = reinterpret_cast<float *>(tiles);  // [wave][head][HD]
+    constexpr int OS = o_stride(HD);
+    constexpr bool kBehind = o_behind(TPW, G8);
+    if constexpr (!kBehind) __syncthreads();  // the tiles are read
+    float *opw = reinterpret_cast<float *>(tiles + (kBehind ? 2 * P * HD : 0));  // [wave][head][OS]
 #pragma unroll
     for (int h = 0; h < HP; h++) {
         // Rows added: a swap of odd and even 16-lane rows of two values and an add leave
@@ -540,7 +553,7 @@ __global__ __launch_bounds__(kSpanThreads, HD == 128 && G8 ? 4 : 6) void attn_sp
         }
         const int head = 4 * h + (int)(lane & 3u);
         if (head < G) {
-            float *dst = opw + ((size_t)wv * G + head) * HD + DB * (4 * (int)(li >> 2) + (int)lg);
+            float *dst = opw + ((size_t)wv * G + head) * OS + DB * (4 * (int)(li >> 2) + (int)lg);
 #pragma unroll
             for (int k = 0; k < DB; k += 4) *reinterpret_cast<float4 *>(dst + k) = make_float4(v[k], v[k + 1], v[k + 2], v[k + 3]);
         }
@@ -550,8 +563,13 @@ __global__ __launch_bounds__(kSpanThreads, HD == 128 && G8 ? 4 : 6) void attn_sp
     unsigned long long *pbase = A.words + (size_t)(kvh * G) * pstride + (size_t)span * (2 + HD);
     for (int i = (int)tid; i < G * HD; i += NTH) {
         const int h = i / HD, c = i % HD;
-        float ov = opw[(size_t)h * HD + c];
-        for (int u = 1; u < NW; u++) ov += opw[((size_t)u * G + h) * HD + c];
+        float ov = opw[(size_t)h * OS + c];
+        for (int u = 1; u < NW; u++) ov += opw[((size_t)u * G + h) * OS + c];
+        unsigned long long *pp = pbase + (size_t)h * pstride;
+        if (nact != 1) {
+            ll_word_store(pp + 2 + c, __float_as_uint(ov), ep);
+            if (c != 0) continue;
+        }
         float mm = red_m[h][0], l = red_l[h][0];
         for (int u = 1; u < NW; u++) {
             mm = fmaxf(mm, red_m[h][u]);
@@ -559,11 +577,7 @@ __global__ __launch_bounds__(kSpanThreads, HD == 128 && G8 ? 4 : 6) void attn_sp
         }
         if (nact == 1) {
             fin[i] = ov * (1.0f / l);
-            continue;
-        }
-        unsigned long long *pp = pbase + (size_t)h * pstride;
-        ll_word_store(pp + 2 + c, __float_as_uint(ov), ep);
-        if (c == 0) {
+        } else {
             ll_word_store(pp, __float_as_uint(mm), ep);
             ll_word_store(pp + 1, __float_as_uint(l), ep);
         }
