@@ -1454,9 +1454,11 @@ static void launch_swiglu_fmt(hipStream_t st, const MfArgs &A) {
 template <int FMT, int HP>
 static void launch_qkv_fmt(hipStream_t st, const MfArgs &A) {
     // A head and 16 tokens per workgroup while those are few: 48 heads, K 2048, 128 tokens (384
-    // workgroups) 3.5 us a layer less than 64-token tiles, 512 tokens 14 us more.
+    // workgroups) 3.5 us a layer less than 64-token tiles, 512 tokens 14 us more.  The NF4 cache's
+    // epilogue takes its tokens one by one, so tiles hold 16 of them in a row on each wave: 96
+    // heads, 100 / 256 tokens 22.6 and 14.6 us a layer more than here, 400 tokens 3 more, 512 tokens 4 less.
     const dim3 grid(A.stripes / 4, A.nblk);
-    if (grid.x * grid.y <= 512) hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 1, kMfmaDepth, true>), grid, dim3(256), 0, st, A);
+    if (grid.x * grid.y <= (A.qp.kr.bits == 8 ? 512u : 2560u)) hipLaunchKernelGGL((gemm_mfma_kernel<FMT, HP, 1, kMfmaDepth, true>), grid, dim3(256), 0, st, A);
     else launch_tile<FMT, HP, 2, 1, 2, 2>(st, A);
 }
 

@@ -226,7 +226,7 @@ def test_nf3_batch_equals_one_token(gpu_ctx, rows, cols, ntok, cap):
 
 
 # gate_up with the SwiGLU epilogue in 64-token (n 250) and 128-token tiles (n 300), qkv's epilogue in
-# 64-token tiles (28 heads x 19 token blocks) and 16-token ones (28 x 16), partial tiles in each
+# 64-token tiles (28 heads x 19 token blocks, int8 cache) and 16-token ones, partial tiles in each
 @pytest.mark.parametrize("fmt,planes,kv_bits,n", [("nf4", None, 8, 250), ("nf4", None, 4, 300), ("n4", "p55454", 8, 300)])
 def test_prefill_epilogues_equal_separate_kernels(gpu_ctx, fmt, planes, kv_bits, n):
     """A prefill whose qkv and gate_up products end in the fused epilogues gives the logits of
@@ -239,6 +239,34 @@ def test_prefill_epilogues_equal_separate_kernels(gpu_ctx, fmt, planes, kv_bits,
     gm, mats = _gpu_model(gpu_ctx, cfg, layers, head, fn, max_batch=320)
     gm.set_kv_bits(kv_bits)
     toks = np.random.default_rng(44).integers(0, cfg["vocab"], n).astype(np.int32)
+    got = {}
+    try:
+        for mode in (1, 2):
+            gpu_ctx.set_mfma(mode)
+            gm.reset()
+            got[mode] = gm.prefill(toks, want_logits=True), gm.decode(3)
+    finally:
+        gpu_ctx.set_mfma(True)
+        gm.close()
+        for m in mats:
+            m.close()
+    for a, b in zip(got[1], got[2]):
+        assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+# the NF4 cache: 100 heads x 25 token blocks are 16-token workgroups, x 26 are 64-token tiles
+@pytest.mark.parametrize("n", [400, 401])
+def test_qkv_epilogue_of_the_nf4_cache(gpu_ctx, n):
+    """The fused epilogue of many heads gives the logits of the separate kernel (mode 2), bit for
+    bit, and so does a decode step after it (which reads the stored cache)."""
+    from model_oracle import random_model
+    from test_gpu_model import _gpu_model
+    cfg = dict(n_layers=1, hidden=256, n_heads=92, n_kv_heads=4, head_dim=64, intermediate=256, vocab=128, max_seq=416,
+               rms_eps=1e-5, rope_theta=10000.0)
+    layers, head, fn = random_model(cfg, seed=45, fmt="nf4")
+    gm, mats = _gpu_model(gpu_ctx, cfg, layers, head, fn, max_batch=416)
+    gm.set_kv_bits(4)
+    toks = np.random.default_rng(46).integers(0, cfg["vocab"], n).astype(np.int32)
     got = {}
     try:
         for mode in (1, 2):
