@@ -7,7 +7,7 @@
 // nibble4_sdot_batch_stripe_range, 4101-4320).  Here a 16-row stripe's codes of a 64-column
 // chunk are decoded to int8 once per up to 128 tokens, with one MFMA per 16-token block
 // (A: 16 rows x 64 codes, B: 64 activation bytes x 16 tokens).  Three kernels share that step and
-// differ in how stripes, tokens and chunks are dealt to waves (launch_plain_fmt's rule).
+// differ in how stripes, tokens and chunks are dealt to waves (plain_form's rule).
 //  - NF4: the codebook value of each code (the codebook as two v_perm XOR tables,
 //    nf4_xlut); the MFMA gives the chunk dot.
 //  - NF3: the same through one v_perm per four codes, from the row's triplet of dwords, in
@@ -1317,13 +1317,22 @@ void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, cons
     hip_check(hipGetLastError(), "mfma gemv launch");
 }
 
-// Whether `blocks` 16-token blocks run on gemm_ks_kernel: few stripes, and no more (stripe,
+// Where gemm_ks_kernel is considered for `blocks` 16-token blocks: few stripes, and no more (stripe,
 // block) pairs than keep its exchange through LDS cheaper than a long chain per wave.  NF4
 // 4096 x 14336 (256 stripes), 16 / 64 / 128 / 256 tokens: 16.5 / 28.9 / 41.5 / 76 us there,
 // 40.5 / 46 / 47 / 58 us on the others; 2048 x 2048, 128: 8.6 and 10.8.  The bit planes' chains
 // also subtract the code sums: b6 4096 x 14336, 64 / 128 tokens 33 / 63 us there, 40 / 49 us.
-static bool ks_split(const k2t_mat *m, int blocks) {
+static bool ks_range(const k2t_mat *m, int blocks) {
     return m->stripes < 512 && (long)m->stripes * blocks <= (m->fmt == K2T_FMT_NIBBLE4 ? 1024 : 2048);
+}
+
+// And its workgroups (of four blocks from the third on, the last group padded) are one round: two per
+// CU for NF, one for the bit planes.  A second round of a few workgroups costs as much as the
+// first: NF4 5000 x 2112, 96 tokens (626 workgroups) 15.7 us there, 12.4 on a wave per stripe and
+// block; b4, 48 tokens (313) 11.7 and 9.5.
+static bool ks_fits(const k2t_ctx *ctx, const k2t_mat *m, int blocks) {
+    return ks_range(m, blocks) &&
+           (blocks <= 2 || m->stripes * ((blocks + 3) / 4) <= ctx->num_cus * (m->fmt == K2T_FMT_NIBBLE4 ? 1 : 2));
 }
 
 // Whether gemm_ks_kernel then reads a plain activation as its rows lie, rather than a tile-major
@@ -1331,9 +1340,25 @@ static bool ks_split(const k2t_mat *m, int blocks) {
 // gathers them again).  960 x 576, 16 tokens 7.3 -> 4.2 us, NF4 128 tokens 7.4 -> 6.6; NF4
 // 2048 x 2048, 16 tokens 7.1 -> 6.0; not taken: 32 tokens of it 7.2 -> 8.1, 6144 x 2048, 16 tokens
 // 7.6 -> 10.2, b6 960 x 576, 64 tokens 7.4 -> 8.0.
-static bool ks_rows(const k2t_mat *m, int blocks) {
-    return ks_split(m, blocks) && (long)m->stripes * m->nc * blocks <= 6000 &&
+static bool ks_rows(const k2t_ctx *ctx, const k2t_mat *m, int blocks) {
+    return ks_fits(ctx, m, blocks) && (long)m->stripes * m->nc * blocks <= 6000 &&
            m->nc * (blocks < 4 ? blocks : 4) <= (m->fmt == K2T_FMT_NIBBLE4 ? 20 : 40);
+}
+
+// The kernel of `blocks` blocks: gemm_ks_kernel unless its rounds of eight chunks are mostly padding
+// (nine chunks: b4 3072 x 576, 64 tokens 7.0 us there, 6.3 on a wave per stripe and block; NF4 512
+// tokens 8.6 and 7.7, but 64 tokens 6.8 and 6.6: from 900 pairs on); then a wave per stripe and
+// block where those are at most 8 per CU and 64-token tiles would be more than one per CU (b4 5000 x
+// 4096, 96 tokens, 314 tiles: 21.8 us and 19.2; 8192 x 4096, 64 tokens, 256 tiles: 17.5 and 18.1,
+// not taken); else tiles.
+enum class PlainForm { kKs, kWave, kTile };
+static PlainForm plain_form(const k2t_ctx *ctx, const k2t_mat *m, int blocks) {
+    const long pairs = (long)m->stripes * blocks;
+    const bool full = (m->nc + 7) / 8 * 16 <= 3 * m->nc || (m->fmt == K2T_FMT_NF && pairs < 900);
+    if (ks_fits(ctx, m, blocks) && (full || ks_rows(ctx, m, blocks))) return PlainForm::kKs;
+    const int tiles = (m->stripes + 1) / 2 * ((blocks + 3) / 4);
+    if (blocks <= 2 || (pairs <= 8 * ctx->num_cus && (ks_range(m, blocks) || tiles > ctx->num_cus))) return PlainForm::kWave;
+    return PlainForm::kTile;
 }
 
 static bool stream_captured(k2t_ctx *ctx) {
@@ -1347,7 +1372,7 @@ static bool stream_captured(k2t_ctx *ctx) {
 
 bool gemm_mfma_nf3_passes(k2t_ctx *ctx, const k2t_mat *m, int ntok) {
     if (ntok <= 128 && (long)m->stripes * m->nc * ((ntok + 3) / 4) <= 36000) return true;
-    return !ks_rows(m, (ntok + 15) / 16) && stream_captured(ctx);
+    return !ks_rows(ctx, m, (ntok + 15) / 16) && stream_captured(ctx);
 }
 
 // Arguments of one launch over all of m's stripes, and the tile-major activation (the
@@ -1423,16 +1448,16 @@ static void launch_ks(hipStream_t st, const MfArgs &A) {
 }
 
 template <int FMT, int HP>
-static void launch_plain_fmt(hipStream_t st, bool ks, const MfArgs &A) {
+static void launch_plain_fmt(hipStream_t st, PlainForm form, const MfArgs &A) {
     const int S = A.stripes, B = A.nblk;
-    // Many stripes and up to 32 tokens: a wave per stripe (NF4 14336 x 4096, 16 tokens 16 us,
+    // Up to 32 tokens (and plain_form's cases): a wave per stripe (NF4 14336 x 4096, 16 tokens 16 us,
     // 18.6 in 64-token tiles).  Above, tiles of 32 rows x 64 tokens, or x 128 once those give 448
     // workgroups: NF4 14336 x 4096, 64 / 128 / 512 tokens 22 / 38 / 105 us in 64-token tiles,
     // 25 / 30 / 81 in 128-token ones (a wave per stripe and block, or 16 rows x 64 tokens per
     // wave: 31 / 41 / 94); 2048 x 8192, 512 tokens (256 workgroups of 128) 38 and 42.5.
-    if (ks) {
+    if (form == PlainForm::kKs) {
         launch_ks<FMT, HP>(st, A);
-    } else if (B <= 2) {
+    } else if (form == PlainForm::kWave) {
         // two blocks per wave only where that leaves 8 waves per CU
         const int nb = B == 2 && S >= 2048 ? 2 : 1;
         const dim3 grid((S + 3) / 4, (B + nb - 1) / nb);
@@ -1466,13 +1491,13 @@ void launch_gemm_mfma(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, const fl
                       int ntok, float *out, size_t out_stride, bool accum, ActTiles tiles) {
     if (!gemm_mfma_supported(m, ntok)) throw Error(K2T_E_INTERNAL, "mfma gemm: unsupported matrix");
     MfArgs A;
-    mfma_args(ctx, m, xq, xs, xsum, ntok, tiles, ks_rows(m, (ntok + 15) / 16), A);
+    mfma_args(ctx, m, xq, xs, xsum, ntok, tiles, ks_rows(ctx, m, (ntok + 15) / 16), A);
     A.out = out;
     A.out_stride = out_stride;
     A.accum = accum ? 1 : 0;
-    const bool ks = ks_split(m, A.nblk);
-    if (is_nf3(m)) launch_plain_fmt<2, 0>(ctx->stream, ks, A);
-    else MF_FORMATS(m, launch_plain_fmt, ctx->stream, ks, A);
+    const PlainForm form = plain_form(ctx, m, A.nblk);
+    if (is_nf3(m)) launch_plain_fmt<2, 0>(ctx->stream, form, A);
+    else MF_FORMATS(m, launch_plain_fmt, ctx->stream, form, A);
     hip_check(hipGetLastError(), "mfma gemm launch");
 }
 

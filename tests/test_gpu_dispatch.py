@@ -192,6 +192,15 @@ def test_batched_gemv_equals_exact_passes(gpu_ctx, fmt, rows, cols, ntok):
     m.close()
 
 
+# three and more blocks of tokens on a wave per stripe and block: K dealt over a workgroup would be a
+# round and a few workgroups (313 and 626 of them), or mostly padding (nine chunks); more tiles than CUs
+@pytest.mark.parametrize("fmt", ["nf4", "nf3", "b4", "b6"])
+@pytest.mark.parametrize("rows,cols,ntok", [(5000, 2112, 48), (5000, 2112, 90), (3080, 576, 70), (6160, 1088, 65)])
+def test_batched_gemv_of_a_wave_per_block(gpu_ctx, fmt, rows, cols, ntok):
+    """The same bits on the wave-per-stripe kernel beyond 32 tokens."""
+    test_batched_gemv_equals_exact_passes(gpu_ctx, fmt, rows, cols, ntok)
+
+
 # the ordered kernel with 1, 2 and 4 blocks of tokens, stripe and pair mode, partial blocks, ragged
 # segments, a tail stripe; the 16-token passes of small products, one block over many stripes, short
 # rows; K segments capped at 3 (more visits per accumulator than one) and at 1
