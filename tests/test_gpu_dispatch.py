@@ -458,6 +458,57 @@ def test_span_attention_in_decode_steps(gpu_ctx, nq, nkv, hd, bits, window):
         x.close()
 
 
+# spans of 128 positions (up to four q heads a group, and eight) and of 256; the last place of a span,
+# then a span of one position; one span, then two; a full window whose ring wraps between the steps
+@pytest.mark.parametrize("nq,nkv,hd,window,pos", [(4, 4, 64, 0, 1279), (32, 32, 64, 0, 1279), (8, 1, 128, 0, 1279),
+                                                  (8, 2, 128, 0, 126), (8, 2, 128, 1100, 1611), (32, 32, 64, 1100, 1610)])
+@pytest.mark.parametrize("bits", [8, 4])
+def test_span_attention_stores_and_reads_the_current_position(gpu_ctx, nq, nkv, hd, window, pos, bits):
+    """Decode steps through the span kernel against the same tokens as a batch of two (K / V stored
+    by a launch of their own, split partials and a merge).  One layer, so the cache depends on
+    the tokens alone and a batch has the one-token bits: a later step's logits are equal bit for
+    bit only if the stored K / V are.  The steps' own logits agree to 5e-3 of their norm, a few
+    moved int8 codes of the attention output (one is about 1.5e-3 of 256 elements); the first q head
+    of each group has its K's projection, so the current position takes about half of the weight
+    there, and a stale or missing row would move them by far more."""
+    rng = np.random.default_rng(nq + hd + pos + bits)
+    d, V = 256, 64
+    up = lambda W: (lambda c: gpu_ctx.upload_nf(*W.shape, 4, 2, c[0], c[2], c[3]))(k2t.compile_nf4(W, 2))  # noqa: E731
+    dense = lambda r, c: (0.1 * rng.standard_normal((r, c))).astype(np.float32)  # noqa: E731
+    W = dense((nq + 2 * nkv) * hd, d)
+    for g in range(nkv):
+        q0 = g * (nq // nkv) * hd
+        W[q0:q0 + hd] = W[(nq + g) * hd:(nq + g + 1) * hd]
+    mats = [up(w) for w in (W, dense(d, nq * hd), dense(256, d), dense(d, 128), dense(V, d))]
+    m = k2t.Model(gpu_ctx, dict(n_layers=1, hidden=d, n_heads=nq, n_kv_heads=nkv, head_dim=hd, intermediate=128, vocab=V,
+                                rms_eps=1e-5, rope_theta=10000.0, max_seq=2048), max_batch=300)
+    ones = np.ones(d, np.float32)
+    m.set_layer(0, *mats[:4], ones, ones)
+    m.set_qk_norm(0, np.ones(hd, np.float32), np.ones(hd, np.float32))
+    m.set_head(mats[4], ones)
+    m.set_persistent(False)
+    m.set_kv_bits(bits)
+    if window:
+        m.set_kv_window(window, 4)
+    toks = rng.integers(0, V, pos + 3).astype(np.int32)
+    got = []
+    for batch in (False, True):
+        m.reset()
+        m.prefill(toks[:pos], want_logits=False)
+        if batch:
+            last = m.prefill(toks[pos:pos + 2])
+        else:
+            m.decode(int(toks[pos]), want_logits=False)
+            last = m.decode(int(toks[pos + 1]))
+        got.append((last, m.decode(int(toks[pos + 2]))))
+    (a, a3), (b, b3) = got
+    assert np.linalg.norm(a - b) <= 5e-3 * np.linalg.norm(b) and np.isfinite(a).all()
+    assert np.array_equal(a3.view(np.uint32), b3.view(np.uint32))
+    m.close()
+    for x in mats:
+        x.close()
+
+
 # banks of different expert counts on one context (its hand-off words are shared), calls with and
 # without the route's outputs, the wide router (d > 2048)
 def test_moe_ffn_calls_share_the_context_state(gpu_ctx):
