@@ -901,6 +901,11 @@ __global__ __launch_bounds__(256) void mf_tile_kernel(const int8_t *xq, const fl
 // lane groups: 4 in pair mode, 8 in stripe mode), which are added pairwise as the lane
 // butterfly does, then the waves' sums in wave order.  (A chunk with scale 0 adds +-0.)
 // Any number of tokens in groups of up to 16, a weight pass each.
+// XL, groups of up to 4 tokens and K segments of up to 16 chunks: a wave first copies its segment's
+// activation into LDS (4 KB, loads ahead of its first weights), so its ring holds weights alone and
+// all G chunks are in flight where the planes' registers otherwise allow four, and a chunk's
+// activation is one LDS read instead of three gathers.  b6 4096 x 14336, 4 tokens: 16.4 -> 11.3 us
+// from HBM (4-token passes 15.5), 14.3 -> 10.6 us from the Infinity Cache (15.1).
 struct GvArgs {
     const uint8_t *pair, *tail;
     size_t ptot;
@@ -929,11 +934,14 @@ struct GvFrag {
     int32_t su;
 };
 
-template <int FMT, int HP, bool SM, bool GRP = false>
+constexpr int kXlTokens = 4, kXlChunks = 16;
+constexpr int kXlBytes = kXlChunks * kXlTokens * (64 + 4 + 4);  // a wave's codes, scales, code sums
+
+template <int FMT, int HP, bool SM, bool GRP = false, bool XL = false>
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
     constexpr int RS = SM ? 1 : 2, G = SM ? 8 : 4, RB = 16 * RS;
-    constexpr int P = SM && FMT == 0 && HP > 0 ? 4 : G;  // chunks in flight (128 VGPRs at 16 waves)
-    extern __shared__ float part[];  // [nseg][16 tokens][RB rows + 1]
+    constexpr int P = SM && FMT == 0 && HP > 0 && !XL ? 4 : G;  // chunks in flight (128 VGPRs at 16 waves)
+    extern __shared__ __align__(16) float part[];  // [nseg][16 tokens][RB rows + 1], XL: then [nseg][kXlBytes]
     const uint32_t lane = threadIdx.x & 63u, li = lane & 15u, lg = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     int rbi = (int)blockIdx.x;
@@ -981,11 +989,31 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
             const v2u sw = __builtin_amdgcn_raw_buffer_load_b64(rw, L[s].s_off, sgb, 0);
             f.sw[s] = make_uint2(sw[0], sw[1]);
         }
-        const v4u x = __builtin_amdgcn_raw_buffer_load_b128(rx, x_off, (uint32_t)c * 64u, 0);
-        f.x = v4i{(int)x[0], (int)x[1], (int)x[2], (int)x[3]};
-        f.sx = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, sx_off, (uint32_t)c * 4u, 0));
-        if constexpr (FMT == 0) f.su = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(ru, sx_off, (uint32_t)c * 4u, 0);
+        if constexpr (!XL) {
+            const v4u x = __builtin_amdgcn_raw_buffer_load_b128(rx, x_off, (uint32_t)c * 64u, 0);
+            f.x = v4i{(int)x[0], (int)x[1], (int)x[2], (int)x[3]};
+            f.sx = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, sx_off, (uint32_t)c * 4u, 0));
+            if constexpr (FMT == 0) f.su = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(ru, sx_off, (uint32_t)c * 4u, 0);
+        }
     };
+    // XL: this wave's [chunk][token][64 codes], [chunk][token] scales and sums (chunks past the
+    // segment and tokens past nt repeat the last ones)
+    unsigned char *xl = nullptr;
+    v4u xr[XL ? kXlChunks / 4 : 1];
+    uint32_t sr = 0, ur = 0;
+    if constexpr (XL) {
+        static_assert(kXlTokens == 4 && kXlChunks == 16, "the lane layout of the copies");
+        xl = reinterpret_cast<unsigned char *>(part) + ((size_t)A.nseg * 16 * (RB + 1) * 4) + (size_t)wave * kXlBytes;
+#pragma unroll
+        for (int g = 0; g < kXlChunks / 4; g++) {
+            const uint32_t c = (uint32_t)min(cw0 + 4 * g + (int)lg, cw1 - 1), t = (uint32_t)min((int)(li >> 2), nt - 1);
+            xr[g] = __builtin_amdgcn_raw_buffer_load_b128(rx, t * (uint32_t)A.K + c * 64u + (li & 3u) * 16u, 0, 0);
+        }
+        const uint32_t c = (uint32_t)min(cw0 + (int)(lane >> 2), cw1 - 1), t = (uint32_t)min((int)(lane & 3u), nt - 1);
+        const uint32_t at = (t * (uint32_t)A.nc + c) * 4u;
+        sr = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0);
+        if constexpr (FMT == 0) ur = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(ru, at, 0, 0);
+    }
     float acc[G][RS][4];
 #pragma unroll
     for (int g = 0; g < G; g++)
@@ -993,7 +1021,14 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
         for (int s = 0; s < RS; s++)
 #pragma unroll
             for (int r = 0; r < 4; r++) acc[g][s][r] = 0.0f;
-    auto compute = [&](const GvFrag<FMT, RS> &f, float (&o)[RS][4]) {
+    auto compute = [&](const GvFrag<FMT, RS> &w, int i, float (&o)[RS][4]) {  // i: chunk of the segment
+        GvFrag<FMT, RS> f = w;
+        if constexpr (XL) {
+            const uint32_t t = li & 3u;
+            f.x = *reinterpret_cast<const v4i *>(xl + i * 256 + t * 64u + lg * 16u);
+            f.sx = *reinterpret_cast<const float *>(xl + kXlChunks * 256 + i * 16 + t * 4u);
+            if constexpr (FMT == 0) f.su = *reinterpret_cast<const int32_t *>(xl + kXlChunks * 272 + i * 16 + t * 4u);
+        }
 #pragma unroll
         for (int s = 0; s < RS; s++) {
             const v4i a = mf_decode<FMT, HP>(f.d0[s], f.d1[s], f.hv[s], A.t0, A.t1, A.u0, A.u1, lane);
@@ -1014,11 +1049,18 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
     GvFrag<FMT, RS> ring[P];
 #pragma unroll
     for (int u = 0; u < P; u++) fetch(ring[u], min(cw0 + u, cw1 - 1));
+    if constexpr (XL) {
+        __builtin_amdgcn_sched_barrier(0);  // (the copies' loads and the first weights are under way)
+#pragma unroll
+        for (int g = 0; g < kXlChunks / 4; g++) *reinterpret_cast<v4u *>(xl + g * 1024 + lane * 16u) = xr[g];
+        *reinterpret_cast<uint32_t *>(xl + kXlChunks * 256 + lane * 4u) = sr;
+        if constexpr (FMT == 0) *reinterpret_cast<uint32_t *>(xl + kXlChunks * 272 + lane * 4u) = ur;
+    }
     int i0 = 0;
     for (; i0 + G < n; i0 += G) {
 #pragma unroll
         for (int u = 0; u < G; u++) {
-            compute(ring[u % P], acc[u]);
+            compute(ring[u % P], i0 + u, acc[u]);
             __builtin_amdgcn_sched_barrier(0);
             fetch(ring[u % P], min(cw0 + i0 + P + u, cw1 - 1));
             __builtin_amdgcn_sched_barrier(0);
@@ -1026,7 +1068,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
     }
 #pragma unroll
     for (int u = 0; u < G; u++) {
-        if (i0 + u < n) compute(ring[u % P], acc[u]);
+        if (i0 + u < n) compute(ring[u % P], i0 + u, acc[u]);
         if (u + P < G) fetch(ring[u % P], min(cw0 + i0 + P + u, cw1 - 1));
     }
     // the accumulators pairwise (neighbours, then pairs, ...), then into LDS
@@ -1197,32 +1239,27 @@ bool gemv_mfma_supported(const k2t_mat *m, int ntok) {
     return ntok >= 2 && ntok < kMfmaMinTokens && gemm_mfma_supported(m, kMfmaMinTokens);
 }
 
-// Where the 4-token passes stay the better form.  Their 16-byte loads stream weights better than
-// this kernel's dwords; what they pay is decode and dots per token.  So only calls that are one
-// launch of one round of workgroups count (up to 4 tokens, or whole groups of 4 side by side),
-// and of those (weights from HBM, us in passes and here):
-//  - 2 tokens: NF4 14336 x 4096 10.1 and 11.4, b4 4096 x 4096 5.4 and 6.9, b6 4096 x 14336 12.4 and
-//    15.8 (b5 2048 x 2048 6.7 and 5.6, the one kind of exception);
-//  - NF3 up to 4 tokens, or with long rows: 4096 x 14336, 4 tokens 11.0 and 11.3; 2048 x 8192, 8
-//    tokens 7.9 and 8.9; not taken: 2048 x 4096, 8 tokens 6.6 and 5.8;
-//  - pair mode, b4 with 3 tokens: 14336 x 4096 11.5 and 12.2 (4 tokens 12.8 and 12.5; b5 3 tokens
-//    14.2 and 13.8, NF4 12.1 and 11.4: not taken);
-//  - stripe mode, by the row length where they meet: b4 4096 x 4096, 4 tokens 6.8 and 7.4; b5 2048 x
-//    8192, 4 tokens 9.5 and 9.9 (2048 x 5632: 8.0 and 7.6); NF4, b6 4096 x 14336, 3 tokens 12.1 and
-//    12.9, 15.6 and 16.1, 2048 x 16384, 8 tokens 12.9 and 13.5, 15.5 and 16.9 (2048 x 8192: 8.7 and
-//    8.8, 10.1 and 10.0; NF4 with 3 tokens 8.0 and 8.5).
-bool gemv_four_token_passes(const k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, int ntok) {
-    if (ntok > 4 && (ntok % 4 != 0 || (plan.rb_hi - plan.rb_lo) * (ntok / 4) > ctx->num_cus)) return false;
-    if (m->fmt == K2T_FMT_NF && m->bits == 3) return ntok <= 4 || m->nc > 96;
-    if (ntok == 2) return true;
-    const bool b4 = m->fmt == K2T_FMT_NIBBLE4 && m->hp == 0, b5 = m->fmt == K2T_FMT_NIBBLE4 && m->hp == 1;
-    if (!plan.stripe_mode) return b4 && ntok == 3;
-    return b4 || m->nc > (b5 || (ntok == 3 && m->fmt == K2T_FMT_NF) ? 96 : 160);
+// Where the 4-token passes stay the better form: their 16-byte loads stream weights better than this
+// kernel's dwords, and what they pay is decode and dots per token.  NF3 with 2 or 3 tokens (weights
+// from HBM, us in passes and here: 4096 x 14336 8.9 and 9.9, 9.7 and 10.0; 2048 x 8192 5.8 and 6.9, 6.5 and
+// 6.9; 4 tokens 10.7 and 10.0, 7.2 and 6.9: not taken), and up to 4 tokens over K segments too long for
+// the activation in LDS (b6 4096 x 14336 without it, 2 / 4 tokens 12.3 and 15.8, 15.5 and 16.4).
+bool gemv_four_token_passes(const k2t_mat *m, const GemvPlan &plan, int ntok) {
+    return (m->fmt == K2T_FMT_NF && m->bits == 3 && ntok <= 3) || (ntok <= 4 && plan.cps > kXlChunks);
 }
 
 template <int FMT, int HP>
 static void launch_gemv_mfma_fmt(hipStream_t st, const GemvPlan &plan, dim3 grid, size_t lds, const GvArgs &A) {
     const dim3 block(64 * plan.nseg);
+    // Activation in LDS for groups of up to four tokens, but over the shortest rows, which have little
+    // to keep in flight (NF4 960 x 576, 4 tokens 3.4 us without and 3.7, 2048 x 2048 4.0 and 3.9; b5 3.4
+    // and 3.4, 1536 x 1536 3.7 and 3.6).
+    if (A.tg <= kXlTokens && plan.cps <= kXlChunks && A.nc > (FMT == 0 ? 16 : 24)) {
+        const size_t l = lds + (size_t)plan.nseg * kXlBytes;
+        if (plan.stripe_mode) hipLaunchKernelGGL((gemv_mfma_kernel<FMT, HP, true, false, true>), grid, block, l, st, A);
+        else hipLaunchKernelGGL((gemv_mfma_kernel<FMT, HP, false, false, true>), grid, block, l, st, A);
+        return;
+    }
     if (plan.stripe_mode) hipLaunchKernelGGL((gemv_mfma_kernel<FMT, HP, true>), grid, block, lds, st, A);
     else hipLaunchKernelGGL((gemv_mfma_kernel<FMT, HP, false>), grid, block, lds, st, A);
 }

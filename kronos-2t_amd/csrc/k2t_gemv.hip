@@ -989,7 +989,7 @@ static void launch_gemv_impl(k2t_ctx *ctx, const k2t_mat *m, const int8_t *xq, c
     // 2 .. 15 tokens with the fast epilogue: one weight pass on the matrix cores, the same
     // plan and sum order (each token's bits are the one-token GEMV's)
     if (!dots && !grp && xsm == 0 && gu_split == 0 && !ctx->exact && ctx->mfma && gemv_mfma_supported(m, ntok) &&
-        !gemv_four_token_passes(ctx, m, plan, ntok)) {
+        !gemv_four_token_passes(m, plan, ntok)) {
         launch_gemv_mfma(ctx, m, plan, xq, xs, xsum, ntok, s0, s1, out, out_stride, accum);
         return;
     }

@@ -168,7 +168,7 @@ void launch_gemm_ordered(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, c
 // 2 .. 15 tokens with the fast epilogue on the matrix cores (any number of tokens where asked
 // for): the same split and order.
 bool gemv_mfma_supported(const k2t_mat *m, int ntok);
-bool gemv_four_token_passes(const k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, int ntok);
+bool gemv_four_token_passes(const k2t_mat *m, const GemvPlan &plan, int ntok);
 void launch_gemv_mfma(k2t_ctx *ctx, const k2t_mat *m, const GemvPlan &plan, const int8_t *xq, const float *xs,
                       const int32_t *xsum, int ntok, int s0, int s1, float *out, size_t out_stride, bool accum);
 // The same over sparse-MoE experts: work items {expert, first entry of `list`, pairs (1 .. 16)}

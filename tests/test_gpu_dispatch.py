@@ -156,6 +156,16 @@ def test_small_batch_gemv_equals_one_token(gpu_ctx, fmt, rows, cols, ntok):
     m.close()
 
 
+# the activation in LDS: stripe and pair mode, segments of 16 chunks, of a round and a few, of less than a
+# round; 2, 3 and 4 tokens, more of them dealt to several workgroups; the shortest rows that take it
+@pytest.mark.parametrize("fmt", ["nf4", "nf3", "b4", "b5", "b6"])
+@pytest.mark.parametrize("rows,cols,ntok", [(1030, 4160, 4), (1040, 16384, 7), (8300, 8256, 3), (8208, 16320, 2), (40, 1600, 4),
+                                            (48, 1088, 3), (64, 12288, 13)])
+def test_few_tokens_equal_one_token(gpu_ctx, fmt, rows, cols, ntok):
+    """The same bits with up to four tokens a workgroup."""
+    test_small_batch_gemv_equals_one_token(gpu_ctx, fmt, rows, cols, ntok)
+
+
 # the batched GEMV's kernels at their edges: K dealt over a workgroup with 1, 2 and 4 blocks of
 # tokens, from rows and from tiles, ragged rounds and a tail stripe; a wave per stripe (512 or more
 # stripes, up to 32 tokens); 64-token and 128-token tiles, partial ones, a last stage of one chunk,
@@ -823,6 +833,7 @@ def test_attention_of_a_cache_at_any_address(gpu_ctx, bits, hd, seq):
 # small-batch kernel, the K-split one (ordered and chain) and the tiles; rows 0 and 33 have an
 # infinite and a NaN scale in the first chunk
 @pytest.mark.parametrize("fmt,ntok,rows,cols", [("nf4", 5, 64, 576), ("b4", 7, 64, 576), ("b6", 15, 64, 576), ("nf3", 5, 64, 576),
+                                                ("nf4", 3, 64, 2112), ("b6", 4, 64, 2112), ("nf3", 4, 64, 2112),
                                                 ("nf3", 20, 64, 576), ("nf3", 200, 1040, 4160), ("nf3", 40, 8200, 1088),
                                                 ("nf3", 16, 8200, 2112), ("nf3", 130, 8200, 576)])
 @pytest.mark.parametrize("exact", [False, True])
