@@ -25,9 +25,9 @@
 // What bounds it is latency: a context of one span takes 5.5 us, the hand-off and the merge 2
 // to 4 more; 9 MB of K / V at copy rate are 1.8 us.  Against one workgroup per q head and
 // 256-position span with a merge launch (which had the position stored by a launch of its
-// own): 32 heads x 64, 4100 positions, NF4 cache 18.4 -> 12.1 us, int8 13.6 -> 12.9; 32 / 4
-// heads x 128, 12000 positions, NF4 49.3 -> 14.5, int8 (grouped before too) 22.0 -> 14.6;
-// a 1000-position window of it 18.3 -> 10.6.
+// own), back to back: 32 heads x 64, 4100 positions, NF4 cache 15.4 -> 12.3 us, int8 12.1 -> 13.0 (waited
+// for 26.1 -> 25.0; 12000 positions 30.6 -> 21.7); 32 / 4 heads x 128, 12000 positions, NF4 49.0 -> 13.7, int8
+// (grouped before too) 21.0 -> 14.2; a 1000-position window of it 18.4 -> 9.9.
 #include <float.h>
 #include <math.h>
 

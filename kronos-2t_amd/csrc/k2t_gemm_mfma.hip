@@ -893,8 +893,8 @@ __global__ __launch_bounds__(256) void mf_tile_kernel(const int8_t *xq, const fl
 // cost the same for 2 tokens as for 16, so what bounds it is the weight stream and, past
 // about 8 tokens, the gather of the activation rows (16 lines per load).  Weights from the
 // Infinity Cache, NF4 14336 x 4096, 4 / 8 / 15 tokens: 12.6 / 21.1 / 40.3 us as 4-token passes,
-// 9.2 / 10.6 / 12.7 us here (one token 8.7); b6 4096 x 14336, 8 / 15 tokens: 27.7 / 54.8 us, 18.2 /
-// 23.8 us here; from HBM, 4 / 8 tokens of the first 13.0 / 21.8 us and 11.8 / 12.3 us.
+// 8.4 / 10.6 / 12.7 us here (one token 8.7); b6 4096 x 14336, 8 / 15 tokens: 27.7 / 54.8 us, 18.2 /
+// 23.8 us here; from HBM, 4 / 8 tokens of the first 13.0 / 21.8 us and 10.1 / 12.1 us.
 // gemv_four_token_passes says where the passes stay.
 // Sums: the order of gemv_kernel's fast epilogue, so a batch gives each token the bits of
 // the one-token GEMV.  A wave's chunks are dealt round-robin to G accumulators (the GEMV's
