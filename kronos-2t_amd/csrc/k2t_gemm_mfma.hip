@@ -1000,7 +1000,8 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
     // segment and tokens past nt repeat the last ones)
     unsigned char *xl = nullptr;
     v4u xr[XL ? kXlChunks / 4 : 1];
-    uint32_t sr = 0, ur = 0;
+    float sr = 0.0f;
+    int32_t ur = 0;
     if constexpr (XL) {
         static_assert(kXlTokens == 4 && kXlChunks == 16, "the lane layout of the copies");
         xl = reinterpret_cast<unsigned char *>(part) + ((size_t)A.nseg * 16 * (RB + 1) * 4) + (size_t)wave * kXlBytes;
@@ -1011,8 +1012,8 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
         }
         const uint32_t c = (uint32_t)min(cw0 + (int)(lane >> 2), cw1 - 1), t = (uint32_t)min((int)(lane & 3u), nt - 1);
         const uint32_t at = (t * (uint32_t)A.nc + c) * 4u;
-        sr = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0);
-        if constexpr (FMT == 0) ur = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(ru, at, 0, 0);
+        sr = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0));
+        if constexpr (FMT == 0) ur = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(ru, at, 0, 0);
     }
     float acc[G][RS][4];
 #pragma unroll
@@ -1052,9 +1053,9 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(GvArgs A) {
     if constexpr (XL) {
         __builtin_amdgcn_sched_barrier(0);  // (the copies' loads and the first weights are under way)
 #pragma unroll
-        for (int g = 0; g < kXlChunks / 4; g++) *reinterpret_cast<v4u *>(xl + g * 1024 + lane * 16u) = xr[g];
-        *reinterpret_cast<uint32_t *>(xl + kXlChunks * 256 + lane * 4u) = sr;
-        if constexpr (FMT == 0) *reinterpret_cast<uint32_t *>(xl + kXlChunks * 272 + lane * 4u) = ur;
+        for (int g = 0; g < kXlChunks / 4; g++) *reinterpret_cast<v4i *>(xl + g * 1024 + lane * 16u) = v4i{(int)xr[g][0], (int)xr[g][1], (int)xr[g][2], (int)xr[g][3]};
+        *reinterpret_cast<float *>(xl + kXlChunks * 256 + lane * 4u) = sr;
+        if constexpr (FMT == 0) *reinterpret_cast<int32_t *>(xl + kXlChunks * 272 + lane * 4u) = ur;
     }
     int i0 = 0;
     for (; i0 + G < n; i0 += G) {
